@@ -206,15 +206,12 @@ static void allocate(Ctx& c) {
   }
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc(FLAG_COUNT * 4);
-  c.tile_q.alloc(kQueueWords * 4);
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {
     c.movcell.alloc(((size_t)c.grid.n_cells + 1) * 4);
     PR_HIP(hipMemsetAsync(c.movcell.p, 0, ((size_t)c.grid.n_cells + 1) * 4, c.stream));
     c.dry_pass.alloc(nn * 4);
     PR_HIP(hipMemsetAsync(c.dry_pass.p, 0, nn * 4, c.stream));
   }
-  PR_HIP(hipMemsetAsync(c.tile_q.p, 0, kQueueWords * 4, c.stream));
-  PR_HIP(hipDeviceGetAttribute(&c.n_cus, hipDeviceAttributeMultiprocessorCount, c.device));
   PR_HIP(hipMemsetAsync(c.flags.p, 0, FLAG_COUNT * 4, c.stream));
   const size_t es = f32 || (mixed && c.desc.model == PRESTIGE_MODEL_WCSPH) ? 4 : 8;
   c.rp.alloc(nn * 2 * es);

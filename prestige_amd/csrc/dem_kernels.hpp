@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_dem_force(
     uint32_t* __restrict__ events, uint32_t ev_weight) {
   using real = typename DemForm<F>::real;
   using G4 = typename DemForm<F>::G4;
-  const uint32_t i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t i = xcd_tile(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t me = ids[i];
   const uint32_t mc = kc.max_contacts;
@@ -277,7 +277,7 @@ void dem_step_impl(Ctx& c) {
   DemHist hist{c.hcnt[h].as<uint32_t>(), c.hid[h].as<uint32_t>(), c.hxi[h].p, c.wxi[h].p,
                c.hcnt[h ^ 1].as<uint32_t>(), c.hid[h ^ 1].as<uint32_t>(), c.hxi[h ^ 1].p, c.wxi[h ^ 1].p};
   // one wavefront per block: small scenes (the 10k lattice) spread over more CUs
-  const uint32_t grid = xcd_grid(blocks_for(n, 64));
+  const uint32_t grid = tile_grid(blocks_for(n, 64));
   const double ge = (double)sizeof(real);
   const double lb_bytes = 4.0 * (double)c.grid.n_cells / (double)n;
   // gathered: pos 3 + r, vel 3 + m, omega 3; ids + key; state in/out (pos, vel, omega) 3 x 24 x 2;

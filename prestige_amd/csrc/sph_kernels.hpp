@@ -21,8 +21,8 @@
 //            opposite runs in LDS and walk the stored masks: momentum +
 //            viscosity, then symplectic Euler, the next step's cell key and
 //            the moved-slot mask of the next incremental sort.
-// Both passes take their 64-slot tiles from per-XCD queues (for_each_tile),
-// and the density pass keeps the values of wall particles that had no moving
+// A block is one wavefront on one 64-slot tile (xcd_tile), and the density pass
+// keeps the values of wall particles that had no moving
 // particle nearby at this pass and the previous one (DryWalls).
 // Scanning in FP32 halves the bytes each candidate costs, and the expensive
 // pair bodies only run over the set bits.  Runs in the order of sph_run and
@@ -598,10 +598,8 @@ struct DryWalls {
 };
 
 constexpr int kDensBlock = 64;  // one wavefront: block barriers are wave barriers
-// Wavefronts per SIMD the register budget is held to: the tile loop lets the
-// compiler keep more values live, and these are the budgets that measured
-// fastest (density: 7 in every form, one fewer than the occupancy before the
-// loop, which avoids spills).
+// Wavefronts per SIMD the register budget is held to: the budget that measured
+// fastest (8: spills).
 template <int F>
 constexpr int kDensWaves = 7;
 constexpr uint32_t kStageCap = 256;   // scan offsets staged per run (4 KB)
@@ -642,276 +640,276 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
     const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ lb, Grid g, SphConst kc, SphUnits u,
     uint2* __restrict__ meta, uint32_t* __restrict__ words, typename SphForm<F>::R2* __restrict__ rp,
     typename SphForm<F>::G4* wpos, typename SphForm<F>::G4* wvel,
-    typename SphForm<F>::real* __restrict__ pres, uint32_t* flags, TileQueue tq, DryWalls dw) {
+    typename SphForm<F>::real* __restrict__ pres, uint32_t* flags, uint32_t n_tiles, DryWalls dw) {
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using S4 = typename SphForm<F>::S4;
   __shared__ float4 s_q[kStageCap + kScanUnr];
   const uint32_t lane = threadIdx.x;
-  for_each_tile(tq, [&](uint32_t tile) {
-    const uint32_t wbase = tile * kDensBlock;
-    const uint32_t i = wbase + lane;
-    const bool live = i < n;
-    // reference point of the wavefront (n >= 1 whenever the kernel runs)
-    const S4 p0 = spos[wbase < n ? wbase : n - 1];
-    const double xr = (double)p0.x, yr = (double)p0.y, zr = (double)p0.z, ih = u.scan_inv_h;
-    auto offset = [&](const S4& p) {
-      return make_float4((float)(((double)p.x - xr) * ih), (float)(((double)p.y - yr) * ih),
-                         (float)(((double)p.z - zr) * ih), 0.0f);
-    };
-    ScanPoint sp{0.0f, 0.0f, 0.0f, u.H2_probe};
-    CellRows cr{};
-    G4 pi{};
-    if (live) {
-      cr = decode_cell(skeys[i], g);
-      pi = pos[i];
-    }
-    // Mixed form, wavefront within one row of cells (the common case): scan
-    // offsets are taken from the 16-byte probes and the cell keys, in a frame
-    // at the origin of cell (cx_ref, row) in units of h, instead of from the
-    // 32-byte FP64 state.  Every candidate of run r then lies in the run's
-    // row, cells cx_ref + (key - row base), shifted by the run's (dy, dz).
-    bool probe_frame = false;
-    uint32_t cx_ref = 0, row_ref = 0;
-    if constexpr (F == kMixed) {
-      const uint32_t rowid = (uint32_t)cr.cz * (uint32_t)g.dims[1] + (uint32_t)cr.cy;
-      const uint32_t rmin = wave_min(live ? rowid : 0xFFFFFFFFu);
-      probe_frame = rmin == wave_max(live ? rowid : 0u);
-      row_ref = rmin;
-      cx_ref = wave_min(live ? (uint32_t)cr.cx : 0xFFFFFFFFu);
-    }
-    auto probe_offset = [&](uint32_t j, uint32_t rowbase, float oy, float oz) {
-      const float4 q = reinterpret_cast<const float4*>(pos)[j];
-      const int cx = (int)(skeys[j] - rowbase) - (int)cx_ref;
-      return make_float4(q.x + (float)cx * u.cs_u, q.y + oy, q.z + oz, 0.0f);
-    };
-    if (live) {
-      if (probe_frame) {
-        sp.x = (float)pi.x + (float)(cr.cx - (int)cx_ref) * u.cs_u;
-        sp.y = (float)pi.y;
-        sp.z = (float)pi.z;
-      } else {
-        const float4 o = offset(spos[i]);
-        sp.x = o.x;
-        sp.y = o.y;
-        sp.z = o.z;
-      }
-    }
-    // a wavefront of fixed particles whose densities cannot have changed
-    // since the last pass keeps them (see DryWalls)
-    using R2 = typename SphForm<F>::R2;
-    uint64_t dry_mask = 0;   // lanes seen dry at this pass
-    if (dw.stamps && __ballot(live && (uint64_t)dw.ids[i] < dw.n_moving) == 0ull) {
-      bool keep = true, dry = false;
-      uint32_t id = 0;
-      if (live) {
-        id = dw.ids[i];
-        dry = dry_cells(cr, g, dw);
-        keep = dry && dw.reuse && dw.dry_pass[id] == dw.pass - 1u;
-        if (dry) dw.dry_pass[id] = dw.pass;
-      }
-      dry_mask = __ballot(dry);
-      if (__ballot(!keep) == 0ull) {
-        if (live && dw.zero_masks)
-          for (uint32_t r = 0; r < kRuns; ++r) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
-        if (live) {
-          if constexpr (F == kF64) {
-            const double rho = pi.w, pr = reinterpret_cast<const double*>(wvel + i)[3];
-            rp[i] = make_double2(rho, pr);
-            pres[i] = tait_p(rho, kc);
-          } else {
-            rp[i] = static_cast<const R2*>(dw.rp_id)[id];
-            pres[i] = static_cast<const real*>(dw.pres_id)[id];
-          }
-        }
-        return;
-      }
-    }
-    // dot-form scan of staged runs: a = -2 s, and |s|^2 for the threshold
-    const float ax = -2.0f * sp.x, ay = -2.0f * sp.y, az = -2.0f * sp.z;
-    const float ss = __builtin_fmaf(sp.x, sp.x, __builtin_fmaf(sp.y, sp.y, sp.z * sp.z));
-    const float ss_max = wave_max_pos(ss);
-    const real H2 = (real)u.H2, inv_h = (real)u.inv_h;
-    Sum<real, F == kMixed> acc;
-    bool overflow = false;
-    const int nx = g.dims[0], ny = g.dims[1], nz = g.dims[2];
-    // Runs in the WCSPH order, scanned one at a time and walked a group at a
-    // time: a run and its opposite row ({0, 8}, {1, 7}, {2, 6}, {3, 5}, {4})
-    // as one stream of set bits, so a lane with few hits in one row and many
-    // in the other idles less of the lockstep walk (at 4M: FP64 1147 -> 1106
-    // us a pass, mixed 941 -> 892, FP32 904 -> 844).  The order of the pairs
-    // stays the scan order.
-    constexpr uint32_t G = 2u;   // runs per group
-    for (uint32_t grp = 0; grp < kGroups; ++grp) {
-      const uint32_t nrun = grp + 1u < kGroups ? 2u : 1u;
-      uint64_t m[2 * G];
-      uint32_t gj0[G];
-      float gby[G], gbz[G];   // mixed form: per-run bases of the pair vector
-#pragma unroll
-      for (uint32_t t = 0; t < G; ++t) {
-        m[2u * t] = m[2u * t + 1u] = 0u;
-        gj0[t] = 0u;
-        gby[t] = gbz[t] = 0.0f;
-      }
-#pragma unroll
-      for (uint32_t t = 0; t < G; ++t) {
-        if (t >= nrun) break;
-        const uint32_t r = sph_run(G * grp + t);
-        const int zz = cr.cz + (int)(r / 3u) - 1, yy = cr.cy + (int)(r % 3u) - 1;
-        const bool row_ok = live && zz >= 0 && zz < nz && yy >= 0 && yy < ny;
-        uint32_t j0 = 0, len = 0;
-        if (row_ok) {
-          const uint32_t row = ((uint32_t)zz * (uint32_t)ny + (uint32_t)yy) * (uint32_t)nx;
-          j0 = lb[row + (uint32_t)cr.x0];
-          len = lb[row + (uint32_t)cr.x1 + 1] - j0;
-          if (len > 128u) {
-            overflow = true;
-            len = 128u;
-          }
-        }
-        gj0[t] = j0;
-        // probe pair vector (o_i - o_j) - (c_j - c_i) cs/h: the y and z shifts
-        // are the run's (folded into bases), x comes from the cell codes
-        if constexpr (F == kMixed) {
-          gby[t] = (float)pi.y - (float)((int)(r % 3u) - 1) * u.cs_u;
-          gbz[t] = (float)pi.z - (float)((int)(r / 3u) - 1) * u.cs_u;
-        }
-        if (live) meta[meta_index(r, n, i)] = make_uint2(j0, len);
-        // union of the wavefront's candidate ranges of this run
-        const uint32_t base = wave_min(len ? j0 : 0xFFFFFFFFu);
-        const uint32_t top = wave_max(len ? j0 + len : 0u);
-        if (top <= base) continue;
-        const bool staged = top - base <= kStageCap;
-        // scan offset of candidate j in this wavefront's frame
-        const int rdy = (int)(r % 3u) - 1, rdz = (int)(r / 3u) - 1;
-        const uint32_t rowbase = (row_ref + (uint32_t)(rdz * g.dims[1] + rdy)) * (uint32_t)nx;
-        const float ofy = (float)rdy * u.cs_u, ofz = (float)rdz * u.cs_u;
-        auto cand = [&](uint32_t j) {
-          return probe_frame ? probe_offset(j, rowbase, ofy, ofz) : offset(spos[j]);
-        };
-        float thr = 0.0f;
-        if (staged) {
-          float mq = 0.0f;
-          for (uint32_t kk = lane; kk < top - base; kk += kDensBlock) {
-            float4 q = cand(base + kk);
-            q.w = __builtin_fmaf(q.x, q.x, __builtin_fmaf(q.y, q.y, q.z * q.z));
-            s_q[kk] = q;
-            mq = q.w > mq ? q.w : mq;
-          }
-          // Rounding of the dot form with |s|, |q| <= M: |q|^2 (3 roundings),
-          // the three FMAs (partial sums up to 3 M^2), |s|^2 and the threshold,
-          // and the FP32 offsets themselves (2 u M per component on a pair vector
-          // of length < 2) stay below u (22 M^2 + 14 M + 5); the margin is
-          // 32 u (M^2 + M + 1), u = 2^-24, on top of the common probe margin.
-          const float m2 = fmaxf(ss_max, wave_max_pos(mq));
-          const float h2p = u.H2_probe + 0x1.0p-19f * (m2 + __builtin_sqrtf(m2) + 1.0f);
-          thr = h2p - ss;
-          __syncthreads();
-        }
-        if (len) {
-          if (staged) {
-            scan_run([&](uint32_t k0, uint32_t cnt) {
-                       return scan_word_dot([&](uint32_t j) { return s_q[j - base]; }, k0, cnt, ax, ay, az, thr);
-                     },
-                     j0, len, r, words, n, i, m[2u * t], m[2u * t + 1u]);
-          } else {
-            scan_run([&](uint32_t k0, uint32_t cnt) {
-                       return scan_word([&](uint32_t j) { return cand(j < n ? j : n - 1); }, k0, cnt, sp);
-                     },
-                     j0, len, r, words, n, i, m[2u * t], m[2u * t + 1u]);
-          }
-        }
-        if (staged) __syncthreads();  // the next run's staging overwrites s_q
-      }
-      // the group's words in stream order, each with the slot of its bit 0
-      uint32_t wb[2 * G];
-#pragma unroll
-      for (uint32_t t = 0; t < G; ++t) {
-        // mixed form: bit 31 names the run of the group (slots stay below 2^31)
-        const uint32_t tag = F == kMixed ? t << 31 : 0u;
-        wb[2u * t] = gj0[t] | tag;
-        wb[2u * t + 1u] = (gj0[t] + 64u) | tag;
-      }
-      walk_bits_q<kDensUnr>(m, wb, [&](const uint32_t* jj) {
-        uint32_t js[kDensUnr], tv[kDensUnr];
-#pragma unroll
-        for (int v = 0; v < kDensUnr; ++v) {
-          const uint32_t q = jj[v] == kPad ? jj[0] : jj[v];
-          tv[v] = F == kMixed ? q >> 31 : 0u;
-          js[v] = F == kMixed ? q & 0x7FFFFFFFu : q;
-        }
-        G4 pj[kDensUnr];
-#pragma unroll
-        for (int v = 0; v < kDensUnr; ++v) pj[v] = pos[js[v]];
-#pragma unroll
-        for (int v = 0; v < kDensUnr; ++v) {
-          if (jj[v] == kPad) continue;
-          real dx, dy, dz;
-          if constexpr (F == kMixed) {
-            dx = (pi.x - pj[v].x) - (float)cell_shift(__float_as_uint(pi.w), __float_as_uint(pj[v].w), 0) * u.cs_u;
-            dy = (tv[v] ? gby[1] : gby[0]) - pj[v].y;
-            dz = (tv[v] ? gbz[1] : gbz[0]) - pj[v].z;
-          } else {
-            form_pair<F>(pi, pj[v], u.cs_u, dx, dy, dz);
-          }
-          real r2 = dot3(dx, dy, dz, dx, dy, dz);
-          if (r2 < H2) {
-            // the self pair (and coincident slots) has r2 = 0, q = 0
-            real q = r2 > real(0.0) ? sqrt_pos(r2) * inv_h : real(0.0);
-            acc.add(spline_f(q));
-          }
-        }
-      });
-    }
-    if (!live) return;
-    if (overflow) atomicOr(&flags[FLAG_CAPACITY], 1u);
-    if constexpr (F == kF64) {
-      const double rho = kc.msig * acc.s;
-      const double p = tait_p(rho, kc);
-      const double pr = p / (rho * rho);
-      rp[i] = make_double2(rho, pr);
-      reinterpret_cast<double*>(wpos + i)[3] = rho;
-      reinterpret_cast<double*>(wvel + i)[3] = pr;
-      pres[i] = p;
-    } else if constexpr (F == kF32) {
-      float rho = (float)kc.msig * acc.s;
-      float ratio = rho * (float)kc.inv_rho0;
-      float r2_ = ratio * ratio;
-      float r4 = r2_ * r2_;
-      float r7 = r4 * r2_ * ratio;
-      float p = (float)kc.B * (r7 - 1.0f);
-      if (p < 0.0f) p = 0.0f;
-      const float pr = p / (rho * rho);
-      rp[i] = make_float2(rho, pr);
-      reinterpret_cast<float*>(wpos + i)[3] = rho;
-      reinterpret_cast<float*>(wvel + i)[3] = pr;
-      pres[i] = p;
-      if ((dry_mask >> lane) & 1ull) {
-        const uint32_t id = dw.ids[i];
-        static_cast<float2*>(dw.rp_id)[id] = make_float2(rho, pr);
-        static_cast<float*>(dw.pres_id)[id] = p;
-      }
+  const uint32_t tile = xcd_tile(blockIdx.x);
+  if (tile >= n_tiles) return;
+  const uint32_t wbase = tile * kDensBlock;
+  const uint32_t i = wbase + lane;
+  const bool live = i < n;
+  // reference point of the wavefront (n >= 1 whenever the kernel runs)
+  const S4 p0 = spos[wbase < n ? wbase : n - 1];
+  const double xr = (double)p0.x, yr = (double)p0.y, zr = (double)p0.z, ih = u.scan_inv_h;
+  auto offset = [&](const S4& p) {
+    return make_float4((float)(((double)p.x - xr) * ih), (float)(((double)p.y - yr) * ih),
+                       (float)(((double)p.z - zr) * ih), 0.0f);
+  };
+  ScanPoint sp{0.0f, 0.0f, 0.0f, u.H2_probe};
+  CellRows cr{};
+  G4 pi{};
+  if (live) {
+    cr = decode_cell(skeys[i], g);
+    pi = pos[i];
+  }
+  // Mixed form, wavefront within one row of cells (the common case): scan
+  // offsets are taken from the 16-byte probes and the cell keys, in a frame
+  // at the origin of cell (cx_ref, row) in units of h, instead of from the
+  // 32-byte FP64 state.  Every candidate of run r then lies in the run's
+  // row, cells cx_ref + (key - row base), shifted by the run's (dy, dz).
+  bool probe_frame = false;
+  uint32_t cx_ref = 0, row_ref = 0;
+  if constexpr (F == kMixed) {
+    const uint32_t rowid = (uint32_t)cr.cz * (uint32_t)g.dims[1] + (uint32_t)cr.cy;
+    const uint32_t rmin = wave_min(live ? rowid : 0xFFFFFFFFu);
+    probe_frame = rmin == wave_max(live ? rowid : 0u);
+    row_ref = rmin;
+    cx_ref = wave_min(live ? (uint32_t)cr.cx : 0xFFFFFFFFu);
+  }
+  auto probe_offset = [&](uint32_t j, uint32_t rowbase, float oy, float oz) {
+    const float4 q = reinterpret_cast<const float4*>(pos)[j];
+    const int cx = (int)(skeys[j] - rowbase) - (int)cx_ref;
+    return make_float4(q.x + (float)cx * u.cs_u, q.y + oy, q.z + oz, 0.0f);
+  };
+  if (live) {
+    if (probe_frame) {
+      sp.x = (float)pi.x + (float)(cr.cx - (int)cx_ref) * u.cs_u;
+      sp.y = (float)pi.y;
+      sp.z = (float)pi.z;
     } else {
-      // EOS in FP64 from the compensated sum: gamma = 7 amplifies the relative
-      // error of rho by 7 rho^7 / (rho^7 - rho0^7), so rho is never rounded to
-      // FP32 before p is formed.
-      double rho = kc.msig * acc.wide();
-      double ratio = rho * kc.inv_rho0;
-      double r2_ = ratio * ratio;
-      double r4 = r2_ * r2_;
-      double r7 = r4 * r2_ * ratio;
-      double p = kc.B * (r7 - 1.0);
-      if (p < 0.0) p = 0.0;
-      const float2 rpi = make_float2((float)rho, (float)(p / (rho * rho)));
-      rp[i] = rpi;
-      pres[i] = (float)p;
-      if ((dry_mask >> lane) & 1ull) {
-        const uint32_t id = dw.ids[i];
-        static_cast<float2*>(dw.rp_id)[id] = rpi;
-        static_cast<float*>(dw.pres_id)[id] = (float)p;
-      }
+      const float4 o = offset(spos[i]);
+      sp.x = o.x;
+      sp.y = o.y;
+      sp.z = o.z;
     }
-  });
+  }
+  // a wavefront of fixed particles whose densities cannot have changed
+  // since the last pass keeps them (see DryWalls)
+  using R2 = typename SphForm<F>::R2;
+  uint64_t dry_mask = 0;   // lanes seen dry at this pass
+  if (dw.stamps && __ballot(live && (uint64_t)dw.ids[i] < dw.n_moving) == 0ull) {
+    bool keep = true, dry = false;
+    uint32_t id = 0;
+    if (live) {
+      id = dw.ids[i];
+      dry = dry_cells(cr, g, dw);
+      keep = dry && dw.reuse && dw.dry_pass[id] == dw.pass - 1u;
+      if (dry) dw.dry_pass[id] = dw.pass;
+    }
+    dry_mask = __ballot(dry);
+    if (__ballot(!keep) == 0ull) {
+      if (live && dw.zero_masks)
+        for (uint32_t r = 0; r < kRuns; ++r) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
+      if (live) {
+        if constexpr (F == kF64) {
+          const double rho = pi.w, pr = reinterpret_cast<const double*>(wvel + i)[3];
+          rp[i] = make_double2(rho, pr);
+          pres[i] = tait_p(rho, kc);
+        } else {
+          rp[i] = static_cast<const R2*>(dw.rp_id)[id];
+          pres[i] = static_cast<const real*>(dw.pres_id)[id];
+        }
+      }
+      return;
+    }
+  }
+  // dot-form scan of staged runs: a = -2 s, and |s|^2 for the threshold
+  const float ax = -2.0f * sp.x, ay = -2.0f * sp.y, az = -2.0f * sp.z;
+  const float ss = __builtin_fmaf(sp.x, sp.x, __builtin_fmaf(sp.y, sp.y, sp.z * sp.z));
+  const float ss_max = wave_max_pos(ss);
+  const real H2 = (real)u.H2, inv_h = (real)u.inv_h;
+  Sum<real, F == kMixed> acc;
+  bool overflow = false;
+  const int nx = g.dims[0], ny = g.dims[1], nz = g.dims[2];
+  // Runs in the WCSPH order, scanned one at a time and walked a group at a
+  // time: a run and its opposite row ({0, 8}, {1, 7}, {2, 6}, {3, 5}, {4})
+  // as one stream of set bits, so a lane with few hits in one row and many
+  // in the other idles less of the lockstep walk (at 4M: FP64 1147 -> 1106
+  // us a pass, mixed 941 -> 892, FP32 904 -> 844).  The order of the pairs
+  // stays the scan order.
+  constexpr uint32_t G = 2u;   // runs per group
+  for (uint32_t grp = 0; grp < kGroups; ++grp) {
+    const uint32_t nrun = grp + 1u < kGroups ? 2u : 1u;
+    uint64_t m[2 * G];
+    uint32_t gj0[G];
+    float gby[G], gbz[G];   // mixed form: per-run bases of the pair vector
+#pragma unroll
+    for (uint32_t t = 0; t < G; ++t) {
+      m[2u * t] = m[2u * t + 1u] = 0u;
+      gj0[t] = 0u;
+      gby[t] = gbz[t] = 0.0f;
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < G; ++t) {
+      if (t >= nrun) break;
+      const uint32_t r = sph_run(G * grp + t);
+      const int zz = cr.cz + (int)(r / 3u) - 1, yy = cr.cy + (int)(r % 3u) - 1;
+      const bool row_ok = live && zz >= 0 && zz < nz && yy >= 0 && yy < ny;
+      uint32_t j0 = 0, len = 0;
+      if (row_ok) {
+        const uint32_t row = ((uint32_t)zz * (uint32_t)ny + (uint32_t)yy) * (uint32_t)nx;
+        j0 = lb[row + (uint32_t)cr.x0];
+        len = lb[row + (uint32_t)cr.x1 + 1] - j0;
+        if (len > 128u) {
+          overflow = true;
+          len = 128u;
+        }
+      }
+      gj0[t] = j0;
+      // probe pair vector (o_i - o_j) - (c_j - c_i) cs/h: the y and z shifts
+      // are the run's (folded into bases), x comes from the cell codes
+      if constexpr (F == kMixed) {
+        gby[t] = (float)pi.y - (float)((int)(r % 3u) - 1) * u.cs_u;
+        gbz[t] = (float)pi.z - (float)((int)(r / 3u) - 1) * u.cs_u;
+      }
+      if (live) meta[meta_index(r, n, i)] = make_uint2(j0, len);
+      // union of the wavefront's candidate ranges of this run
+      const uint32_t base = wave_min(len ? j0 : 0xFFFFFFFFu);
+      const uint32_t top = wave_max(len ? j0 + len : 0u);
+      if (top <= base) continue;
+      const bool staged = top - base <= kStageCap;
+      // scan offset of candidate j in this wavefront's frame
+      const int rdy = (int)(r % 3u) - 1, rdz = (int)(r / 3u) - 1;
+      const uint32_t rowbase = (row_ref + (uint32_t)(rdz * g.dims[1] + rdy)) * (uint32_t)nx;
+      const float ofy = (float)rdy * u.cs_u, ofz = (float)rdz * u.cs_u;
+      auto cand = [&](uint32_t j) {
+        return probe_frame ? probe_offset(j, rowbase, ofy, ofz) : offset(spos[j]);
+      };
+      float thr = 0.0f;
+      if (staged) {
+        float mq = 0.0f;
+        for (uint32_t kk = lane; kk < top - base; kk += kDensBlock) {
+          float4 q = cand(base + kk);
+          q.w = __builtin_fmaf(q.x, q.x, __builtin_fmaf(q.y, q.y, q.z * q.z));
+          s_q[kk] = q;
+          mq = q.w > mq ? q.w : mq;
+        }
+        // Rounding of the dot form with |s|, |q| <= M: |q|^2 (3 roundings),
+        // the three FMAs (partial sums up to 3 M^2), |s|^2 and the threshold,
+        // and the FP32 offsets themselves (2 u M per component on a pair vector
+        // of length < 2) stay below u (22 M^2 + 14 M + 5); the margin is
+        // 32 u (M^2 + M + 1), u = 2^-24, on top of the common probe margin.
+        const float m2 = fmaxf(ss_max, wave_max_pos(mq));
+        const float h2p = u.H2_probe + 0x1.0p-19f * (m2 + __builtin_sqrtf(m2) + 1.0f);
+        thr = h2p - ss;
+        __syncthreads();
+      }
+      if (len) {
+        if (staged) {
+          scan_run([&](uint32_t k0, uint32_t cnt) {
+                     return scan_word_dot([&](uint32_t j) { return s_q[j - base]; }, k0, cnt, ax, ay, az, thr);
+                   },
+                   j0, len, r, words, n, i, m[2u * t], m[2u * t + 1u]);
+        } else {
+          scan_run([&](uint32_t k0, uint32_t cnt) {
+                     return scan_word([&](uint32_t j) { return cand(j < n ? j : n - 1); }, k0, cnt, sp);
+                   },
+                   j0, len, r, words, n, i, m[2u * t], m[2u * t + 1u]);
+        }
+      }
+      if (staged) __syncthreads();  // the next run's staging overwrites s_q
+    }
+    // the group's words in stream order, each with the slot of its bit 0
+    uint32_t wb[2 * G];
+#pragma unroll
+    for (uint32_t t = 0; t < G; ++t) {
+      // mixed form: bit 31 names the run of the group (slots stay below 2^31)
+      const uint32_t tag = F == kMixed ? t << 31 : 0u;
+      wb[2u * t] = gj0[t] | tag;
+      wb[2u * t + 1u] = (gj0[t] + 64u) | tag;
+    }
+    walk_bits_q<kDensUnr>(m, wb, [&](const uint32_t* jj) {
+      uint32_t js[kDensUnr], tv[kDensUnr];
+#pragma unroll
+      for (int v = 0; v < kDensUnr; ++v) {
+        const uint32_t q = jj[v] == kPad ? jj[0] : jj[v];
+        tv[v] = F == kMixed ? q >> 31 : 0u;
+        js[v] = F == kMixed ? q & 0x7FFFFFFFu : q;
+      }
+      G4 pj[kDensUnr];
+#pragma unroll
+      for (int v = 0; v < kDensUnr; ++v) pj[v] = pos[js[v]];
+#pragma unroll
+      for (int v = 0; v < kDensUnr; ++v) {
+        if (jj[v] == kPad) continue;
+        real dx, dy, dz;
+        if constexpr (F == kMixed) {
+          dx = (pi.x - pj[v].x) - (float)cell_shift(__float_as_uint(pi.w), __float_as_uint(pj[v].w), 0) * u.cs_u;
+          dy = (tv[v] ? gby[1] : gby[0]) - pj[v].y;
+          dz = (tv[v] ? gbz[1] : gbz[0]) - pj[v].z;
+        } else {
+          form_pair<F>(pi, pj[v], u.cs_u, dx, dy, dz);
+        }
+        real r2 = dot3(dx, dy, dz, dx, dy, dz);
+        if (r2 < H2) {
+          // the self pair (and coincident slots) has r2 = 0, q = 0
+          real q = r2 > real(0.0) ? sqrt_pos(r2) * inv_h : real(0.0);
+          acc.add(spline_f(q));
+        }
+      }
+    });
+  }
+  if (!live) return;
+  if (overflow) atomicOr(&flags[FLAG_CAPACITY], 1u);
+  if constexpr (F == kF64) {
+    const double rho = kc.msig * acc.s;
+    const double p = tait_p(rho, kc);
+    const double pr = p / (rho * rho);
+    rp[i] = make_double2(rho, pr);
+    reinterpret_cast<double*>(wpos + i)[3] = rho;
+    reinterpret_cast<double*>(wvel + i)[3] = pr;
+    pres[i] = p;
+  } else if constexpr (F == kF32) {
+    float rho = (float)kc.msig * acc.s;
+    float ratio = rho * (float)kc.inv_rho0;
+    float r2_ = ratio * ratio;
+    float r4 = r2_ * r2_;
+    float r7 = r4 * r2_ * ratio;
+    float p = (float)kc.B * (r7 - 1.0f);
+    if (p < 0.0f) p = 0.0f;
+    const float pr = p / (rho * rho);
+    rp[i] = make_float2(rho, pr);
+    reinterpret_cast<float*>(wpos + i)[3] = rho;
+    reinterpret_cast<float*>(wvel + i)[3] = pr;
+    pres[i] = p;
+    if ((dry_mask >> lane) & 1ull) {
+      const uint32_t id = dw.ids[i];
+      static_cast<float2*>(dw.rp_id)[id] = make_float2(rho, pr);
+      static_cast<float*>(dw.pres_id)[id] = p;
+    }
+  } else {
+    // EOS in FP64 from the compensated sum: gamma = 7 amplifies the relative
+    // error of rho by 7 rho^7 / (rho^7 - rho0^7), so rho is never rounded to
+    // FP32 before p is formed.
+    double rho = kc.msig * acc.wide();
+    double ratio = rho * kc.inv_rho0;
+    double r2_ = ratio * ratio;
+    double r4 = r2_ * r2_;
+    double r7 = r4 * r2_ * ratio;
+    double p = kc.B * (r7 - 1.0);
+    if (p < 0.0) p = 0.0;
+    const float2 rpi = make_float2((float)rho, (float)(p / (rho * rho)));
+    rp[i] = rpi;
+    pres[i] = (float)p;
+    if ((dry_mask >> lane) & 1ull) {
+      const uint32_t id = dw.ids[i];
+      static_cast<float2*>(dw.rp_id)[id] = rpi;
+      static_cast<float*>(dw.pres_id)[id] = (float)p;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1007,7 +1005,7 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
     SphUnits u, const typename SphForm<F>::S4* __restrict__ spos,
     const typename SphForm<F>::S4* __restrict__ svel, typename SphForm<F>::S4* __restrict__ opos,
     typename SphForm<F>::S4* __restrict__ ovel, uint32_t* __restrict__ okeys,
-    typename SphForm<F>::S4* __restrict__ oacc, MovedOut moved, uint32_t* flags, TileQueue tq,
+    typename SphForm<F>::S4* __restrict__ oacc, MovedOut moved, uint32_t* flags, uint32_t n_tiles,
     uint32_t* __restrict__ movcell, uint32_t next_pass) {
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
@@ -1017,145 +1015,145 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
   __shared__ StageArr<G4, kForceCap> s_p, s_v;
   __shared__ R2 s_rp[F == kMixed ? kForceCap : 1];
   const uint32_t lane = threadIdx.x;
-  for_each_tile(tq, [&](uint32_t tile) {
-    const uint32_t i = tile * kForceBlock + lane;
-    const bool live = i < n && (uint64_t)ids[i] < n_moving;
-    // (rho, p/rho^2) of a slot: the density pass also left them in the .w
-    // lanes of the FP64 / FP32 gather copies
-    G4 pi{}, vi{};
-    real rhoi = real(0.0), pri = real(0.0);
-    if (live) {
-      pi = gpos[i];
-      vi = gvel[i];
-      if constexpr (F == kMixed) {
-        const R2 rpi = rp[i];
-        rhoi = rpi.x;
-        pri = rpi.y;
-      } else {
-        rhoi = pi.w;
-        pri = vi.w;
-      }
+  const uint32_t tile = xcd_tile(blockIdx.x);
+  if (tile >= n_tiles) return;
+  const uint32_t i = tile * kForceBlock + lane;
+  const bool live = i < n && (uint64_t)ids[i] < n_moving;
+  // (rho, p/rho^2) of a slot: the density pass also left them in the .w
+  // lanes of the FP64 / FP32 gather copies
+  G4 pi{}, vi{};
+  real rhoi = real(0.0), pri = real(0.0);
+  if (live) {
+    pi = gpos[i];
+    vi = gvel[i];
+    if constexpr (F == kMixed) {
+      const R2 rpi = rp[i];
+      rhoi = rpi.x;
+      pri = rpi.y;
+    } else {
+      rhoi = pi.w;
+      pri = vi.w;
     }
-    const real alpha_c0 = (real)kc.alpha_c0, ach = alpha_c0 * (real)u.hv;
-    Sum<real, F == kMixed> sx, sy, sz;
-    ProbeRunBases rb;   // mixed form: per-run bases of the pair vector
-    auto begin_group = [&](uint32_t grp) {
-      if constexpr (F == kMixed) rb.begin(pi, grp, u.cs_u);
-    };
-    // pair bodies over a batch of neighbours fetched by get(j, p, v, rho, pr)
-    auto body = [&](const uint32_t* jj, const uint32_t* tt, auto&& get) {
-      G4 pj[kUnr], vj[kUnr];
-      real rhoj[kUnr], prj[kUnr];
+  }
+  const real alpha_c0 = (real)kc.alpha_c0, ach = alpha_c0 * (real)u.hv;
+  Sum<real, F == kMixed> sx, sy, sz;
+  ProbeRunBases rb;   // mixed form: per-run bases of the pair vector
+  auto begin_group = [&](uint32_t grp) {
+    if constexpr (F == kMixed) rb.begin(pi, grp, u.cs_u);
+  };
+  // pair bodies over a batch of neighbours fetched by get(j, p, v, rho, pr)
+  auto body = [&](const uint32_t* jj, const uint32_t* tt, auto&& get) {
+    G4 pj[kUnr], vj[kUnr];
+    real rhoj[kUnr], prj[kUnr];
   #pragma unroll
-      for (int v = 0; v < kUnr; ++v) get(jj[v] == kPad ? jj[0] : jj[v], pj[v], vj[v], rhoj[v], prj[v]);
+    for (int v = 0; v < kUnr; ++v) get(jj[v] == kPad ? jj[0] : jj[v], pj[v], vj[v], rhoj[v], prj[v]);
   #pragma unroll
-      for (int v = 0; v < kUnr; ++v) {
-        if (jj[v] == kPad) continue;
-        real dx, dy, dz, sc;
-        if constexpr (F == kMixed) rb.pair(pi, pj[v], tt[v], u.cs_u, dx, dy, dz);
-        else form_pair<F>(pi, pj[v], u.cs_u, dx, dy, dz);
-        if (force_pair_sc<F>(dx, dy, dz, vi, rhoi, pri, vj[v], rhoj[v], prj[v], u, ach, sc)) {
-          if constexpr (F == kMixed) {
-            // compensated sums of the FP32 terms
-            sx.add(sc * dx);
-            sy.add(sc * dy);
-            sz.add(sc * dz);
-          } else {
-            sx.s = fmad(sc, dx, sx.s);
-            sy.s = fmad(sc, dy, sy.s);
-            sz.s = fmad(sc, dz, sz.s);
-          }
+    for (int v = 0; v < kUnr; ++v) {
+      if (jj[v] == kPad) continue;
+      real dx, dy, dz, sc;
+      if constexpr (F == kMixed) rb.pair(pi, pj[v], tt[v], u.cs_u, dx, dy, dz);
+      else form_pair<F>(pi, pj[v], u.cs_u, dx, dy, dz);
+      if (force_pair_sc<F>(dx, dy, dz, vi, rhoi, pri, vj[v], rhoj[v], prj[v], u, ach, sc)) {
+        if constexpr (F == kMixed) {
+          // compensated sums of the FP32 terms
+          sx.add(sc * dx);
+          sy.add(sc * dy);
+          sz.add(sc * dz);
+        } else {
+          sx.s = fmad(sc, dx, sx.s);
+          sy.s = fmad(sc, dy, sy.s);
+          sz.s = fmad(sc, dz, sz.s);
         }
       }
-    };
-    walk_runs_staged<kUnr, kForceCap, kForcePrefetch<F>>(
-        meta, words, n, i, live, lane, begin_group,
-        [&](uint32_t k, uint32_t j) {
-          s_p.put(k, gpos[j]);
-          s_v.put(k, gvel[j]);
-          if constexpr (F == kMixed) s_rp[k] = rp[j];
-        },
-        [&](const uint32_t* jj, const uint32_t* tt) {
-          body(jj, tt, [&](uint32_t k, G4& p, G4& v, real& rho, real& pr) {
-            p = s_p.get(k);
-            v = s_v.get(k);
-            if constexpr (F == kMixed) {
-              const R2 t = s_rp[k];
-              rho = t.x;
-              pr = t.y;
-            } else {
-              rho = p.w;
-              pr = v.w;
-            }
-          });
-        },
-        [&](const uint32_t* jj, const uint32_t* tt) {
-          body(jj, tt, [&](uint32_t j, G4& p, G4& v, real& rho, real& pr) {
-            p = gpos[j];
-            v = gvel[j];
-            if constexpr (F == kMixed) {
-              const R2 t = rp[j];
-              rho = t.x;
-              pr = t.y;
-            } else {
-              rho = p.w;
-              pr = v.w;
-            }
-          });
-        },
-        [] {});
-    if (i >= n) return;
-    const uint64_t live_mask = __ballot(live);
-    if (!live) {
-      opos[i] = spos[i];
-      ovel[i] = svel[i];
-      okeys[i] = skeys[i];
-      if (oacc) oacc[i] = S4{0, 0, 0, 0};
-      moved_word_fixed(moved, i, live_mask);
-      return;
     }
-    const S4 xs = spos[i];
-    const S4 vs = svel[i];
-    sreal ax, ay, az;
-    if constexpr (F == kF32) {
-      const float msh = (float)kc.msh;
-      ax = (float)kc.g[0] - msh * sx.s;
-      ay = (float)kc.g[1] - msh * sy.s;
-      az = (float)kc.g[2] - msh * sz.s;
-    } else {
-      ax = kc.g[0] - kc.msh * sx.wide();
-      ay = kc.g[1] - kc.msh * sy.wide();
-      az = kc.g[2] - kc.msh * sz.wide();
-    }
-    const sreal dt = (sreal)kc.dt;
-    S4 v2 = vs, x2 = xs;
-    v2.x = vs.x + dt * ax;
-    v2.y = vs.y + dt * ay;
-    v2.z = vs.z + dt * az;
-    x2.x = xs.x + dt * v2.x;
-    x2.y = xs.y + dt * v2.y;
-    x2.z = xs.z + dt * v2.z;
-    opos[i] = x2;
-    ovel[i] = v2;
-    if (oacc) oacc[i] = S4{ax, ay, az, 0};
-    if (!isfinite(ax) || !isfinite(ay) || !isfinite(az)) atomicOr(&flags[FLAG_NONFINITE], 1u);
-    if ((double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2)
-      atomicOr(&flags[FLAG_CFL], 1u);
-    // next step's cell key, same FP64 floor as the key kernel
-    double fx = floor(((double)x2.x - g.lo[0]) * g.inv_cs);
-    double fy = floor(((double)x2.y - g.lo[1]) * g.inv_cs);
-    double fz = floor(((double)x2.z - g.lo[2]) * g.inv_cs);
-    bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
-              fy < (double)g.dims[1] && fz < (double)g.dims[2];
-    uint32_t key = 0;
-    if (ok)
-      key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
-    else
-      atomicOr(&flags[FLAG_DOMAIN], 1u);
-    okeys[i] = key;
-    movcell[key] = next_pass;   // this cell holds a moving particle at the next density pass
-    moved_word_live(moved, i, key != skeys[i], live_mask);
-  });
+  };
+  walk_runs_staged<kUnr, kForceCap, kForcePrefetch<F>>(
+      meta, words, n, i, live, lane, begin_group,
+      [&](uint32_t k, uint32_t j) {
+        s_p.put(k, gpos[j]);
+        s_v.put(k, gvel[j]);
+        if constexpr (F == kMixed) s_rp[k] = rp[j];
+      },
+      [&](const uint32_t* jj, const uint32_t* tt) {
+        body(jj, tt, [&](uint32_t k, G4& p, G4& v, real& rho, real& pr) {
+          p = s_p.get(k);
+          v = s_v.get(k);
+          if constexpr (F == kMixed) {
+            const R2 t = s_rp[k];
+            rho = t.x;
+            pr = t.y;
+          } else {
+            rho = p.w;
+            pr = v.w;
+          }
+        });
+      },
+      [&](const uint32_t* jj, const uint32_t* tt) {
+        body(jj, tt, [&](uint32_t j, G4& p, G4& v, real& rho, real& pr) {
+          p = gpos[j];
+          v = gvel[j];
+          if constexpr (F == kMixed) {
+            const R2 t = rp[j];
+            rho = t.x;
+            pr = t.y;
+          } else {
+            rho = p.w;
+            pr = v.w;
+          }
+        });
+      },
+      [] {});
+  if (i >= n) return;
+  const uint64_t live_mask = __ballot(live);
+  if (!live) {
+    opos[i] = spos[i];
+    ovel[i] = svel[i];
+    okeys[i] = skeys[i];
+    if (oacc) oacc[i] = S4{0, 0, 0, 0};
+    moved_word_fixed(moved, i, live_mask);
+    return;
+  }
+  const S4 xs = spos[i];
+  const S4 vs = svel[i];
+  sreal ax, ay, az;
+  if constexpr (F == kF32) {
+    const float msh = (float)kc.msh;
+    ax = (float)kc.g[0] - msh * sx.s;
+    ay = (float)kc.g[1] - msh * sy.s;
+    az = (float)kc.g[2] - msh * sz.s;
+  } else {
+    ax = kc.g[0] - kc.msh * sx.wide();
+    ay = kc.g[1] - kc.msh * sy.wide();
+    az = kc.g[2] - kc.msh * sz.wide();
+  }
+  const sreal dt = (sreal)kc.dt;
+  S4 v2 = vs, x2 = xs;
+  v2.x = vs.x + dt * ax;
+  v2.y = vs.y + dt * ay;
+  v2.z = vs.z + dt * az;
+  x2.x = xs.x + dt * v2.x;
+  x2.y = xs.y + dt * v2.y;
+  x2.z = xs.z + dt * v2.z;
+  opos[i] = x2;
+  ovel[i] = v2;
+  if (oacc) oacc[i] = S4{ax, ay, az, 0};
+  if (!isfinite(ax) || !isfinite(ay) || !isfinite(az)) atomicOr(&flags[FLAG_NONFINITE], 1u);
+  if ((double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2)
+    atomicOr(&flags[FLAG_CFL], 1u);
+  // next step's cell key, same FP64 floor as the key kernel
+  double fx = floor(((double)x2.x - g.lo[0]) * g.inv_cs);
+  double fy = floor(((double)x2.y - g.lo[1]) * g.inv_cs);
+  double fz = floor(((double)x2.z - g.lo[2]) * g.inv_cs);
+  bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
+            fy < (double)g.dims[1] && fz < (double)g.dims[2];
+  uint32_t key = 0;
+  if (ok)
+    key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
+  else
+    atomicOr(&flags[FLAG_DOMAIN], 1u);
+  okeys[i] = key;
+  movcell[key] = next_pass;   // this cell holds a moving particle at the next density pass
+  moved_word_live(moved, i, key != skeys[i], live_mask);
 }
 
 template <int F>
@@ -1203,7 +1201,7 @@ struct SphStepIO {
   const typename SphForm<F>::G4* gpos;
   const typename SphForm<F>::G4* gvel;
   const uint32_t* skeys;
-  TileQueue tq;
+  uint32_t n_tiles;
   DryWalls dw;
   uint32_t pass;
 };
@@ -1217,8 +1215,7 @@ SphStepIO<F> sph_step_io(Ctx& c) {
   io.gvel = (F == kMixed) ? c.vel32.as<G4>() : c.vel[c.cur].as<G4>();
   io.skeys = c.keys[c.cur_key].as<uint32_t>();
   static_assert(kDensBlock == kForceBlock, "both gathers walk the same tiles");
-  const uint32_t n_tiles = blocks_for((uint32_t)c.n, kDensBlock);
-  io.tq = TileQueue{c.tile_q.as<uint32_t>(), n_tiles, (n_tiles + 7u) / 8u};
+  io.n_tiles = blocks_for((uint32_t)c.n, kDensBlock);
   io.pass = c.dens_pass;
   io.dw = DryWalls{c.ids[c.cur_ids].as<uint32_t>(), c.n_moving, c.movcell.as<uint32_t>(),
                    c.dry_pass.as<uint32_t>(), c.rp_id.p, c.pres_id.p, io.pass, c.stamp_pass == io.pass,
@@ -1241,12 +1238,10 @@ void sph_density_launch(Ctx& c, const SphStepIO<F>& io, typename SphForm<F>::R2*
   double per = (F == kMixed ? 12.0 : 3.0 * ge) + 3.0 * ge;
   LaunchScope ls(&c, F == kF64 ? "sph_density_f64" : (F == kF32 ? "sph_density_f32" : "sph_density_mixed"),
                  per * n);
-  static const int per_cu = blocks_per_cu(k_sph_density<F>, kDensBlock);
-  const uint32_t dgrid = queue_grid(per_cu, c.n_cus, io.tq.n_tiles);
-  k_sph_density<F><<<dgrid, kDensBlock, 0, c.stream>>>(n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys,
+  k_sph_density<F><<<tile_grid(io.n_tiles), kDensBlock, 0, c.stream>>>(n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys,
                                                       c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nmeta.as<uint2>(),
                                                       c.nword.as<uint32_t>(), rp, wpos, wvel, pres,
-                                                      c.flags.as<uint32_t>(), io.tq, io.dw);
+                                                      c.flags.as<uint32_t>(), io.n_tiles, io.dw);
   PR_HIP(hipGetLastError());
 }
 
@@ -1266,7 +1261,6 @@ void sph_step_impl(Ctx& c) {
   const G4* gpos = io.gpos;
   const G4* gvel = io.gvel;
   const uint32_t* skeys = io.skeys;
-  const TileQueue& tq = io.tq;
   const uint32_t pass = io.pass;
   const double se = (F == kF32) ? 4.0 : 8.0;   // bytes per state scalar
   const double ge = (double)sizeof(real);     // bytes per scalar of the pair arithmetic
@@ -1287,14 +1281,12 @@ void sph_step_impl(Ctx& c) {
     LaunchScope ls(&c, F == kF64 ? "sph_force_f64" : (F == kF32 ? "sph_force_f32" : "sph_force_mixed"), per * nm);
     const int dst = c.cur ^ 1;
     const int kdst = c.cur_key ^ 1;
-    static const int per_cu = blocks_per_cu(k_sph_force<F>, kForceBlock);
-    const uint32_t fgrid = queue_grid(per_cu, c.n_cus, tq.n_tiles);
-    k_sph_force<F><<<fgrid, kForceBlock, 0, c.stream>>>(
+    k_sph_force<F><<<tile_grid(io.n_tiles), kForceBlock, 0, c.stream>>>(
         n, c.n_moving, gpos, gvel, c.rp.as<R2>(), c.ids[c.cur_ids].as<uint32_t>(), skeys,
         c.nmeta.as<uint2>(), c.nword.as<uint32_t>(), c.grid, c.sph, u, c.pos[c.cur].as<S4>(), c.vel[c.cur].as<S4>(),
         c.pos[dst].as<S4>(), c.vel[dst].as<S4>(), c.keys[kdst].as<uint32_t>(),
         c.keep_acc ? c.acc.as<S4>() : nullptr, MovedOut{c.inc_mask.as<uint64_t>(), c.inc_tiles.as<uint32_t>()},
-        c.flags.as<uint32_t>(), tq, c.movcell.as<uint32_t>(), pass + 1u);
+        c.flags.as<uint32_t>(), io.n_tiles, c.movcell.as<uint32_t>(), pass + 1u);
     PR_HIP(hipGetLastError());
     c.cur = dst;
     c.cur_key = kdst;
