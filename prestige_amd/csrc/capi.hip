@@ -242,6 +242,23 @@ static void allocate(Ctx& c) {
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {
     c.nmeta.alloc(nn * 9 * sizeof(uint2));
     c.nword.alloc(nn * 36 * sizeof(uint32_t));
+    // Four lanes per particle (sph_quad.hpp) where one lane per particle
+    // leaves the device idle.  Density + force, one lane / four lanes, us, at
+    // 8k, 64k, 250k and 500k moving particles: FP64 128/45, 158/98, 269/226,
+    // 425/458; FP32 115/39, 135/80, 193/167, 301/320; mixed 144/44, 175/98,
+    // 228/211, 359/424.  The line lies where the two meet (mixed a little
+    // lower: its compensated sums run under a mask).  The lists take 516 B a
+    // particle, so a context of over a million particles does without.
+    const uint64_t most = mixed ? 290000u : 380000u;
+    c.quad = c.n_moving <= most && n <= 1000000u;
+    if (const char* e = std::getenv("PRESTIGE_QUAD")) {
+      if (std::string(e) == "on") c.quad = true;
+      else if (std::string(e) == "off") c.quad = false;
+    }
+    if (c.quad) {
+      c.nlist.alloc(((nn + 15) / 16) * 2048 * sizeof(uint32_t));
+      c.ncnt.alloc(nn * sizeof(uint32_t));
+    }
   }
   c.scratch.alloc(nn * 8);
   if (dem) {

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -292,6 +293,11 @@ struct Ctx {
   // candidate slot, candidate count) at nmeta[r n + i] (uint2) and its hit
   // words at nword[(4 r + w) n + i] (uint32, written for 32 w < count)
   DevBuf nmeta, nword;
+  // WCSPH gathers with four lanes per particle (sph_quad.hpp) and their
+  // neighbour lists and counts.  PRESTIGE_QUAD=on|off overrides the choice by
+  // size (comparisons and tests).
+  bool quad = false;
+  DevBuf nlist, ncnt;
   // eq1 probe
   DevBuf force, mass, scratch;
   bool have_force = false, have_mass = false;

@@ -219,6 +219,17 @@ __device__ inline void form_pair(const typename SphForm<F>::G4& pi, const typena
   }
 }
 
+// The same vector without the run: y and z shifts from the cell codes too,
+// rounded as ProbeRunBases rounds them (base first, then the neighbour).
+__device__ inline void quad_probe_pair(const float4& pi, const float4& pj, float cs_u, float& dx, float& dy,
+                                       float& dz) {
+  const uint32_t wi = __float_as_uint(pi.w), wj = __float_as_uint(pj.w);
+  dx = (pi.x - pj.x) - (float)cell_shift(wi, wj, 0) * cs_u;
+  const float by = pi.y - (float)cell_shift(wi, wj, 1) * cs_u, bz = pi.z - (float)cell_shift(wi, wj, 2) * cs_u;
+  dy = by - pj.y;
+  dz = bz - pj.z;
+}
+
 // Fused multiply-add, one rounding (a correctly rounded a b + c in either
 // precision).  The WCSPH pair arithmetic writes its dot products and spline
 // polynomials with it, in the same places as the oracle.
@@ -634,6 +645,77 @@ __device__ inline bool dry_cells(const CellRows& cr, const Grid& g, const DryWal
   return dry;
 }
 
+// Outputs of a dry particle whose density is the previous pass's (DryWalls).
+template <int F>
+__device__ inline void density_keep(uint32_t i, uint32_t id, const typename SphForm<F>::G4& pi,
+                                    const typename SphForm<F>::G4* wvel, const SphConst& kc, const DryWalls& dw,
+                                    typename SphForm<F>::R2* __restrict__ rp,
+                                    typename SphForm<F>::real* __restrict__ pres) {
+  if constexpr (F == kF64) {
+    const double rho = pi.w, pr = reinterpret_cast<const double*>(wvel + i)[3];
+    rp[i] = make_double2(rho, pr);
+    pres[i] = tait_p(rho, kc);
+  } else {
+    rp[i] = static_cast<const typename SphForm<F>::R2*>(dw.rp_id)[id];
+    pres[i] = static_cast<const typename SphForm<F>::real*>(dw.pres_id)[id];
+  }
+}
+
+// Density, pressure and p/rho^2 of slot i from its kernel sum; dry: the
+// FP32 and mixed forms leave a copy by particle id (DryWalls).
+template <int F>
+__device__ inline void density_store(uint32_t i, const Sum<typename SphForm<F>::real, F == kMixed>& acc,
+                                     const SphConst& kc, bool dry, const DryWalls& dw,
+                                     typename SphForm<F>::R2* __restrict__ rp, typename SphForm<F>::G4* wpos,
+                                     typename SphForm<F>::G4* wvel, typename SphForm<F>::real* __restrict__ pres) {
+  if constexpr (F == kF64) {
+    const double rho = kc.msig * acc.s;
+    const double p = tait_p(rho, kc);
+    const double pr = p / (rho * rho);
+    rp[i] = make_double2(rho, pr);
+    reinterpret_cast<double*>(wpos + i)[3] = rho;
+    reinterpret_cast<double*>(wvel + i)[3] = pr;
+    pres[i] = p;
+  } else if constexpr (F == kF32) {
+    float rho = (float)kc.msig * acc.s;
+    float ratio = rho * (float)kc.inv_rho0;
+    float r2_ = ratio * ratio;
+    float r4 = r2_ * r2_;
+    float r7 = r4 * r2_ * ratio;
+    float p = (float)kc.B * (r7 - 1.0f);
+    if (p < 0.0f) p = 0.0f;
+    const float pr = p / (rho * rho);
+    rp[i] = make_float2(rho, pr);
+    reinterpret_cast<float*>(wpos + i)[3] = rho;
+    reinterpret_cast<float*>(wvel + i)[3] = pr;
+    pres[i] = p;
+    if (dry) {
+      const uint32_t id = dw.ids[i];
+      static_cast<float2*>(dw.rp_id)[id] = make_float2(rho, pr);
+      static_cast<float*>(dw.pres_id)[id] = p;
+    }
+  } else {
+    // EOS in FP64 from the compensated sum: gamma = 7 amplifies the relative
+    // error of rho by 7 rho^7 / (rho^7 - rho0^7), so rho is never rounded to
+    // FP32 before p is formed.
+    double rho = kc.msig * acc.wide();
+    double ratio = rho * kc.inv_rho0;
+    double r2_ = ratio * ratio;
+    double r4 = r2_ * r2_;
+    double r7 = r4 * r2_ * ratio;
+    double p = kc.B * (r7 - 1.0);
+    if (p < 0.0) p = 0.0;
+    const float2 rpi = make_float2((float)rho, (float)(p / (rho * rho)));
+    rp[i] = rpi;
+    pres[i] = (float)p;
+    if (dry) {
+      const uint32_t id = dw.ids[i];
+      static_cast<float2*>(dw.rp_id)[id] = rpi;
+      static_cast<float*>(dw.pres_id)[id] = (float)p;
+    }
+  }
+}
+
 template <int F>
 __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
     uint32_t n, const typename SphForm<F>::S4* __restrict__ spos, const typename SphForm<F>::G4* pos,
@@ -698,7 +780,6 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
   }
   // a wavefront of fixed particles whose densities cannot have changed
   // since the last pass keeps them (see DryWalls)
-  using R2 = typename SphForm<F>::R2;
   uint64_t dry_mask = 0;   // lanes seen dry at this pass
   if (dw.stamps && __ballot(live && (uint64_t)dw.ids[i] < dw.n_moving) == 0ull) {
     bool keep = true, dry = false;
@@ -713,16 +794,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
     if (__ballot(!keep) == 0ull) {
       if (live && dw.zero_masks)
         for (uint32_t r = 0; r < kRuns; ++r) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
-      if (live) {
-        if constexpr (F == kF64) {
-          const double rho = pi.w, pr = reinterpret_cast<const double*>(wvel + i)[3];
-          rp[i] = make_double2(rho, pr);
-          pres[i] = tait_p(rho, kc);
-        } else {
-          rp[i] = static_cast<const R2*>(dw.rp_id)[id];
-          pres[i] = static_cast<const real*>(dw.pres_id)[id];
-        }
-      }
+      if (live) density_keep<F>(i, id, pi, wvel, kc, dw, rp, pres);
       return;
     }
   }
@@ -864,52 +936,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
   }
   if (!live) return;
   if (overflow) atomicOr(&flags[FLAG_CAPACITY], 1u);
-  if constexpr (F == kF64) {
-    const double rho = kc.msig * acc.s;
-    const double p = tait_p(rho, kc);
-    const double pr = p / (rho * rho);
-    rp[i] = make_double2(rho, pr);
-    reinterpret_cast<double*>(wpos + i)[3] = rho;
-    reinterpret_cast<double*>(wvel + i)[3] = pr;
-    pres[i] = p;
-  } else if constexpr (F == kF32) {
-    float rho = (float)kc.msig * acc.s;
-    float ratio = rho * (float)kc.inv_rho0;
-    float r2_ = ratio * ratio;
-    float r4 = r2_ * r2_;
-    float r7 = r4 * r2_ * ratio;
-    float p = (float)kc.B * (r7 - 1.0f);
-    if (p < 0.0f) p = 0.0f;
-    const float pr = p / (rho * rho);
-    rp[i] = make_float2(rho, pr);
-    reinterpret_cast<float*>(wpos + i)[3] = rho;
-    reinterpret_cast<float*>(wvel + i)[3] = pr;
-    pres[i] = p;
-    if ((dry_mask >> lane) & 1ull) {
-      const uint32_t id = dw.ids[i];
-      static_cast<float2*>(dw.rp_id)[id] = make_float2(rho, pr);
-      static_cast<float*>(dw.pres_id)[id] = p;
-    }
-  } else {
-    // EOS in FP64 from the compensated sum: gamma = 7 amplifies the relative
-    // error of rho by 7 rho^7 / (rho^7 - rho0^7), so rho is never rounded to
-    // FP32 before p is formed.
-    double rho = kc.msig * acc.wide();
-    double ratio = rho * kc.inv_rho0;
-    double r2_ = ratio * ratio;
-    double r4 = r2_ * r2_;
-    double r7 = r4 * r2_ * ratio;
-    double p = kc.B * (r7 - 1.0);
-    if (p < 0.0) p = 0.0;
-    const float2 rpi = make_float2((float)rho, (float)(p / (rho * rho)));
-    rp[i] = rpi;
-    pres[i] = (float)p;
-    if ((dry_mask >> lane) & 1ull) {
-      const uint32_t id = dw.ids[i];
-      static_cast<float2*>(dw.rp_id)[id] = rpi;
-      static_cast<float*>(dw.pres_id)[id] = (float)p;
-    }
-  }
+  density_store<F>(i, acc, kc, ((dry_mask >> lane) & 1ull) != 0ull, dw, rp, wpos, wvel, pres);
 }
 
 // ---------------------------------------------------------------------------
@@ -996,6 +1023,85 @@ __device__ inline bool force_pair_sc(typename SphForm<F>::real dx, typename SphF
   return true;
 }
 
+// Where a force pass writes the integrated state, the next cell keys and the
+// moved-slot mask of the next incremental sort.
+template <int F>
+struct ForceOut {
+  using S4 = typename SphForm<F>::S4;
+  const S4 *spos, *svel;
+  S4 *opos, *ovel;
+  const uint32_t* skeys;
+  uint32_t* okeys;
+  S4* oacc;
+  uint32_t* movcell;
+  uint32_t next_pass;
+  uint32_t* flags;
+  MovedOut moved;
+  Grid g;
+  SphConst kc;
+};
+
+// Integrate slot i from its force sums (a fixed particle copies through) and
+// find its next cell; true when the cell changed.
+template <int F>
+__device__ inline bool force_store(uint32_t i, bool live, const Sum<typename SphForm<F>::real, F == kMixed>& sx,
+                                   const Sum<typename SphForm<F>::real, F == kMixed>& sy,
+                                   const Sum<typename SphForm<F>::real, F == kMixed>& sz, const ForceOut<F>& o) {
+  using S4 = typename SphForm<F>::S4;
+  using sreal = typename SphForm<F>::sreal;
+  const Grid& g = o.g;
+  const SphConst& kc = o.kc;
+  const uint32_t old_key = o.skeys[i];
+  const S4 xs = o.spos[i];
+  const S4 vs = o.svel[i];
+  if (!live) {
+    o.opos[i] = xs;
+    o.ovel[i] = vs;
+    o.okeys[i] = old_key;
+    if (o.oacc) o.oacc[i] = S4{0, 0, 0, 0};
+    return false;
+  }
+  sreal ax, ay, az;
+  if constexpr (F == kF32) {
+    const float msh = (float)kc.msh;
+    ax = (float)kc.g[0] - msh * sx.s;
+    ay = (float)kc.g[1] - msh * sy.s;
+    az = (float)kc.g[2] - msh * sz.s;
+  } else {
+    ax = kc.g[0] - kc.msh * sx.wide();
+    ay = kc.g[1] - kc.msh * sy.wide();
+    az = kc.g[2] - kc.msh * sz.wide();
+  }
+  const sreal dt = (sreal)kc.dt;
+  S4 v2 = vs, x2 = xs;
+  v2.x = vs.x + dt * ax;
+  v2.y = vs.y + dt * ay;
+  v2.z = vs.z + dt * az;
+  x2.x = xs.x + dt * v2.x;
+  x2.y = xs.y + dt * v2.y;
+  x2.z = xs.z + dt * v2.z;
+  o.opos[i] = x2;
+  o.ovel[i] = v2;
+  if (o.oacc) o.oacc[i] = S4{ax, ay, az, 0};
+  if (!isfinite(ax) || !isfinite(ay) || !isfinite(az)) atomicOr(&o.flags[FLAG_NONFINITE], 1u);
+  if ((double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2)
+    atomicOr(&o.flags[FLAG_CFL], 1u);
+  // next step's cell key, same FP64 floor as the key kernel
+  double fx = floor(((double)x2.x - g.lo[0]) * g.inv_cs);
+  double fy = floor(((double)x2.y - g.lo[1]) * g.inv_cs);
+  double fz = floor(((double)x2.z - g.lo[2]) * g.inv_cs);
+  bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
+            fy < (double)g.dims[1] && fz < (double)g.dims[2];
+  uint32_t key = 0;
+  if (ok)
+    key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
+  else
+    atomicOr(&o.flags[FLAG_DOMAIN], 1u);
+  o.okeys[i] = key;
+  o.movcell[key] = o.next_pass;   // this cell holds a moving particle at the next density pass
+  return key != old_key;
+}
+
 template <int F>
 __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
     uint32_t n, uint64_t n_moving, const typename SphForm<F>::G4* __restrict__ gpos,
@@ -1010,8 +1116,6 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using R2 = typename SphForm<F>::R2;
-  using S4 = typename SphForm<F>::S4;
-  using sreal = typename SphForm<F>::sreal;
   __shared__ StageArr<G4, kForceCap> s_p, s_v;
   __shared__ R2 s_rp[F == kMixed ? kForceCap : 1];
   const uint32_t lane = threadIdx.x;
@@ -1103,57 +1207,14 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
         });
       },
       [] {});
-  if (i >= n) return;
-  const uint64_t live_mask = __ballot(live);
-  if (!live) {
-    opos[i] = spos[i];
-    ovel[i] = svel[i];
-    okeys[i] = skeys[i];
-    if (oacc) oacc[i] = S4{0, 0, 0, 0};
-    moved_word_fixed(moved, i, live_mask);
-    return;
+  const ForceOut<F> out{spos, svel, opos, ovel, skeys, okeys, oacc, movcell, next_pass, flags, moved, g, kc};
+  bool mv = false;
+  if (i < n) mv = force_store<F>(i, live, sx, sy, sz, out);
+  const uint64_t b = __ballot(mv);
+  if (lane == 0u && moved.mask) {
+    moved.mask[tile] = b;
+    if (b) atomicAdd(&moved.tile_cnt[i / kSortTile], (uint32_t)__popcll(b));
   }
-  const S4 xs = spos[i];
-  const S4 vs = svel[i];
-  sreal ax, ay, az;
-  if constexpr (F == kF32) {
-    const float msh = (float)kc.msh;
-    ax = (float)kc.g[0] - msh * sx.s;
-    ay = (float)kc.g[1] - msh * sy.s;
-    az = (float)kc.g[2] - msh * sz.s;
-  } else {
-    ax = kc.g[0] - kc.msh * sx.wide();
-    ay = kc.g[1] - kc.msh * sy.wide();
-    az = kc.g[2] - kc.msh * sz.wide();
-  }
-  const sreal dt = (sreal)kc.dt;
-  S4 v2 = vs, x2 = xs;
-  v2.x = vs.x + dt * ax;
-  v2.y = vs.y + dt * ay;
-  v2.z = vs.z + dt * az;
-  x2.x = xs.x + dt * v2.x;
-  x2.y = xs.y + dt * v2.y;
-  x2.z = xs.z + dt * v2.z;
-  opos[i] = x2;
-  ovel[i] = v2;
-  if (oacc) oacc[i] = S4{ax, ay, az, 0};
-  if (!isfinite(ax) || !isfinite(ay) || !isfinite(az)) atomicOr(&flags[FLAG_NONFINITE], 1u);
-  if ((double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2)
-    atomicOr(&flags[FLAG_CFL], 1u);
-  // next step's cell key, same FP64 floor as the key kernel
-  double fx = floor(((double)x2.x - g.lo[0]) * g.inv_cs);
-  double fy = floor(((double)x2.y - g.lo[1]) * g.inv_cs);
-  double fz = floor(((double)x2.z - g.lo[2]) * g.inv_cs);
-  bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
-            fy < (double)g.dims[1] && fz < (double)g.dims[2];
-  uint32_t key = 0;
-  if (ok)
-    key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
-  else
-    atomicOr(&flags[FLAG_DOMAIN], 1u);
-  okeys[i] = key;
-  movcell[key] = next_pass;   // this cell holds a moving particle at the next density pass
-  moved_word_live(moved, i, key != skeys[i], live_mask);
 }
 
 template <int F>
@@ -1194,6 +1255,10 @@ SphUnits sph_units(const Ctx& c) {
   return u;
 }
 
+}  // namespace prestige
+#include "sph_quad.hpp"
+namespace prestige {
+
 // Per-step inputs of both gathers of form F.
 template <int F>
 struct SphStepIO {
@@ -1201,6 +1266,7 @@ struct SphStepIO {
   const typename SphForm<F>::G4* gpos;
   const typename SphForm<F>::G4* gvel;
   const uint32_t* skeys;
+  bool quad;   // four lanes per particle (sph_quad.hpp)
   uint32_t n_tiles;
   DryWalls dw;
   uint32_t pass;
@@ -1215,7 +1281,8 @@ SphStepIO<F> sph_step_io(Ctx& c) {
   io.gvel = (F == kMixed) ? c.vel32.as<G4>() : c.vel[c.cur].as<G4>();
   io.skeys = c.keys[c.cur_key].as<uint32_t>();
   static_assert(kDensBlock == kForceBlock, "both gathers walk the same tiles");
-  io.n_tiles = blocks_for((uint32_t)c.n, kDensBlock);
+  io.quad = c.quad && !c.record_all;
+  io.n_tiles = blocks_for((uint32_t)c.n, io.quad ? (int)kQuadSlots : kDensBlock);
   io.pass = c.dens_pass;
   io.dw = DryWalls{c.ids[c.cur_ids].as<uint32_t>(), c.n_moving, c.movcell.as<uint32_t>(),
                    c.dry_pass.as<uint32_t>(), c.rp_id.p, c.pres_id.p, io.pass, c.stamp_pass == io.pass,
@@ -1238,6 +1305,13 @@ void sph_density_launch(Ctx& c, const SphStepIO<F>& io, typename SphForm<F>::R2*
   double per = (F == kMixed ? 12.0 : 3.0 * ge) + 3.0 * ge;
   LaunchScope ls(&c, F == kF64 ? "sph_density_f64" : (F == kF32 ? "sph_density_f32" : "sph_density_mixed"),
                  per * n);
+  if (io.quad) {
+    k_sph_density_quad<F><<<tile_grid(io.n_tiles), 64, 0, c.stream>>>(
+        n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys, c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nlist.as<uint32_t>(),
+        c.ncnt.as<uint32_t>(), rp, wpos, wvel, pres, c.flags.as<uint32_t>(), io.n_tiles, io.dw);
+    PR_HIP(hipGetLastError());
+    return;
+  }
   k_sph_density<F><<<tile_grid(io.n_tiles), kDensBlock, 0, c.stream>>>(n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys,
                                                       c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nmeta.as<uint2>(),
                                                       c.nword.as<uint32_t>(), rp, wpos, wvel, pres,
@@ -1281,12 +1355,22 @@ void sph_step_impl(Ctx& c) {
     LaunchScope ls(&c, F == kF64 ? "sph_force_f64" : (F == kF32 ? "sph_force_f32" : "sph_force_mixed"), per * nm);
     const int dst = c.cur ^ 1;
     const int kdst = c.cur_key ^ 1;
-    k_sph_force<F><<<tile_grid(io.n_tiles), kForceBlock, 0, c.stream>>>(
-        n, c.n_moving, gpos, gvel, c.rp.as<R2>(), c.ids[c.cur_ids].as<uint32_t>(), skeys,
-        c.nmeta.as<uint2>(), c.nword.as<uint32_t>(), c.grid, c.sph, u, c.pos[c.cur].as<S4>(), c.vel[c.cur].as<S4>(),
-        c.pos[dst].as<S4>(), c.vel[dst].as<S4>(), c.keys[kdst].as<uint32_t>(),
-        c.keep_acc ? c.acc.as<S4>() : nullptr, MovedOut{c.inc_mask.as<uint64_t>(), c.inc_tiles.as<uint32_t>()},
-        c.flags.as<uint32_t>(), io.n_tiles, c.movcell.as<uint32_t>(), pass + 1u);
+    const MovedOut moved{c.inc_mask.as<uint64_t>(), c.inc_tiles.as<uint32_t>()};
+    S4* acc = c.keep_acc ? c.acc.as<S4>() : nullptr;
+    if (io.quad) {
+      const ForceOut<F> out{c.pos[c.cur].as<S4>(), c.vel[c.cur].as<S4>(), c.pos[dst].as<S4>(), c.vel[dst].as<S4>(),
+                            skeys, c.keys[kdst].as<uint32_t>(), acc, c.movcell.as<uint32_t>(), pass + 1u,
+                            c.flags.as<uint32_t>(), moved, c.grid, c.sph};
+      k_sph_force_quad<F><<<tile_grid(io.n_tiles), 64, 0, c.stream>>>(
+          n, c.n_moving, gpos, gvel, c.rp.as<R2>(), c.ids[c.cur_ids].as<uint32_t>(), skeys, c.lb.as<uint32_t>(),
+          c.nlist.as<uint32_t>(), c.ncnt.as<uint32_t>(), u, out, io.n_tiles);
+    } else {
+      k_sph_force<F><<<tile_grid(io.n_tiles), kForceBlock, 0, c.stream>>>(
+          n, c.n_moving, gpos, gvel, c.rp.as<R2>(), c.ids[c.cur_ids].as<uint32_t>(), skeys,
+          c.nmeta.as<uint2>(), c.nword.as<uint32_t>(), c.grid, c.sph, u, c.pos[c.cur].as<S4>(), c.vel[c.cur].as<S4>(),
+          c.pos[dst].as<S4>(), c.vel[dst].as<S4>(), c.keys[kdst].as<uint32_t>(), acc, moved, c.flags.as<uint32_t>(),
+          io.n_tiles, c.movcell.as<uint32_t>(), pass + 1u);
+    }
     PR_HIP(hipGetLastError());
     c.cur = dst;
     c.cur_key = kdst;
