@@ -52,6 +52,20 @@ __device__ inline void for_quad(Fn&& fn) {
   fn(std::integral_constant<int, 3>{});
 }
 
+// Moved-slot bits of a 16-slot tile (its quarter of the mask word) from the
+// quads' first lanes; every lane calls.
+__device__ inline void moved_word_quad(const MovedOut& mo, uint32_t tile, bool moved) {
+  uint64_t m = __ballot(moved);   // bits 4 p, packed to bits p
+  m = (m | (m >> 3)) & 0x0303030303030303ull;
+  m = (m | (m >> 6)) & 0x000F000F000F000Full;
+  m = (m | (m >> 12)) & 0x000000FF000000FFull;
+  m = (m | (m >> 24)) & 0xFFFFull;
+  if (__lane_id() == 0u && mo.mask) {
+    reinterpret_cast<uint16_t*>(mo.mask)[tile] = (uint16_t)m;
+    if (m) atomicAdd(&mo.tile_cnt[tile * kQuadSlots / kSortTile], (uint32_t)__popcll(m));
+  }
+}
+
 // Row runs of a particle's cell in the WCSPH order: first slot and length of
 // each (0 outside the grid; cut to 128 candidates, reported in over).
 struct QuadRuns {
@@ -401,15 +415,7 @@ __global__ __launch_bounds__(64, kQuadForceWaves<F>) void k_sph_force_quad(
   const bool mine = sub == 0u && i < n;
   bool mv = false;
   if (mine) mv = force_store<F>(i, live, sx, sy, sz, out);
-  uint64_t m = __ballot(mv);   // bits 4 p: to bits p of this tile's quarter of the mask word
-  m = (m | (m >> 3)) & 0x0303030303030303ull;
-  m = (m | (m >> 6)) & 0x000F000F000F000Full;
-  m = (m | (m >> 12)) & 0x000000FF000000FFull;
-  m = (m | (m >> 24)) & 0xFFFFull;
-  if (lane == 0u && out.moved.mask) {
-    reinterpret_cast<uint16_t*>(out.moved.mask)[tile] = (uint16_t)m;
-    if (m) atomicAdd(&out.moved.tile_cnt[wbase / kSortTile], (uint32_t)__popcll(m));
-  }
+  moved_word_quad(out.moved, tile, mv);
 }
 
 }  // namespace prestige
