@@ -189,21 +189,17 @@ static void allocate(Ctx& c) {
   const uint64_t tiles = sort_tiles(n) + 1;
   c.sort_hist.alloc(256 * tiles * 4);
   c.sort_tot.alloc(256 * 4);
-  c.inc_mask.alloc(((nn + 63) / 64) * 8);
-  c.inc_woff.alloc(((nn + 63) / 64) * 4);
-  c.inc_tiles.alloc((2 * tiles + 1) * 4);
-  PR_HIP(hipMemsetAsync(c.inc_tiles.p, 0, (2 * tiles + 1) * 4, c.stream));
-  c.inc_count.alloc(4);
-  c.inc_mov.alloc(nn * 8);
-  c.inc_tmp.alloc(nn * 8);
-  PR_HIP(hipHostMalloc((void**)&c.inc_host, sizeof(uint32_t), hipHostMallocMapped));
-  *c.inc_host = 0;
-  PR_HIP(hipHostGetDevicePointer((void**)&c.inc_host_dev, c.inc_host, 0));
-  if (const char* dr = std::getenv("PRESTIGE_DRY")) c.dry_reuse = std::string(dr) != "off";
-  if (const char* sp = std::getenv("PRESTIGE_SORT")) {
-    if (std::string(sp) == "radix") c.sort_policy = Ctx::kSortRadix;
-    else if (std::string(sp) == "incremental") c.sort_policy = Ctx::kSortIncremental;
+  if (c.desc.model != PRESTIGE_MODEL_PAIRS) {
+    const size_t cells = (size_t)c.grid.n_cells + 1;
+    c.inc_tiles = (cells + kCellTile - 1) / kCellTile;
+    c.inc_mask.alloc(((nn + 63) / 64) * 8);
+    c.inc_next.alloc(nn * 4);
+    c.lb_spare.alloc(cells * 4);
+    c.inc_cells.alloc(c.inc_tiles * kCellTile * 8 + c.inc_count_bytes());
+    PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, c.inc_cells.bytes, c.stream));
   }
+  if (const char* dr = std::getenv("PRESTIGE_DRY")) c.dry_reuse = std::string(dr) != "off";
+  if (const char* sp = std::getenv("PRESTIGE_SORT")) c.sort_radix = std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc(FLAG_COUNT * 4);
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {

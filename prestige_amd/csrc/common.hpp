@@ -143,15 +143,47 @@ struct Timing {
 
 struct Ctx;
 
-// Moved-slot mask of the next incremental sort, written by the step kernels:
-// word w has bit l set when slot 64 w + l gets a different cell key from the
-// step (fixed particles never move), and tile_cnt[t] counts the moved slots of
-// sort tile t (kSortTile slots; cleared by the sort that consumes it).
-constexpr uint32_t kSortTile = 2048;
+// What the step kernels leave for the next build's incremental sort.  A slot
+// whose particle changes cell ("moved", fixed particles never do) counts into
+// its new cell (cin) and out of its old one (cout), into the same totals per
+// tile of kCellTile cells (tin, tout), and is linked into its new cell's list:
+// head[c] holds (epoch << 32 | last slot linked), next[slot] the slot linked
+// before it (kListEnd for the first of this epoch, so heads need no clearing).
+// Word w of mask has bit l set when slot 64 w + l moved.
+constexpr uint32_t kCellTile = 1024;
+constexpr uint32_t kListEnd = 0xFFFFFFFFu;
+// Slots one cell's list takes in one step.  Steps within the CFL bounds stay
+// far below; a runaway that throws more than this into one cell leaves the
+// rest in their old cells and raises the capacity flag, so that every list
+// walk stays short.
+constexpr uint32_t kMaxIn = 1u << 16;
 struct MovedOut {
   uint64_t* mask;
-  uint32_t* tile_cnt;
+  uint32_t *cin, *cout, *tin, *tout;
+  uint64_t* head;
+  uint32_t* next;
+  uint32_t epoch;
+  uint32_t* flags;
 };
+// Slot i goes from cell old_key to cell key: record it; false when it stays
+// (key is then old_key).
+__device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old_key, uint32_t& key) {
+  if (key == old_key) return false;
+  if (atomicAdd(&mo.cin[key], 1u) >= kMaxIn) {
+    atomicSub(&mo.cin[key], 1u);
+    atomicOr(&mo.flags[FLAG_CAPACITY], 1u);
+    key = old_key;
+    return false;
+  }
+  atomicAdd(&mo.cout[old_key], 1u);
+  atomicAdd(&mo.tin[key / kCellTile], 1u);
+  atomicAdd(&mo.tout[old_key / kCellTile], 1u);
+  const unsigned long long mine = ((unsigned long long)mo.epoch << 32) | i;
+  const unsigned long long last = atomicExch(reinterpret_cast<unsigned long long*>(&mo.head[key]), mine);
+  mo.next[i] = (uint32_t)(last >> 32) == mo.epoch ? (uint32_t)last : kListEnd;
+  return true;
+}
+
 // Hand a buffer a step just wrote to an adjoint record without copying: the
 // next step only writes into the context side of the swap before reading it.
 inline void take_buffer(DevBuf& ctx_buf, DevBuf& rec_buf) {
@@ -212,9 +244,6 @@ struct Ctx {
   Ctx() = default;
   Ctx(const Ctx&) = delete;
   Ctx& operator=(const Ctx&) = delete;
-  ~Ctx() {
-    if (inc_host) (void)hipHostFree(inc_host);
-  }
   prestige_desc desc{};
   int device = 0;
   hipStream_t stream = nullptr;
@@ -241,16 +270,21 @@ struct Ctx {
   DevBuf keys[2], vals[2];       // radix-sort ping-pong
   int perm_buf = 0;              // which vals[] holds the last permutation
   DevBuf sort_hist, sort_tot;    // per-tile digit counts, per-digit totals
-  // incremental sort: moved-slot mask (bit per slot), per-tile moved counts
-  // and offsets, moved count, moved entries (key << 32 | slot), the same
-  // sorted, and the moved slots before each mask word
-  DevBuf inc_mask, inc_tiles, inc_count, inc_mov, inc_tmp, inc_woff;
-  uint32_t* inc_host = nullptr;  // pinned, mapped: moved count of the last incremental sort
-  uint32_t* inc_host_dev = nullptr;  // the same word as the device writes it
+  // incremental sort (MovedOut): moved-slot mask, links per slot, the spare
+  // cell table, and in one buffer the list heads per cell and the counts cin,
+  // cout (inc_tiles * kCellTile each), tin, tout (inc_tiles each)
+  DevBuf inc_mask, inc_next, lb_spare, inc_cells;
+  size_t inc_tiles = 0;
+  uint64_t* inc_head() const { return inc_cells.as<uint64_t>(); }
+  uint32_t* inc_cin() const { return reinterpret_cast<uint32_t*>(inc_head() + inc_tiles * kCellTile); }
+  uint32_t* inc_cout() const { return inc_cin() + inc_tiles * kCellTile; }
+  uint32_t* inc_tin() const { return inc_cout() + inc_tiles * kCellTile; }
+  uint32_t* inc_tout() const { return inc_tin() + inc_tiles; }
+  size_t inc_count_bytes() const { return inc_tiles * (2 * kCellTile + 2) * 4; }   // from inc_cin() on
+  uint32_t inc_epoch = 1;
   bool inc_ready = false;        // keys[cur_key] are the next keys of the last build's slots
-  uint32_t inc_skipped = 0;      // radix builds since the moved count was last measured
-  enum SortPolicy { kSortAuto = 0, kSortRadix = 1, kSortIncremental = 2 };
-  int sort_policy = kSortAuto;   // PRESTIGE_SORT=radix|incremental overrides the choice
+  bool inc_counts = false;       // a step's counts are waiting (a build that does not use them clears them)
+  bool sort_radix = false;       // PRESTIGE_SORT=radix: every build sorts anew (comparisons and tests)
   DevBuf lb;                     // n_cells + 1
   // WCSPH wall particles far from the fluid (DryWalls): cell stamps (n_cells),
   // last dry pass per particle id, pass counter, the pass the stamps describe,
@@ -400,6 +434,7 @@ void set_context_free_error(const std::string& msg);
 
 // Per-form kernel entry points (defined in the .hip files).
 void neighbors_build(Ctx& c);
+MovedOut moved_out(Ctx& c);        // for the next step kernel; its counts then wait for the build
 uint64_t sort_tiles(uint64_t n);   // radix-sort tiles of n keys (histogram rows per digit)
 void keys_from_positions(Ctx& c);
 void eq1_eval(Ctx& c, int loop, double cutoff);

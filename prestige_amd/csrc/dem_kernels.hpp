@@ -106,7 +106,7 @@ __global__ __launch_bounds__(64) void k_dem_force(
     }
     for (int c = (int)sub; c < 18; c += 4) wxi_out[(size_t)c * n + me] = real(0.0);
   }
-  uint32_t key = key_i;
+  bool mv = false;
   if (__ballot(live) != 0ull) {
     const CellRows cr = decode_cell(key_i, g);
     const G4 pi = gpos[self], vi = gvel[self], wi = gom[self];
@@ -309,8 +309,10 @@ __global__ __launch_bounds__(64) void k_dem_force(
       double fz = floor((x2.z - g.lo[2]) * g.inv_cs);
       const bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
                       fy < (double)g.dims[1] && fz < (double)g.dims[2];
-      key = ok ? ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx : 0u;
       if (sub == 0u) {
+        uint32_t key = key_i;   // a sphere outside the grid keeps its cell
+        if (ok) key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
+        mv = move_to_cell(moved, i, key_i, key);
         opos[i] = x2;
         ovel[i] = v2;
         oom[i] = w2;
@@ -329,7 +331,7 @@ __global__ __launch_bounds__(64) void k_dem_force(
       }
     }
   }
-  moved_word_quad(moved, tile, sub == 0u && live && key != key_i);
+  moved_word_quad(moved, tile, mv);
 }
 
 template <int F>
@@ -359,7 +361,7 @@ void dem_step_impl(Ctx& c) {
       c.lb.as<uint32_t>(), c.grid, c.dem, c.pos[c.cur].as<double4>(), c.vel[c.cur].as<double4>(),
       c.omega[c.cur].as<double4>(), c.pos[dst].as<double4>(), c.vel[dst].as<double4>(),
       c.omega[dst].as<double4>(), c.keys[kdst].as<uint32_t>(), c.keep_acc ? c.acc.as<double4>() : nullptr,
-      hist, MovedOut{c.inc_mask.as<uint64_t>(), c.inc_tiles.as<uint32_t>()}, c.flags.as<uint32_t>(),
+      hist, moved_out(c), c.flags.as<uint32_t>(),
       c.ev_weight ? c.events.as<uint32_t>() : nullptr, c.ev_weight, n_tiles);
   PR_HIP(hipGetLastError());
   c.cur = dst;

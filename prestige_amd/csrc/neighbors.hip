@@ -66,7 +66,6 @@ constexpr int kBuckets = 1 << kRadixBits;
 constexpr int kSortThreads = 256;
 constexpr int kSortItems = 8;   // keys per thread and tile
 constexpr int kTile = kSortThreads * kSortItems;
-static_assert(kTile == (int)kSortTile, "the step kernels count moved slots per sort tile");
 static_assert(kSortThreads == kBuckets, "one thread per bucket in the scan phases");
 
 // Lanes of this wavefront whose digit equals mine (and whose item is valid):
@@ -89,8 +88,7 @@ __device__ inline uint64_t lanes_below() {
 __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const uint32_t* __restrict__ keys,
                                                             uint32_t n, int shift,
                                                             uint32_t n_tiles,
-                                                            uint32_t* __restrict__ hist,
-                                                            uint32_t* __restrict__ tile_cnt) {
+                                                            uint32_t* __restrict__ hist) {
   __shared__ uint32_t h[kBuckets];
   const uint32_t t = threadIdx.x;
   h[t] = 0;
@@ -105,9 +103,6 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const uint32_t* __re
   }
   __syncthreads();
   hist[t * n_tiles + blockIdx.x] = h[t];
-  // the moved-slot counts the last step kernel left for an incremental sort
-  // this build does not use start again from zero
-  if (t == 0 && tile_cnt) tile_cnt[blockIdx.x] = 0;
 }
 
 // Inclusive scan within a wavefront of 64 lanes.
@@ -217,14 +212,12 @@ static int key_bits(uint32_t n_cells) {
 }
 
 // Buffers of one radix sort: key and value ping-pong pairs, the per-tile digit
-// histogram (kBuckets x tiles), the digit totals, and optionally the moved-slot
-// tile counts the sort clears for the next incremental sort.
+// histogram (kBuckets x tiles) and the digit totals.
 struct SortBufs {
   uint32_t* keys[2];
   uint32_t* vals[2];
   uint32_t* hist;
   uint32_t* tot;
-  uint32_t* tile_cnt;
 };
 
 // Sorts the n keys (< n_cells) in keys[src]; *key_out and *val_out receive
@@ -249,8 +242,7 @@ static void radix_sort_bufs(Ctx* c, const SortBufs& b, int src, uint32_t n, uint
     const int vdst = (vsrc < 0) ? 0 : (vsrc ^ 1);
     {
       LaunchScope ls(c, "sort_hist", 4.0 * n);
-      k_sort_hist<<<n_tiles, kSortThreads, 0, st>>>(b.keys[src], n, shift, n_tiles, b.hist,
-                                                    p == 0 ? b.tile_cnt : nullptr);
+      k_sort_hist<<<n_tiles, kSortThreads, 0, st>>>(b.keys[src], n, shift, n_tiles, b.hist);
       PR_HIP(hipGetLastError());
     }
     {
@@ -276,7 +268,7 @@ static void radix_sort_bufs(Ctx* c, const SortBufs& b, int src, uint32_t n, uint
 static void radix_sort(Ctx& c) {
   const SortBufs b{{c.keys[0].as<uint32_t>(), c.keys[1].as<uint32_t>()},
                    {c.vals[0].as<uint32_t>(), c.vals[1].as<uint32_t>()},
-                   c.sort_hist.as<uint32_t>(), c.sort_tot.as<uint32_t>(), c.inc_tiles.as<uint32_t>()};
+                   c.sort_hist.as<uint32_t>(), c.sort_tot.as<uint32_t>()};
   radix_sort_bufs(&c, b, c.cur_key, (uint32_t)c.n, c.grid.n_cells, c.stream, &c.cur_key, &c.perm_buf);
 }
 
@@ -383,34 +375,28 @@ double reorder_bytes(const Ctx& c) {
 
 // ---------------------------------------------------------------------------
 // incremental stable sort.  Between two builds only the slots whose particle
-// changed cell ("moved", key_new != key_old) break the order: slots are in
-// key_old order, so the slots that kept their key are still sorted and keep
-// their relative order, and the stable sort of key_new merges them with the
-// few moved ones sorted by (key_new, slot).  With P(t) = moved slots before
-// slot t and M the moved entries sorted by (key, slot):
-//   kept slot i (key c):  position i - P(i) + #{M entries < (c, i)}
-//   moved entry b = (c, i): position b + t - P(t), t = lb_old[c] if i <
-//                           lb_old[c], else lb_old[c + 1]
-// (the kept slots before (c, i) are the slots before t that kept their key;
-// i never lies inside cell c's old range, whose slots all had key c).  The
-// step kernel that computed the keys also wrote the moved-slot mask and the
-// per-tile moved counts; three launches (gather, sort of M, placement, which
-// also moves the particle state) replace the radix sort's nine and the
-// reorder, and the permutation and keys are exactly the stable sort's, as
-// the radix sort would give them.
+// changed cell ("moved") break the order: slots are in key_old order, and the
+// kept slots of a cell keep their relative order.  The stable sort puts into
+// cell c, in this order, the slots that moved in from lower cells, the kept
+// ones and those from higher cells, each by slot (old slot order is old key
+// order), so with the new cell table lb and the list of c's incoming slots
+//   kept slot i:               lb[c] + #{incoming < i} + i - lb_old[c]
+//                                - #{moved slots in [lb_old[c], i)}
+//   incoming, i < lb_old[c]:   lb[c] + #{incoming < i}
+//   incoming, i >= lb_old[c+1]: lb[c+1] - #{incoming >= i}
+// and lb[c] is lb_old[c] plus the prefix of (in - out) over the cells before
+// c.  The step kernel counted and listed the moved slots (MovedOut), so two
+// launches, the cell table and the placement, which also moves the particle
+// state, replace the radix sort's launches, the reorder and the cell table's;
+// permutation and keys are exactly the stable sort's.  Lists have no order (the
+// step's atomics link them), but only counts are taken from them.
+//
+// Us per step, against gathering the moved entries, sorting them, merging and
+// a cell table (up to 8,192 moved; the radix path above): 42,866 particles 19
+// -> 11, 10,000 spheres 14 -> 9, 1.8M mixed 95 -> 66, 6M FP64 (about 20,000
+// moved a step) 334 -> 181.  The table costs 8 bytes a cell, the placement is
+// bound by the state it moves (6 TB/s at 6M).
 // ---------------------------------------------------------------------------
-// Up to kRankMax moved entries are ordered by counting their ranks, one
-// block per 64 entries; more take a one-block radix sort (the host then
-// prefers the full radix sort for the next builds).
-constexpr uint32_t kRankMax = 8192;
-constexpr int kIncSortThreads = 1024;
-
-// The gather walks a sort tile with kIncThreads threads, kIncItems slots
-// each.
-constexpr int kIncThreads = 1024;
-constexpr int kIncItems = kTile / kIncThreads;
-constexpr uint32_t kIncWaves = kIncThreads / 64;
-static_assert(kIncItems * kIncThreads == kTile, "whole tiles");
 
 __device__ inline uint32_t wave_sum(uint32_t x) {
 #pragma unroll
@@ -418,319 +404,116 @@ __device__ inline uint32_t wave_sum(uint32_t x) {
   return x;
 }
 
-// Block b of n_tiles: sums the per-tile moved counts (from the step kernel
-// that wrote the keys) of the tiles before b, writes that to tile_off[b] and
-// the count before each mask word to word_off, and lists its moved slots at
-// their rank, as (key << 32 | slot) in slot order.  Block 0 sums every tile
-// and writes the total to tile_off[n_tiles], *count and the host-mapped word
-// *host_count, which the host reads without waiting when it picks the next
-// build's sort.  The tile's mask words are read before the counts are summed,
-// so one barrier serves both.  The placement clears the tile counts.
-__global__ __launch_bounds__(kIncThreads) void k_inc_gather(
-    uint32_t n, uint32_t n_tiles, const uint32_t* __restrict__ tile_cnt, const uint32_t* __restrict__ knew,
-    const uint64_t* __restrict__ mask, uint32_t* __restrict__ tile_off, uint32_t* __restrict__ word_off,
-    uint32_t* __restrict__ count, uint32_t* __restrict__ host_count, uint64_t* __restrict__ mov) {
-  __shared__ uint32_t s_red[kIncWaves];
-  __shared__ uint32_t s_w[kIncItems * kIncWaves];
-  const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
-  const uint32_t base = blockIdx.x * (uint32_t)kTile;
-  uint64_t word[kIncItems];
-#pragma unroll
-  for (int it = 0; it < kIncItems; ++it) {
-    const uint32_t i0 = base + (uint32_t)it * kIncThreads + 64u * w;   // the wavefront's first slot
-    word[it] = i0 < n ? mask[i0 >> 6] : 0ull;
-  }
-  const uint32_t lim = blockIdx.x == 0 ? n_tiles : blockIdx.x;
+// New cell table of tile b (kCellTile cells): the offset before it from the
+// tile totals, then a block scan of the cells' net counts, which are cleared
+// for the next step.  A tile nothing entered or left only adds its offset.
+__global__ __launch_bounds__(kBlock) void k_inc_cells(uint32_t n_cells, const uint32_t* __restrict__ lb_old,
+                                                      const uint32_t* __restrict__ tin,
+                                                      const uint32_t* __restrict__ tout, uint4* __restrict__ cin,
+                                                      uint4* __restrict__ cout, uint32_t* __restrict__ lb) {
+  static_assert(kCellTile == 4 * kBlock, "four cells per thread");
+  __shared__ uint32_t s4[4];
+  const uint32_t b = blockIdx.x, t = threadIdx.x;
+  const bool busy = (tin[b] | tout[b]) != 0u;
   uint32_t part = 0;
-  for (uint32_t t = threadIdx.x; t < lim; t += kIncThreads) part += tile_cnt[t];
+  for (uint32_t k = t; k < b; k += kBlock) part += tin[k] - tout[k];
   part = wave_sum(part);
-  if (lane == 0) {
-    s_red[w] = part;
-#pragma unroll
-    for (int it = 0; it < kIncItems; ++it) s_w[it * kIncWaves + w] = (uint32_t)__popcll(word[it]);
-  }
+  if (__lane_id() == 0) s4[t >> 6] = part;
   __syncthreads();
-  uint32_t sum = 0;
-  for (uint32_t k = 0; k < kIncWaves; ++k) sum += s_red[k];
-  const uint32_t pre = blockIdx.x == 0 ? 0u : sum;
-  if (threadIdx.x == 0) {
-    tile_off[blockIdx.x] = pre;
-    if (blockIdx.x == 0) {
-      tile_off[n_tiles] = sum;
-      count[0] = sum;
-      *host_count = sum;
-      __threadfence_system();
-    }
+  uint32_t run = s4[0] + s4[1] + s4[2] + s4[3];
+  uint32_t d[4] = {0u, 0u, 0u, 0u};
+  if (busy) {
+    __syncthreads();
+    const uint32_t q = b * kBlock + t;
+    const uint4 in = cin[q], out = cout[q];
+    d[0] = in.x - out.x; d[1] = in.y - out.y; d[2] = in.z - out.z; d[3] = in.w - out.w;
+    if (in.x | in.y | in.z | in.w) cin[q] = make_uint4(0u, 0u, 0u, 0u);
+    if (out.x | out.y | out.z | out.w) cout[q] = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t total;
+    run += block_excl_scan(d[0] + d[1] + d[2] + d[3], s4, &total);
   }
-  uint32_t run = pre;
+  const uint32_t c0 = b * kCellTile + 4u * t;
 #pragma unroll
-  for (int it = 0; it < kIncItems; ++it) {
-    uint32_t before = run, total = 0;
-    for (uint32_t k = 0; k < kIncWaves; ++k) {
-      const uint32_t cnt = s_w[it * kIncWaves + k];
-      before += k < w ? cnt : 0u;
-      total += cnt;
-    }
-    const uint32_t i = base + (uint32_t)it * kIncThreads + 64u * w + lane;
-    before += (uint32_t)__popcll(word[it] & lanes_below());
-    if (i < n && (i & 63u) == 0u) word_off[i >> 6] = before;
-    if (i < n && ((word[it] >> lane) & 1ull) != 0ull) mov[before] = ((uint64_t)knew[i] << 32) | i;
-    run += total;
+  for (uint32_t k = 0; k < 4u; ++k) {
+    if (c0 + k <= n_cells) lb[c0 + k] = lb_old[c0 + k] + run;
+    run += d[k];
   }
 }
 
-// Writes the moved entries sorted by (key, slot) to out.  Up to kRankMax
-// entries, block b places the 64-entry chunk b of them at its rank
-// #{y : (key_y, y) < (key_x, x)}, counted by its 16 wavefronts over
-// interleaved 64-entry chunks of y and summed in LDS.  The entries are in
-// slot order, so (key_y, y) < (key_x, x) is key_y < key_x + [y < x]: one
-// 32-bit compare per pair, the y keys read by scalar loads.  Above kRankMax
-// entries block 0 runs a stable LSD radix sort on the key over mov and out
-// (entries arrive in slot order, so key order alone keeps (key, slot) order).
-__global__ __launch_bounds__(kIncSortThreads) void k_inc_sort(const uint32_t* __restrict__ count, int key_bits,
-                                                              uint64_t* __restrict__ mov,
-                                                              uint64_t* __restrict__ out) {
-  constexpr uint32_t kW = kIncSortThreads / 64;
-  const uint32_t m = count[0];
-  const uint32_t t = threadIdx.x;
-  if (m <= kRankMax) {
-    const uint32_t nch = (m + 63u) >> 6;
-    const uint32_t xc = blockIdx.x;
-    if (xc >= nch) return;
-    __shared__ uint32_t s_cnt[kW][64];
-    const uint32_t lane = __lane_id();
-    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
-    const uint32_t* keys = reinterpret_cast<const uint32_t*>(mov) + 1;   // high halves, stride 2
-    const uint32_t x = xc * 64u + lane;
-    const uint32_t kx = x < m ? keys[2u * x] : 0u;
-    uint32_t cnt = 0;
-    for (uint32_t c = w; c < nch; c += kW) {
-      const uint32_t y0 = c * 64u;
-      if (c != xc && y0 + 64u <= m) {
-        const uint32_t thr = c < xc ? kx + 1u : kx;   // all y before x, or all after
-#pragma unroll 16
-        for (uint32_t y = y0; y < y0 + 64u; ++y) cnt += keys[2u * y] < thr ? 1u : 0u;
-      } else {
-        const uint32_t y1 = min(y0 + 64u, m);
-        for (uint32_t y = y0; y < y1; ++y) cnt += keys[2u * y] < (y < x ? kx + 1u : kx) ? 1u : 0u;
-      }
-    }
-    s_cnt[w][lane] = cnt;
-    __syncthreads();
-    if (w == 0 && x < m) {
-      uint32_t r = 0;
-#pragma unroll
-      for (uint32_t k = 0; k < kW; ++k) r += s_cnt[k][lane];
-      if (r < m) out[r] = mov[x];   // always
-    }
-    return;
-  }
-  if (blockIdx.x != 0) return;
-  // digit histogram, then a stable scatter in chunks of kIncSortThreads
-  // entries (wavefront rank by ballot match + counts of the earlier
-  // wavefronts of the chunk)
-  __shared__ uint32_t hist[kBuckets];
-  __shared__ uint32_t wcnt[kW * kBuckets];
-  const uint32_t w = t >> 6;
-  uint64_t* src = mov;
-  uint64_t* dst = out;
-  const int passes = (key_bits + kRadixBits - 1) / kRadixBits;
-  for (int p = 0; p < passes; ++p) {
-    const int shift = 32 + p * kRadixBits;
-    for (uint32_t k = t; k < kBuckets; k += kIncSortThreads) hist[k] = 0;
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < m; c0 += kIncSortThreads) {
-      const uint32_t k = c0 + t;
-      const bool valid = k < m;
-      const uint32_t d = valid ? (uint32_t)(src[k] >> shift) & (kBuckets - 1) : 0u;
-      const uint64_t peers = match_digit(d, valid);
-      if (valid && (peers & lanes_below()) == 0ull) atomicAdd(&hist[d], (uint32_t)__popcll(peers));
-    }
-    __syncthreads();
-    if (t < 64) {   // exclusive scan of the 256 counts by one wavefront, 4 per lane
-      uint32_t v[4], sum = 0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[q] = hist[4 * t + q];
-        sum += v[q];
-      }
-      const uint32_t incl = wave_incl_scan(sum);
-      uint32_t run = incl - sum;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        hist[4 * t + q] = run;
-        run += v[q];
-      }
-    }
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < m; c0 += kIncSortThreads) {
-      const uint32_t k = c0 + t;
-      const bool valid = k < m;
-      const uint64_t e = valid ? src[k] : 0ull;
-      const uint32_t d = (uint32_t)(e >> shift) & (kBuckets - 1);
-      for (uint32_t q = t; q < kW * kBuckets; q += kIncSortThreads) wcnt[q] = 0;
-      __syncthreads();
-      const uint64_t peers = match_digit(d, valid);
-      const uint32_t r = (uint32_t)__popcll(peers & lanes_below());
-      if (valid && r == 0) wcnt[w * kBuckets + d] = (uint32_t)__popcll(peers);
-      __syncthreads();
-      if (t < kBuckets) {   // per digit: offsets of the wavefronts of this chunk
-        uint32_t run = hist[t];
-        for (uint32_t q = 0; q < kW; ++q) {
-          const uint32_t c = wcnt[q * kBuckets + t];
-          wcnt[q * kBuckets + t] = run;
-          run += c;
-        }
-        hist[t] = run;
-      }
-      __syncthreads();
-      if (valid) dst[wcnt[w * kBuckets + d] + r] = e;
-      __syncthreads();
-    }
-    uint64_t* x = src;
-    src = dst;
-    dst = x;
-  }
-  if (src != out)
-    for (uint32_t k = t; k < m; k += kIncSortThreads) out[k] = src[k];
+// Set bits of the moved-slot mask in [a, b).
+__device__ inline uint32_t moved_in(const uint64_t* __restrict__ mask, uint32_t a, uint32_t b) {
+  if (a >= b) return 0u;
+  const uint32_t wa = a >> 6, wb = (b - 1u) >> 6;
+  uint64_t w = mask[wa] & (~0ull << (a & 63u));
+  uint32_t cnt = 0;
+  for (uint32_t k = wa; k < wb; w = mask[++k]) cnt += (uint32_t)__popcll(w);
+  const uint32_t top = b & 63u;   // 0: the last word counts whole
+  return cnt + (uint32_t)__popcll(top ? w & ((1ull << top) - 1ull) : w);
 }
 
-// Moved slots before slot t (t <= n; m = all moved slots).
-__device__ inline uint32_t inc_moved_before(uint32_t t, uint32_t n, uint32_t m, const uint64_t* __restrict__ mask,
-                                            const uint32_t* __restrict__ word_off) {
-  if (t >= n) return m;
-  const uint32_t r = t & 63u;
-  return word_off[t >> 6] + (r ? (uint32_t)__popcll(mask[t >> 6] & ((1ull << r) - 1ull)) : 0u);
-}
-
-// Lower bounds in the sorted moved entries mov[0 .. m) of ea (returned in .x)
-// and eb >= ea (in .y), one per half-wavefront: each step probes 32 evenly
-// spaced entries of the remaining range and keeps the gap that holds the
-// bound, so m = 32k entries take three dependent loads.  Every lane of the
-// wavefront calls.
-__device__ inline uint2 wave_lower_bounds(const uint64_t* __restrict__ mov, uint32_t m, uint64_t ea, uint64_t eb) {
-  const uint32_t lane = __lane_id();
-  const bool upper = lane >= 32u;
-  const uint64_t e = upper ? eb : ea;
-  const uint32_t j = lane & 31u;
-  uint32_t lo = 0, hi = m;   // the bound lies in [lo, hi]
-  while (__ballot(lo < hi)) {
-    const uint32_t chunk = (hi - lo + 31u) >> 5;   // 0 when this half is done
-    const uint32_t idx = lo + j * chunk;
-    const bool below = chunk != 0u && idx < hi && mov[idx] < e;
-    const uint64_t bal = __ballot(below);
-    const uint32_t c = (uint32_t)__popcll(upper ? (bal >> 32) : (bal & 0xffffffffull));
-    if (chunk != 0u) {
-      if (c == 0u) {
-        hi = lo;   // mov[lo] >= e
-      } else {
-        const uint32_t nlo = lo + (c - 1u) * chunk + 1u;
-        hi = min(lo + c * chunk, hi);
-        lo = nlo;
-      }
-    }
-  }
-  return make_uint2((uint32_t)__builtin_amdgcn_readlane((int)lo, 0),
-                    (uint32_t)__builtin_amdgcn_readlane((int)lo, 32));
-}
-
-// One thread per slot (a wavefront covers one mask word, so the moved slots
-// before slot i are word_off[i / 64] plus a popcount), then the moved
-// entries spread over the blocks.
+// One thread per slot: its place in the new order; key, permutation and the
+// particle's state go there.  Also clears the tile totals.
 template <class T4, bool OMEGA, bool PROBE, bool MIXED>
 __global__ __launch_bounds__(kBlock) void k_inc_place(
-    uint32_t n, uint32_t n_tiles, const uint32_t* __restrict__ knew, const uint64_t* __restrict__ mask,
-    const uint32_t* __restrict__ word_off, const uint64_t* __restrict__ mov, const uint32_t* __restrict__ count,
-    const uint32_t* __restrict__ lb_old, uint32_t* __restrict__ tile_cnt, uint32_t* __restrict__ kout,
-    uint32_t* __restrict__ perm, ReorderIO<T4> io) {
-  static_assert(kBlock % 64 == 0, "wavefronts cover whole mask words");
-  const uint32_t m = count[0];
+    uint32_t n, uint32_t cell_tiles, const uint32_t* __restrict__ knew, const uint64_t* __restrict__ mask,
+    const uint64_t* __restrict__ head, const uint32_t* __restrict__ next, uint32_t epoch,
+    const uint32_t* __restrict__ lb_old, const uint32_t* __restrict__ lb, uint32_t* __restrict__ tin,
+    uint32_t* __restrict__ tout, uint32_t* __restrict__ kout, uint32_t* __restrict__ perm, ReorderIO<T4> io) {
   const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
-  const uint32_t lane = __lane_id();
-  if (i < n_tiles) tile_cnt[i] = 0;   // for the next step's counts
-  const bool valid = i < n;
-  const uint64_t word = valid ? mask[i >> 6] : 0ull;
-  const bool kept = valid && ((word >> lane) & 1ull) == 0ull;
-  const uint64_t km = __ballot(kept);
-  if (km != 0ull) {
-    const uint32_t key = kept ? knew[i] : 0u;
-    const uint64_t e = ((uint64_t)key << 32) | i;
-    // kept slots are in (key, slot) order, so the wavefront's bounds lie
-    // between those of its first and last kept slot
-    const int first = __builtin_ctzll(km), last = 63 - __builtin_clzll(km);
-    const uint64_t ea = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)key, first) << 32) |
-                        (uint32_t)__builtin_amdgcn_readlane((int)i, first);
-    const uint64_t eb = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)key, last) << 32) |
-                        (uint32_t)__builtin_amdgcn_readlane((int)i, last);
-    const uint2 bnd = wave_lower_bounds(mov, m, ea, eb);
-    if (kept) {
-      const uint32_t before = word_off[i >> 6] + (uint32_t)__popcll(word & lanes_below());
-      uint32_t lo = bnd.x, hi = bnd.y;   // moved entries below (key, i)
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (mov[mid] < e) lo = mid + 1;
-        else hi = mid;
-      }
-      const uint32_t pos = i - before + lo;
-      if (pos < n) {   // always, when the moved counts are consistent
-        kout[pos] = key;
-        perm[pos] = i;
-        move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, key);
-      }
+  for (uint32_t k = i; k < cell_tiles; k += gridDim.x * (uint32_t)kBlock) tin[k] = tout[k] = 0u;
+  if (i >= n) return;
+  const uint32_t c = knew[i];
+  const uint32_t o0 = lb_old[c], l0 = lb[c];
+  const uint64_t hd = head[c];
+  uint32_t below = 0, above = 0;   // incoming slots before i, and i or after it
+  if ((uint32_t)(hd >> 32) == epoch)
+    for (uint32_t e = (uint32_t)hd; e != kListEnd; e = next[e]) {
+      below += e < i ? 1u : 0u;
+      above += e < i ? 0u : 1u;
     }
-  }
-  // moved entries, spread over the blocks
-  for (uint32_t b = threadIdx.x * gridDim.x + blockIdx.x; b < m; b += (uint32_t)kBlock * gridDim.x) {
-    const uint64_t e = mov[b];
-    const uint32_t key = (uint32_t)(e >> 32), s = (uint32_t)e;
-    const uint32_t t = s < lb_old[key] ? lb_old[key] : lb_old[key + 1];
-    const uint32_t pos = b + t - inc_moved_before(t, n, m, mask, word_off);
-    if (pos >= n) continue;   // never, when the moved counts are consistent
-    kout[pos] = key;
-    perm[pos] = s;
-    move_slot<T4, OMEGA, PROBE, MIXED>(io, s, pos, key);
-  }
+  uint32_t pos;
+  if (i < o0) pos = l0 + below;
+  else if (i >= lb_old[c + 1u]) pos = lb[c + 1u] - above;
+  else pos = l0 + below + (i - o0) - moved_in(mask, o0, i);
+  if (pos >= n) return;   // never, when the counts are consistent
+  kout[pos] = c;
+  perm[pos] = i;
+  move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, c);
+}
+
+MovedOut moved_out(Ctx& c) {
+  c.inc_counts = true;
+  return MovedOut{c.inc_mask.as<uint64_t>(), c.inc_cin(), c.inc_cout(), c.inc_tin(), c.inc_tout(), c.inc_head(),
+                  c.inc_next.as<uint32_t>(), ++c.inc_epoch, c.flags.as<uint32_t>()};
 }
 
 // Stable sort of keys[cur_key] from the previous build's order (keys[cur_key
-// ^ 1] = its sorted keys, lb its cell table); same outputs as radix_sort.
+// ^ 1] = its sorted keys, lb its cell table), with the new cell table and the
+// state moved; same outputs as radix_sort, k_reorder and k_cell_lb.
 static void incremental_sort(Ctx& c) {
   const uint32_t n = (uint32_t)c.n;
-  const uint32_t n_tiles = (uint32_t)sort_tiles(n);
-  const uint32_t* knew = c.keys[c.cur_key].as<uint32_t>();
-  uint32_t* kold = c.keys[c.cur_key ^ 1].as<uint32_t>();   // overwritten with the sorted keys
-  const uint64_t* mask = c.inc_mask.as<uint64_t>();         // written by the step kernel
-  uint32_t* cnt = c.inc_count.as<uint32_t>();
-  uint32_t* tile_cnt = c.inc_tiles.as<uint32_t>();      // n_tiles, from the step kernel
-  uint32_t* tiles = tile_cnt + n_tiles;                  // tile offsets, n_tiles + 1
-  uint32_t* woff = c.inc_woff.as<uint32_t>();            // moved slots before each mask word
+  const uint32_t cells = c.grid.n_cells;
+  const uint32_t tiles = (uint32_t)c.inc_tiles;
   {
-    LaunchScope ls(&c, "sort_inc_gather", 2.0 * n_tiles * n_tiles + 8.5 * n);
-    k_inc_gather<<<n_tiles, kIncThreads, 0, c.stream>>>(n, n_tiles, tile_cnt, knew, mask, tiles, woff, cnt,
-                                                        c.inc_host_dev, c.inc_mov.as<uint64_t>());
+    LaunchScope ls(&c, "sort_inc_cells", 8.0 * cells);
+    k_inc_cells<<<tiles, kBlock, 0, c.stream>>>(cells, c.lb.as<uint32_t>(), c.inc_tin(), c.inc_tout(),
+                                                reinterpret_cast<uint4*>(c.inc_cin()),
+                                                reinterpret_cast<uint4*>(c.inc_cout()), c.lb_spare.as<uint32_t>());
     PR_HIP(hipGetLastError());
   }
   {
-    LaunchScope ls(&c, "sort_inc_sort", 0.0);
-    k_inc_sort<<<kRankMax / 64u, kIncSortThreads, 0, c.stream>>>(cnt, key_bits(c.grid.n_cells),
-                                                                 c.inc_mov.as<uint64_t>(),
-                                                                 c.inc_tmp.as<uint64_t>());
-    PR_HIP(hipGetLastError());
-  }
-  {
-    // placement and the reorder in one pass: each slot's state goes straight
-    // to its sorted position
     LaunchScope ls(&c, "sort_inc_place", (12.0 + reorder_bytes(c)) * n);
-    const uint64_t* mov = c.inc_tmp.as<uint64_t>();   // sorted
-    const uint32_t* lb_old = c.lb.as<uint32_t>();
-    uint32_t* perm = c.vals[0].as<uint32_t>();
     with_reorder_form(c, c.cur, c.cur ^ 1, [&](auto form, auto io) {
       using F = decltype(form);
       k_inc_place<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(
-          n, n_tiles, knew, mask, woff, mov, cnt, lb_old, tile_cnt, kold, perm, io);
+          n, tiles, c.keys[c.cur_key].as<uint32_t>(), c.inc_mask.as<uint64_t>(), c.inc_head(),
+          c.inc_next.as<uint32_t>(), c.inc_epoch, c.lb.as<uint32_t>(), c.lb_spare.as<uint32_t>(), c.inc_tin(),
+          c.inc_tout(), c.keys[c.cur_key ^ 1].as<uint32_t>(), c.vals[0].as<uint32_t>(), io);
     });
     PR_HIP(hipGetLastError());
   }
+  std::swap(c.lb.p, c.lb_spare.p);
+  c.inc_counts = false;
   c.cur_key ^= 1;
   c.perm_buf = 0;
 }
@@ -793,38 +576,33 @@ void neighbors_build(Ctx& c) {
     c.sorted = true; c.built = true;
     return;
   }
-  // incremental sort when the state is still in the previous build's slot
-  // order with fresh keys (right after a step) and the last moved count seen
-  // was small; every few radix builds the moved count is measured again
-  bool inc = false;
-  if (c.inc_ready && c.sort_policy != Ctx::kSortRadix) {
-    const uint32_t seen = *(volatile const uint32_t*)c.inc_host;
-    inc = c.sort_policy == Ctx::kSortIncremental || seen <= kRankMax || ++c.inc_skipped >= 16u;
-  }
-  if (inc) {
-    c.inc_skipped = 0;
+  // incremental when the state is still in the previous build's slot order
+  // with fresh keys (right after a step)
+  const int src = c.cur, dst = c.cur ^ 1;
+  if (c.inc_ready && !c.sort_radix) {
     incremental_sort(c);
   } else {
+    if (c.inc_counts) {   // counts of a step this build does not continue
+      PR_HIP(hipMemsetAsync(c.inc_cin(), 0, c.inc_count_bytes(), c.stream));
+      c.inc_counts = false;
+    }
     radix_sort(c);
-  }
-  c.inc_ready = false;
-  const uint32_t* skeys = c.keys[c.cur_key].as<uint32_t>();
-  const int src = c.cur, dst = c.cur ^ 1;
-  if (!inc) {   // the incremental sort moved the state itself
+    const uint32_t* skeys = c.keys[c.cur_key].as<uint32_t>();
     const uint32_t* perm = c.vals[c.perm_buf].as<uint32_t>();
-    LaunchScope ls(&c, "reorder", reorder_bytes(c) * n);
-    with_reorder_form(c, src, dst, [&](auto form, auto io) {
-      using F = decltype(form);
-      k_reorder<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(n, perm, skeys, io);
-    });
-    PR_HIP(hipGetLastError());
-  }
-  c.cur = dst;
-  c.cur_ids ^= 1;
-  {
+    {
+      LaunchScope ls(&c, "reorder", reorder_bytes(c) * n);
+      with_reorder_form(c, src, dst, [&](auto form, auto io) {
+        using F = decltype(form);
+        k_reorder<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(n, perm, skeys, io);
+      });
+      PR_HIP(hipGetLastError());
+    }
     LaunchScope ls(&c, "cell_lb", 8.0 * n + 4.0 * c.grid.n_cells);
     launch_cell_lb(c, skeys);
   }
+  c.inc_ready = false;
+  c.cur = dst;
+  c.cur_ids ^= 1;
   c.sorted = true;
   c.built = true;
 }
@@ -1196,7 +974,7 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
                     reinterpret_cast<uint32_t*>(base + kNaKeys + na_round(4 * kNoAllocMaxN))},
                    {reinterpret_cast<uint32_t*>(base + kNaVals),
                     reinterpret_cast<uint32_t*>(base + kNaVals + na_round(4 * kNoAllocMaxN))},
-                   reinterpret_cast<uint32_t*>(base + kNaHist), reinterpret_cast<uint32_t*>(base + kNaTot), nullptr};
+                   reinterpret_cast<uint32_t*>(base + kNaHist), reinterpret_cast<uint32_t*>(base + kNaTot)};
   double4* spos = reinterpret_cast<double4*>(base + kNaPos);
   uint32_t* lb = reinterpret_cast<uint32_t*>(base + kNaLb);
   k_noalloc_clear<<<1, 64, 0, st>>>(flags);

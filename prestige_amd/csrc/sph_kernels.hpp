@@ -1092,14 +1092,15 @@ __device__ inline bool force_store(uint32_t i, bool live, const Sum<typename Sph
   double fz = floor(((double)x2.z - g.lo[2]) * g.inv_cs);
   bool ok = fx >= 0.0 && fy >= 0.0 && fz >= 0.0 && fx < (double)g.dims[0] &&
             fy < (double)g.dims[1] && fz < (double)g.dims[2];
-  uint32_t key = 0;
+  uint32_t key = old_key;   // a particle outside the grid keeps its cell
   if (ok)
     key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
   else
     atomicOr(&o.flags[FLAG_DOMAIN], 1u);
+  const bool mv = move_to_cell(o.moved, i, old_key, key);
   o.okeys[i] = key;
   o.movcell[key] = o.next_pass;   // this cell holds a moving particle at the next density pass
-  return key != old_key;
+  return mv;
 }
 
 template <int F>
@@ -1211,10 +1212,7 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
   bool mv = false;
   if (i < n) mv = force_store<F>(i, live, sx, sy, sz, out);
   const uint64_t b = __ballot(mv);
-  if (lane == 0u && moved.mask) {
-    moved.mask[tile] = b;
-    if (b) atomicAdd(&moved.tile_cnt[i / kSortTile], (uint32_t)__popcll(b));
-  }
+  if (lane == 0u) moved.mask[tile] = b;
 }
 
 template <int F>
@@ -1355,7 +1353,7 @@ void sph_step_impl(Ctx& c) {
     LaunchScope ls(&c, F == kF64 ? "sph_force_f64" : (F == kF32 ? "sph_force_f32" : "sph_force_mixed"), per * nm);
     const int dst = c.cur ^ 1;
     const int kdst = c.cur_key ^ 1;
-    const MovedOut moved{c.inc_mask.as<uint64_t>(), c.inc_tiles.as<uint32_t>()};
+    const MovedOut moved = moved_out(c);
     S4* acc = c.keep_acc ? c.acc.as<S4>() : nullptr;
     if (io.quad) {
       const ForceOut<F> out{c.pos[c.cur].as<S4>(), c.vel[c.cur].as<S4>(), c.pos[dst].as<S4>(), c.vel[dst].as<S4>(),

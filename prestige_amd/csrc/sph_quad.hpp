@@ -60,10 +60,7 @@ __device__ inline void moved_word_quad(const MovedOut& mo, uint32_t tile, bool m
   m = (m | (m >> 6)) & 0x000F000F000F000Full;
   m = (m | (m >> 12)) & 0x000000FF000000FFull;
   m = (m | (m >> 24)) & 0xFFFFull;
-  if (__lane_id() == 0u && mo.mask) {
-    reinterpret_cast<uint16_t*>(mo.mask)[tile] = (uint16_t)m;
-    if (m) atomicAdd(&mo.tile_cnt[tile * kQuadSlots / kSortTile], (uint32_t)__popcll(m));
-  }
+  if (__lane_id() == 0u) reinterpret_cast<uint16_t*>(mo.mask)[tile] = (uint16_t)m;
 }
 
 // Row runs of a particle's cell in the WCSPH order: first slot and length of
