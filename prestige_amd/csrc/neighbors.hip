@@ -670,51 +670,66 @@ void gather_from_ids(Ctx& c, const double* d_in, void* dst, int dst_kind, int co
 
 // All pairs: thread t is particle id t, j runs over ids 0..n-1 in id order,
 // exactly the generated loop.  force and mass are held in id order.
-// The sum is one dependent FP64 add per pair (about 7 cycles each).  The
-// masses pass through LDS a block-wide tile at a time, in two alternating
-// buffers (one barrier per tile): the next tile is loaded from global memory
-// while the current one is summed, and a full tile is read 32 masses ahead of
-// the adds, enough to cover the LDS latency at one wavefront per SIMD.
-__global__ __launch_bounds__(kBlock) void k_eq1_allpairs(uint32_t n,
-                                                         const double* __restrict__ mass,
-                                                         double* __restrict__ force) {
-  __shared__ double2 tiles[2][kBlock / 2];
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = i < n ? force[i] : 0.0;
-  double next = threadIdx.x < n ? mass[threadIdx.x] : 0.0;
-  uint32_t buf = 0;
-  for (uint32_t j0 = 0; j0 < n; j0 += kBlock, buf ^= 1u) {
-    double2* tile = tiles[buf];
-    double* tile1 = reinterpret_cast<double*>(tile);
-    tile1[threadIdx.x] = next;
-    __syncthreads();
-    const uint32_t jn = j0 + kBlock + threadIdx.x;
-    next = jn < n ? mass[jn] : 0.0;
-    uint32_t m = n - j0 < (uint32_t)kBlock ? n - j0 : (uint32_t)kBlock;
-    if (m == (uint32_t)kBlock) {
-      double2 cur[16], nxt[16];
+// Each force is one chain of dependent FP64 adds (8 cycles each), so the
+// masses must reach every lane without costing issue slots or LDS bandwidth:
+// each row of 16 lanes holds 16 consecutive masses, one per lane, and adds the
+// k-th to all its lanes with a row broadcast in the instruction itself
+// (acc = mass * 1 + acc, the same rounding as the add).  128 masses are held
+// and the next 128 load meanwhile.  Read through LDS (16 bytes to 64 lanes is
+// 8 cycles of a CU's LDS) the four wavefronts of a block took 13.4 cycles a
+// mass at 10,000 particles, 57 us; this takes 8 cycles
+// a mass, 35 us (60,000: 322 -> 199 us).
+__device__ inline double add_row16(double acc, double x, double one) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+      : "+v"(acc)
+      : "v"(x), "v"(one));
+  return acc;
+}
+
+constexpr uint32_t kPairBatch = 8;   // rows of 16 masses held
+__global__ __launch_bounds__(64) void k_eq1_allpairs(uint32_t n, const double* __restrict__ mass,
+                                                     double* __restrict__ force) {
+  const uint32_t i = blockIdx.x * 64u + threadIdx.x, l = threadIdx.x & 15u;
+  double acc = i < n ? force[i] : 0.0;   // every lane stays active: the broadcasts read them all
+  const double one = 1.0;
+  constexpr uint32_t kStep = 16u * kPairBatch;
+  const uint32_t whole = n / kStep * kStep;
+  double cur[kPairBatch], nxt[kPairBatch];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) cur[u] = tile[u];
-      for (uint32_t t = 16; t < (uint32_t)kBlock / 2; t += 16) {
+  for (uint32_t u = 0; u < kPairBatch; ++u) cur[u] = mass[min(16u * u + l, n - 1u)];
+  for (uint32_t j0 = 0; j0 < whole; j0 += kStep) {
 #pragma unroll
-        for (int u = 0; u < 16; ++u) nxt[u] = tile[t + u];
+    for (uint32_t u = 0; u < kPairBatch; ++u) nxt[u] = mass[min(j0 + kStep + 16u * u + l, n - 1u)];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          acc += cur[u].x;
-          acc += cur[u].y;
-        }
+    for (uint32_t u = 0; u < kPairBatch; ++u) acc = add_row16(acc, cur[u], one);
 #pragma unroll
-        for (int u = 0; u < 16; ++u) cur[u] = nxt[u];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        acc += cur[u].x;
-        acc += cur[u].y;
-      }
-    } else {
-      for (uint32_t t = 0; t < m; ++t) acc += tile1[t];
-    }
+    for (uint32_t u = 0; u < kPairBatch; ++u) cur[u] = nxt[u];
   }
+  // the last n % 128 masses: whole rows from the registers, then one by one
+  uint32_t j = whole;
+#pragma unroll
+  for (uint32_t u = 0; u < kPairBatch; ++u)
+    if (j + 16u <= n) {
+      acc = add_row16(acc, cur[u], one);
+      j += 16u;
+    }
+  for (; j < n; ++j) acc += mass[j];
   if (i < n) force[i] = acc;
 }
 
@@ -859,7 +874,7 @@ void eq1_eval(Ctx& c, int loop, double cutoff) {
   if (!n) return;
   if (loop == PRESTIGE_LOOP_ALLPAIRS) {
     LaunchScope ls(&c, "eq1_allpairs", 24.0 * n);
-    k_eq1_allpairs<<<blocks_for(n), kBlock, 0, c.stream>>>(n, c.mass.as<double>(), c.force.as<double>());
+    k_eq1_allpairs<<<blocks_for(n, 64), 64, 0, c.stream>>>(n, c.mass.as<double>(), c.force.as<double>());
     PR_HIP(hipGetLastError());
     return;
   }
