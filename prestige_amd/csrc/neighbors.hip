@@ -738,13 +738,21 @@ __global__ __launch_bounds__(64) void k_eq1_allpairs(uint32_t n, const double* _
 //
 // One wavefront per block (64 consecutive slots).  Per row run the wavefront
 // copies the union of its lanes' candidate ranges into LDS as FP32 offsets
-// from its first slot in units of the cutoff (|q|^2 in .w), with their masses;
-// each lane scans its own range with the dot form q.w - 2 s.q < t, whose
-// threshold carries the rounding margin of the FP32 form (so the scan keeps a
-// superset of the exact neighbours), then walks the set bits in ascending slot
-// order and applies the exact FP64 test: the pairs and the order of the plain
-// loop, so each force is the plain loop's sum bit for bit.  A union wider than
-// the stage is scanned from global memory.
+// from its first slot in units of the cutoff (|q|^2 in .w), with their masses.
+// Each lane then takes its own candidates in slot order with the dot form
+// q.w - 2 s.q, which decides almost every pair: below 1 - m it lies inside the
+// cutoff, at 1 + m or above outside, with m twice the rounding bound of the
+// form (32 u (M^2 + M + 1), u = 2^-24, M the largest offset); a mass inside is
+// added at once.  A wavefront in which some lane's candidate falls between (a
+// few pairs in 10^5) takes the exact FP64 test for it.  So the pairs and the
+// order are the plain loop's, and each force is its sum bit for bit.
+// A union wider than the stage takes the exact test throughout.
+// 1M random particles at 2.4 spacings: 236 us; scanning into masks, walking the
+// set bits and testing each exactly took 403 (1.8M of a jittered dam break: 522
+// -> 361).  What bounds it is instruction issue, six a candidate, then the
+// LDS reads, 24 bytes a candidate and lane.  Where many pairs lie at the
+// cutoff to seven digits (an undisturbed lattice with a lattice distance for
+// a cutoff) the exact tests cost what the direct sums save: 395 -> 413.
 constexpr uint32_t kEq1Stage = 256;
 
 template <class T4>
@@ -752,118 +760,99 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
                                                   const uint32_t* __restrict__ ids,
                                                   const uint32_t* __restrict__ skeys,
                                                   const uint32_t* __restrict__ lb, Grid g, double c2,
-                                                  double inv_cut, float thr, const double* __restrict__ mass,
-                                                  double* __restrict__ force) {
+                                                  double inv_cut, const double* __restrict__ mass,
+                                                  double* __restrict__ force, uint32_t n_tiles) {
 #pragma clang fp contract(off)
-  __shared__ float4 s_q[kEq1Stage + 4];   // 4 entries of padding for the scan's last trip
-  __shared__ double s_m[kEq1Stage];        // mass of the staged slots, gathered once per row run
-  const uint32_t lane = threadIdx.x, wbase = blockIdx.x * 64u, i = wbase + lane;
+  __shared__ float4 s_q[kEq1Stage];
+  __shared__ double s_m[kEq1Stage];   // mass of the staged slots, gathered once per row run
+  const uint32_t tile = xcd_tile(blockIdx.x);
+  if (tile >= n_tiles) return;
+  const uint32_t lane = threadIdx.x, wbase = tile * 64u, i = wbase + lane;
   const bool live = i < n;
-  const T4 pi = pos[live ? i : wbase];
+  const uint32_t self = live ? i : wbase;
+  const T4 pi = pos[self];
   const T4 p0 = pos[wbase];
   const double xr = (double)p0.x, yr = (double)p0.y, zr = (double)p0.z;
   auto offset = [&](const T4& p) {
-    return make_float4((float)(((double)p.x - xr) * inv_cut), (float)(((double)p.y - yr) * inv_cut),
-                       (float)(((double)p.z - zr) * inv_cut), 0.0f);
+    float4 q = make_float4((float)(((double)p.x - xr) * inv_cut), (float)(((double)p.y - yr) * inv_cut),
+                           (float)(((double)p.z - zr) * inv_cut), 0.0f);
+    q.w = __builtin_fmaf(q.x, q.x, __builtin_fmaf(q.y, q.y, q.z * q.z));
+    return q;
   };
-  const uint32_t me = live ? ids[i] : 0u;
+  auto exact = [&](uint32_t j) {
+    const T4 pj = pos[j];
+    const double ex = (double)pi.x - (double)pj.x, ey = (double)pi.y - (double)pj.y, ez = (double)pi.z - (double)pj.z;
+    return ex * ex + ey * ey + ez * ez < c2;
+  };
+  const uint32_t me = ids[self];
   double acc = live ? force[me] : 0.0;
   const uint32_t nx = (uint32_t)g.dims[0], ny = (uint32_t)g.dims[1], nz = (uint32_t)g.dims[2];
-  const uint32_t key = live ? skeys[i] : 0u;
+  const uint32_t key = skeys[self];
   const int cx = (int)(key % nx), cy = (int)((key / nx) % ny), cz = (int)(key / (nx * ny));
   const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx < (int)nx - 1 ? cx + 1 : (int)nx - 1;
+  // the nine row runs' ranges, read at once
+  uint32_t j0[9], len[9];
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    const int zz = cz + r / 3 - 1, yy = cy + r % 3 - 1;
+    const bool ok = live && zz >= 0 && zz < (int)nz && yy >= 0 && yy < (int)ny;
+    const uint32_t row = ok ? ((uint32_t)zz * ny + (uint32_t)yy) * nx : 0u;
+    j0[r] = lb[row + (uint32_t)x0];
+    len[r] = ok ? lb[row + (uint32_t)x1 + 1u] - j0[r] : 0u;
+  }
   const float4 so = offset(pi);
   const float ax = -2.0f * so.x, ay = -2.0f * so.y, az = -2.0f * so.z;
-  const float ss = __builtin_fmaf(so.x, so.x, __builtin_fmaf(so.y, so.y, so.z * so.z));
-  const float ss_max = wave_max_pos(live ? ss : 0.0f);
-  for (int dz = -1; dz <= 1; ++dz) {
-    for (int dy = -1; dy <= 1; ++dy) {
-      const int zz = cz + dz, yy = cy + dy;
-      uint32_t j0 = 0u, len = 0u;
-      if (live && zz >= 0 && zz < (int)nz && yy >= 0 && yy < (int)ny) {
-        const uint32_t row = ((uint32_t)zz * ny + (uint32_t)yy) * nx;
-        j0 = lb[row + (uint32_t)x0];
-        len = lb[row + (uint32_t)x1 + 1] - j0;
-      }
-      const uint32_t base = wave_min(len ? j0 : 0xFFFFFFFFu);
-      const uint32_t top = wave_max(len ? j0 + len : 0u);
-      if (top <= base) continue;
-      const bool staged = top - base <= kEq1Stage;
-      float t = 0.0f;
-      if (staged) {
-        float mq = 0.0f;
-        for (uint32_t kk = lane; kk < top - base; kk += 64u) {
-          float4 q = offset(pos[base + kk]);
-          q.w = __builtin_fmaf(q.x, q.x, __builtin_fmaf(q.y, q.y, q.z * q.z));
-          s_q[kk] = q;
-          s_m[kk] = mass[ids[base + kk]];
-          mq = q.w > mq ? q.w : mq;
-        }
-        // rounding of the dot form with |s|, |q| <= M, as in the WCSPH scan
-        const float m2 = fmaxf(ss_max, wave_max_pos(mq));
-        t = thr + 0x1.0p-19f * (m2 + __builtin_sqrtf(m2) + 1.0f) - ss;
-        __syncthreads();
-      }
-      // up to 128 candidates at a time: four scan words, then a walk of their set bits
-      for (uint32_t c0 = 0u; c0 < len; c0 += 128u) {
-        const uint32_t clen = len - c0 < 128u ? len - c0 : 128u;
-        uint32_t wd[4] = {0u, 0u, 0u, 0u};
+  const float ss_max = wave_max_pos(live ? so.w : 0.0f);
 #pragma unroll
-        for (uint32_t w = 0u; w < 4u; ++w) {
-          if (32u * w >= clen) break;
-          const uint32_t cnt = clen - 32u * w < 32u ? clen - 32u * w : 32u;
-          uint32_t word = 0u;
-          for (uint32_t b = 0u; b < cnt; b += 4u) {
-            uint32_t hb = 0u;
-#pragma unroll
-            for (uint32_t u = 0u; u < 4u; ++u) {
-              const uint32_t jc = j0 + c0 + 32u * w + b + u;
-              bool hit;
-              if (staged) {
-                const float4 q = s_q[jc - base];
-                hit = __builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w))) < t;
-              } else {
-                const float4 q = offset(pos[jc < n ? jc : n - 1u]);
-                const float ddx = so.x - q.x, ddy = so.y - q.y, ddz = so.z - q.z;
-                hit = __builtin_fmaf(ddx, ddx, __builtin_fmaf(ddy, ddy, ddz * ddz)) < thr;
-              }
-              hb |= (hit ? 1u : 0u) << u;
-            }
-            word |= hb << b;
-          }
-          wd[w] = cnt < 32u ? word & ((1u << cnt) - 1u) : word;
-        }
-        uint64_t m0 = (uint64_t)wd[0] | ((uint64_t)wd[1] << 32);
-        uint64_t m1 = (uint64_t)wd[2] | ((uint64_t)wd[3] << 32);
-        auto pop = [&]() -> uint32_t {
-          uint32_t b;
-          if (m0) {
-            b = (uint32_t)__builtin_ctzll(m0);
-            m0 &= m0 - 1;
-          } else {
-            b = 64u + (uint32_t)__builtin_ctzll(m1);
-            m1 &= m1 - 1;
-          }
-          return b;
-        };
-        // two neighbours a trip, so their loads overlap; the sum still runs in slot order
-        while (m0 | m1) {
-          const uint32_t ja = j0 + c0 + pop();
-          const bool two = (m0 | m1) != 0u;
-          const uint32_t jb = two ? j0 + c0 + pop() : ja;
-          const T4 pa = pos[ja], pb = pos[jb];
-          const double ma = staged ? s_m[ja - base] : mass[ids[ja]];
-          const double mb = staged ? s_m[jb - base] : mass[ids[jb]];
-          const double ex = (double)pi.x - (double)pa.x, ey = (double)pi.y - (double)pa.y,
-                       ez = (double)pi.z - (double)pa.z;
-          const double fx = (double)pi.x - (double)pb.x, fy = (double)pi.y - (double)pb.y,
-                       fz = (double)pi.z - (double)pb.z;
-          if (ex * ex + ey * ey + ez * ez < c2) acc += ma;
-          if (two && fx * fx + fy * fy + fz * fz < c2) acc += mb;
-        }
-      }
-      if (staged) __syncthreads();
+  for (int r = 0; r < 9; ++r) {
+    // union of the lanes' ranges: slots are in key order, so the first and
+    // last lane with candidates bound it
+    const uint64_t any = __ballot(len[r] != 0u);
+    if (any == 0ull) continue;
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)j0[r], __builtin_ctzll(any));
+    const uint32_t span = (uint32_t)__builtin_amdgcn_readlane((int)(j0[r] + len[r]), 63 - __builtin_clzll(any)) - base;
+    if (span > kEq1Stage) {
+      for (uint32_t b = 0; b < len[r]; ++b)
+        if (exact(j0[r] + b)) acc += mass[ids[j0[r] + b]];
+      continue;
     }
+    float mq = 0.0f;
+    for (uint32_t kk = lane; kk < span; kk += 64u) {
+      const float4 q = offset(pos[base + kk]);
+      s_q[kk] = q;
+      s_m[kk] = mass[ids[base + kk]];
+      mq = q.w > mq ? q.w : mq;
+    }
+    const float m2 = fmaxf(ss_max, wave_max_pos(mq));
+    const float margin = 0x1.0p-18f * (m2 + __builtin_sqrtf(m2) + 1.0f);
+    const float lo = (1.0f - margin) - so.w, hi = (1.0f + margin) - so.w;
+    __builtin_amdgcn_wave_barrier();   // one wavefront: its LDS operations complete in order
+    const uint32_t first = j0[r] - base;
+    auto take = [&](float v, double m, uint32_t j) {
+      bool in = v < lo;
+      if (__ballot(in != (v < hi)) != 0ull) {   // some lane cannot tell
+        if (v < hi && !in) in = exact(j);
+      }
+      if (in) acc += m;
+    };
+    uint32_t b = 0;
+    for (; b + 4u <= len[r]; b += 4u) {
+      float v[4];
+      double m[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4u; ++u) {
+        const float4 q = s_q[first + b + u];
+        v[u] = __builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w)));
+        m[u] = s_m[first + b + u];
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 4u; ++u) take(v[u], m[u], j0[r] + b + u);
+    }
+    for (; b < len[r]; ++b) {
+      const float4 q = s_q[first + b];
+      take(__builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w))), s_m[first + b], j0[r] + b);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
   if (live) force[me] = acc;
 }
@@ -883,15 +872,15 @@ void eq1_eval(Ctx& c, int loop, double cutoff) {
   if (!c.sorted) neighbors_build(c);
   LaunchScope ls(&c, "eq1_cells", 56.0 * n);
   const uint32_t* ids = c.ids[c.cur_ids].as<uint32_t>();
-  const float thr = cell_scan_threshold(c.grid, cutoff);
+  const uint32_t tiles = blocks_for(n, 64);
   if (c.desc.precision == PRESTIGE_F32)
-    k_eq1_cells<float4><<<blocks_for(n, 64), 64, 0, c.stream>>>(
+    k_eq1_cells<float4><<<tile_grid(tiles), 64, 0, c.stream>>>(
         n, c.pos[c.cur].as<float4>(), ids, c.keys[c.cur_key].as<uint32_t>(), c.lb.as<uint32_t>(),
-        c.grid, cutoff * cutoff, 1.0 / cutoff, thr, c.mass.as<double>(), c.force.as<double>());
+        c.grid, cutoff * cutoff, 1.0 / cutoff, c.mass.as<double>(), c.force.as<double>(), tiles);
   else
-    k_eq1_cells<double4><<<blocks_for(n, 64), 64, 0, c.stream>>>(
+    k_eq1_cells<double4><<<tile_grid(tiles), 64, 0, c.stream>>>(
         n, c.pos[c.cur].as<double4>(), ids, c.keys[c.cur_key].as<uint32_t>(), c.lb.as<uint32_t>(),
-        c.grid, cutoff * cutoff, 1.0 / cutoff, thr, c.mass.as<double>(), c.force.as<double>());
+        c.grid, cutoff * cutoff, 1.0 / cutoff, c.mass.as<double>(), c.force.as<double>(), tiles);
   PR_HIP(hipGetLastError());
 }
 
@@ -1005,8 +994,9 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
   const uint32_t key_blocks = (uint32_t)blocks_for(n);
   k_cell_lb<<<key_blocks + kTailBlocks, kBlock, 0, st>>>(n, g.n_cells, skeys, lb, key_blocks);
   PR_HIP(hipGetLastError());
-  k_eq1_cells<double4><<<blocks_for(n, 64), 64, 0, st>>>(n, spos, perm, skeys, lb, g, cutoff * cutoff, 1.0 / cutoff,
-                                                          cell_scan_threshold(g, cutoff), mass, force);
+  const uint32_t tiles = blocks_for(n, 64);
+  k_eq1_cells<double4><<<tile_grid(tiles), 64, 0, st>>>(n, spos, perm, skeys, lb, g, cutoff * cutoff, 1.0 / cutoff,
+                                                        mass, force, tiles);
   PR_HIP(hipGetLastError());
   uint32_t h[FLAG_COUNT] = {0, 0, 0, 0};
   PR_HIP(hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, st));
