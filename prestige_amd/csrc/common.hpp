@@ -373,23 +373,31 @@ __device__ inline uint32_t xcd_tile(uint32_t b) {
 // Blocks that cover n_tiles tiles (the last ones may have none).
 inline uint32_t tile_grid(uint32_t n_tiles) { return (n_tiles + 8u * kTileRun - 1u) / (8u * kTileRun) * (8u * kTileRun); }
 
-// Minimum / maximum over the wavefront, returned as a wave-uniform value.
-__device__ inline uint32_t wave_min(uint32_t v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const uint32_t t = __shfl_xor(v, d, 64);
-    v = t < v ? t : v;
-  }
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+// Reductions over the wavefront, returned as a wave-uniform value; every lane
+// calls.  Row shifts and row broadcasts in the operation itself (its first
+// operand through DPP) carry them into lane 63: six instructions and no LDS,
+// where shuffles go through the LDS crossbar six times in turn.  The WCSPH
+// passes do up to four reductions per run: the FP64 force pass went from 126 to
+// 111 registers and from 1362 to 1305 us at 6M particles.
+template <class Op>
+__device__ inline uint32_t wave_reduce(uint32_t v, uint32_t id, Op&& op) {
+  // lanes a control does not reach combine with the identity
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x111, 0xF, 0xF, false));   // row_shr:1
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x112, 0xF, 0xF, false));   // row_shr:2
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x114, 0xF, 0xF, false));   // row_shr:4
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x118, 0xF, 0xF, false));   // row_shr:8
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x142, 0xA, 0xF, false));   // row_bcast:15
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x143, 0xC, 0xF, false));   // row_bcast:31
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-
+__device__ inline uint32_t wave_min(uint32_t v) {
+  return wave_reduce(v, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return b < a ? b : a; });
+}
 __device__ inline uint32_t wave_max(uint32_t v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const uint32_t t = __shfl_xor(v, d, 64);
-    v = t > v ? t : v;
-  }
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+  return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return b > a ? b : a; });
+}
+__device__ inline uint32_t wave_sum(uint32_t v) {
+  return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 // Maximum of a non-negative float over the wavefront (their bit patterns

@@ -398,12 +398,6 @@ double reorder_bytes(const Ctx& c) {
 // bound by the state it moves (6 TB/s at 6M).
 // ---------------------------------------------------------------------------
 
-__device__ inline uint32_t wave_sum(uint32_t x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
-}
-
 // New cell table of tile b (kCellTile cells): the offset before it from the
 // tile totals, then a block scan of the cells' net counts, which are cleared
 // for the next step.  A tile nothing entered or left only adds its offset.
