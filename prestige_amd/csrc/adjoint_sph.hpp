@@ -99,36 +99,49 @@ __global__ __launch_bounds__(kBlock) void k_adj_prep(uint32_t n, uint64_t n_movi
   cvec[k] = C4{(decltype(C4{}.x))(s * vt.x), (decltype(C4{}.x))(s * vt.y), (decltype(C4{}.x))(s * vt.z), 0};
 }
 
-// Block sum of two doubles into partial[slot] (deterministic); W wavefronts
-// per block.
-template <uint32_t W>
-__device__ inline void block_sum2(double a, double b, double2* __restrict__ partial, uint32_t slot) {
-  __shared__ double sa[W], sb[W];
+// K sums of a block's wavefronts 1 .. kGroups - 1.
+template <int K>
+struct GroupSums {
+  double v[kGroups - 1][K][64];
+};
+// Adds them to the first wavefront's, in wavefront order; false in the others,
+// which are done.
+template <int K>
+__device__ inline bool gather_groups(double* (&sums)[K], GroupSums<K>& st, uint32_t wave, uint32_t lane) {
+  if (wave != 0u) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) st.v[wave - 1u][q][lane] = *sums[q];
+  }
+  __syncthreads();
+  if (wave != 0u) return false;
+  for (uint32_t w = 0; w + 1u < kGroups; ++w) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) *sums[q] += st.v[w][q][lane];
+  }
+  return true;
+}
+
+// Sum of two doubles over the wavefront into partial[slot] (deterministic).
+__device__ inline void wave_sum2(double a, double b, double2* __restrict__ partial, uint32_t slot) {
   for (int o = 32; o > 0; o >>= 1) {
     a += __shfl_down(a, (unsigned)o, 64);
     b += __shfl_down(b, (unsigned)o, 64);
   }
-  const uint32_t w = threadIdx.x >> 6;
-  if (__lane_id() == 0) {
-    sa[w] = a;
-    sb[w] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double ta = 0.0, tb = 0.0;
-    for (uint32_t k = 0; k < W; ++k) {
-      ta += sa[k];
-      tb += sb[k];
-    }
-    partial[slot] = make_double2(ta, tb);
-  }
+  if (__lane_id() == 0) partial[slot] = make_double2(0.0 + a, 0.0 + b);
 }
 
 // Force + EOS adjoint (all slots; fixed particles collect Pbar and rhobar as
 // neighbours of moving ones).  Writes xbar of the force rows (metres), adds
 // the viscosity part of vbar, writes rhobar, and block partials of
-// (dalpha, dc0).  One wavefront per block; each row run's neighbour data are
-// staged in LDS as in the forward force pass.
+// (dalpha, dc0).  Each row run's neighbour data are staged in LDS as in the
+// forward force pass.
+//
+// SPLIT: a block is five wavefronts on one 64-slot tile, each walking one run
+// group straight from global memory (with a stage each, a mixed block's 45 KB
+// of LDS made 118k particles 58 us instead of 50); the first adds the groups'
+// sums, which are formed apart in either variant, in group order, so the
+// results are the same bits.  For contexts whose tiles leave the device idle
+// (the rule stands in sph_reverse_step).
 constexpr int kAdjBlock = 64;
 // Wavefronts per SIMD the register budgets are held to, as measured fastest
 // (mixed density adjoint at 1M: 6 256 us, 7 263, 8 273).
@@ -144,7 +157,14 @@ template <int F>
 constexpr bool kAdjPrefetch = F == kMixed;
 
 template <int F>
-__global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
+struct AdjForceStage {
+  StageArr<typename SphForm<F>::G4, kForceCap> p, v;
+  typename SphForm<F>::R2 rp[kForceCap];
+  StageArr<typename AdjForm<F>::C4, kForceCap> c;
+};
+
+template <int F, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
     uint32_t n, uint64_t n_moving, SphStepRecord rec, Grid g, SphConst kc, SphUnits u, double alpha, double c0,
     double rho0, const typename AdjForm<F>::C4* __restrict__ cvec, double4* __restrict__ xbf,
     double4* __restrict__ vb, typename AdjForm<F>::ar* __restrict__ rhob, double2* __restrict__ partial,
@@ -157,10 +177,9 @@ __global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
   const G4* gpos = (const G4*)rec.gpos;
   const G4* gvel = (const G4*)rec.gvel;
   const R2* rp = (const R2*)rec.rp;
-  __shared__ StageArr<G4, kForceCap> s_p, s_v;
-  __shared__ R2 s_rp[kForceCap];
-  __shared__ StageArr<C4, kForceCap> s_c;
-  const uint32_t lane = threadIdx.x;
+  __shared__ typename std::conditional<SPLIT, GroupSums<9>, AdjForceStage<F>>::type st;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = SPLIT ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0u;
   const uint32_t tile = xcd_tile(blockIdx.x);
   if (tile >= n_tiles) return;
   const uint32_t i = tile * kAdjBlock + lane;
@@ -247,23 +266,27 @@ __global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
         }
       }
     };
-    walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F>>(
-        rec.meta, rec.words, n, i, live, lane,
+    walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
+        rec.meta, rec.words, n, i, live, lane, SPLIT ? wave : 0u, SPLIT ? wave + 1u : kGroups,
         [&](uint32_t grp) {
           if constexpr (F == kMixed) pb_.begin(pi, grp, u.cs_u);
         },
         [&](uint32_t k, uint32_t j) {
-          s_p.put(k, gpos[j]);
-          s_v.put(k, gvel[j]);
-          s_rp[k] = rp[j];
-          s_c.put(k, cvec[j]);
+          if constexpr (!SPLIT) {
+            st.p.put(k, gpos[j]);
+            st.v.put(k, gvel[j]);
+            st.rp[k] = rp[j];
+            st.c.put(k, cvec[j]);
+          }
         },
         [&](const uint32_t* jj, const uint32_t* tt) {
           body(jj, tt, [&](uint32_t k, G4& p, G4& v, R2& r, C4& cc) {
-            p = s_p.get(k);
-            v = s_v.get(k);
-            r = s_rp[k];
-            cc = s_c.get(k);
+            if constexpr (!SPLIT) {
+              p = st.p.get(k);
+              v = st.v.get(k);
+              r = st.rp[k];
+              cc = st.c.get(k);
+            }
           });
         },
         [&](const uint32_t* jj, const uint32_t* tt) {
@@ -275,6 +298,10 @@ __global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
           });
         },
         end_run);
+    if constexpr (SPLIT) {
+      double* sums[9] = {&xx, &xy, &xz, &vx, &vy, &vz, &pb, &rb, &sa};
+      if (!gather_groups(sums, st, wave, lane)) return;
+    }
     if (live) {
       pa = sa * c0;
       pc = sa * alpha;
@@ -300,7 +327,7 @@ __global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
       }
     }
   }
-  block_sum2<kAdjBlock / 64>(pa, pc, partial, tile);   // one partial per tile: a fixed sum order
+  wave_sum2(pa, pc, partial, tile);   // one partial per tile: a fixed sum order
 }
 
 // Density adjoint + assembly: xbar_k = xbar'_k + force part + density part
@@ -308,7 +335,13 @@ __global__ __launch_bounds__(kAdjBlock, kAdjForceWaves<F>) void k_adj_force(
 // step's slot order through the frozen permutation.  One wavefront per
 // block, neighbour data staged per row run.
 template <int F>
-__global__ __launch_bounds__(kAdjBlock, kAdjDensityWaves<F>) void k_adj_density(
+struct AdjDensityStage {
+  StageArr<typename SphForm<F>::G4, kForceCap> p;
+  typename AdjForm<F>::ar rb[kForceCap];
+};
+
+template <int F, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjDensityWaves<F>) void k_adj_density(
     uint32_t n, uint64_t n_moving, SphStepRecord rec, Grid g, SphConst kc, SphUnits u,
     const typename AdjForm<F>::ar* __restrict__ rhob, const double4* __restrict__ xb_in,
     const double4* __restrict__ xbf, const double4* __restrict__ vb_in, double4* __restrict__ xb_out,
@@ -317,9 +350,9 @@ __global__ __launch_bounds__(kAdjBlock, kAdjDensityWaves<F>) void k_adj_density(
   using G4 = typename SphForm<F>::G4;
   using ar = typename AdjForm<F>::ar;
   const G4* gpos = (const G4*)rec.gpos;
-  __shared__ StageArr<G4, kForceCap> s_p;
-  __shared__ ar s_rb[kForceCap];
-  const uint32_t lane = threadIdx.x;
+  __shared__ typename std::conditional<SPLIT, GroupSums<3>, AdjDensityStage<F>>::type st;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = SPLIT ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0u;
   const uint32_t tile = xcd_tile(blockIdx.x);
   if (tile >= n_tiles) return;
   const uint32_t i = tile * kAdjBlock + lane;
@@ -356,19 +389,23 @@ __global__ __launch_bounds__(kAdjBlock, kAdjDensityWaves<F>) void k_adj_density(
       qz += s * (ar)dzr;
     }
   };
-  walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F>>(
-      rec.meta, rec.words, n, i, live, lane,
+  walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
+      rec.meta, rec.words, n, i, live, lane, SPLIT ? wave : 0u, SPLIT ? wave + 1u : kGroups,
       [&](uint32_t grp) {
         if constexpr (F == kMixed) pb_.begin(pi, grp, u.cs_u);
       },
       [&](uint32_t k, uint32_t j) {
-        s_p.put(k, gpos[j]);
-        s_rb[k] = rhob[j];
+        if constexpr (!SPLIT) {
+          st.p.put(k, gpos[j]);
+          st.rb[k] = rhob[j];
+        }
       },
       [&](const uint32_t* jj, const uint32_t* tt) {
         body(jj, tt, [&](uint32_t k, G4& p, ar& rb) {
-          p = s_p.get(k);
-          rb = s_rb[k];
+          if constexpr (!SPLIT) {
+            p = st.p.get(k);
+            rb = st.rb[k];
+          }
         });
       },
       [&](const uint32_t* jj, const uint32_t* tt) {
@@ -383,6 +420,10 @@ __global__ __launch_bounds__(kAdjBlock, kAdjDensityWaves<F>) void k_adj_density(
         sz += (double)qz;
         qx = qy = qz = ar(0.0);
       });
+  if constexpr (SPLIT) {
+    double* sums[3] = {&sx, &sy, &sz};
+    if (!gather_groups(sums, st, wave, lane)) return;
+  }
   if (i >= n) return;
   const uint32_t dst = rec.perm[i];
   if (!live) {
@@ -450,6 +491,12 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
   const uint32_t n = (uint32_t)c.n;
   const SphUnits u = sph_units<F>(c);
   const uint32_t n_tiles = blocks_for(n, kAdjBlock);
+  // Five wavefronts per tile (SPLIT) up to where the device is full with one:
+  // us at 10k, 43k, 118k, 196k, 329k particles, one / five: mixed force 61/27,
+  // 66/31, 68/50, 82/88; FP64 force 85/37, 91/66, 99/121; density mixed 37/17,
+  // 40/18, 42/22, 47/38, 54/54, FP64 48/20, 52/23, 53/33, 68/56, 92/83.
+  const bool split_force = c.quad && n <= (F == kMixed ? 150000u : 64000u);
+  const bool split_density = c.quad && n <= 300000u;
   {
     LaunchScope ls(&c, "adj_prep", 2.0 * 32.0 * n + 32.0 * n);
     k_adj_prep<F><<<blocks_for(n), kBlock, 0, c.stream>>>(n, c.n_moving, rec.ids, A.xb, A.vb,
@@ -459,9 +506,13 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
   {
     const double ge = (double)sizeof(typename SphForm<F>::real);
     LaunchScope ls(&c, F == kF64 ? "adj_force_f64" : "adj_force_mixed", (8.0 * ge + 24.0 + 24.0 + 8.0 + 48.0) * n);
-    k_adj_force<F><<<tile_grid(n_tiles), kAdjBlock, 0, c.stream>>>(
-        n, c.n_moving, rec, c.grid, c.sph, u, c.desc.alpha, c.desc.c0, c.desc.rho0,
-        (const typename AdjForm<F>::C4*)A.cvec, A.xbf, A.vb, (typename AdjForm<F>::ar*)A.rhob, A.partial, n_tiles);
+    auto launch = [&](auto kernel, int block) {
+      kernel<<<tile_grid(n_tiles), block, 0, c.stream>>>(
+          n, c.n_moving, rec, c.grid, c.sph, u, c.desc.alpha, c.desc.c0, c.desc.rho0,
+          (const typename AdjForm<F>::C4*)A.cvec, A.xbf, A.vb, (typename AdjForm<F>::ar*)A.rhob, A.partial, n_tiles);
+    };
+    if (split_force) launch(k_adj_force<F, true>, 64 * kGroups);
+    else launch(k_adj_force<F, false>, kAdjBlock);
     PR_HIP(hipGetLastError());
     k_adj_reduce<<<1, kAdjReduceBlock, 0, c.stream>>>(n_tiles, A.partial, A.acc);
     PR_HIP(hipGetLastError());
@@ -470,9 +521,13 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
     const double ge = (double)sizeof(typename SphForm<F>::real);
     LaunchScope ls(&c, F == kF64 ? "adj_density_f64" : "adj_density_mixed",
                    (3.0 * ge + 8.0 + 24.0 * 3 + 24.0 * 2 + 8.0) * n);
-    k_adj_density<F><<<tile_grid(n_tiles), kAdjBlock, 0, c.stream>>>(
-        n, c.n_moving, rec, c.grid, c.sph, u, (const typename AdjForm<F>::ar*)A.rhob, A.xb, A.xbf, A.vb, A.xb2,
-        A.vb2, n_tiles);
+    auto launch = [&](auto kernel, int block) {
+      kernel<<<tile_grid(n_tiles), block, 0, c.stream>>>(
+          n, c.n_moving, rec, c.grid, c.sph, u, (const typename AdjForm<F>::ar*)A.rhob, A.xb, A.xbf, A.vb, A.xb2, A.vb2,
+          n_tiles);
+    };
+    if (split_density) launch(k_adj_density<F, true>, 64 * kGroups);
+    else launch(k_adj_density<F, false>, kAdjBlock);
     PR_HIP(hipGetLastError());
   }
   std::swap(A.xb, A.xb2);

@@ -267,6 +267,7 @@ __device__ inline real spline_df(real q) {
 constexpr int kScanUnr = 2;
 constexpr int kDensUnr = 2;
 constexpr int kUnr = 2;
+constexpr int kMaskUnr = 8;   // candidates in flight in the scan that only keeps masks
 static_assert(kScanUnr == 1 || kScanUnr == 2 || kScanUnr == 4, "scan batch divides 32");
 static_assert(kDensUnr >= 1 && kUnr >= 1, "walk batches hold at least one neighbour");
 constexpr uint32_t kPad = 0xFFFFFFFFu;
@@ -323,21 +324,21 @@ __device__ inline uint32_t shift_in(uint32_t w, bool hit) {
 // H2p is tested as q.w - 2 s.q < H2p - |s|^2, three FMAs per candidate with
 // a = -2 s and t = H2p - |s|^2 precomputed.  The rounding of this form grows
 // with the offsets' magnitude M, so t carries a margin in M (density kernel).
-template <class Ld>
+template <int U, class Ld>
 __device__ inline uint32_t scan_word_dot(Ld&& ld, uint32_t k0, uint32_t cnt, float ax, float ay, float az,
                                          float t) {
   uint32_t word = 0;
-  for (uint32_t b = 0; b < cnt; b += kScanUnr) {
-    float4 q[kScanUnr];
+  for (uint32_t b = 0; b < cnt; b += U) {
+    float4 q[U];
 #pragma unroll
-    for (int u = 0; u < kScanUnr; ++u) q[u] = ld(k0 + b + (uint32_t)u);
+    for (int u = 0; u < U; ++u) q[u] = ld(k0 + b + (uint32_t)u);
 #pragma unroll
-    for (int u = 0; u < kScanUnr; ++u) {
+    for (int u = 0; u < U; ++u) {
       const float v = __builtin_fmaf(ax, q[u].x, __builtin_fmaf(ay, q[u].y, __builtin_fmaf(az, q[u].z, q[u].w)));
       word = shift_in(word, v < t);
     }
   }
-  const uint32_t P = (cnt + (uint32_t)kScanUnr - 1u) & ~((uint32_t)kScanUnr - 1u);
+  const uint32_t P = (cnt + (uint32_t)U - 1u) & ~((uint32_t)U - 1u);
   word = __builtin_bitreverse32(word) >> (32u - P);
   return cnt < 32u ? word & ((1u << cnt) - 1u) : word;
 }
@@ -449,8 +450,15 @@ __device__ inline void ProbeRunBases::begin(const float4& pi, uint32_t grp, floa
   }
 }
 
-// Walk of a wavefront over its lanes' stored masks (one wavefront per block;
-// every lane calls it, live or not), run groups in the WCSPH order.  For each
+// Orders a wavefront's LDS accesses before and after it (they complete in
+// order; the compiler must not move them).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Walk of a wavefront over its lanes' stored masks (its own LDS stage; every
+// lane calls it, live or not), run groups [g0, g1) in the WCSPH order.  For each
 // group begin(grp) runs first; then the wavefront copies the gather data of
 // the union of its lanes' hit ranges of the group's runs into LDS with
 // stage(k, j) (slot j -> stage entry k), then each lane walks its own masks B
@@ -460,10 +468,14 @@ __device__ inline void ProbeRunBases::begin(const float4& pi, uint32_t grp, floa
 // walked run by run, and a run whose union alone exceeds CAP with glob(jj,
 // tt) (jj: slots).  Lanes visit their neighbours in group order and scan
 // order either way; end_run() follows each group.
-template <int B, uint32_t CAP, bool PF = false, class Begin, class Stage, class Lds, class Glob, class End>
+//
+// DIRECT: nothing is staged and every walk uses glob; the groups are still
+// walked as one stream or run by run by the same rule, so that the entries
+// come in the same batches.
+template <int B, uint32_t CAP, bool PF = false, bool DIRECT = false, class Begin, class Stage, class Lds, class Glob, class End>
 __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const uint32_t* __restrict__ words,
-                                        uint32_t n, uint32_t i, bool live, uint32_t lane, Begin&& begin,
-                                        Stage&& stage, Lds&& lds, Glob&& glob, End&& end_run) {
+                                        uint32_t n, uint32_t i, bool live, uint32_t lane, uint32_t g0, uint32_t g1,
+                                        Begin&& begin, Stage&& stage, Lds&& lds, Glob&& glob, End&& end_run) {
   // PF: the next group's row metadata and the first two mask words of each of
   // its runs (candidates 0..63, nearly every run) are loaded one group ahead,
   // masked by the run's length on use, so their latency overlaps the current
@@ -483,8 +495,8 @@ __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const ui
       }
     }
   };
-  if constexpr (PF) prefetch(0u);
-  for (uint32_t grp = 0; grp < kGroups; ++grp) {
+  if constexpr (PF) prefetch(g0);
+  for (uint32_t grp = g0; grp < g1; ++grp) {
     begin(grp);
     const uint32_t nrun = grp + 1u == kGroups ? 1u : 2u;
     uint64_t m[4] = {0u, 0u, 0u, 0u};
@@ -503,7 +515,7 @@ __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const ui
         m[2u * t] = (uint64_t)wd[0] | ((uint64_t)wd[1] << 32);
         m[2u * t + 1u] = (uint64_t)wd[2] | ((uint64_t)wd[3] << 32);
       }
-      if (grp + 1u < kGroups) prefetch(grp + 1u);
+      if (grp + 1u < g1) prefetch(grp + 1u);
     }
 #pragma unroll
     for (uint32_t t = 0; t < 2u; ++t) {
@@ -525,11 +537,35 @@ __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const ui
       end_run();
       continue;
     }
-    if (total <= CAP) {
+    if constexpr (DIRECT) {
+      if (total <= CAP) {
+        // bit 31 names the run of the group (slots stay below 2^31)
+        uint32_t wb[4] = {j0[0], j0[0] + 64u, j0[1] | 0x80000000u, (j0[1] + 64u) | 0x80000000u};
+        walk_bits_q<B>(m, wb, [&](const uint32_t* jj) {
+          uint32_t js[B], tt[B];
+#pragma unroll
+          for (int v = 0; v < B; ++v) {
+            js[v] = jj[v] == kPad ? kPad : jj[v] & 0x7FFFFFFFu;
+            tt[v] = jj[v] == kPad ? 0u : jj[v] >> 31;
+          }
+          glob(js, tt);
+        });
+      } else {
+#pragma unroll
+        for (uint32_t t = 0; t < 2u; ++t) {
+          uint32_t tt[B];
+#pragma unroll
+          for (int v = 0; v < B; ++v) tt[v] = t;
+          uint64_t mm[2] = {m[2u * t], m[2u * t + 1u]};
+          uint32_t wb[2] = {j0[t], j0[t] + 64u};
+          walk_bits_q<B>(mm, wb, [&](const uint32_t* jj) { glob(jj, tt); });
+        }
+      }
+    } else if (total <= CAP) {
       // both runs' unions side by side: run 0 at [0, span0), run 1 after it
       for (uint32_t k = lane; k < total; k += 64u)
         stage(k, k < span[0] ? base[0] + k : base[1] + (k - span[0]));
-      __syncthreads();
+      wave_lds_fence();
       // stage entry of bit 0 of each mask word
       uint32_t wb[4] = {j0[0] - base[0], j0[0] - base[0] + 64u, span[0] + j0[1] - base[1],
                         span[0] + j0[1] - base[1] + 64u};
@@ -540,7 +576,7 @@ __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const ui
         for (int v = 0; v < B; ++v) tt[v] = jj[v] != kPad && jj[v] >= s0 ? 1u : 0u;
         lds(jj, tt);
       });
-      __syncthreads();  // the next group's staging overwrites the stage
+      wave_lds_fence();  // the next group's staging overwrites the stage
     } else {
 #pragma unroll
       for (uint32_t t = 0; t < 2u; ++t) {
@@ -551,10 +587,10 @@ __device__ inline void walk_runs_staged(const uint2* __restrict__ meta, const ui
         uint64_t mm[2] = {m[2u * t], m[2u * t + 1u]};
         if (span[t] <= CAP) {
           for (uint32_t k = lane; k < span[t]; k += 64u) stage(k, base[t] + k);
-          __syncthreads();
+          wave_lds_fence();
           uint32_t wb[2] = {j0[t] - base[t], j0[t] - base[t] + 64u};
           walk_bits_q<B>(mm, wb, [&](const uint32_t* jj) { lds(jj, tt); });
-          __syncthreads();
+          wave_lds_fence();
         } else {
           uint32_t wb[2] = {j0[t], j0[t] + 64u};
           walk_bits_q<B>(mm, wb, [&](const uint32_t* jj) { glob(jj, tt); });
@@ -716,8 +752,14 @@ __device__ inline void density_store(uint32_t i, const Sum<typename SphForm<F>::
   }
 }
 
-template <int F>
-__global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
+// WALK false: only the row masks (of a step recorded for the mixed adjoint,
+// whose sums the four-lane passes form, sph_quad.hpp): the same scan from the
+// same points, so the same masks; wavefronts of dry wall particles get empty
+// ones.  Block row y scans run sph_run(y) alone: a small tank leaves most of
+// the device idle, and nothing ties the runs together (110k particles: 69 us
+// with the nine runs in turn, 26 so).
+template <int F, bool WALK>
+__global__ __launch_bounds__(kDensBlock, WALK ? kDensWaves<F> : 4) void k_sph_density(
     uint32_t n, const typename SphForm<F>::S4* __restrict__ spos, const typename SphForm<F>::G4* pos,
     const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ lb, Grid g, SphConst kc, SphUnits u,
     uint2* __restrict__ meta, uint32_t* __restrict__ words, typename SphForm<F>::R2* __restrict__ rp,
@@ -726,7 +768,8 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using S4 = typename SphForm<F>::S4;
-  __shared__ float4 s_q[kStageCap + kScanUnr];
+  constexpr int kUnrolled = WALK ? kScanUnr : kMaskUnr;
+  __shared__ float4 s_q[kStageCap + kUnrolled];
   const uint32_t lane = threadIdx.x;
   const uint32_t tile = xcd_tile(blockIdx.x);
   if (tile >= n_tiles) return;
@@ -787,14 +830,16 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
     if (live) {
       id = dw.ids[i];
       dry = dry_cells(cr, g, dw);
-      keep = dry && dw.reuse && dw.dry_pass[id] == dw.pass - 1u;
-      if (dry) dw.dry_pass[id] = dw.pass;
+      keep = dry && (!WALK || (dw.reuse && dw.dry_pass[id] == dw.pass - 1u));
+      if (WALK && dry) dw.dry_pass[id] = dw.pass;
     }
     dry_mask = __ballot(dry);
     if (__ballot(!keep) == 0ull) {
       if (live && dw.zero_masks)
-        for (uint32_t r = 0; r < kRuns; ++r) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
-      if (live) density_keep<F>(i, id, pi, wvel, kc, dw, rp, pres);
+        for (uint32_t r = 0; r < kRuns; ++r)
+        if (WALK || r == sph_run(blockIdx.y)) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
+      if constexpr (WALK)
+        if (live) density_keep<F>(i, id, pi, wvel, kc, dw, rp, pres);
       return;
     }
   }
@@ -827,6 +872,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
 #pragma unroll
     for (uint32_t t = 0; t < G; ++t) {
       if (t >= nrun) break;
+      if (!WALK && G * grp + t != blockIdx.y) continue;
       const uint32_t r = sph_run(G * grp + t);
       const int zz = cr.cz + (int)(r / 3u) - 1, yy = cr.cy + (int)(r % 3u) - 1;
       const bool row_ok = live && zz >= 0 && zz < nz && yy >= 0 && yy < ny;
@@ -882,7 +928,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
       if (len) {
         if (staged) {
           scan_run([&](uint32_t k0, uint32_t cnt) {
-                     return scan_word_dot([&](uint32_t j) { return s_q[j - base]; }, k0, cnt, ax, ay, az, thr);
+                     return scan_word_dot<kUnrolled>([&](uint32_t j) { return s_q[j - base]; }, k0, cnt, ax, ay, az, thr);
                    },
                    j0, len, r, words, n, i, m[2u * t], m[2u * t + 1u]);
         } else {
@@ -894,6 +940,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
       }
       if (staged) __syncthreads();  // the next run's staging overwrites s_q
     }
+    if constexpr (!WALK) continue;
     // the group's words in stream order, each with the slot of its bit 0
     uint32_t wb[2 * G];
 #pragma unroll
@@ -934,7 +981,7 @@ __global__ __launch_bounds__(kDensBlock, kDensWaves<F>) void k_sph_density(
       }
     });
   }
-  if (!live) return;
+  if (!WALK || !live) return;
   if (overflow) atomicOr(&flags[FLAG_CAPACITY], 1u);
   density_store<F>(i, acc, kc, ((dry_mask >> lane) & 1ull) != 0ull, dw, rp, wpos, wvel, pres);
 }
@@ -1173,7 +1220,7 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
     }
   };
   walk_runs_staged<kUnr, kForceCap, kForcePrefetch<F>>(
-      meta, words, n, i, live, lane, begin_group,
+      meta, words, n, i, live, lane, 0u, kGroups, begin_group,
       [&](uint32_t k, uint32_t j) {
         s_p.put(k, gpos[j]);
         s_v.put(k, gvel[j]);
@@ -1279,7 +1326,11 @@ SphStepIO<F> sph_step_io(Ctx& c) {
   io.gvel = (F == kMixed) ? c.vel32.as<G4>() : c.vel[c.cur].as<G4>();
   io.skeys = c.keys[c.cur_key].as<uint32_t>();
   static_assert(kDensBlock == kForceBlock, "both gathers walk the same tiles");
-  io.quad = c.quad && !c.record_all;
+  // a recorded step also stores masks, which the four-lane passes pay more for:
+  // density + masks + force, us, four lanes / one, at 27k, 64k, 125k, 200k moving
+  // particles: FP64 86/138, 120/159, 182/203, 262/244; mixed 107/161, 144/172,
+  // 206/197, 283/234
+  io.quad = c.quad && (!c.record_all || c.n_moving <= (F == kF64 ? 160000u : 100000u));
   io.n_tiles = blocks_for((uint32_t)c.n, io.quad ? (int)kQuadSlots : kDensBlock);
   io.pass = c.dens_pass;
   io.dw = DryWalls{c.ids[c.cur_ids].as<uint32_t>(), c.n_moving, c.movcell.as<uint32_t>(),
@@ -1304,13 +1355,28 @@ void sph_density_launch(Ctx& c, const SphStepIO<F>& io, typename SphForm<F>::R2*
   LaunchScope ls(&c, F == kF64 ? "sph_density_f64" : (F == kF32 ? "sph_density_f32" : "sph_density_mixed"),
                  per * n);
   if (io.quad) {
-    k_sph_density_quad<F><<<tile_grid(io.n_tiles), 64, 0, c.stream>>>(
-        n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys, c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nlist.as<uint32_t>(),
-        c.ncnt.as<uint32_t>(), rp, wpos, wvel, pres, c.flags.as<uint32_t>(), io.n_tiles, io.dw);
+    auto launch = [&](auto kernel) {
+      kernel<<<tile_grid(io.n_tiles), 64, 0, c.stream>>>(
+          n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys, c.lb.as<uint32_t>(), c.grid, c.sph, io.u,
+          c.nlist.as<uint32_t>(), c.ncnt.as<uint32_t>(), c.nmeta.as<uint2>(), c.nword.as<uint32_t>(), rp, wpos, wvel,
+          pres, c.flags.as<uint32_t>(), io.n_tiles, io.dw);
+    };
+    if (F == kF64 && c.record_all) launch(k_sph_density_quad<F, F == kF64>);
+    else launch(k_sph_density_quad<F, false>);
     PR_HIP(hipGetLastError());
+    if (F == kMixed && c.record_all) {
+      // the mixed reverse passes round by how a lane's hits pair up in its
+      // walk, so their masks are the one-lane scan's to the last bit
+      LaunchScope lm(&c, "sph_masks", 0.0);
+      const uint32_t tiles = blocks_for(n, kDensBlock);
+      k_sph_density<F, F != kMixed><<<dim3(tile_grid(tiles), kRuns), kDensBlock, 0, c.stream>>>(
+          n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys, c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nmeta.as<uint2>(),
+          c.nword.as<uint32_t>(), rp, wpos, wvel, pres, c.flags.as<uint32_t>(), tiles, io.dw);
+      PR_HIP(hipGetLastError());
+    }
     return;
   }
-  k_sph_density<F><<<tile_grid(io.n_tiles), kDensBlock, 0, c.stream>>>(n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys,
+  k_sph_density<F, true><<<tile_grid(io.n_tiles), kDensBlock, 0, c.stream>>>(n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys,
                                                       c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nmeta.as<uint2>(),
                                                       c.nword.as<uint32_t>(), rp, wpos, wvel, pres,
                                                       c.flags.as<uint32_t>(), io.n_tiles, io.dw);

@@ -153,17 +153,28 @@ __device__ inline uint2 rows_prefix(uint32_t x, uint32_t lane) {
   return make_uint2(((lane & 16u) ? a[0] : 0u) + ((lane & 32u) ? b[0] : 0u), b[0] + b[1]);
 }
 
+// The four 16-bit words of lanes l, l + 16, l + 32, l + 48 as one, in that order.
+__device__ inline uint64_t rows_gather16(uint32_t x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const uint32_t pair = a[0] | (a[1] << 16);
+  const auto b = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+  return (uint64_t)b[0] | ((uint64_t)b[1] << 32);
+}
+
 // Six wavefronts per SIMD: 500k fluid mixed 245 us a pass; with 32-bit list
 // entries in LDS, which leave room for four, 281.
 template <int F>
 constexpr int kQuadDensWaves = 6;
-template <int F>
+// REC: the step is recorded for the adjoint, so every particle's row masks are
+// stored too, in the layout of k_sph_density (42,866 particles: 27 -> 31 us).
+template <int F, bool REC>
 __global__ __launch_bounds__(64, kQuadDensWaves<F>) void k_sph_density_quad(
     uint32_t n, const typename SphForm<F>::S4* __restrict__ spos, const typename SphForm<F>::G4* pos,
     const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ lb, Grid g, SphConst kc, SphUnits u,
-    uint32_t* __restrict__ nlist, uint32_t* __restrict__ ncnt, typename SphForm<F>::R2* __restrict__ rp,
-    typename SphForm<F>::G4* wpos, typename SphForm<F>::G4* wvel, typename SphForm<F>::real* __restrict__ pres,
-    uint32_t* flags, uint32_t n_tiles, DryWalls dw) {
+    uint32_t* __restrict__ nlist, uint32_t* __restrict__ ncnt, uint2* __restrict__ meta,
+    uint32_t* __restrict__ words, typename SphForm<F>::R2* __restrict__ rp, typename SphForm<F>::G4* wpos,
+    typename SphForm<F>::G4* wvel, typename SphForm<F>::real* __restrict__ pres, uint32_t* flags, uint32_t n_tiles,
+    DryWalls dw) {
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using S4 = typename SphForm<F>::S4;
@@ -187,6 +198,9 @@ __global__ __launch_bounds__(64, kQuadDensWaves<F>) void k_sph_density_quad(
     const bool keep = !live || (dry && dw.reuse && dw.dry_pass[id] == dw.pass - 1u);
     if (dry) dw.dry_pass[id] = dw.pass;
     if (__ballot(!keep) == 0ull) {
+      if constexpr (REC)
+        if (live)
+          for (uint32_t r = sub; r < kRuns; r += 4u) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
       if (live && sub == 0u) density_keep<F>(i, id, pi, wvel, kc, dw, rp, pres);
       return;
     }
@@ -234,6 +248,7 @@ __global__ __launch_bounds__(64, kQuadDensWaves<F>) void k_sph_density_quad(
   for (uint32_t k = 0; k < kRuns; ++k) {
     S4 cand = next;
     if (lane == 0u) s_base[k] = base[k];
+    uint64_t m0 = 0, m1 = 0;   // REC: the run's mask, bit 0 its first candidate
     if (k + 1u < kRuns) next = spos[min(base[k + 1u] + lane, n - 1u)];
     for (uint32_t c = 0; c < span[k]; c += 64u) {
       if (c) cand = spos[min(base[k] + c + lane, n - 1u)];
@@ -242,6 +257,18 @@ __global__ __launch_bounds__(64, kQuadDensWaves<F>) void k_sph_density_quad(
       const uint32_t first = base[k] + c + 16u * h;   // slot of bit 0
       const int lo = max((int)(qr.j0[k] - first), 0), hi = min((int)(qr.j0[k] + qr.len[k] - first), 16);
       word = hi > lo ? word & (((1u << (hi - lo)) - 1u) << lo) : 0u;
+      if constexpr (REC) {
+        const uint64_t all = rows_gather16(word);   // bit b: slot base + c + b
+        const int at = (int)(base[k] + c - qr.j0[k]);   // mask bit of bit 0
+        if (at <= 0) {
+          if (at > -64) m0 |= all >> -at;
+        } else if (at < 64) {
+          m0 |= all << at;
+          m1 |= all >> (64 - at);
+        } else if (at < 128) {
+          m1 |= all << (at - 64);
+        }
+      }
       const uint2 pre = rows_prefix((uint32_t)__popc(word), lane);
       fits = fits && c < 4096u && __ballot(scnt + pre.y > kQuadCap) == 0ull;
       if (fits) {
@@ -254,6 +281,13 @@ __global__ __launch_bounds__(64, kQuadDensWaves<F>) void k_sph_density_quad(
       }
       scnt += pre.y;
     }
+    if constexpr (REC)
+      if (slive) {
+        const uint32_t r = sph_run(k);
+        if (h == 0u) meta[meta_index(r, n, sself)] = make_uint2(qr.j0[k], qr.len[k]);
+        const uint64_t m = h < 2u ? m0 : m1;
+        if (qr.len[k] > 32u * h) words[word_index(r, h, n, sself)] = (uint32_t)((h & 1u) ? m >> 32 : m);
+      }
   }
   __builtin_amdgcn_wave_barrier();
   const uint32_t cnt = __shfl(scnt, (int)p, 64);

@@ -96,3 +96,22 @@ def test_lists_that_do_not_fit(scene, monkeypatch):
     for precision in (pa.F32, pa.MIXED):
         d.precision = precision
         _same(_run(d, arrs, 2, "on", monkeypatch), _run(d, arrs, 2, "off", monkeypatch))
+
+
+@pytest.mark.parametrize("precision", [pa.F64, pa.MIXED])
+@pytest.mark.parametrize("n_target", [27, 8000])
+def test_adjoint_same_bits(n_target, precision, monkeypatch):
+    """Steps recorded by the four-lane passes and reverse passes split over a block's wavefronts give the
+    gradients of the one-lane, one-wavefront passes bit for bit."""
+    d, arrs = _stirred(n_target, precision)
+    rng = np.random.default_rng(2)
+    seeds = [rng.standard_normal((3, d.n_particles)) for _ in range(2)]
+    out = {}
+    for mode in ("on", "off"):
+        monkeypatch.setenv("PRESTIGE_QUAD", mode)
+        with pa.Context(d) as ctx:
+            upload_all(ctx, arrs)
+            ctx.forward_tape(14, 4)
+            out[mode] = ctx.adjoint(*seeds)
+    assert np.array_equal(out["on"][0], out["off"][0])
+    assert np.array_equal(out["on"][1], out["off"][1])
