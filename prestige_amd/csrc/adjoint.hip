@@ -6,13 +6,47 @@
 
 namespace prestige {
 
-static void copy_dev(Ctx& c, DevBuf& dst, const DevBuf& src, size_t bytes) {
-  dst.alloc(bytes ? bytes : 1);
-  if (bytes) PR_HIP(hipMemcpyAsync(dst.p, src.p, bytes, hipMemcpyDeviceToDevice, c.stream));
+// Up to kCopies device buffers in one launch, block column y copying the y-th
+// (a checkpoint is up to nine buffers, which a small context copies in less
+// time than their launches take).
+constexpr int kCopies = 9;
+struct CopyList {
+  const uint4* src[kCopies];
+  uint4* dst[kCopies];
+  size_t bytes[kCopies];
+};
+__global__ __launch_bounds__(kBlock) void k_copy_many(CopyList l) {
+  const uint4* src = l.src[blockIdx.y];
+  uint4* dst = l.dst[blockIdx.y];
+  const size_t bytes = l.bytes[blockIdx.y], n = bytes / 16;
+  const size_t stride = (size_t)gridDim.x * kBlock, t = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  for (size_t k = t; k < n; k += stride) dst[k] = src[k];
+  const size_t done = n * 4, words = bytes / 4;   // the last words
+  if (t < words - done)
+    reinterpret_cast<uint32_t*>(dst)[done + t] = reinterpret_cast<const uint32_t*>(src)[done + t];
 }
 
-static void copy_back(Ctx& c, DevBuf& dst, const DevBuf& src, size_t bytes) {
-  if (bytes) PR_HIP(hipMemcpyAsync(dst.p, src.p, bytes, hipMemcpyDeviceToDevice, c.stream));
+static void launch_copies(Ctx& c, const std::vector<Copy>& list) {
+  CopyList l{};
+  size_t most = 0;
+  int k = 0;
+  for (const Copy& p : list) {
+    if (!p.bytes) continue;
+    PR_CHECK(k < kCopies && p.bytes % 4 == 0, PRESTIGE_E_INVALID, "copy list");
+    l.src[k] = p.src->as<uint4>();
+    l.dst[k] = p.dst->as<uint4>();
+    l.bytes[k++] = p.bytes;
+    most = std::max(most, p.bytes);
+  }
+  if (!k) return;
+  const uint32_t blocks = (uint32_t)std::min<size_t>(2048, most / (16 * kBlock) + 1);
+  k_copy_many<<<dim3(blocks, (uint32_t)k), kBlock, 0, c.stream>>>(l);
+  PR_HIP(hipGetLastError());
+}
+
+void copy_many(Ctx& c, const std::vector<Copy>& list) {
+  for (const Copy& p : list) p.dst->alloc(p.bytes ? p.bytes : 1);
+  launch_copies(c, list);
 }
 
 static size_t elem4(const Ctx& c) { return c.desc.precision == PRESTIGE_F32 ? sizeof(float4) : sizeof(double4); }
@@ -21,38 +55,40 @@ void snapshot_state(Ctx& c, Snapshot& s) {
   const size_t n = c.n, e4 = elem4(c);
   s.cur = c.cur; s.cur_ids = c.cur_ids; s.cur_key = c.cur_key; s.cur_hist = c.cur_hist;
   s.sorted = c.sorted; s.keys_valid = c.keys_valid; s.built = c.built;
-  copy_dev(c, s.pos, c.pos[c.cur], n * e4);
-  copy_dev(c, s.vel, c.vel[c.cur], n * e4);
-  copy_dev(c, s.ids, c.ids[c.cur_ids], n * 4);
-  copy_dev(c, s.keys, c.keys[c.cur_key], n * 4);
+  std::vector<Copy> l{{&s.pos, &c.pos[c.cur], n * e4},
+                      {&s.vel, &c.vel[c.cur], n * e4},
+                      {&s.ids, &c.ids[c.cur_ids], n * 4},
+                      {&s.keys, &c.keys[c.cur_key], n * 4}};
   if (c.desc.model == PRESTIGE_MODEL_DEM) {
     const size_t mc = c.desc.max_contacts, hr = c.desc.precision == PRESTIGE_MIXED ? 4 : 8;
-    copy_dev(c, s.omega, c.omega[c.cur], n * e4);
-    copy_dev(c, s.hcnt, c.hcnt[c.cur_hist], n * 4);
-    copy_dev(c, s.hid, c.hid[c.cur_hist], n * mc * 4);
-    copy_dev(c, s.hxi, c.hxi[c.cur_hist], n * mc * 3 * hr);
-    copy_dev(c, s.wxi, c.wxi[c.cur_hist], n * 18 * hr);
+    l.insert(l.end(), {{&s.omega, &c.omega[c.cur], n * e4},
+                       {&s.hcnt, &c.hcnt[c.cur_hist], n * 4},
+                       {&s.hid, &c.hid[c.cur_hist], n * mc * 4},
+                       {&s.hxi, &c.hxi[c.cur_hist], n * mc * 3 * hr},
+                       {&s.wxi, &c.wxi[c.cur_hist], n * 18 * hr}});
   }
+  copy_many(c, l);
 }
 
-void restore_state(Ctx& c, const Snapshot& s) {
+void restore_state(Ctx& c, Snapshot& s) {
   const size_t n = c.n, e4 = elem4(c);
   c.cur = s.cur; c.cur_ids = s.cur_ids; c.cur_key = s.cur_key; c.cur_hist = s.cur_hist;
   c.sorted = s.sorted; c.keys_valid = s.keys_valid; c.built = s.built;
   c.inc_ready = false;   // the previous build's keys and cell table are not restored
   c.forget_dry();
-  copy_back(c, c.pos[c.cur], s.pos, n * e4);
-  copy_back(c, c.vel[c.cur], s.vel, n * e4);
-  copy_back(c, c.ids[c.cur_ids], s.ids, n * 4);
-  copy_back(c, c.keys[c.cur_key], s.keys, n * 4);
+  std::vector<Copy> l{{&c.pos[c.cur], &s.pos, n * e4},
+                      {&c.vel[c.cur], &s.vel, n * e4},
+                      {&c.ids[c.cur_ids], &s.ids, n * 4},
+                      {&c.keys[c.cur_key], &s.keys, n * 4}};
   if (c.desc.model == PRESTIGE_MODEL_DEM) {
     const size_t mc = c.desc.max_contacts, hr = c.desc.precision == PRESTIGE_MIXED ? 4 : 8;
-    copy_back(c, c.omega[c.cur], s.omega, n * e4);
-    copy_back(c, c.hcnt[c.cur_hist], s.hcnt, n * 4);
-    copy_back(c, c.hid[c.cur_hist], s.hid, n * mc * 4);
-    copy_back(c, c.hxi[c.cur_hist], s.hxi, n * mc * 3 * hr);
-    copy_back(c, c.wxi[c.cur_hist], s.wxi, n * 18 * hr);
+    l.insert(l.end(), {{&c.omega[c.cur], &s.omega, n * e4},
+                       {&c.hcnt[c.cur_hist], &s.hcnt, n * 4},
+                       {&c.hid[c.cur_hist], &s.hid, n * mc * 4},
+                       {&c.hxi[c.cur_hist], &s.hxi, n * mc * 3 * hr},
+                       {&c.wxi[c.cur_hist], &s.wxi, n * 18 * hr}});
   }
+  launch_copies(c, l);
 }
 
 __global__ void k_seed_gather(uint32_t n, const uint32_t* __restrict__ ids, const double* __restrict__ sx,
@@ -76,12 +112,11 @@ __global__ void k_grad_scatter(uint32_t n, uint64_t n_moving, const uint32_t* __
   out[2 * (size_t)n + id] = mv ? v.z : 0.0;
 }
 
-void ensure_adj_buffers(Ctx& c, uint32_t grid_blocks) {
+void ensure_adj_buffers(Ctx& c) {
   Tape& T = c.tape;
   const size_t n = c.n ? c.n : 1;
   for (DevBuf* b : {&T.xb, &T.vb, &T.xb2, &T.vb2, &T.cvec, &T.xbf, &T.wb, &T.wb2}) b->alloc(n * sizeof(double4));
   T.rhob.alloc(n * sizeof(double));
-  T.partial.alloc((size_t)grid_blocks * sizeof(double2) + 64);
   T.acc.alloc(8 * sizeof(double));
   T.seeds.alloc(6 * n * sizeof(double));
 }

@@ -170,11 +170,20 @@ __device__ inline RowBar row_vjp(bool wall, V3 d, V3 nwall, double delta_wall, V
   return b;
 }
 
-template <class H>
+// Index of partner among the owner's cnt contacts (-1: none), eight ids read
+// at a time.
 __device__ inline int find_slot(const uint32_t* __restrict__ hid, uint32_t cnt, uint32_t n, uint32_t owner,
                                 uint32_t partner) {
-  for (uint32_t c = 0; c < cnt; ++c)
-    if (hid[(size_t)c * n + owner] == partner) return (int)c;
+  for (uint32_t c0 = 0; c0 < cnt; c0 += 8u) {
+    uint32_t id[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8u; ++u) id[u] = hid[(size_t)(c0 + u < cnt ? c0 + u : c0) * n + owner];
+    int at = -1;
+#pragma unroll
+    for (uint32_t u = 8u; u-- > 0u;)
+      if (c0 + u < cnt && id[u] == partner) at = (int)(c0 + u);
+    if (at >= 0) return at;
+  }
   return -1;
 }
 
@@ -204,22 +213,19 @@ struct DemStepView {
   const uint32_t *cnt_out, *hid_out;   // contacts the step found (its frozen list)
 };
 
-static __global__ __launch_bounds__(kBlock) void k_dem_slot_of(uint32_t n, const uint32_t* __restrict__ ids,
-                                                                uint32_t* __restrict__ slot_of) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) slot_of[ids[k]] = k;
-}
-
-// vbt = vbar' + dt xbar', Fbar = dt vbt / m, Tbar = dt wbar' / I.
+// vbt = vbar' + dt xbar', Fbar = dt vbt / m, Tbar = dt wbar' / I; and the slot of
+// each id.
 static __global__ __launch_bounds__(kBlock) void k_dem_adj_prep(uint32_t n, uint64_t n_moving, DemStepView s,
                                                                  const double4* __restrict__ xb,
                                                                  double4* __restrict__ vb,
                                                                  const double4* __restrict__ wb,
                                                                  double4* __restrict__ Fb, double4* __restrict__ Tb,
-                                                                 double dt) {
+                                                                 double dt, uint32_t* __restrict__ slot_of) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  if ((uint64_t)s.ids[k] >= n_moving) {
+  const uint32_t id = s.ids[k];
+  slot_of[id] = k;
+  if ((uint64_t)id >= n_moving) {
     vb[k] = make_double4(0, 0, 0, 0);
     Fb[k] = make_double4(0, 0, 0, 0);
     Tb[k] = make_double4(0, 0, 0, 0);
@@ -235,160 +241,180 @@ static __global__ __launch_bounds__(kBlock) void k_dem_adj_prep(uint32_t n, uint
   Tb[k] = make_double4(ti * w.x, ti * w.y, ti * w.z, 0.0);
 }
 
-__device__ inline void block_sum3(double a, double b, double c, double4* __restrict__ partial) {
-  __shared__ double s[3][kBlock / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_down(a, (unsigned)o, 64);
-    b += __shfl_down(b, (unsigned)o, 64);
-    c += __shfl_down(c, (unsigned)o, 64);
-  }
-  const uint32_t w = threadIdx.x >> 6;
-  if (__lane_id() == 0) {
-    s[0][w] = a;
-    s[1][w] = b;
-    s[2][w] = c;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t0 = 0, t1 = 0, t2 = 0;
-    for (uint32_t q = 0; q < kBlock / 64; ++q) {
-      t0 += s[0][q];
-      t1 += s[1][q];
-      t2 += s[2][q];
-    }
-    partial[blockIdx.x] = make_double4(t0, t1, t2, 0.0);
-  }
-}
-
-// Contact adjoint + integrator assembly for one reverse step.
+// Contact adjoint + integrator assembly for one reverse step, four lanes per
+// particle (a quad): each lane takes one of the particle's contacts at a time,
+// the quad's sums are added in lane order.  A contact is two row products of
+// some 200 FP64 operations behind a chain of reads (partner id, its slot, its
+// state, three searches); with one lane per particle 20,000 spheres were 313
+// wavefronts that ran their contacts in turn: 40 us, 18 with quads.
 template <class H>
-__global__ __launch_bounds__(kBlock) void k_dem_adj(uint32_t n, uint64_t n_moving, DemStepView s, DemAdjConst kc,
-                                                    const double4* __restrict__ xb_in,
-                                                    const double4* __restrict__ vb_in,
-                                                    const double4* __restrict__ wb_in,
-                                                    const double4* __restrict__ Fb, const double4* __restrict__ Tb,
-                                                    const double* __restrict__ hb_next,
-                                                    const double* __restrict__ wallb_next,
-                                                    double* __restrict__ hb_prev, double* __restrict__ wallb_prev,
-                                                    double4* __restrict__ xb_out, double4* __restrict__ vb_out,
-                                                    double4* __restrict__ wb_out, double4* __restrict__ partial) {
+__global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, DemStepView s, DemAdjConst kc,
+                                                const double4* __restrict__ xb_in,
+                                                const double4* __restrict__ vb_in,
+                                                const double4* __restrict__ wb_in,
+                                                const double4* __restrict__ Fb, const double4* __restrict__ Tb,
+                                                const double* __restrict__ hb_next,
+                                                const double* __restrict__ wallb_next,
+                                                double* __restrict__ hb_prev, double* __restrict__ wallb_prev,
+                                                double4* __restrict__ xb_out, double4* __restrict__ vb_out,
+                                                double4* __restrict__ wb_out, double4* __restrict__ partial,
+                                                uint32_t n_tiles) {
+  __shared__ uint32_t s_had[kQuadSlots];   // history slots a contact of the step continues
+  const uint32_t tile = xcd_tile(blockIdx.x);
+  if (tile >= n_tiles) return;
   const H* xi_in = (const H*)s.xi_in;
   const H* wxi_in = (const H*)s.wxi_in;
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = threadIdx.x, sub = lane & 3u, p = lane >> 2;
+  const uint32_t k = tile * kQuadSlots + p;
+  const bool in = k < n;
+  const uint32_t self = in ? k : tile * kQuadSlots;
+  const uint32_t me = s.ids[self], dst = s.perm[self];
+  const bool live = in && (uint64_t)me < n_moving;
+  const uint32_t cin = in ? s.cnt_in[me] : 0u, cout = live ? s.cnt_out[me] : 0u;
   double pk = 0.0, pt = 0.0, pm = 0.0;
-  if (k < n) {
-    const uint32_t me = s.ids[k];
-    const uint32_t dst = s.perm[k];
-    const uint32_t cin = s.cnt_in[me];
-    for (uint32_t c = 0; c < cin; ++c) store3(hb_prev, c, n, me, v3(0, 0, 0));
-    if ((uint64_t)me >= n_moving) {
-      for (int w = 0; w < 6; ++w) store3(wallb_prev, (uint32_t)w, n, me, v3(0, 0, 0));
-      xb_out[dst] = make_double4(0, 0, 0, 0);
-      vb_out[dst] = make_double4(0, 0, 0, 0);
-      wb_out[dst] = make_double4(0, 0, 0, 0);
-    } else {
-      const double4 pk4 = s.pos[k], vk4 = s.vel[k], wk4 = s.om[k];
-      const V3 xk = xyz(pk4), vk = xyz(vk4), wk = xyz(wk4);
-      const double rk = pk4.w, mk = vk4.w;
-      const V3 Fbk = xyz(Fb[k]), Tbk = xyz(Tb[k]);
-      V3 X = v3(0, 0, 0), V = v3(0, 0, 0), W = v3(0, 0, 0);
-      const uint32_t cout = s.cnt_out[me];
-      for (uint32_t c = 0; c < cout; ++c) {
-        const uint32_t pid = s.hid_out[(size_t)c * n + me];
-        const uint32_t j = s.slot_of[pid];
-        const double4 pj4 = s.pos[j], vj4 = s.vel[j], wj4 = s.om[j];
-        const V3 xj = xyz(pj4), vj = xyz(vj4), wj = xyz(wj4);
-        const double rj = pj4.w, mj = vj4.w;
-        // own row (k, j)
-        const int ci = find_slot<H>(s.hid_in, cin, n, me, pid);
-        const V3 xo = ci >= 0 ? load_xi(xi_in, (uint32_t)ci, n, me) : v3(0, 0, 0);
-        const V3 xnb = load3(hb_next, c, n, me);
-        RowBar a = row_vjp(false, xk - xj, v3(0, 0, 0), 0.0, vk, vj, wk, wj, rk, rj, mk, mj, xo, Fbk, Tbk, xnb, kc);
-        X = X + a.d;
-        V = V + a.vi;
-        W = W + a.wi;
-        if (ci >= 0) store3(hb_prev, (uint32_t)ci, n, me, a.xo);
-        pk += a.kn;
-        pt += a.tz;
-        pm += a.mu;
-        // partner row (j, k): keep the terms of k
-        const uint32_t cjin = s.cnt_in[pid], cjout = s.cnt_out[pid];
-        const int cj = find_slot<H>(s.hid_in, cjin, n, pid, me);
-        const V3 xoj = cj >= 0 ? load_xi(xi_in, (uint32_t)cj, n, pid) : v3(0, 0, 0);
-        const int co = find_slot<H>(s.hid_out, cjout, n, pid, me);
-        const V3 xnbj = co >= 0 ? load3(hb_next, (uint32_t)co, n, pid) : v3(0, 0, 0);
-        const bool jm = (uint64_t)pid < n_moving;
-        const V3 Fbj = jm ? xyz(Fb[j]) : v3(0, 0, 0), Tbj = jm ? xyz(Tb[j]) : v3(0, 0, 0);
-        RowBar b = row_vjp(false, xj - xk, v3(0, 0, 0), 0.0, vj, vk, wj, wk, rj, rk, mj, mk, xoj, Fbj, Tbj, xnbj, kc);
-        X = X - b.d;
-        V = V + b.vj;
-        W = W + b.wj;
+  V3 X = v3(0, 0, 0), V = v3(0, 0, 0), W = v3(0, 0, 0);
+  if (sub == 0u) s_had[p] = 0u;
+  wave_lds_fence();
+  const double4 pk4 = s.pos[self], vk4 = s.vel[self], wk4 = s.om[self];
+  const V3 xk = xyz(pk4), vk = xyz(vk4), wk = xyz(wk4);
+  const double rk = pk4.w, mk = vk4.w;
+  const V3 Fbk = xyz(Fb[self]), Tbk = xyz(Tb[self]);
+  for (uint32_t c = sub; c < cout; c += 4u) {
+    const uint32_t pid = s.hid_out[(size_t)c * n + me];
+    const uint32_t j = s.slot_of[pid];
+    const uint32_t cjin = s.cnt_in[pid], cjout = s.cnt_out[pid];
+    const double4 pj4 = s.pos[j], vj4 = s.vel[j], wj4 = s.om[j];
+    const bool jm = (uint64_t)pid < n_moving;
+    const V3 Fbj = jm ? xyz(Fb[j]) : v3(0, 0, 0), Tbj = jm ? xyz(Tb[j]) : v3(0, 0, 0);
+    const V3 xj = xyz(pj4), vj = xyz(vj4), wj = xyz(wj4);
+    const double rj = pj4.w, mj = vj4.w;
+    const int ci = find_slot(s.hid_in, cin, n, me, pid);
+    const int cj = find_slot(s.hid_in, cjin, n, pid, me);
+    const int co = find_slot(s.hid_out, cjout, n, pid, me);
+    // own row (k, j)
+    const V3 xo = ci >= 0 ? load_xi(xi_in, (uint32_t)ci, n, me) : v3(0, 0, 0);
+    const V3 xnb = load3(hb_next, c, n, me);
+    const RowBar a = row_vjp(false, xk - xj, v3(0, 0, 0), 0.0, vk, vj, wk, wj, rk, rj, mk, mj, xo, Fbk, Tbk, xnb, kc);
+    X = X + a.d;
+    V = V + a.vi;
+    W = W + a.wi;
+    if (ci >= 0) {
+      store3(hb_prev, (uint32_t)ci, n, me, a.xo);
+      atomicOr(&s_had[p], 1u << ci);   // max_contacts <= 32
+    }
+    pk += a.kn;
+    pt += a.tz;
+    pm += a.mu;
+    // partner row (j, k): keep the terms of k
+    const V3 xoj = cj >= 0 ? load_xi(xi_in, (uint32_t)cj, n, pid) : v3(0, 0, 0);
+    const V3 xnbj = co >= 0 ? load3(hb_next, (uint32_t)co, n, pid) : v3(0, 0, 0);
+    const RowBar b = row_vjp(false, xj - xk, v3(0, 0, 0), 0.0, vj, vk, wj, wk, rj, rk, mj, mk, xoj, Fbj, Tbj, xnbj, kc);
+    X = X - b.d;
+    V = V + b.vj;
+    W = W + b.wj;
+  }
+  wave_lds_fence();
+  // history slots no contact continues get zero adjoints
+  const uint32_t had = s_had[p];
+  for (uint32_t c = sub; c < cin; c += 4u)
+    if (!((had >> c) & 1u)) store3(hb_prev, c, n, me, v3(0, 0, 0));
+  // the quad's sums, in lane order, in all its lanes
+  auto quad_sum = [](double v) {
+    return ((quad_bcast<0>(v) + quad_bcast<1>(v)) + quad_bcast<2>(v)) + quad_bcast<3>(v);
+  };
+  auto quad_sum3 = [&](V3 v) { return v3(quad_sum(v.x), quad_sum(v.y), quad_sum(v.z)); };
+  X = quad_sum3(X);
+  V = quad_sum3(V);
+  W = quad_sum3(W);
+  if (in) {
+    // walls: the quad's lanes compute the same, each stores its share
+    for (int w = 0; w < 6; ++w) {
+      bool on = false;
+      double delta = 0.0;
+      V3 nw = v3(0, 0, 0);
+      if (live && (kc.wall_mask & (1u << w))) {
+        const int ax = w >> 1;
+        const double pa = ax == 0 ? xk.x : (ax == 1 ? xk.y : xk.z);
+        const double dist = (w & 1) ? (kc.wall_hi[ax] - pa) : (pa - kc.wall_lo[ax]);
+        delta = rk - dist;
+        on = delta > 0.0;
+        const double sgn = (w & 1) ? -1.0 : 1.0;
+        nw = v3(ax == 0 ? sgn : 0.0, ax == 1 ? sgn : 0.0, ax == 2 ? sgn : 0.0);
       }
-      // walls
-      for (int w = 0; w < 6; ++w) {
-        bool on = false;
-        double delta = 0.0;
-        V3 nw = v3(0, 0, 0);
-        if (kc.wall_mask & (1u << w)) {
-          const int ax = w >> 1;
-          const double pa = ax == 0 ? xk.x : (ax == 1 ? xk.y : xk.z);
-          const double dist = (w & 1) ? (kc.wall_hi[ax] - pa) : (pa - kc.wall_lo[ax]);
-          delta = rk - dist;
-          on = delta > 0.0;
-          const double sgn = (w & 1) ? -1.0 : 1.0;
-          nw = v3(ax == 0 ? sgn : 0.0, ax == 1 ? sgn : 0.0, ax == 2 ? sgn : 0.0);
-        }
-        if (!on) {
-          store3(wallb_prev, (uint32_t)w, n, me, v3(0, 0, 0));
-          continue;
-        }
+      V3 xob = v3(0, 0, 0);
+      if (on) {
         const V3 xo = load_xi(wxi_in, (uint32_t)w, n, me);
         const V3 xnb = load3(wallb_next, (uint32_t)w, n, me);
-        RowBar a = row_vjp(true, v3(0, 0, 0), nw, delta, vk, v3(0, 0, 0), wk, v3(0, 0, 0), rk, 0.0, mk, 0.0, xo,
-                           Fbk, Tbk, xnb, kc);
+        const RowBar a = row_vjp(true, v3(0, 0, 0), nw, delta, vk, v3(0, 0, 0), wk, v3(0, 0, 0), rk, 0.0, mk, 0.0, xo,
+                                 Fbk, Tbk, xnb, kc);
         X = X + a.d;
         V = V + a.vi;
         W = W + a.wi;
-        store3(wallb_prev, (uint32_t)w, n, me, a.xo);
-        pk += a.kn;
-        pt += a.tz;
-        pm += a.mu;
+        xob = a.xo;
+        if (sub == 0u) {
+          pk += a.kn;
+          pt += a.tz;
+          pm += a.mu;
+        }
       }
-      const double4 x0 = xb_in[k], v0 = vb_in[k], w0 = wb_in[k];
-      xb_out[dst] = make_double4(x0.x + X.x, x0.y + X.y, x0.z + X.z, 0.0);
-      vb_out[dst] = make_double4(v0.x + V.x, v0.y + V.y, v0.z + V.z, 0.0);
-      wb_out[dst] = make_double4(w0.x + W.x, w0.y + W.y, w0.z + W.z, 0.0);
+      if ((uint32_t)(w & 3) == sub) store3(wallb_prev, (uint32_t)w, n, me, xob);
+    }
+    const V3 z = v3(0, 0, 0);
+    if (sub < 3u) {
+      const double4* from = sub == 0u ? xb_in : (sub == 1u ? vb_in : wb_in);
+      double4* to = sub == 0u ? xb_out : (sub == 1u ? vb_out : wb_out);
+      const V3 d = sub == 0u ? X : (sub == 1u ? V : W);
+      const double4 v0 = from[k];
+      const V3 r = live ? v3(v0.x + d.x, v0.y + d.y, v0.z + d.z) : z;
+      to[dst] = make_double4(r.x, r.y, r.z, 0.0);
     }
   }
-  block_sum3(pk, pt * kc.dtz_de, pm, partial);
+  pt *= kc.dtz_de;
+  for (int o = 32; o > 0; o >>= 1) {
+    pk += __shfl_down(pk, (unsigned)o, 64);
+    pt += __shfl_down(pt, (unsigned)o, 64);
+    pm += __shfl_down(pm, (unsigned)o, 64);
+  }
+  if (lane == 0u) partial[tile] = make_double4(pk, pt, pm, 0.0);
 }
 
-static __global__ void k_dem_adj_reduce(uint32_t nparts, const double4* __restrict__ partial,
-                                        double* __restrict__ acc) {
+// Parameter sums of one reverse step per block (its partials lie nparts apart
+// per step), in a fixed order, into its first partial.
+static __global__ void k_dem_adj_reduce(uint32_t nparts, double4* __restrict__ partial) {
   __shared__ double s[3][256];
+  double4* part = partial + (size_t)blockIdx.x * nparts;
   double a = 0.0, b = 0.0, c = 0.0;
   for (uint32_t q = threadIdx.x; q < nparts; q += blockDim.x) {
-    a += partial[q].x;
-    b += partial[q].y;
-    c += partial[q].z;
+    const double4 v = part[q];
+    a += v.x;
+    b += v.y;
+    c += v.z;
   }
   s[0][threadIdx.x] = a;
   s[1][threadIdx.x] = b;
   s[2][threadIdx.x] = c;
   __syncthreads();
   for (uint32_t st = blockDim.x / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      s[0][threadIdx.x] += s[0][threadIdx.x + st];
-      s[1][threadIdx.x] += s[1][threadIdx.x + st];
-      s[2][threadIdx.x] += s[2][threadIdx.x + st];
-    }
+    if (threadIdx.x < st)
+      for (int k = 0; k < 3; ++k) s[k][threadIdx.x] += s[k][threadIdx.x + st];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    acc[0] += s[0][0];
-    acc[1] += s[1][0];
-    acc[2] += s[2][0];
+  if (threadIdx.x == 0) part[0] = make_double4(s[0][0], s[1][0], s[2][0], 0.0);
+}
+
+// acc[0..2] += the sums of `steps` reverse steps, step by step.
+static __global__ void k_dem_adj_acc(uint32_t nparts, uint32_t steps, const double4* __restrict__ partial,
+                                     double* __restrict__ acc) {
+  double a = acc[0], b = acc[1], c = acc[2];
+  for (uint32_t t = 0; t < steps; ++t) {
+    const double4 v = partial[(size_t)t * nparts];
+    a += v.x;
+    b += v.y;
+    c += v.z;
   }
+  acc[0] = a;
+  acc[1] = b;
+  acc[2] = c;
 }
 
 }  // namespace prestige
@@ -396,24 +422,23 @@ static __global__ void k_dem_adj_reduce(uint32_t nparts, const double4* __restri
 namespace prestige {
 
 void snapshot_state(Ctx& c, Snapshot& s);
-void restore_state(Ctx& c, const Snapshot& s);
+void restore_state(Ctx& c, Snapshot& s);
+void copy_many(Ctx& c, const std::vector<Copy>& list);
 void adj_seed_gather(Ctx& c, const uint32_t* ids, const double* seed_x, const double* seed_v);
 void adj_grad_scatter(Ctx& c, const uint32_t* ids, const double4* vb, double* grad_v0_host);
-void ensure_adj_buffers(Ctx& c, uint32_t grid_blocks);
+void ensure_adj_buffers(Ctx& c);
 
-// Keep what the reverse sweep needs from the step that just ran.  Taken by
-// swap (the next step overwrites them before reading): the sorted pre-step
-// state, the permutation and the contact history the step read.  Copied:
-// ids (the next reorder reads them) and the history the step wrote (the next
-// step's input).
+// Keep what the reverse sweep needs from step t of a segment, which just ran,
+// in rec[t].  Taken by swap (the next step overwrites them before reading): the
+// sorted pre-step state, the permutation, the contact history the step read and
+// the previous step's ids, whose order this step's build left.  The history a
+// step writes is the one the next step reads, so rec[t + 1] holds step t's
+// contacts; the segment's last step copies both.
 template <class H>
-void record_dem_step(Ctx& c, StepRecord& r) {
+void record_dem_step(Ctx& c, Tape& T, uint32_t t, bool last) {
+  StepRecord& r = *T.rec[t];
   const size_t n = c.n ? c.n : 1, mc = c.desc.max_contacts;
   const int prev = c.cur ^ 1, hin = c.cur_hist ^ 1, hout = c.cur_hist;
-  auto cp = [&](DevBuf& d, const DevBuf& s, size_t b) {
-    d.alloc(b);
-    PR_HIP(hipMemcpyAsync(d.p, s.p, b, hipMemcpyDeviceToDevice, c.stream));
-  };
   take_buffer(c.pos[prev], r.state_pos);
   take_buffer(c.vel[prev], r.state_vel);
   take_buffer(c.omega[prev], r.state_om);
@@ -422,9 +447,10 @@ void record_dem_step(Ctx& c, StepRecord& r) {
   take_buffer(c.hid[hin], r.hid);
   take_buffer(c.hxi[hin], r.hxi);
   take_buffer(c.wxi[hin], r.wxi);
-  cp(r.ids, c.ids[c.cur_ids], n * 4);
-  cp(r.hcnt_out, c.hcnt[hout], n * 4);
-  cp(r.hid_out, c.hid[hout], n * mc * 4);
+  if (t > 0) take_buffer(c.ids[c.cur_ids ^ 1], T.rec[t - 1]->ids);
+  if (!last) return;
+  copy_many(c, {{&r.ids, &c.ids[c.cur_ids], n * 4}, {&r.hcnt_out, &c.hcnt[hout], n * 4},
+                {&r.hid_out, &c.hid[hout], n * mc * 4}});
 }
 
 inline DemAdjConst dem_adj_const(const Ctx& c) {
@@ -463,7 +489,7 @@ void dem_tape_forward(Ctx& c, uint32_t nsteps, uint32_t every) {
       snapshot_state(c, T.next_ckpt());
     }
     dem_step_impl<F>(c);
-    if (s >= last0) record_dem_step<H>(c, *T.rec[s - last0]);
+    if (s >= last0) record_dem_step<H>(c, T, s - last0, s + 1 == nsteps);
   }
   T.last_recorded = nsteps > 0;
   if (!c.tape.final_state) c.tape.final_state.reset(new Snapshot());
@@ -477,9 +503,9 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
   Tape& T = c.tape;
   const uint32_t n = (uint32_t)c.n;
   const size_t nn = n ? n : 1, mc = c.desc.max_contacts;
-  const uint32_t nb = blocks_for(n);
-  ensure_adj_buffers(c, nb);
-  T.partial.alloc((size_t)nb * sizeof(double4) + 64);
+  const uint32_t nb = blocks_for(n), tiles = blocks_for(n, (int)kQuadSlots);
+  ensure_adj_buffers(c);
+  T.partial.alloc((size_t)tiles * std::min(T.every, T.nsteps) * sizeof(double4) + 64);
   T.hb[0].alloc(nn * mc * 3 * sizeof(double));
   T.hb[1].alloc(nn * mc * 3 * sizeof(double));
   T.wallb[0].alloc(nn * 18 * sizeof(double));
@@ -504,7 +530,7 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       restore_state(c, *T.ckpt[seg]);
       for (uint32_t t = 0; t < len; ++t) {
         dem_step_impl<F>(c);
-        record_dem_step<H>(c, *T.rec[t]);
+        record_dem_step<H>(c, T, t, t + 1 == len);
       }
     }
     T.last_recorded = false;   // records are overwritten by the recompute of earlier segments
@@ -513,22 +539,27 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       DemStepView v{r.state_pos.as<double4>(), r.state_vel.as<double4>(), r.state_om.as<double4>(),
                     r.ids.as<uint32_t>(), r.perm.as<uint32_t>(), T.slot_of.as<uint32_t>(),
                     r.hcnt.as<uint32_t>(), r.hid.as<uint32_t>(), r.hxi.p, r.wxi.p,
-                    r.hcnt_out.as<uint32_t>(), r.hid_out.as<uint32_t>()};
+                    (t + 1 == len ? r.hcnt_out : T.rec[t + 1]->hcnt).as<uint32_t>(),
+                    (t + 1 == len ? r.hid_out : T.rec[t + 1]->hid).as<uint32_t>()};
       if (!n) continue;
       LaunchScope ls(&c, F == kF64 ? "dem_adjoint_f64" : "dem_adjoint_mixed", 0.0);
-      k_dem_slot_of<<<nb, kBlock, 0, c.stream>>>(n, v.ids, T.slot_of.as<uint32_t>());
       k_dem_adj_prep<<<nb, kBlock, 0, c.stream>>>(n, c.n_moving, v, xb, vb, wb, T.cvec.as<double4>(),
-                                                  T.xbf.as<double4>(), c.dem.dt);
-      k_dem_adj<H><<<nb, kBlock, 0, c.stream>>>(n, c.n_moving, v, kc, xb, vb, wb, T.cvec.as<double4>(),
-                                                T.xbf.as<double4>(), hn, wn, hp, wp, xb2, vb2, wb2,
-                                                T.partial.as<double4>());
-      k_dem_adj_reduce<<<1, 256, 0, c.stream>>>(nb, T.partial.as<double4>(), T.acc.as<double>());
+                                                  T.xbf.as<double4>(), c.dem.dt, T.slot_of.as<uint32_t>());
+      k_dem_adj<H><<<tile_grid(tiles), 64, 0, c.stream>>>(
+          n, c.n_moving, v, kc, xb, vb, wb, T.cvec.as<double4>(), T.xbf.as<double4>(), hn, wn, hp, wp, xb2, vb2, wb2,
+          T.partial.as<double4>() + (size_t)tiles * (len - 1u - t), tiles);
       PR_HIP(hipGetLastError());
       std::swap(xb, xb2);
       std::swap(vb, vb2);
       std::swap(wb, wb2);
       std::swap(hn, hp);
       std::swap(wn, wp);
+    }
+    if (n) {   // the segment's parameter sums
+      k_dem_adj_reduce<<<len, 256, 0, c.stream>>>(tiles, T.partial.as<double4>());
+      PR_HIP(hipGetLastError());
+      k_dem_adj_acc<<<1, 1, 0, c.stream>>>(tiles, len, T.partial.as<double4>(), T.acc.as<double>());
+      PR_HIP(hipGetLastError());
     }
   }
   if (grad_params) {

@@ -75,8 +75,20 @@ __device__ inline void adj_len(T r2, T& rr, T& irr) {
   }
 }
 
-// Reverse of the symplectic-Euler update for one slot: vbt = vbar' + dt xbar',
-// c = -(m sigma/h) dt vbt; fixed particles get zero.
+// Reverse of the symplectic-Euler update of a moving particle: vbt = vbar' +
+// dt xbar', c = -(m sigma/h) dt vbt.
+template <int F>
+__device__ inline void adj_integrator(const double4& x, const double4& v, double dt, double msh, double4& vt_out,
+                                      typename AdjForm<F>::C4& c_out) {
+  using C4 = typename AdjForm<F>::C4;
+  const double4 vt = make_double4(v.x + dt * x.x, v.y + dt * x.y, v.z + dt * x.z, 0.0);
+  vt_out = vt;
+  const double s = -msh * dt;
+  c_out = C4{(decltype(C4{}.x))(s * vt.x), (decltype(C4{}.x))(s * vt.y), (decltype(C4{}.x))(s * vt.z), 0};
+}
+
+// The same for every slot; fixed particles get zero.  Only the sweep's first
+// step needs it: k_adj_density does it for the step before its own.
 template <int F>
 __global__ __launch_bounds__(kBlock) void k_adj_prep(uint32_t n, uint64_t n_moving,
                                                      const uint32_t* __restrict__ ids,
@@ -92,11 +104,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_prep(uint32_t n, uint64_t n_movi
     cvec[k] = C4{0, 0, 0, 0};
     return;
   }
-  double4 x = xb[k], v = vb[k];
-  double4 vt = make_double4(v.x + dt * x.x, v.y + dt * x.y, v.z + dt * x.z, 0.0);
-  vb[k] = vt;
-  double s = -msh * dt;
-  cvec[k] = C4{(decltype(C4{}.x))(s * vt.x), (decltype(C4{}.x))(s * vt.y), (decltype(C4{}.x))(s * vt.z), 0};
+  adj_integrator<F>(xb[k], vb[k], dt, msh, vb[k], cvec[k]);
 }
 
 // K sums of a block's wavefronts 1 .. kGroups - 1.
@@ -332,7 +340,8 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjForceWaves<F>
 
 // Density adjoint + assembly: xbar_k = xbar'_k + force part + density part
 // (moving particles; fixed ones 0), then both adjoints move to the previous
-// step's slot order through the frozen permutation.  One wavefront per
+// step's slot order through the frozen permutation.  With cvec the integrator's
+// adjoint of that step (k_adj_prep) is taken on the way.  One wavefront per
 // block, neighbour data staged per row run.
 template <int F>
 struct AdjDensityStage {
@@ -345,10 +354,11 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjDensityWaves<
     uint32_t n, uint64_t n_moving, SphStepRecord rec, Grid g, SphConst kc, SphUnits u,
     const typename AdjForm<F>::ar* __restrict__ rhob, const double4* __restrict__ xb_in,
     const double4* __restrict__ xbf, const double4* __restrict__ vb_in, double4* __restrict__ xb_out,
-    double4* __restrict__ vb_out, uint32_t n_tiles) {
+    double4* __restrict__ vb_out, typename AdjForm<F>::C4* __restrict__ cvec, uint32_t n_tiles) {
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using ar = typename AdjForm<F>::ar;
+  using C4 = typename AdjForm<F>::C4;
   const G4* gpos = (const G4*)rec.gpos;
   __shared__ typename std::conditional<SPLIT, GroupSums<3>, AdjDensityStage<F>>::type st;
   const uint32_t lane = threadIdx.x & 63u;
@@ -429,30 +439,33 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjDensityWaves<
   if (!live) {
     xb_out[dst] = make_double4(0, 0, 0, 0);
     vb_out[dst] = make_double4(0, 0, 0, 0);
+    if (cvec) cvec[dst] = C4{0, 0, 0, 0};
     return;
   }
   const double k = kc.msig * u.inv_h * u.unit_scale;
   const double4 a = xb_in[i], b = xbf[i];
-  xb_out[dst] = make_double4(a.x + b.x + k * sx, a.y + b.y + k * sy, a.z + b.z + k * sz, 0.0);
-  vb_out[dst] = vb_in[i];
+  const double4 x = make_double4(a.x + b.x + k * sx, a.y + b.y + k * sy, a.z + b.z + k * sz, 0.0);
+  const double4 v = vb_in[i];
+  xb_out[dst] = x;
+  if (cvec) adj_integrator<F>(x, v, kc.dt, kc.msh, vb_out[dst], cvec[dst]);
+  else vb_out[dst] = v;
 }
 
-// Sum the block partials of one reverse step into acc[0..1] (one block).
-constexpr uint32_t kAdjReduceBlock = 1024;
-// One block, fixed order: thread t sums partials t + 1024 (4 q + s) into its
+// Sum of one reverse step's partials per block (nparts apart per step) into its
+// first one.  Fixed order: thread t sums partials t + 1024 (4 q + s) into its
 // accumulator s (four independent load chains, so the loads overlap), then the
 // four and the block's threads are combined in a fixed tree.
-static __global__ __launch_bounds__(kAdjReduceBlock) void k_adj_reduce(uint32_t nparts,
-                                                                       const double2* __restrict__ partial,
-                                                                       double* __restrict__ acc) {
+constexpr uint32_t kAdjReduceBlock = 1024;
+static __global__ __launch_bounds__(kAdjReduceBlock) void k_adj_reduce(uint32_t nparts, double2* __restrict__ partial) {
   __shared__ double sa[kAdjReduceBlock], sb[kAdjReduceBlock];
+  double2* part = partial + (size_t)blockIdx.x * nparts;
   double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0};
   for (uint32_t k0 = 0; k0 < nparts; k0 += 4u * kAdjReduceBlock) {
     double2 v[4];
 #pragma unroll
     for (uint32_t s = 0; s < 4u; ++s) {
       const uint32_t k = k0 + s * kAdjReduceBlock + threadIdx.x;
-      v[s] = k < nparts ? partial[k] : make_double2(0.0, 0.0);
+      v[s] = k < nparts ? part[k] : make_double2(0.0, 0.0);
     }
 #pragma unroll
     for (uint32_t s = 0; s < 4u; ++s) {
@@ -470,10 +483,20 @@ static __global__ __launch_bounds__(kAdjReduceBlock) void k_adj_reduce(uint32_t 
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    acc[0] += sa[0];
-    acc[1] += sb[0];
+  if (threadIdx.x == 0) part[0] = make_double2(sa[0], sb[0]);
+}
+
+// acc[0..1] += the sums of `steps` reverse steps, step by step.
+static __global__ void k_adj_acc(uint32_t nparts, uint32_t steps, const double2* __restrict__ partial,
+                                 double* __restrict__ acc) {
+  double a = acc[0], b = acc[1];
+  for (uint32_t t = 0; t < steps; ++t) {
+    const double2 v = partial[(size_t)t * nparts];
+    a += v.x;
+    b += v.y;
   }
+  acc[0] = a;
+  acc[1] = b;
 }
 
 // Device buffers of the reverse sweep.
@@ -486,8 +509,10 @@ struct AdjBufs {
   double* acc;
 };
 
+// One reverse step; step: its place in the segment's partials, first / last: of
+// the whole sweep.
 template <int F>
-void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
+void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A, uint32_t step, bool first, bool last) {
   const uint32_t n = (uint32_t)c.n;
   const SphUnits u = sph_units<F>(c);
   const uint32_t n_tiles = blocks_for(n, kAdjBlock);
@@ -497,7 +522,7 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
   // 40/18, 42/22, 47/38, 54/54, FP64 48/20, 52/23, 53/33, 68/56, 92/83.
   const bool split_force = c.quad && n <= (F == kMixed ? 150000u : 64000u);
   const bool split_density = c.quad && n <= 300000u;
-  {
+  if (first) {
     LaunchScope ls(&c, "adj_prep", 2.0 * 32.0 * n + 32.0 * n);
     k_adj_prep<F><<<blocks_for(n), kBlock, 0, c.stream>>>(n, c.n_moving, rec.ids, A.xb, A.vb,
                                                           (typename AdjForm<F>::C4*)A.cvec, c.sph.dt, c.sph.msh);
@@ -509,12 +534,11 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
     auto launch = [&](auto kernel, int block) {
       kernel<<<tile_grid(n_tiles), block, 0, c.stream>>>(
           n, c.n_moving, rec, c.grid, c.sph, u, c.desc.alpha, c.desc.c0, c.desc.rho0,
-          (const typename AdjForm<F>::C4*)A.cvec, A.xbf, A.vb, (typename AdjForm<F>::ar*)A.rhob, A.partial, n_tiles);
+          (const typename AdjForm<F>::C4*)A.cvec, A.xbf, A.vb, (typename AdjForm<F>::ar*)A.rhob,
+          A.partial + (size_t)step * n_tiles, n_tiles);
     };
     if (split_force) launch(k_adj_force<F, true>, 64 * kGroups);
     else launch(k_adj_force<F, false>, kAdjBlock);
-    PR_HIP(hipGetLastError());
-    k_adj_reduce<<<1, kAdjReduceBlock, 0, c.stream>>>(n_tiles, A.partial, A.acc);
     PR_HIP(hipGetLastError());
   }
   {
@@ -524,7 +548,7 @@ void sph_reverse_step(Ctx& c, const SphStepRecord& rec, AdjBufs& A) {
     auto launch = [&](auto kernel, int block) {
       kernel<<<tile_grid(n_tiles), block, 0, c.stream>>>(
           n, c.n_moving, rec, c.grid, c.sph, u, (const typename AdjForm<F>::ar*)A.rhob, A.xb, A.xbf, A.vb, A.xb2, A.vb2,
-          n_tiles);
+          last ? nullptr : (typename AdjForm<F>::C4*)A.cvec, n_tiles);
     };
     if (split_density) launch(k_adj_density<F, true>, 64 * kGroups);
     else launch(k_adj_density<F, false>, kAdjBlock);
@@ -540,18 +564,21 @@ namespace prestige {
 
 // Host helpers shared by the forms (adjoint.hip).
 void snapshot_state(Ctx& c, Snapshot& s);
-void restore_state(Ctx& c, const Snapshot& s);
+void restore_state(Ctx& c, Snapshot& s);
+void copy_many(Ctx& c, const std::vector<Copy>& list);
 void adj_seed_gather(Ctx& c, const uint32_t* ids, const double* seed_x, const double* seed_v);
 void adj_grad_scatter(Ctx& c, const uint32_t* ids, const double4* vb, double* grad_v0_host);
-void ensure_adj_buffers(Ctx& c, uint32_t grid_blocks);
+void ensure_adj_buffers(Ctx& c);
 
-// Keep what the reverse sweep needs from the step that just ran.  Taken by
-// swap: the pair geometry (sorted pre-step state or FP32 probes), the
-// permutation and the row-run masks, all of which the next step
-// regenerates.  Copied: ids (the next reorder reads them) and (rho, p/rho^2),
-// which stays downloadable.
+// Keep what the reverse sweep needs from step t of a segment, which just ran,
+// in rec[t].  Taken by swap: the pair geometry (sorted pre-step state or FP32
+// probes), the permutation, the row-run masks and (rho, p/rho^2), all of which
+// the next step regenerates, and the previous step's ids, whose order this
+// step's build left.  The segment's last step copies its ids, and the taped
+// run's last (rho, p/rho^2), which stay downloadable.
 template <int F>
-void record_sph_step(Ctx& c, StepRecord& r) {
+void record_sph_step(Ctx& c, Tape& T, uint32_t t, bool last, bool keep_rp) {
+  StepRecord& r = *T.rec[t];
   const size_t n = c.n ? c.n : 1;
   const size_t r2 = (F == kF64) ? sizeof(double2) : sizeof(float2);
   const int prev = c.cur ^ 1;   // the step left its sorted input in the other buffer
@@ -565,13 +592,10 @@ void record_sph_step(Ctx& c, StepRecord& r) {
   take_buffer(c.vals[c.perm_buf], r.perm);
   take_buffer(c.nmeta, r.nmeta);
   take_buffer(c.nword, r.nword);
-  r.rp.alloc(n * r2);
-  r.ids.alloc(n * 4);
-  auto cp = [&](DevBuf& d, const void* s, size_t b) {
-    PR_HIP(hipMemcpyAsync(d.p, s, b, hipMemcpyDeviceToDevice, c.stream));
-  };
-  cp(r.rp, c.rp.p, c.n * r2);
-  cp(r.ids, c.ids[c.cur_ids].p, c.n * 4);
+  if (t > 0) take_buffer(c.ids[c.cur_ids ^ 1], T.rec[t - 1]->ids);
+  if (keep_rp) copy_many(c, {{&r.rp, &c.rp, n * r2}});
+  else take_buffer(c.rp, r.rp);
+  if (last) copy_many(c, {{&r.ids, &c.ids[c.cur_ids], n * 4}});
 }
 
 // Steps taken while this is alive leave every particle usable row masks
@@ -600,7 +624,7 @@ void sph_tape_forward(Ctx& c, uint32_t nsteps, uint32_t every) {
     }
     c.record_all = s >= last0;   // only recorded steps need usable masks for every particle
     sph_step_impl<F>(c);
-    if (s >= last0) record_sph_step<F>(c, *T.rec[s - last0]);
+    if (s >= last0) record_sph_step<F>(c, T, s - last0, s + 1 == nsteps, s + 1 == nsteps);
   }
   T.last_recorded = true;
   if (!c.tape.final_state) c.tape.final_state.reset(new Snapshot());
@@ -613,7 +637,9 @@ template <int F>
 void sph_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* grad_params, double* grad_v0) {
   Tape& T = c.tape;
   const uint32_t n = (uint32_t)c.n;
-  ensure_adj_buffers(c, blocks_for(n, kAdjBlock));   // one force partial per tile
+  const uint32_t n_tiles = blocks_for(n, kAdjBlock);
+  ensure_adj_buffers(c);
+  T.partial.alloc((size_t)n_tiles * std::min(T.every, T.nsteps) * sizeof(double2) + 64);   // one per tile and step
   AdjBufs A{T.xb.as<double4>(), T.vb.as<double4>(), T.xb2.as<double4>(), T.vb2.as<double4>(),
             T.cvec.p, T.xbf.as<double4>(), T.rhob.p, T.partial.as<double2>(),
             T.acc.as<double>()};
@@ -629,7 +655,7 @@ void sph_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       RecordAll keep_masks(c);
       for (uint32_t t = 0; t < len; ++t) {
         sph_step_impl<F>(c);
-        record_sph_step<F>(c, *T.rec[t]);
+        record_sph_step<F>(c, T, t, t + 1 == len, false);
       }
     }
     T.last_recorded = false;   // records are overwritten by the recompute of earlier segments
@@ -637,8 +663,13 @@ void sph_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       const StepRecord& r = *T.rec[t];
       SphStepRecord sr{r.gpos.p, r.gvel.p, r.rp.p, r.ids.as<uint32_t>(), r.perm.as<uint32_t>(),
                        r.nmeta.as<uint2>(), r.nword.as<uint32_t>()};
-      sph_reverse_step<F>(c, sr, A);
+      sph_reverse_step<F>(c, sr, A, len - 1u - t, s0 + t + 1u == T.nsteps, s0 + t == 0u);
     }
+    if (!n) continue;
+    k_adj_reduce<<<len, kAdjReduceBlock, 0, c.stream>>>(n_tiles, A.partial);
+    PR_HIP(hipGetLastError());
+    k_adj_acc<<<1, 1, 0, c.stream>>>(n_tiles, len, A.partial, A.acc);
+    PR_HIP(hipGetLastError());
   }
   // A.xb / A.vb now hold the adjoints of the state the tape started from
   if (grad_params) {

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <map>
@@ -198,6 +199,13 @@ struct LaunchScope {
   hipEvent_t a = nullptr, b = nullptr;
   LaunchScope(Ctx* c, const char* name, double bytes);
   ~LaunchScope() noexcept(false);
+};
+
+// One device-to-device copy of a list (copy_many allocates dst).
+struct Copy {
+  DevBuf* dst;
+  DevBuf* src;
+  size_t bytes;
 };
 
 // Device copy of the full integration state (used as an adjoint checkpoint).
