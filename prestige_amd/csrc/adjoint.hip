@@ -128,11 +128,11 @@ void adj_seed_gather(Ctx& c, const uint32_t* ids, const double* seed_x, const do
   double* dsv = nullptr;
   if (seed_x) {
     dsx = T.seeds.as<double>();
-    PR_HIP(hipMemcpyAsync(dsx, seed_x, 3 * n * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    to_device(c, dsx, seed_x, 3 * n * sizeof(double));
   }
   if (seed_v) {
     dsv = T.seeds.as<double>() + 3 * n;
-    PR_HIP(hipMemcpyAsync(dsv, seed_v, 3 * n * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    to_device(c, dsv, seed_v, 3 * n * sizeof(double));
   }
   if (n) {
     k_seed_gather<<<blocks_for(n), kBlock, 0, c.stream>>>((uint32_t)n, ids, dsx, dsv, T.xb.as<double4>(),
@@ -149,8 +149,7 @@ void adj_grad_scatter(Ctx& c, const uint32_t* ids, const double4* vb, double* gr
   double* d = T.seeds.as<double>();
   k_grad_scatter<<<blocks_for(n), kBlock, 0, c.stream>>>((uint32_t)n, c.n_moving, ids, vb, d);
   PR_HIP(hipGetLastError());
-  PR_HIP(hipMemcpyAsync(grad_v0_host, d, 3 * n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  PR_HIP(hipStreamSynchronize(c.stream));
+  to_host(c, grad_v0_host, d, 3 * n * sizeof(double));
 }
 
 void sph_tape_forward_mixed(Ctx& c, uint32_t nsteps, uint32_t every);

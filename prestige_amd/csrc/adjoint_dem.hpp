@@ -564,8 +564,7 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
   }
   if (grad_params) {
     double acc[3];
-    PR_HIP(hipMemcpyAsync(acc, T.acc.p, sizeof(acc), hipMemcpyDeviceToHost, c.stream));
-    PR_HIP(hipStreamSynchronize(c.stream));
+    to_host(c, acc, T.acc.p, sizeof(acc));
     for (int q = 0; q < 3; ++q) grad_params[q] = acc[q];
   }
   if (grad_v0) adj_grad_scatter(c, T.ckpt[0]->ids.as<uint32_t>(), vb, grad_v0);

@@ -674,8 +674,7 @@ void sph_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
   // A.xb / A.vb now hold the adjoints of the state the tape started from
   if (grad_params) {
     double acc[2];
-    PR_HIP(hipMemcpyAsync(acc, A.acc, sizeof(acc), hipMemcpyDeviceToHost, c.stream));
-    PR_HIP(hipStreamSynchronize(c.stream));
+    to_host(c, acc, A.acc, sizeof(acc));
     grad_params[0] = acc[0];
     grad_params[1] = acc[1];
   }

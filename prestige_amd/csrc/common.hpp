@@ -252,6 +252,9 @@ struct Ctx {
   Ctx() = default;
   Ctx(const Ctx&) = delete;
   Ctx& operator=(const Ctx&) = delete;
+  ~Ctx() {
+    if (pin) (void)hipHostFree(pin);
+  }
   prestige_desc desc{};
   int device = 0;
   hipStream_t stream = nullptr;
@@ -302,7 +305,8 @@ struct Ctx {
   bool record_all = false;
   bool dry_reuse = true;         // PRESTIGE_DRY=off turns the reuse off (comparisons and tests)
   void forget_dry() { dens_pass += 2; }   // state changed outside a step
-  DevBuf flags;                  // FLAG_COUNT uint32
+  DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word
+  void *pin = nullptr, *pin_dev = nullptr;   // pinned block for small transfers (host and device address)
   // gather outputs
   DevBuf rp;                     // (rho, p/rho^2) per slot: double2 or float2
   DevBuf pres;                   // p per slot (double or float)
@@ -447,6 +451,11 @@ __device__ inline int cell_shift(uint32_t wi, uint32_t wj, int axis) {
 
 // Error message of calls without a context (prestige_last_error(NULL)).
 void set_context_free_error(const std::string& msg);
+
+// Copies to and from host memory that is only borrowed for the call; to_host
+// waits for the stream (capi.hip).
+void to_device(Ctx& c, void* dst, const void* host, size_t bytes);
+void to_host(Ctx& c, void* host, const void* src, size_t bytes);
 
 // Per-form kernel entry points (defined in the .hip files).
 void neighbors_build(Ctx& c);

@@ -614,12 +614,13 @@ __global__ void k_scatter_ids(uint32_t n, const T* __restrict__ src, int stride,
   if (k < n) out[ids[k]] = (double)src[(size_t)k * stride + comp];
 }
 
+// (of an upload: nothing when *bad is set, the field's values failed their check)
 template <class T>
 __global__ void k_gather_ids(uint32_t n, const double* __restrict__ in,
                              const uint32_t* __restrict__ ids, T* __restrict__ dst, int stride,
-                             int comp) {
+                             int comp, const uint32_t* __restrict__ bad) {
   uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) dst[(size_t)k * stride + comp] = (T)in[ids[k]];
+  if (k < n && *bad == 0u) dst[(size_t)k * stride + comp] = (T)in[ids[k]];
 }
 
 __global__ void k_scatter_keys(uint32_t n, const uint32_t* __restrict__ keys,
@@ -648,12 +649,13 @@ void gather_from_ids(Ctx& c, const double* d_in, void* dst, int dst_kind, int co
   const uint32_t n = (uint32_t)c.n;
   if (!n) return;
   const uint32_t* ids = c.ids[c.cur_ids].as<uint32_t>();
+  const uint32_t* bad = c.flags.as<uint32_t>() + FLAG_COUNT;
   int stride = comp >= 0 ? (comp >= 100 ? 2 : 4) : 1;
   int cc = comp >= 100 ? comp - 100 : (comp >= 0 ? comp : 0);
   if (dst_kind == 0)
-    k_gather_ids<double><<<blocks_for(n), kBlock, 0, c.stream>>>(n, d_in, ids, (double*)dst, stride, cc);
+    k_gather_ids<double><<<blocks_for(n), kBlock, 0, c.stream>>>(n, d_in, ids, (double*)dst, stride, cc, bad);
   else
-    k_gather_ids<float><<<blocks_for(n), kBlock, 0, c.stream>>>(n, d_in, ids, (float*)dst, stride, cc);
+    k_gather_ids<float><<<blocks_for(n), kBlock, 0, c.stream>>>(n, d_in, ids, (float*)dst, stride, cc, bad);
   PR_HIP(hipGetLastError());
 }
 
