@@ -244,7 +244,7 @@ const char* prestige_last_error(const prestige_ctx* ctx);
  * prestige_desc; stream is a hipStream_t (NULL: the null stream).  The work
  * runs on that stream and the call returns once it has finished (it reads
  * back the domain flag).  Intermediate arrays live in a fixed device array
- * of about 64.5 MiB per GPU, held until the process ends: n <= 1,048,576
+ * of about 96 MiB per GPU, held until the process ends: n <= 1,048,576
  * particles and at most 4,194,304 cells, else PRESTIGE_E_CAPACITY.  Calls on
  * one GPU share that array, so calls that overlap on one GPU race.
  * PRESTIGE_E_DOMAIN when a particle lies outside the grid.  Errors are read

@@ -512,6 +512,184 @@ static void incremental_sort(Ctx& c) {
   c.perm_buf = 0;
 }
 
+// ---------------------------------------------------------------------------
+// counting sort: the first build of a state, and eq1 without allocating
+// ---------------------------------------------------------------------------
+// Every slot takes a number within its cell as it arrives, a scan of the cell
+// counts is the cell table, and the cell lists that follow from both give each
+// slot its place: the start of its cell plus the slots of the cell before it
+// (a stable sort, whatever the order of arrival).  The placement moves the
+// state, so keys, permutation, cell table and sorted state are those of the
+// radix sort with its reorder and cell table, in six launches for its eleven
+// (three digits).  Us: 1M scattered points 146 -> 93, 571k particles in tank
+// order 83 -> 35, 1,000 in 1,000 cells 60 -> 32.
+//
+// The radix sort keeps what does not pay here.  The table costs 16 bytes a
+// cell: 4.1M cells with 300k particles 110 -> 59, but with 20k 107 either way, so
+// the line lies at kCountCells.  A slot reads its cell's whole list: 2,000
+// particles in one cell 81 -> 65, but 20,000 84 -> 340, so the mean may not pass
+// kCountMean (a crowd in one cell of many costs any pass over the cells far
+// more than the build).
+constexpr uint32_t kCountCells = 1u << 22;
+constexpr uint32_t kCountMean = 2048;
+
+static bool count_sort_fits(uint32_t n, uint32_t n_cells) {
+  if ((uint64_t)n > (uint64_t)kCountMean * n_cells) return false;
+  // the tile totals live in the radix sort's histogram
+  const uint64_t tiles = ((uint64_t)n_cells + 1u + kCellTile - 1u) / kCellTile;
+  return n_cells <= kCountCells && tiles <= (uint64_t)kBuckets * sort_tiles(n);
+}
+
+__global__ __launch_bounds__(kBlock) void k_count_clear(uint32_t n, uint32_t* __restrict__ cnt, uint32_t* flags) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (i < n) cnt[i] = 0u;
+  if (flags && i < (uint32_t)FLAG_COUNT) flags[i] = 0u;
+}
+
+// This lane's number in cell key; the lanes of a wavefront that follow each
+// other into one cell take theirs with one atomic (571k particles in tank order:
+// 40 -> 4.5 us; points in no order find nothing to share).  All lanes call.
+__device__ inline uint32_t cell_arrival(uint32_t* __restrict__ cnt, uint32_t key, bool live) {
+  const uint32_t lane = __lane_id();
+  const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
+  const uint64_t starts = __ballot(lane == 0u || key != before || !live);
+  const uint32_t first = 63u - (uint32_t)__builtin_clzll(starts & (~0ull >> (63u - lane)));
+  const uint64_t after = lane == 63u ? 0ull : starts & (~0ull << (lane + 1u));
+  const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
+  uint32_t base = 0;
+  if (live && first == lane) base = atomicAdd(&cnt[key], end - first);
+  return (uint32_t)__shfl((int)base, (int)first, 64) + lane - first;
+}
+
+__global__ __launch_bounds__(kBlock) void k_count_keys(uint32_t n, const uint32_t* __restrict__ keys,
+                                                       uint32_t* __restrict__ cnt, uint32_t* __restrict__ arr) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  const bool live = i < n;
+  const uint32_t a = cell_arrival(cnt, live ? keys[i] : 0u, live);
+  if (live) arr[i] = a;
+}
+
+__global__ __launch_bounds__(kBlock) void k_count_tiles(uint32_t n_cells, const uint32_t* __restrict__ cnt,
+                                                        uint32_t* __restrict__ tot) {
+  __shared__ uint32_t s4[4];
+  uint32_t sum = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kCellTile / kBlock; ++k) {
+    const uint32_t c = blockIdx.x * kCellTile + k * kBlock + threadIdx.x;
+    if (c < n_cells) sum += cnt[c];
+  }
+  sum = wave_sum(sum);
+  if (__lane_id() == 0) s4[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) tot[blockIdx.x] = s4[0] + s4[1] + s4[2] + s4[3];
+}
+
+// Counts to cell table, in place.
+__global__ __launch_bounds__(kBlock) void k_count_table(uint32_t n_cells, const uint32_t* __restrict__ tot,
+                                                        uint32_t* __restrict__ lb) {
+  __shared__ uint32_t s4[4];
+  const uint32_t b = blockIdx.x, t = threadIdx.x;
+  uint32_t part = 0;
+  for (uint32_t k = t; k < b; k += kBlock) part += tot[k];
+  part = wave_sum(part);
+  if (__lane_id() == 0) s4[t >> 6] = part;
+  __syncthreads();
+  uint32_t run = s4[0] + s4[1] + s4[2] + s4[3];
+  __syncthreads();
+  const uint32_t c0 = b * kCellTile + 4u * t;
+  uint32_t d[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k) d[k] = c0 + k < n_cells ? lb[c0 + k] : 0u;
+  uint32_t total;
+  run += block_excl_scan(d[0] + d[1] + d[2] + d[3], s4, &total);
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k) {
+    if (c0 + k <= n_cells) lb[c0 + k] = run;
+    run += d[k];
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_count_list(uint32_t n, const uint32_t* __restrict__ keys,
+                                                       const uint32_t* __restrict__ arr,
+                                                       const uint32_t* __restrict__ lb, uint32_t* __restrict__ list) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (i < n) list[lb[keys[i]] + arr[i]] = i;
+}
+
+// Place of slot i of a cell with entries [l0, l1) of the lists: l0 plus the
+// entries below i.  A crowded cell is read 128 bytes at a time (20,000 slots in
+// one cell: 620 -> 310 us, of the 5,700 that eq1 then takes over them).
+__device__ inline uint32_t place_in_cell(const uint32_t* __restrict__ list, uint32_t l0, uint32_t l1, uint32_t i) {
+  uint32_t pos = l0, q = l0;
+  if (l1 - l0 > 64u) {
+    for (; q & 3u; ++q) pos += list[q] < i ? 1u : 0u;
+    const uint4* l4 = reinterpret_cast<const uint4*>(list);
+    for (; q + 32u <= l1; q += 32u) {
+      uint4 v[8];
+#pragma unroll
+      for (uint32_t k = 0; k < 8u; ++k) v[k] = l4[(q >> 2) + k];
+#pragma unroll
+      for (uint32_t k = 0; k < 8u; ++k)
+        pos += (v[k].x < i ? 1u : 0u) + (v[k].y < i ? 1u : 0u) + (v[k].z < i ? 1u : 0u) + (v[k].w < i ? 1u : 0u);
+    }
+  }
+#pragma unroll 4
+  for (; q < l1; ++q) pos += list[q] < i ? 1u : 0u;
+  return pos;
+}
+
+template <class T4, bool OMEGA, bool PROBE, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_count_place(uint32_t n, const uint32_t* __restrict__ keys,
+                                                        const uint32_t* __restrict__ lb,
+                                                        const uint32_t* __restrict__ list,
+                                                        uint32_t* __restrict__ skeys, uint32_t* __restrict__ perm,
+                                                        ReorderIO<T4> io) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t c = keys[i];
+  const uint32_t pos = place_in_cell(list, lb[c], lb[c + 1u], i);
+  skeys[pos] = c;
+  perm[pos] = i;
+  move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, c);
+}
+
+// n_cells + 1 counts (the last unused) to the cell table; tot: a total per tile.
+static void count_table(Ctx* c, uint32_t n_cells, uint32_t* cnt, uint32_t* tot, hipStream_t st) {
+  LaunchScope ls(c, "sort_count_cells", 12.0 * n_cells);
+  const uint32_t tiles = blocks_for((uint64_t)n_cells + 1u, (int)kCellTile);
+  k_count_tiles<<<tiles, kBlock, 0, st>>>(n_cells, cnt, tot);
+  PR_HIP(hipGetLastError());
+  k_count_table<<<tiles, kBlock, 0, st>>>(n_cells, tot, cnt);
+  PR_HIP(hipGetLastError());
+}
+// The counting sort of keys[cur_key] with the state moved; same outputs as
+// radix_sort, k_reorder and k_cell_lb.
+static void context_count_sort(Ctx& c) {
+  const uint32_t n = (uint32_t)c.n, cells = c.grid.n_cells;
+  const uint32_t* keys = c.keys[c.cur_key].as<uint32_t>();
+  uint32_t* arr = c.vals[0].as<uint32_t>();
+  {
+    LaunchScope ls(&c, "sort_count", 4.0 * cells + 12.0 * n);
+    k_count_clear<<<blocks_for(cells + 1u), kBlock, 0, c.stream>>>(cells + 1u, c.lb.as<uint32_t>(), nullptr);
+    PR_HIP(hipGetLastError());
+    k_count_keys<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, c.lb.as<uint32_t>(), arr);
+    PR_HIP(hipGetLastError());
+  }
+  count_table(&c, cells, c.lb.as<uint32_t>(), c.sort_hist.as<uint32_t>(), c.stream);
+  LaunchScope ls(&c, "sort_count_place", (24.0 + reorder_bytes(c)) * n);
+  uint32_t* list = c.vals[1].as<uint32_t>();
+  k_count_list<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, arr, c.lb.as<uint32_t>(), list);
+  PR_HIP(hipGetLastError());
+  with_reorder_form(c, c.cur, c.cur ^ 1, [&](auto form, auto io) {
+    using F = decltype(form);
+    k_count_place<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(
+        n, keys, c.lb.as<uint32_t>(), list, c.keys[c.cur_key ^ 1].as<uint32_t>(), arr, io);
+  });
+  PR_HIP(hipGetLastError());
+  c.cur_key ^= 1;
+  c.perm_buf = 0;
+}
+
 // lb[c] = first slot with key >= c, for c = 0 .. n_cells.  Thread k < n owns
 // the cells [lo, hi) whose lower bound is k: lo = key[k-1] + 1 (0 for k = 0),
 // hi = key[k] + 1; the cells after the last key (lower bound n: the empty
@@ -580,19 +758,23 @@ void neighbors_build(Ctx& c) {
       PR_HIP(hipMemsetAsync(c.inc_cin(), 0, c.inc_count_bytes(), c.stream));
       c.inc_counts = false;
     }
-    radix_sort(c);
-    const uint32_t* skeys = c.keys[c.cur_key].as<uint32_t>();
-    const uint32_t* perm = c.vals[c.perm_buf].as<uint32_t>();
-    {
-      LaunchScope ls(&c, "reorder", reorder_bytes(c) * n);
-      with_reorder_form(c, src, dst, [&](auto form, auto io) {
-        using F = decltype(form);
-        k_reorder<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(n, perm, skeys, io);
-      });
-      PR_HIP(hipGetLastError());
+    if (!c.sort_radix && count_sort_fits(n, c.grid.n_cells)) {
+      context_count_sort(c);
+    } else {
+      radix_sort(c);
+      const uint32_t* skeys = c.keys[c.cur_key].as<uint32_t>();
+      const uint32_t* perm = c.vals[c.perm_buf].as<uint32_t>();
+      {
+        LaunchScope ls(&c, "reorder", reorder_bytes(c) * n);
+        with_reorder_form(c, src, dst, [&](auto form, auto io) {
+          using F = decltype(form);
+          k_reorder<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(n, perm, skeys, io);
+        });
+        PR_HIP(hipGetLastError());
+      }
+      LaunchScope ls(&c, "cell_lb", 8.0 * n + 4.0 * c.grid.n_cells);
+      launch_cell_lb(c, skeys);
     }
-    LaunchScope ls(&c, "cell_lb", 8.0 * n + 4.0 * c.grid.n_cells);
-    launch_cell_lb(c, skeys);
   }
   c.inc_ready = false;
   c.cur = dst;
@@ -884,12 +1066,12 @@ void eq1_eval(Ctx& c, int loop, double cutoff) {
 // eq1 over the cell iterator without allocating (prestige_eq1_cells_noalloc)
 // ---------------------------------------------------------------------------
 // The same kernels as prestige_eval_equation(PRESTIGE_EQ1, PRESTIGE_LOOP_CELLS)
-// on a fresh context (cell keys, radix sort, positions in key order, cell
-// table, the eq1 gather), on the caller's device arrays, with every
+// on a fresh context (cell keys, counting sort with the positions moved, the
+// eq1 gather), on the caller's device arrays, with every
 // intermediate array in one file-scope device array: `scratch`.  It holds
-// the sort's key and value ping-pong pairs (16 B per particle), the sorted
-// positions (32 B), the cell table (4 B per cell + 4), the digit histogram
-// and totals, and the error flags, each at a 256-byte boundary, sized for at
+// keys, sorted keys, permutation and arrival numbers (16 B per particle), the
+// positions in order of arrival and sorted (64 B), the cell table (4 B per cell + 4), its tile totals
+// and the error flags, each at a 256-byte boundary, sized for at
 // most kNoAllocMaxN particles and kNoAllocMaxCells cells.  Each device holds
 // its own copy; host code reaches it only through the address
 // hipGetSymbolAddress gives on that device (noalloc_scratch), never through
@@ -900,39 +1082,73 @@ constexpr uint64_t kNoAllocMaxN = 1ull << 20;
 constexpr uint64_t kNoAllocMaxCells = 1ull << 22;
 
 constexpr uint64_t na_round(uint64_t b) { return (b + 255ull) & ~255ull; }
-constexpr uint64_t kNaKeys = 0;                                               // keys[2]: 2 x 4 N
-constexpr uint64_t kNaVals = kNaKeys + 2 * na_round(4 * kNoAllocMaxN);        // vals[2]: 2 x 4 N
-constexpr uint64_t kNaPos = kNaVals + 2 * na_round(4 * kNoAllocMaxN);         // double4 x N
-constexpr uint64_t kNaLb = kNaPos + na_round(32 * kNoAllocMaxN);              // cells + 1
-constexpr uint64_t kNaHist = kNaLb + na_round(4 * (kNoAllocMaxCells + 1));    // kBuckets x tiles
-constexpr uint64_t kNaTot = kNaHist + na_round(4ull * kBuckets * ((kNoAllocMaxN + kTile - 1) / kTile));
-constexpr uint64_t kNaFlags = kNaTot + na_round(4ull * kBuckets);
+constexpr uint64_t kNaKeys = 0;                                               // keys, sorted keys: 2 x 4 N
+constexpr uint64_t kNaVals = kNaKeys + 2 * na_round(4 * kNoAllocMaxN);        // permutation, arrivals: 2 x 4 N
+constexpr uint64_t kNaPos = kNaVals + 2 * na_round(4 * kNoAllocMaxN);         // double4 x N, twice
+constexpr uint64_t kNaLb = kNaPos + 2 * na_round(32 * kNoAllocMaxN);          // cells + 1
+constexpr uint64_t kNaTot = kNaLb + na_round(4 * (kNoAllocMaxCells + 1));     // a total per tile of cells
+constexpr uint64_t kNaFlags = kNaTot + na_round(4ull * (kNoAllocMaxCells / kCellTile + 1));
 constexpr uint64_t kNoAllocBytes = kNaFlags + na_round(4ull * FLAG_COUNT);
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
-__global__ void k_noalloc_clear(uint32_t* flags) {
-  if (threadIdx.x < (uint32_t)FLAG_COUNT) flags[threadIdx.x] = 0u;
-}
-
-__global__ __launch_bounds__(kBlock) void k_cell_keys_soa(uint32_t n, const double* __restrict__ x,
-                                                          const double* __restrict__ y, const double* __restrict__ z,
-                                                          Grid g, uint32_t* __restrict__ keys, uint32_t* flags) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) keys[i] = cell_key_of(x[i], y[i], z[i], g, flags);
-}
-
-// Positions in key order: spos[k] = x[perm[k]] (the ids of a first build are
-// the permutation itself).
-__global__ __launch_bounds__(kBlock) void k_sorted_pos_soa(uint32_t n, const double* __restrict__ x,
-                                                           const double* __restrict__ y, const double* __restrict__ z,
-                                                           const uint32_t* __restrict__ perm,
-                                                           double4* __restrict__ spos) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) {
-    const uint32_t s = perm[k];
-    spos[k] = make_double4(x[s], y[s], z[s], 0.0);
+__global__ __launch_bounds__(kBlock) void k_count_soa(uint32_t n, const double* __restrict__ x,
+                                                      const double* __restrict__ y, const double* __restrict__ z,
+                                                      Grid g, uint32_t* __restrict__ keys, uint32_t* __restrict__ cnt,
+                                                      uint32_t* __restrict__ arr, uint32_t* flags) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  const bool live = i < n;
+  const uint32_t key = live ? cell_key_of(x[i], y[i], z[i], g, flags) : 0u;
+  const uint32_t a = cell_arrival(cnt, key, live);
+  if (live) {
+    keys[i] = key;
+    arr[i] = a;
   }
+}
+
+// The points in order of arrival, with (slot, key) in .w: one write of 32 bytes
+// to a scattered place each, where reading them from there in cell order takes
+// three (1M points in no order: 19 us and 18 for k_count_rank_soa; lists and
+// k_count_place 15 and 65).
+__global__ __launch_bounds__(kBlock) void k_count_scatter_soa(uint32_t n, const double* __restrict__ x,
+                                                              const double* __restrict__ y,
+                                                              const double* __restrict__ z,
+                                                              const uint32_t* __restrict__ keys,
+                                                              const uint32_t* __restrict__ arr,
+                                                              const uint32_t* __restrict__ lb,
+                                                              double4* __restrict__ upos) {
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t key = keys[i];
+  upos[lb[key] + arr[i]] = make_double4(x[i], y[i], z[i], __longlong_as_double((long long)((uint64_t)key << 32 | i)));
+}
+
+// Then by slot within each cell (k_count_place for points that are in cell order
+// already: what it reads and writes lies close together; the ids of a first
+// build are the permutation itself).
+__global__ __launch_bounds__(kBlock) void k_count_rank_soa(uint32_t n, const double4* __restrict__ upos,
+                                                           const uint32_t* __restrict__ lb,
+                                                           double4* __restrict__ spos, uint32_t* __restrict__ skeys,
+                                                           uint32_t* __restrict__ perm) {
+  const uint32_t k = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (k >= n) return;
+  const double4 p = upos[k];
+  const uint64_t w = (uint64_t)__double_as_longlong(p.w);
+  const uint32_t key = (uint32_t)(w >> 32), i = (uint32_t)w;
+  const uint32_t* slot = reinterpret_cast<const uint32_t*>(upos) + 6;   // entry q's slot is slot[8 q]
+  const uint32_t end = lb[key + 1u];
+  uint32_t q = lb[key], pos = q;
+  for (; q + 4u <= end; q += 4u) {
+    uint32_t v[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) v[k] = slot[8u * (size_t)(q + k)];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) pos += v[k] < i ? 1u : 0u;
+  }
+  for (; q < end; ++q) pos += slot[8u * (size_t)q] < i ? 1u : 0u;
+  spos[pos] = make_double4(p.x, p.y, p.z, 0.0);
+  skeys[pos] = key;
+  perm[pos] = i;
 }
 
 // Device address of this device's scratch, looked up once per device with
@@ -970,25 +1186,22 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
   PR_HIP(hipGetDevice(&dev));
   unsigned char* base = static_cast<unsigned char*>(noalloc_scratch(dev));
   uint32_t* flags = reinterpret_cast<uint32_t*>(base + kNaFlags);
-  const SortBufs b{{reinterpret_cast<uint32_t*>(base + kNaKeys),
-                    reinterpret_cast<uint32_t*>(base + kNaKeys + na_round(4 * kNoAllocMaxN))},
-                   {reinterpret_cast<uint32_t*>(base + kNaVals),
-                    reinterpret_cast<uint32_t*>(base + kNaVals + na_round(4 * kNoAllocMaxN))},
-                   reinterpret_cast<uint32_t*>(base + kNaHist), reinterpret_cast<uint32_t*>(base + kNaTot)};
-  double4* spos = reinterpret_cast<double4*>(base + kNaPos);
+  uint32_t* keys = reinterpret_cast<uint32_t*>(base + kNaKeys);
+  uint32_t* skeys = reinterpret_cast<uint32_t*>(base + kNaKeys + na_round(4 * kNoAllocMaxN));
+  uint32_t* perm = reinterpret_cast<uint32_t*>(base + kNaVals);
+  uint32_t* arr = reinterpret_cast<uint32_t*>(base + kNaVals + na_round(4 * kNoAllocMaxN));
+  double4* upos = reinterpret_cast<double4*>(base + kNaPos);
+  double4* spos = reinterpret_cast<double4*>(base + kNaPos + na_round(32 * kNoAllocMaxN));
   uint32_t* lb = reinterpret_cast<uint32_t*>(base + kNaLb);
-  k_noalloc_clear<<<1, 64, 0, st>>>(flags);
+  uint32_t* tot = reinterpret_cast<uint32_t*>(base + kNaTot);
+  k_count_clear<<<blocks_for(g.n_cells + 1u), kBlock, 0, st>>>(g.n_cells + 1u, lb, flags);
   PR_HIP(hipGetLastError());
-  k_cell_keys_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, g, b.keys[0], flags);
+  k_count_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, g, keys, lb, arr, flags);
   PR_HIP(hipGetLastError());
-  int kb = 0, vb = 0;
-  radix_sort_bufs(nullptr, b, 0, n, g.n_cells, st, &kb, &vb);
-  const uint32_t* skeys = b.keys[kb];
-  const uint32_t* perm = b.vals[vb];
-  k_sorted_pos_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, perm, spos);
+  count_table(nullptr, g.n_cells, lb, tot, st);
+  k_count_scatter_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, keys, arr, lb, upos);
   PR_HIP(hipGetLastError());
-  const uint32_t key_blocks = (uint32_t)blocks_for(n);
-  k_cell_lb<<<key_blocks + kTailBlocks, kBlock, 0, st>>>(n, g.n_cells, skeys, lb, key_blocks);
+  k_count_rank_soa<<<blocks_for(n), kBlock, 0, st>>>(n, upos, lb, spos, skeys, perm);
   PR_HIP(hipGetLastError());
   const uint32_t tiles = blocks_for(n, 64);
   k_eq1_cells<double4><<<tile_grid(tiles), 64, 0, st>>>(n, spos, perm, skeys, lb, g, cutoff * cutoff, 1.0 / cutoff,
