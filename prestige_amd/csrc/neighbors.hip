@@ -925,24 +925,29 @@ __global__ __launch_bounds__(64) void k_eq1_allpairs(uint32_t n, const double* _
 // few pairs in 10^5) takes the exact FP64 test for it.  So the pairs and the
 // order are the plain loop's, and each force is its sum bit for bit.
 // A union wider than the stage takes the exact test throughout.
-// 1M random particles at 2.4 spacings: 236 us; scanning into masks, walking the
-// set bits and testing each exactly took 403 (1.8M of a jittered dam break: 522
-// -> 361).  What bounds it is instruction issue, six a candidate, then the
-// LDS reads, 24 bytes a candidate and lane.  Where many pairs lie at the
-// cutoff to seven digits (an undisturbed lattice with a lattice distance for
-// a cutoff) the exact tests cost what the direct sums save: 395 -> 413.
+// The masses come in slot order (smass[mstride j]): gathered by id in here they
+// were 18 of a wavefront's loads of 64 scattered lines each, and what bounded it
+// (236 us below).  Four candidates share the question whether any lane is in doubt.
+// 1M random particles at 2.4 spacings: 191 us (masses in order 12 more);
+// scanning into masks, walking the set bits and testing each exactly took 403
+// (1.8M of a jittered dam break: 522 -> 344 with the masses).  What bounds it are
+// the LDS reads, 24 bytes a candidate and lane, and instruction issue, five a
+// candidate.  Where many pairs lie at the cutoff to seven digits (an undisturbed
+// lattice with a lattice distance for a cutoff) the exact tests cost what the
+// direct sums save: 395 -> 403.
 constexpr uint32_t kEq1Stage = 256;
+constexpr uint32_t kEq1Batch = 4;   // candidates in flight (the exact path picks among four)
 
 template <class T4>
 __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restrict__ pos,
                                                   const uint32_t* __restrict__ ids,
                                                   const uint32_t* __restrict__ skeys,
                                                   const uint32_t* __restrict__ lb, Grid g, double c2,
-                                                  double inv_cut, const double* __restrict__ mass,
+                                                  double inv_cut, const double* __restrict__ smass, uint32_t mstride,
                                                   double* __restrict__ force, uint32_t n_tiles) {
 #pragma clang fp contract(off)
-  __shared__ float4 s_q[kEq1Stage];
-  __shared__ double s_m[kEq1Stage];   // mass of the staged slots, gathered once per row run
+  __shared__ float4 s_q[kEq1Stage + kEq1Batch];   // (a batch may read past the stage's end)
+  __shared__ double s_m[kEq1Stage + kEq1Batch];
   const uint32_t tile = xcd_tile(blockIdx.x);
   if (tile >= n_tiles) return;
   const uint32_t lane = threadIdx.x, wbase = tile * 64u, i = wbase + lane;
@@ -991,14 +996,14 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
     const uint32_t span = (uint32_t)__builtin_amdgcn_readlane((int)(j0[r] + len[r]), 63 - __builtin_clzll(any)) - base;
     if (span > kEq1Stage) {
       for (uint32_t b = 0; b < len[r]; ++b)
-        if (exact(j0[r] + b)) acc += mass[ids[j0[r] + b]];
+        if (exact(j0[r] + b)) acc += smass[(size_t)mstride * (j0[r] + b)];
       continue;
     }
     float mq = 0.0f;
     for (uint32_t kk = lane; kk < span; kk += 64u) {
       const float4 q = offset(pos[base + kk]);
       s_q[kk] = q;
-      s_m[kk] = mass[ids[base + kk]];
+      s_m[kk] = smass[(size_t)mstride * (base + kk)];
       mq = q.w > mq ? q.w : mq;
     }
     const float m2 = fmaxf(ss_max, wave_max_pos(mq));
@@ -1006,33 +1011,47 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
     const float lo = (1.0f - margin) - so.w, hi = (1.0f + margin) - so.w;
     __builtin_amdgcn_wave_barrier();   // one wavefront: its LDS operations complete in order
     const uint32_t first = j0[r] - base;
-    auto take = [&](float v, double m, uint32_t j) {
-      bool in = v < lo;
-      if (__ballot(in != (v < hi)) != 0ull) {   // some lane cannot tell
-        if (v < hi && !in) in = exact(j);
-      }
-      if (in) acc += m;
-    };
-    uint32_t b = 0;
-    for (; b + 4u <= len[r]; b += 4u) {
-      float v[4];
-      double m[4];
+    auto batch = [&](uint32_t b, uint32_t cnt) {
+      float v[kEq1Batch];
+      double m[kEq1Batch];
 #pragma unroll
-      for (uint32_t u = 0; u < 4u; ++u) {
+      for (uint32_t u = 0; u < kEq1Batch; ++u) {
         const float4 q = s_q[first + b + u];
         v[u] = __builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w)));
+        if (u >= cnt) v[u] = 0x1.0p127f;   // past the run: outside
         m[u] = s_m[first + b + u];
       }
+      uint64_t open = 0;   // lanes that cannot tell
 #pragma unroll
-      for (uint32_t u = 0; u < 4u; ++u) take(v[u], m[u], j0[r] + b + u);
-    }
-    for (; b < len[r]; ++b) {
-      const float4 q = s_q[first + b];
-      take(__builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w))), s_m[first + b], j0[r] + b);
-    }
+      for (uint32_t u = 0; u < kEq1Batch; ++u) open |= __ballot(v[u] < lo) ^ __ballot(v[u] < hi);
+      if (open == 0ull) {
+#pragma unroll
+        for (uint32_t u = 0; u < kEq1Batch; ++u)
+          if (v[u] < lo) {
+            acc += m[u];
+            asm volatile("" : "+v"(acc));   // an add under the lane mask; as a select it costs two moves more
+          }
+      } else {
+#pragma unroll 1
+        for (uint32_t u = 0; u < kEq1Batch; ++u) {
+          const float w = u == 0u ? v[0] : (u == 1u ? v[1] : (u == 2u ? v[2] : v[3]));
+          const double mu = u == 0u ? m[0] : (u == 1u ? m[1] : (u == 2u ? m[2] : m[3]));
+          if (w < lo || (w < hi && exact(j0[r] + b + u))) acc += mu;
+        }
+      }
+    };
+    uint32_t b = 0;
+    for (; b + kEq1Batch <= len[r]; b += kEq1Batch) batch(b, kEq1Batch);
+    if (b < len[r]) batch(b, len[r] - b);
     __builtin_amdgcn_wave_barrier();
   }
   if (live) force[me] = acc;
+}
+
+__global__ __launch_bounds__(kBlock) void k_eq1_masses(uint32_t n, const uint32_t* __restrict__ ids,
+                                                       const double* __restrict__ mass, double* __restrict__ smass) {
+  const uint32_t k = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (k < n) smass[k] = mass[ids[k]];
 }
 
 void eq1_eval(Ctx& c, int loop, double cutoff) {
@@ -1051,14 +1070,17 @@ void eq1_eval(Ctx& c, int loop, double cutoff) {
   LaunchScope ls(&c, "eq1_cells", 56.0 * n);
   const uint32_t* ids = c.ids[c.cur_ids].as<uint32_t>();
   const uint32_t tiles = blocks_for(n, 64);
+  double* smass = c.scratch.as<double>();
+  k_eq1_masses<<<blocks_for(n), kBlock, 0, c.stream>>>(n, ids, c.mass.as<double>(), smass);
+  PR_HIP(hipGetLastError());
   if (c.desc.precision == PRESTIGE_F32)
     k_eq1_cells<float4><<<tile_grid(tiles), 64, 0, c.stream>>>(
         n, c.pos[c.cur].as<float4>(), ids, c.keys[c.cur_key].as<uint32_t>(), c.lb.as<uint32_t>(),
-        c.grid, cutoff * cutoff, 1.0 / cutoff, c.mass.as<double>(), c.force.as<double>(), tiles);
+        c.grid, cutoff * cutoff, 1.0 / cutoff, smass, 1u, c.force.as<double>(), tiles);
   else
     k_eq1_cells<double4><<<tile_grid(tiles), 64, 0, c.stream>>>(
         n, c.pos[c.cur].as<double4>(), ids, c.keys[c.cur_key].as<uint32_t>(), c.lb.as<uint32_t>(),
-        c.grid, cutoff * cutoff, 1.0 / cutoff, c.mass.as<double>(), c.force.as<double>(), tiles);
+        c.grid, cutoff * cutoff, 1.0 / cutoff, smass, 1u, c.force.as<double>(), tiles);
   PR_HIP(hipGetLastError());
 }
 
@@ -1128,6 +1150,7 @@ __global__ __launch_bounds__(kBlock) void k_count_scatter_soa(uint32_t n, const 
 // build are the permutation itself).
 __global__ __launch_bounds__(kBlock) void k_count_rank_soa(uint32_t n, const double4* __restrict__ upos,
                                                            const uint32_t* __restrict__ lb,
+                                                           const double* __restrict__ mass,
                                                            double4* __restrict__ spos, uint32_t* __restrict__ skeys,
                                                            uint32_t* __restrict__ perm) {
   const uint32_t k = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
@@ -1146,7 +1169,7 @@ __global__ __launch_bounds__(kBlock) void k_count_rank_soa(uint32_t n, const dou
     for (uint32_t k = 0; k < 4u; ++k) pos += v[k] < i ? 1u : 0u;
   }
   for (; q < end; ++q) pos += slot[8u * (size_t)q] < i ? 1u : 0u;
-  spos[pos] = make_double4(p.x, p.y, p.z, 0.0);
+  spos[pos] = make_double4(p.x, p.y, p.z, mass[i]);
   skeys[pos] = key;
   perm[pos] = i;
 }
@@ -1201,11 +1224,11 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
   count_table(nullptr, g.n_cells, lb, tot, st);
   k_count_scatter_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, keys, arr, lb, upos);
   PR_HIP(hipGetLastError());
-  k_count_rank_soa<<<blocks_for(n), kBlock, 0, st>>>(n, upos, lb, spos, skeys, perm);
+  k_count_rank_soa<<<blocks_for(n), kBlock, 0, st>>>(n, upos, lb, mass, spos, skeys, perm);
   PR_HIP(hipGetLastError());
   const uint32_t tiles = blocks_for(n, 64);
   k_eq1_cells<double4><<<tile_grid(tiles), 64, 0, st>>>(n, spos, perm, skeys, lb, g, cutoff * cutoff, 1.0 / cutoff,
-                                                        mass, force, tiles);
+                                                        &spos->w, 4u, force, tiles);
   PR_HIP(hipGetLastError());
   uint32_t h[FLAG_COUNT] = {0, 0, 0, 0};
   PR_HIP(hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, st));
