@@ -164,11 +164,15 @@ constexpr int kAdjDensityWaves = F == kF64 ? 5 : 6;
 template <int F>
 constexpr bool kAdjPrefetch = F == kMixed;
 
+// Entries staged for a group of runs (which groups walk as one stream decides how
+// the mixed passes round).
+constexpr uint32_t kAdjCap = 160;
+
 template <int F>
 struct AdjForceStage {
-  StageArr<typename SphForm<F>::G4, kForceCap> p, v;
-  typename SphForm<F>::R2 rp[kForceCap];
-  StageArr<typename AdjForm<F>::C4, kForceCap> c;
+  StageArr<typename SphForm<F>::G4, kAdjCap> p, v;
+  typename SphForm<F>::R2 rp[kAdjCap];
+  StageArr<typename AdjForm<F>::C4, kAdjCap> c;
 };
 
 template <int F, bool SPLIT>
@@ -274,7 +278,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjForceWaves<F>
         }
       }
     };
-    walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
+    walk_runs_staged<kUnr, kAdjCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
         rec.meta, rec.words, n, i, live, lane, SPLIT ? wave : 0u, SPLIT ? wave + 1u : kGroups,
         [&](uint32_t grp) {
           if constexpr (F == kMixed) pb_.begin(pi, grp, u.cs_u);
@@ -345,8 +349,8 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjForceWaves<F>
 // block, neighbour data staged per row run.
 template <int F>
 struct AdjDensityStage {
-  StageArr<typename SphForm<F>::G4, kForceCap> p;
-  typename AdjForm<F>::ar rb[kForceCap];
+  StageArr<typename SphForm<F>::G4, kAdjCap> p;
+  typename AdjForm<F>::ar rb[kAdjCap];
 };
 
 template <int F, bool SPLIT>
@@ -399,7 +403,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGroups : kAdjBlock, kAdjDensityWaves<
       qz += s * (ar)dzr;
     }
   };
-  walk_runs_staged<kUnr, kForceCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
+  walk_runs_staged<kUnr, kAdjCap, kAdjPrefetch<F> && !SPLIT, SPLIT>(
       rec.meta, rec.words, n, i, live, lane, SPLIT ? wave : 0u, SPLIT ? wave + 1u : kGroups,
       [&](uint32_t grp) {
         if constexpr (F == kMixed) pb_.begin(pi, grp, u.cs_u);

@@ -1028,7 +1028,13 @@ struct StageArr<double4, N> {
 constexpr int kForceBlock = 64;  // one wavefront: block barriers are wave barriers
 template <int F>
 constexpr int kForceWaves = F == kF64 ? 4 : 5;
-constexpr uint32_t kForceCap = 160;
+// Entries staged for a group of runs.  More let more groups walk their two runs
+// as one stream, until the LDS they take (FP64 64 bytes an entry, mixed 40, FP32
+// 32) costs wavefronts: force pass at 1M / 4M, us, for 136, 160, 192, 256: FP64
+// 1386, 1280, 1400, 1465 (4M); mixed 324, 303, 296, 302 (1M) and 1053, 978, 954,
+// 985; FP32 248, 233, 227, 231 and 821, 760, 738, 786.
+template <int F>
+constexpr uint32_t kForceCap = F == kF64 ? 160 : 192;
 // Mask words loaded one run group ahead in the force walk: in the FP64 form
 // (1152 -> 1098 us at 4M); the mixed form, at 5 wavefronts per SIMD, has no
 // registers to spare for them (888 -> 951 us), and the FP32 form gains
@@ -1164,8 +1170,8 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
   using real = typename SphForm<F>::real;
   using G4 = typename SphForm<F>::G4;
   using R2 = typename SphForm<F>::R2;
-  __shared__ StageArr<G4, kForceCap> s_p, s_v;
-  __shared__ R2 s_rp[F == kMixed ? kForceCap : 1];
+  __shared__ StageArr<G4, kForceCap<F>> s_p, s_v;
+  __shared__ R2 s_rp[F == kMixed ? kForceCap<F> : 1];
   const uint32_t lane = threadIdx.x;
   const uint32_t tile = xcd_tile(blockIdx.x);
   if (tile >= n_tiles) return;
@@ -1219,7 +1225,7 @@ __global__ __launch_bounds__(kForceBlock, kForceWaves<F>) void k_sph_force(
       }
     }
   };
-  walk_runs_staged<kUnr, kForceCap, kForcePrefetch<F>>(
+  walk_runs_staged<kUnr, kForceCap<F>, kForcePrefetch<F>>(
       meta, words, n, i, live, lane, 0u, kGroups, begin_group,
       [&](uint32_t k, uint32_t j) {
         s_p.put(k, gpos[j]);
