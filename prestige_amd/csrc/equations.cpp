@@ -985,8 +985,8 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "        __syncthreads();\n"
              "      }\n"
              "      // up to 128 candidates at a time: four scan words, then one walk of their set bits\n"
-             "      for (unsigned c0 = 0u; c0 < len; c0 += 128u) {\n"
-             "        const unsigned clen = len - c0 < 128u ? len - c0 : 128u;\n"
+             "      for (unsigned c_ = 0u; c_ < len; c_ += 128u) {\n"
+             "        const unsigned clen = len - c_ < 128u ? len - c_ : 128u;\n"
              "        unsigned wd[4] = {0u, 0u, 0u, 0u};\n"
              "#pragma unroll\n"
              "        for (unsigned w = 0u; w < 4u; ++w) {\n"
@@ -998,7 +998,7 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "            unsigned hb = 0u;\n"
              "#pragma unroll\n"
              "            for (unsigned u = 0u; u < 4u; ++u) {\n"
-             "              const unsigned jc = j0 + c0 + 32u * w + b + u;\n"
+             "              const unsigned jc = j0 + c_ + 32u * w + b + u;\n"
              "              bool hit;\n"
              "              if (staged) {\n"
              "                const float4 q = s_q[jc - base];\n"
@@ -1029,9 +1029,9 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "        while (m0 | m1) {\n"
              "          // two neighbours per trip, both positions loaded before either body runs\n"
              "          unsigned jsv[2];\n"
-             "          jsv[0] = j0 + c0 + pop();\n"
+             "          jsv[0] = j0 + c_ + pop();\n"
              "          const bool two = (m0 | m1) != 0ull;\n"
-             "          jsv[1] = two ? j0 + c0 + pop() : jsv[0];\n"
+             "          jsv[1] = two ? j0 + c_ + pop() : jsv[0];\n"
              "          const prestige_pos pjv[2] = {pos[jsv[0]], pos[jsv[1]]};\n"
              "#pragma unroll\n"
              "          for (int u_ = 0; u_ < 2; ++u_) {\n"
