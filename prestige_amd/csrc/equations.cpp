@@ -733,27 +733,43 @@ struct prestige_consts {
   double h, dt, rho0, c0, alpha, kn, kt, mu, gx, gy, gz;
   double two_zeta, neg_inv_kt;   // DEM: 2 zeta from the restitution, -1 / kt
 };
-// Cell-loop passes run one wavefront per block over 64 consecutive slots.  Per row
-// run the wavefront stages the union of its lanes' candidate ranges in LDS as FP32
-// offsets from its first slot in units of the cutoff (|q|^2 in .w); each lane scans
+// Cell-loop passes run one wavefront per block over 64 consecutive slots (pg_tile).
+// Per row run the wavefront stages the union of its lanes' candidate ranges in LDS as
+// FP32 offsets from its first slot in units of the cutoff (|q|^2 in .w); each lane scans
 // its own range into words of 32 candidates with the dot form q.w - 2 s.q < t, up
 // to 128 candidates at a time, and walks their set bits in ascending slot order, two
-// neighbours per trip, applying the exact FP64 test before the bodies.  The threshold t carries the rounding margin of the FP32 form, so the
-// scan keeps a superset of the exact neighbours and the bodies see exactly the
-// pairs and the order of the plain loop.
-__device__ inline unsigned pg_wave_min(unsigned v) {
-  for (int d = 32; d > 0; d >>= 1) {
-    const unsigned t = __shfl_xor(v, d, 64);
-    v = t < v ? t : v;
-  }
-  return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+// neighbours per trip, applying the exact FP64 test before the bodies.  The threshold t
+// carries the rounding margin of the FP32 form, so the scan keeps a superset of the exact
+// neighbours and the bodies see exactly the pairs and the order of the plain loop.
+//
+// pg_tile: blocks go round the 8 XCDs, so runs of 32 consecutive tiles are dealt to each
+// and its L2 keeps the cells they share; the blocks past the last whole round keep their
+// own tile, which makes it a permutation of any grid.
+__device__ inline unsigned pg_tile() {
+  const unsigned b = blockIdx.x;
+  if (b >= (gridDim.x & ~255u)) return b;
+  return (b & ~255u) + (b & 7u) * 32u + ((b >> 3) & 31u);
 }
-__device__ inline unsigned pg_wave_max(unsigned v) {
-  for (int d = 32; d > 0; d >>= 1) {
-    const unsigned t = __shfl_xor(v, d, 64);
-    v = t > v ? t : v;
+// maximum over the wavefront of the bits of a non-negative float, by row shifts and
+// broadcasts within the operation (lanes they do not reach combine with 0)
+__device__ inline float pg_wave_max(float f) {
+  unsigned v = __float_as_uint(f);
+#define PG_STEP(ctrl, rows)                                                                          \
+  {                                                                                                  \
+    const unsigned t = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false);     \
+    v = t > v ? t : v;                                                                               \
   }
-  return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+  PG_STEP(0x111, 0xF) PG_STEP(0x112, 0xF) PG_STEP(0x114, 0xF) PG_STEP(0x118, 0xF)
+  PG_STEP(0x142, 0xA) PG_STEP(0x143, 0xC)
+#undef PG_STEP
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)v, 63));
+}
+// word = 2 word + hit: the wavefront's hits are the carries of one addition
+__device__ inline unsigned pg_shift_in(unsigned w, bool hit) {
+  const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+  unsigned r;
+  asm("v_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(w), "s"(m) : "vcc");
+  return r;
 }
 // Tuples of doubles: (a, b, ..) in a body is pt_make(a, b, ..), t.k is pt_get<k>(t).
 template <int N> struct pt_tuple { double v[N]; };
@@ -928,7 +944,7 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
     s += "#pragma clang fp contract(off)\n";
     if (loop == PRESTIGE_LOOP_CELLS) {
       s += "  __shared__ float4 s_q[256 + 4];\n"
-           "  const unsigned lane = threadIdx.x, wbase = blockIdx.x * 64u, i = wbase + lane;\n"
+           "  const unsigned lane = threadIdx.x, wbase = pg_tile() * 64u, i = wbase + lane;\n"
            "  const bool live = i < n;\n"
            "  const unsigned me = live ? ids[i] : 0u;\n"
            "  const prestige_pos pi = pos[live ? i : wbase];\n"
@@ -957,7 +973,7 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "  const float4 so = offset(pi);\n"
              "  const float ax_ = -2.0f * so.x, ay_ = -2.0f * so.y, az_ = -2.0f * so.z;\n"
              "  const float ss = __builtin_fmaf(so.x, so.x, __builtin_fmaf(so.y, so.y, so.z * so.z));\n"
-             "  const unsigned ss_max = pg_wave_max(live ? __float_as_uint(ss) : 0u);\n"
+             "  const float ss_max = pg_wave_max(live ? ss : 0.0f);\n"
              "  for (int dz = -1; dz <= 1; ++dz) {\n"
              "    for (int dy = -1; dy <= 1; ++dy) {\n"
              "      const int zz = cz + dz, yy = cy + dy;\n"
@@ -967,9 +983,11 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "        j0 = lb[row + (unsigned)x0];\n"
              "        len = lb[row + (unsigned)x1 + 1] - j0;\n"
              "      }\n"
-             "      const unsigned base = pg_wave_min(len ? j0 : 0xFFFFFFFFu);\n"
-             "      const unsigned top = pg_wave_max(len ? j0 + len : 0u);\n"
-             "      if (top <= base) continue;\n"
+             "      // slots are in key order: the first and last lane with candidates bound their union\n"
+             "      const unsigned long long any = __builtin_amdgcn_ballot_w64(len != 0u);\n"
+             "      if (any == 0ull) continue;\n"
+             "      const unsigned base = (unsigned)__builtin_amdgcn_readlane((int)j0, (int)__builtin_ctzll(any));\n"
+             "      const unsigned top = (unsigned)__builtin_amdgcn_readlane((int)(j0 + len), 63 - (int)__builtin_clzll(any));\n"
              "      const bool staged = top - base <= 256u;\n"
              "      float t = 0.0f;\n"
              "      if (staged) {\n"
@@ -980,7 +998,7 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "          s_q[kk] = q;\n"
              "          mq = q.w > mq ? q.w : mq;\n"
              "        }\n"
-             "        const float m2 = fmaxf(__uint_as_float(ss_max), __uint_as_float(pg_wave_max(__float_as_uint(mq))));\n"
+             "        const float m2 = fmaxf(ss_max, pg_wave_max(mq));\n"
              "        t = thr + 0x1.0p-19f * (m2 + __builtin_sqrtf(m2) + 1.0f) - ss;\n"
              "        __syncthreads();\n"
              "      }\n"
@@ -993,25 +1011,30 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "          if (32u * w >= clen) break;\n"
              "          const unsigned cnt = clen - 32u * w < 32u ? clen - 32u * w : 32u;\n"
              "          unsigned word = 0u;\n"
-             "          // four candidates per trip; those past cnt (stage padding, clamped slots) are masked off\n"
-             "          for (unsigned b = 0u; b < cnt; b += 4u) {\n"
-             "            unsigned hb = 0u;\n"
+             "          // four candidates per trip, hits shifted in from the right; those past cnt (stage\n"
+             "          // padding, clamped slots) are masked off\n"
+             "          const unsigned jw = j0 + c_ + 32u * w;\n"
+             "          if (staged) {\n"
+             "            for (unsigned b = 0u; b < cnt; b += 4u) {\n"
+             "              float4 q[4];\n"
              "#pragma unroll\n"
-             "            for (unsigned u = 0u; u < 4u; ++u) {\n"
-             "              const unsigned jc = j0 + c_ + 32u * w + b + u;\n"
-             "              bool hit;\n"
-             "              if (staged) {\n"
-             "                const float4 q = s_q[jc - base];\n"
-             "                hit = __builtin_fmaf(ax_, q.x, __builtin_fmaf(ay_, q.y, __builtin_fmaf(az_, q.z, q.w))) < t;\n"
-             "              } else {\n"
-             "                const float4 q = offset(pos[jc < n ? jc : n - 1u]);\n"
-             "                const float ddx = so.x - q.x, ddy = so.y - q.y, ddz = so.z - q.z;\n"
-             "                hit = __builtin_fmaf(ddx, ddx, __builtin_fmaf(ddy, ddy, ddz * ddz)) < thr;\n"
-             "              }\n"
-             "              hb |= (hit ? 1u : 0u) << u;\n"
+             "              for (unsigned u = 0u; u < 4u; ++u) q[u] = s_q[jw - base + b + u];\n"
+             "#pragma unroll\n"
+             "              for (unsigned u = 0u; u < 4u; ++u)\n"
+             "                word = pg_shift_in(word, __builtin_fmaf(ax_, q[u].x, __builtin_fmaf(ay_, q[u].y,\n"
+             "                                                 __builtin_fmaf(az_, q[u].z, q[u].w))) < t);\n"
              "            }\n"
-             "            word |= hb << b;\n"
+             "          } else {\n"
+             "            for (unsigned b = 0u; b < cnt; b += 4u) {\n"
+             "#pragma unroll\n"
+             "              for (unsigned u = 0u; u < 4u; ++u) {\n"
+             "                const float4 q = offset(pos[jw + b + u < n ? jw + b + u : n - 1u]);\n"
+             "                const float ddx = so.x - q.x, ddy = so.y - q.y, ddz = so.z - q.z;\n"
+             "                word = pg_shift_in(word, __builtin_fmaf(ddx, ddx, __builtin_fmaf(ddy, ddy, ddz * ddz)) < thr);\n"
+             "              }\n"
+             "            }\n"
              "          }\n"
+             "          word = __builtin_bitreverse32(word) >> (32u - ((cnt + 3u) & ~3u));\n"
              "          wd[w] = cnt < 32u ? word & ((1u << cnt) - 1u) : word;\n"
              "        }\n"
              "        unsigned long long m0 = (unsigned long long)wd[0] | ((unsigned long long)wd[1] << 32);\n"
