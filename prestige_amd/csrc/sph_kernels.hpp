@@ -262,14 +262,12 @@ __device__ inline real spline_df(real q) {
 // Loads kept in flight per lane.  The gathers are latency-bound (dependent
 // loads, little arithmetic per byte), so each lane issues a batch of
 // independent loads before it uses any of them: kScanUnr candidates in the
-// density scan, kDensUnr neighbours in the density walk, kUnr neighbours in
-// the walks of the force pass and the adjoint.
+// density scan, kUnr neighbours in the walks of the force pass and the adjoint.
 constexpr int kScanUnr = 2;
-constexpr int kDensUnr = 2;
 constexpr int kUnr = 2;
 constexpr int kMaskUnr = 8;   // candidates in flight in the scan that only keeps masks
 static_assert(kScanUnr == 1 || kScanUnr == 2 || kScanUnr == 4, "scan batch divides 32");
-static_assert(kDensUnr >= 1 && kUnr >= 1, "walk batches hold at least one neighbour");
+static_assert(kUnr >= 1, "walk batches hold at least one neighbour");
 constexpr uint32_t kPad = 0xFFFFFFFFu;
 
 // Candidate coordinates for the scan: offsets from a reference point of the
@@ -849,6 +847,23 @@ __global__ __launch_bounds__(kDensBlock, WALK ? kDensWaves<F> : 4) void k_sph_de
   const float ss_max = wave_max_pos(ss);
   const real H2 = (real)u.H2, inv_h = (real)u.inv_h;
   Sum<real, F == kMixed> acc;
+  // pair with a neighbour in run t of its group (mixed: y and z bases of both runs)
+  auto term = [&](const G4& pj, uint32_t t, const float* by, const float* bz) {
+    real dx, dy, dz;
+    if constexpr (F == kMixed) {
+      dx = (pi.x - pj.x) - (float)cell_shift(__float_as_uint(pi.w), __float_as_uint(pj.w), 0) * u.cs_u;
+      dy = (t ? by[1] : by[0]) - pj.y;
+      dz = (t ? bz[1] : bz[0]) - pj.z;
+    } else {
+      form_pair<F>(pi, pj, u.cs_u, dx, dy, dz);
+    }
+    const real r2 = dot3(dx, dy, dz, dx, dy, dz);
+    if (r2 < H2) {
+      // the self pair (and coincident slots) has r2 = 0, q = 0
+      const real q = r2 > real(0.0) ? sqrt_pos(r2) * inv_h : real(0.0);
+      acc.add(spline_f(q));
+    }
+  };
   bool overflow = false;
   const int nx = g.dims[0], ny = g.dims[1], nz = g.dims[2];
   // Runs in the WCSPH order, scanned one at a time and walked a group at a
@@ -950,36 +965,17 @@ __global__ __launch_bounds__(kDensBlock, WALK ? kDensWaves<F> : 4) void k_sph_de
       wb[2u * t] = gj0[t] | tag;
       wb[2u * t + 1u] = (gj0[t] + 64u) | tag;
     }
-    walk_bits_q<kDensUnr>(m, wb, [&](const uint32_t* jj) {
-      uint32_t js[kDensUnr], tv[kDensUnr];
-#pragma unroll
-      for (int v = 0; v < kDensUnr; ++v) {
-        const uint32_t q = jj[v] == kPad ? jj[0] : jj[v];
-        tv[v] = F == kMixed ? q >> 31 : 0u;
-        js[v] = F == kMixed ? q & 0x7FFFFFFFu : q;
-      }
-      G4 pj[kDensUnr];
-#pragma unroll
-      for (int v = 0; v < kDensUnr; ++v) pj[v] = pos[js[v]];
-#pragma unroll
-      for (int v = 0; v < kDensUnr; ++v) {
-        if (jj[v] == kPad) continue;
-        real dx, dy, dz;
-        if constexpr (F == kMixed) {
-          dx = (pi.x - pj[v].x) - (float)cell_shift(__float_as_uint(pi.w), __float_as_uint(pj[v].w), 0) * u.cs_u;
-          dy = (tv[v] ? gby[1] : gby[0]) - pj[v].y;
-          dz = (tv[v] ? gbz[1] : gbz[0]) - pj[v].z;
-        } else {
-          form_pair<F>(pi, pj[v], u.cs_u, dx, dy, dz);
-        }
-        real r2 = dot3(dx, dy, dz, dx, dy, dz);
-        if (r2 < H2) {
-          // the self pair (and coincident slots) has r2 = 0, q = 0
-          real q = r2 > real(0.0) ? sqrt_pos(r2) * inv_h : real(0.0);
-          acc.add(spline_f(q));
-        }
-      }
+    // one pair at a time, the next neighbour's position read meanwhile
+    G4 pj{};
+    uint32_t tj = kPad;   // run of the pair at hand (kPad: none yet)
+    walk_bits_q<1>(m, wb, [&](const uint32_t* jj) {
+      const uint32_t q = jj[0];
+      const G4 next = pos[F == kMixed ? q & 0x7FFFFFFFu : q];
+      if (tj != kPad) term(pj, tj, gby, gbz);
+      pj = next;
+      tj = F == kMixed ? q >> 31 : 0u;
     });
+    if (tj != kPad) term(pj, tj, gby, gbz);
   }
   if (!WALK || !live) return;
   if (overflow) atomicOr(&flags[FLAG_CAPACITY], 1u);
