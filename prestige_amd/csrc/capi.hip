@@ -315,12 +315,13 @@ static void allocate(Ctx& c) {
     c.nword.alloc(nn * 36 * sizeof(uint32_t));
     // Four lanes per particle (sph_quad.hpp) where one lane per particle
     // leaves the device idle.  Density + force, one lane / four lanes, us, at
-    // 8k, 64k, 250k and 500k moving particles: FP64 128/45, 158/98, 269/226,
-    // 425/458; FP32 115/39, 135/80, 193/167, 301/320; mixed 144/44, 175/98,
-    // 228/211, 359/424.  The line lies where the two meet (mixed a little
-    // lower: its compensated sums run under a mask).  The lists take 516 B a
-    // particle, so a context of over a million particles does without.
-    const uint64_t most = mixed ? 290000u : 380000u;
+    // 8k, 64k, 200k, 300k, 350k and 500k moving particles: FP64 122/45, 157/100,
+    // 228/211, 294/290, 329/335, 424/480; FP32 109/40, 126/82, 165/154, 206/202,
+    // 229/233, 286/330; mixed 138/45, 172/99, 227/193, 257/258, 280/315, 344/440.
+    // The line lies where the two meet (mixed earlier, 225/227 at 250k: its
+    // compensated sums run under a mask).  The lists take 516 B a particle, so a
+    // context of over a million particles does without.
+    const uint64_t most = mixed ? 240000u : 320000u;
     c.quad = c.n_moving <= most && n <= 1000000u;
     if (const char* e = std::getenv("PRESTIGE_QUAD")) {
       if (std::string(e) == "on") c.quad = true;

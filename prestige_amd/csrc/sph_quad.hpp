@@ -13,10 +13,12 @@
 // candidates are loaded while the previous run is scanned, the hits of all
 // runs become one list per particle, and the walk knows every neighbour's
 // address ahead.  Density / force, us, against one lane per particle: 42,866
-// particles FP64 72 / 56 -> 27 / 17, 196k mixed 110 / 65 -> 60 / 38, 571k FP32
-// 108 / 85 -> 115 / 53.  What bounds them now: at 42,866 particles the chain
-// of about eight dependent memory reads; at 571k instruction issue, which for
-// the density pass is 1.2 times the one-lane kernel's.
+// particles FP64 67 / 55 -> 27 / 17, 196k mixed 109 / 63 -> 61 / 38, 571k FP32
+// 98 / 87 -> 120 / 55.  What bounds them now: at 42,866 particles a wavefront's
+// own chain (alone on its SIMD a chunk of 64 candidates takes 1,700 cycles, five
+// trips through LDS and ten rounds of writing hits among them, and a round of
+// the walk 1,000; deeper prefetch changes nothing); at 571k instruction issue
+// and the texture path, each 80 % busy in the density pass.
 #pragma once
 
 namespace prestige {
