@@ -270,7 +270,8 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
   const uint32_t self = in ? k : tile * kQuadSlots;
   const uint32_t me = s.ids[self], dst = s.perm[self];
   const bool live = in && (uint64_t)me < n_moving;
-  const uint32_t cin = in ? s.cnt_in[me] : 0u, cout = live ? s.cnt_out[me] : 0u;
+  const uint32_t had_in = in ? s.cnt_in[me] : 0u;   // contacts and walls (DemHist)
+  const uint32_t cin = had_in & 0xFFu, cout = live ? s.cnt_out[me] & 0xFFu : 0u;
   double pk = 0.0, pt = 0.0, pm = 0.0;
   V3 X = v3(0, 0, 0), V = v3(0, 0, 0), W = v3(0, 0, 0);
   if (sub == 0u) s_had[p] = 0u;
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
   for (uint32_t c = sub; c < cout; c += 4u) {
     const uint32_t pid = s.hid_out[(size_t)c * n + me];
     const uint32_t j = s.slot_of[pid];
-    const uint32_t cjin = s.cnt_in[pid], cjout = s.cnt_out[pid];
+    const uint32_t cjin = s.cnt_in[pid] & 0xFFu, cjout = s.cnt_out[pid] & 0xFFu;
     const double4 pj4 = s.pos[j], vj4 = s.vel[j], wj4 = s.om[j];
     const bool jm = (uint64_t)pid < n_moving;
     const V3 Fbj = jm ? xyz(Fb[j]) : v3(0, 0, 0), Tbj = jm ? xyz(Tb[j]) : v3(0, 0, 0);
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
       }
       V3 xob = v3(0, 0, 0);
       if (on) {
-        const V3 xo = load_xi(wxi_in, (uint32_t)w, n, me);
+        const V3 xo = (had_in >> (8 + w)) & 1u ? load_xi(wxi_in, (uint32_t)w, n, me) : v3(0, 0, 0);
         const V3 xnb = load3(wallb_next, (uint32_t)w, n, me);
         const RowBar a = row_vjp(true, v3(0, 0, 0), nw, delta, vk, v3(0, 0, 0), wk, v3(0, 0, 0), rk, 0.0, mk, 0.0, xo,
                                  Fbk, Tbk, xnb, kc);
