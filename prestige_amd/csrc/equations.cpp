@@ -771,6 +771,11 @@ __device__ inline unsigned pg_shift_in(unsigned w, bool hit) {
   asm("v_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(w), "s"(m) : "vcc");
   return r;
 }
+// the word of cnt candidates shifted in four at a time: candidate 0 in bit 0
+__device__ inline unsigned pg_word(unsigned w, unsigned cnt) {
+  w = __builtin_bitreverse32(w) >> (32u - ((cnt + 3u) & ~3u));
+  return cnt < 32u ? w & ((1u << cnt) - 1u) : w;
+}
 // Tuples of doubles: (a, b, ..) in a body is pt_make(a, b, ..), t.k is pt_get<k>(t).
 template <int N> struct pt_tuple { double v[N]; };
 template <class... A> __device__ inline pt_tuple<(int)sizeof...(A)> pt_make(A... a) {
@@ -1006,36 +1011,46 @@ GenProgram build_program(const int32_t* ids, uint32_t n, int32_t loop, bool f32_
              "      for (unsigned c_ = 0u; c_ < len; c_ += 128u) {\n"
              "        const unsigned clen = len - c_ < 128u ? len - c_ : 128u;\n"
              "        unsigned wd[4] = {0u, 0u, 0u, 0u};\n"
+             "        // four candidates per trip, hits shifted in from the right; those past cnt (stage\n"
+             "        // padding, clamped slots) are masked off\n"
+             "        if (staged) {\n"
              "#pragma unroll\n"
-             "        for (unsigned w = 0u; w < 4u; ++w) {\n"
-             "          if (32u * w >= clen) break;\n"
-             "          const unsigned cnt = clen - 32u * w < 32u ? clen - 32u * w : 32u;\n"
-             "          unsigned word = 0u;\n"
-             "          // four candidates per trip, hits shifted in from the right; those past cnt (stage\n"
-             "          // padding, clamped slots) are masked off\n"
-             "          const unsigned jw = j0 + c_ + 32u * w;\n"
-             "          if (staged) {\n"
+             "          for (unsigned w = 0u; w < 4u; ++w) {\n"
+             "            if (32u * w >= clen) break;\n"
+             "            const unsigned cnt = clen - 32u * w < 32u ? clen - 32u * w : 32u;\n"
+             "            const unsigned first = j0 - base + c_ + 32u * w;\n"
+             "            unsigned word = 0u;\n"
              "            for (unsigned b = 0u; b < cnt; b += 4u) {\n"
              "              float4 q[4];\n"
              "#pragma unroll\n"
-             "              for (unsigned u = 0u; u < 4u; ++u) q[u] = s_q[jw - base + b + u];\n"
+             "              for (unsigned u = 0u; u < 4u; ++u) q[u] = s_q[first + b + u];\n"
              "#pragma unroll\n"
              "              for (unsigned u = 0u; u < 4u; ++u)\n"
              "                word = pg_shift_in(word, __builtin_fmaf(ax_, q[u].x, __builtin_fmaf(ay_, q[u].y,\n"
              "                                                 __builtin_fmaf(az_, q[u].z, q[u].w))) < t);\n"
              "            }\n"
-             "          } else {\n"
+             "            wd[w] = pg_word(word, cnt);\n"
+             "          }\n"
+             "        } else {\n"
+             "#pragma unroll 1\n"
+             "          for (unsigned w = 0u; 32u * w < clen; ++w) {\n"
+             "            const unsigned cnt = clen - 32u * w < 32u ? clen - 32u * w : 32u;\n"
+             "            const unsigned first = j0 + c_ + 32u * w;\n"
+             "            unsigned word = 0u;\n"
              "            for (unsigned b = 0u; b < cnt; b += 4u) {\n"
              "#pragma unroll\n"
              "              for (unsigned u = 0u; u < 4u; ++u) {\n"
-             "                const float4 q = offset(pos[jw + b + u < n ? jw + b + u : n - 1u]);\n"
+             "                const float4 q = offset(pos[first + b + u < n ? first + b + u : n - 1u]);\n"
              "                const float ddx = so.x - q.x, ddy = so.y - q.y, ddz = so.z - q.z;\n"
              "                word = pg_shift_in(word, __builtin_fmaf(ddx, ddx, __builtin_fmaf(ddy, ddy, ddz * ddz)) < thr);\n"
              "              }\n"
              "            }\n"
+             "            word = pg_word(word, cnt);\n"
+             "            if (w == 0u) wd[0] = word;\n"
+             "            else if (w == 1u) wd[1] = word;\n"
+             "            else if (w == 2u) wd[2] = word;\n"
+             "            else wd[3] = word;\n"
              "          }\n"
-             "          word = __builtin_bitreverse32(word) >> (32u - ((cnt + 3u) & ~3u));\n"
-             "          wd[w] = cnt < 32u ? word & ((1u << cnt) - 1u) : word;\n"
              "        }\n"
              "        unsigned long long m0 = (unsigned long long)wd[0] | ((unsigned long long)wd[1] << 32);\n"
              "        unsigned long long m1 = (unsigned long long)wd[2] | ((unsigned long long)wd[3] << 32);\n"
