@@ -255,7 +255,9 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
                                                 const double4* __restrict__ Fb, const double4* __restrict__ Tb,
                                                 const double* __restrict__ hb_next,
                                                 const double* __restrict__ wallb_next,
+                                                const uint32_t* __restrict__ wallm_next,
                                                 double* __restrict__ hb_prev, double* __restrict__ wallb_prev,
+                                                uint32_t* __restrict__ wallm_prev,
                                                 double4* __restrict__ xb_out, double4* __restrict__ vb_out,
                                                 double4* __restrict__ wb_out, double4* __restrict__ partial,
                                                 uint32_t n_tiles) {
@@ -328,7 +330,12 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
   V = quad_sum3(V);
   W = quad_sum3(W);
   if (in) {
-    // walls: the quad's lanes compute the same, each stores its share
+    // walls: the quad's lanes compute the same, each stores its share.  The
+    // spring of a wall has an adjoint where the step touched the wall (wallm);
+    // every other is zero and neither written nor read (100,000 mixed spheres
+    // with few contacts: 26 -> 23 us a pass).
+    const uint32_t later = wallm_next[me];
+    uint32_t walls = 0;
     for (int w = 0; w < 6; ++w) {
       bool on = false;
       double delta = 0.0;
@@ -342,24 +349,24 @@ __global__ __launch_bounds__(64) void k_dem_adj(uint32_t n, uint64_t n_moving, D
         const double sgn = (w & 1) ? -1.0 : 1.0;
         nw = v3(ax == 0 ? sgn : 0.0, ax == 1 ? sgn : 0.0, ax == 2 ? sgn : 0.0);
       }
-      V3 xob = v3(0, 0, 0);
       if (on) {
         const V3 xo = (had_in >> (8 + w)) & 1u ? load_xi(wxi_in, (uint32_t)w, n, me) : v3(0, 0, 0);
-        const V3 xnb = load3(wallb_next, (uint32_t)w, n, me);
+        const V3 xnb = (later >> w) & 1u ? load3(wallb_next, (uint32_t)w, n, me) : v3(0, 0, 0);
         const RowBar a = row_vjp(true, v3(0, 0, 0), nw, delta, vk, v3(0, 0, 0), wk, v3(0, 0, 0), rk, 0.0, mk, 0.0, xo,
                                  Fbk, Tbk, xnb, kc);
         X = X + a.d;
         V = V + a.vi;
         W = W + a.wi;
-        xob = a.xo;
+        walls |= 1u << w;
+        if ((uint32_t)(w & 3) == sub) store3(wallb_prev, (uint32_t)w, n, me, a.xo);
         if (sub == 0u) {
           pk += a.kn;
           pt += a.tz;
           pm += a.mu;
         }
       }
-      if ((uint32_t)(w & 3) == sub) store3(wallb_prev, (uint32_t)w, n, me, xob);
     }
+    if (sub == 0u) wallm_prev[me] = walls;
     const V3 z = v3(0, 0, 0);
     if (sub < 3u) {
       const double4* from = sub == 0u ? xb_in : (sub == 1u ? vb_in : wb_in);
@@ -511,16 +518,18 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
   T.hb[1].alloc(nn * mc * 3 * sizeof(double));
   T.wallb[0].alloc(nn * 18 * sizeof(double));
   T.wallb[1].alloc(nn * 18 * sizeof(double));
+  for (DevBuf& b : T.wallm) b.alloc(nn * 4);
   T.slot_of.alloc(nn * 4);
   PR_HIP(hipMemsetAsync(T.acc.p, 0, 3 * sizeof(double), c.stream));
   PR_HIP(hipMemsetAsync(T.wb.p, 0, nn * sizeof(double4), c.stream));
   PR_HIP(hipMemsetAsync(T.hb[0].p, 0, nn * mc * 3 * sizeof(double), c.stream));
-  PR_HIP(hipMemsetAsync(T.wallb[0].p, 0, nn * 18 * sizeof(double), c.stream));
+  PR_HIP(hipMemsetAsync(T.wallm[0].p, 0, nn * 4, c.stream));
   adj_seed_gather(c, T.final_state->ids.as<uint32_t>(), seed_x, seed_v);
   double4 *xb = T.xb.as<double4>(), *vb = T.vb.as<double4>(), *wb = T.wb.as<double4>();
   double4 *xb2 = T.xb2.as<double4>(), *vb2 = T.vb2.as<double4>(), *wb2 = T.wb2.as<double4>();
   double *hn = T.hb[0].as<double>(), *hp = T.hb[1].as<double>();
   double *wn = T.wallb[0].as<double>(), *wp = T.wallb[1].as<double>();
+  uint32_t *mn = T.wallm[0].as<uint32_t>(), *mp = T.wallm[1].as<uint32_t>();
   const DemAdjConst kc = dem_adj_const(c);
   const uint32_t nseg = (T.nsteps + T.every - 1) / T.every;
   while (T.rec.size() < T.every) T.rec.emplace_back(new StepRecord());
@@ -547,7 +556,7 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       k_dem_adj_prep<<<nb, kBlock, 0, c.stream>>>(n, c.n_moving, v, xb, vb, wb, T.cvec.as<double4>(),
                                                   T.xbf.as<double4>(), c.dem.dt, T.slot_of.as<uint32_t>());
       k_dem_adj<H><<<tile_grid(tiles), 64, 0, c.stream>>>(
-          n, c.n_moving, v, kc, xb, vb, wb, T.cvec.as<double4>(), T.xbf.as<double4>(), hn, wn, hp, wp, xb2, vb2, wb2,
+          n, c.n_moving, v, kc, xb, vb, wb, T.cvec.as<double4>(), T.xbf.as<double4>(), hn, wn, mn, hp, wp, mp, xb2, vb2, wb2,
           T.partial.as<double4>() + (size_t)tiles * (len - 1u - t), tiles);
       PR_HIP(hipGetLastError());
       std::swap(xb, xb2);
@@ -555,6 +564,7 @@ void dem_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       std::swap(wb, wb2);
       std::swap(hn, hp);
       std::swap(wn, wp);
+      std::swap(mn, mp);
     }
     if (n) {   // the segment's parameter sums
       k_dem_adj_reduce<<<len, 256, 0, c.stream>>>(tiles, T.partial.as<double4>());

@@ -236,6 +236,7 @@ struct Tape {
   std::vector<std::unique_ptr<StepRecord>> rec;  // reused across segments
   DevBuf xb, vb, xb2, vb2, cvec, xbf, rhob, partial, acc, seeds, wb, wb2;
   DevBuf hb[2], wallb[2], slot_of;   // DEM history adjoints (ping-pong), id -> slot
+  DevBuf wallm[2];              // walls a step touched, by particle id (bits 0-5)
   // Start a new tape; checkpoint buffers are kept and reused.
   void clear() {
     n_ckpt = 0;
