@@ -264,6 +264,7 @@ static void allocate(Ctx& c) {
   if (c.desc.model != PRESTIGE_MODEL_PAIRS) {
     const size_t cells = (size_t)c.grid.n_cells + 1;
     c.inc_tiles = (cells + kCellTile - 1) / kCellTile;
+    c.inc_one = inc_in_one(n, c.inc_tiles);
     c.inc_mask.alloc(((nn + 63) / 64) * 8);
     c.inc_next.alloc(nn * 4);
     c.lb_spare.alloc(cells * 4);

@@ -143,6 +143,8 @@ struct Timing {
 };
 
 struct Ctx;
+// Whether a context of n slots builds in one launch after a step (neighbors.hip).
+bool inc_in_one(uint64_t n, size_t cell_tiles);
 
 // What the step kernels leave for the next build's incremental sort.  A slot
 // whose particle changes cell ("moved", fixed particles never do) counts into
@@ -150,8 +152,10 @@ struct Ctx;
 // tile of kCellTile cells (tin, tout), and is linked into its new cell's list:
 // head[c] holds (epoch << 32 | last slot linked), next[slot] the slot linked
 // before it (kListEnd for the first of this epoch, so heads need no clearing).
-// Word w of mask has bit l set when slot 64 w + l moved.
+// Word w of mask has bit l set when slot 64 w + l moved.  Contexts whose build is
+// one launch also take what came less what left per kCellGroup cells (gnet).
 constexpr uint32_t kCellTile = 1024;
+constexpr uint32_t kCellGroup = 32;
 constexpr uint32_t kListEnd = 0xFFFFFFFFu;
 // Slots one cell's list takes in one step.  Steps within the CFL bounds stay
 // far below; a runaway that throws more than this into one cell leaves the
@@ -160,7 +164,7 @@ constexpr uint32_t kListEnd = 0xFFFFFFFFu;
 constexpr uint32_t kMaxIn = 1u << 16;
 struct MovedOut {
   uint64_t* mask;
-  uint32_t *cin, *cout, *tin, *tout;
+  uint32_t *cin, *cout, *tin, *tout, *gnet;
   uint64_t* head;
   uint32_t* next;
   uint32_t epoch;
@@ -179,6 +183,10 @@ __device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old
   atomicAdd(&mo.cout[old_key], 1u);
   atomicAdd(&mo.tin[key / kCellTile], 1u);
   atomicAdd(&mo.tout[old_key / kCellTile], 1u);
+  if (mo.gnet && key / kCellGroup != old_key / kCellGroup) {
+    atomicAdd(&mo.gnet[key / kCellGroup], 1u);
+    atomicSub(&mo.gnet[old_key / kCellGroup], 1u);
+  }
   const unsigned long long mine = ((unsigned long long)mo.epoch << 32) | i;
   const unsigned long long last = atomicExch(reinterpret_cast<unsigned long long*>(&mo.head[key]), mine);
   mo.next[i] = (uint32_t)(last >> 32) == mo.epoch ? (uint32_t)last : kListEnd;
@@ -284,15 +292,23 @@ struct Ctx {
   DevBuf sort_hist, sort_tot;    // per-tile digit counts, per-digit totals
   // incremental sort (MovedOut): moved-slot mask, links per slot, the spare
   // cell table, and in one buffer the list heads per cell and the counts cin,
-  // cout (inc_tiles * kCellTile each), tin, tout (inc_tiles each)
+  // cout (inc_tiles * kCellTile each), gnet (a kCellGroup-th of that), tin, tout
+  // (inc_tiles each).  Where the build is one launch there are two sets of
+  // counts: a step writes set inc_set, its build reads it and clears the other.
   DevBuf inc_mask, inc_next, lb_spare, inc_cells;
   size_t inc_tiles = 0;
   uint64_t* inc_head() const { return inc_cells.as<uint64_t>(); }
-  uint32_t* inc_cin() const { return reinterpret_cast<uint32_t*>(inc_head() + inc_tiles * kCellTile); }
-  uint32_t* inc_cout() const { return inc_cin() + inc_tiles * kCellTile; }
-  uint32_t* inc_tin() const { return inc_cout() + inc_tiles * kCellTile; }
-  uint32_t* inc_tout() const { return inc_tin() + inc_tiles; }
-  size_t inc_count_bytes() const { return inc_tiles * (2 * kCellTile + 2) * 4; }   // from inc_cin() on
+  size_t inc_set_words() const { return (inc_tiles * (2 * kCellTile + kCellTile / kCellGroup + 2) + 3) / 4 * 4; }
+  uint32_t* inc_cin(int set) const {
+    return reinterpret_cast<uint32_t*>(inc_head() + inc_tiles * kCellTile) + set * inc_set_words();
+  }
+  uint32_t* inc_cout(int set) const { return inc_cin(set) + inc_tiles * kCellTile; }
+  uint32_t* inc_gnet(int set) const { return inc_cout(set) + inc_tiles * kCellTile; }
+  uint32_t* inc_tin(int set) const { return inc_gnet(set) + inc_tiles * (kCellTile / kCellGroup); }
+  uint32_t* inc_tout(int set) const { return inc_tin(set) + inc_tiles; }
+  size_t inc_count_bytes() const { return (inc_one ? 2 : 1) * inc_set_words() * 4; }   // from inc_cin(0) on
+  bool inc_one = false;          // the build after a step is one launch
+  int inc_set = 0;
   uint32_t inc_epoch = 1;
   bool inc_ready = false;        // keys[cur_key] are the next keys of the last build's slots
   bool inc_counts = false;       // a step's counts are waiting (a build that does not use them clears them)

@@ -389,7 +389,8 @@ double reorder_bytes(const Ctx& c) {
 // launches, the cell table and the placement, which also moves the particle
 // state, replace the radix sort's launches, the reorder and the cell table's;
 // permutation and keys are exactly the stable sort's.  Lists have no order (the
-// step's atomics link them), but only counts are taken from them.
+// step's atomics link them), but only counts are taken from them.  Small scenes
+// do both in one launch (k_inc_one).
 //
 // Us per step, against gathering the moved entries, sorting them, merging and
 // a cell table (up to 8,192 moved; the radix path above): 42,866 particles 19
@@ -401,13 +402,13 @@ double reorder_bytes(const Ctx& c) {
 // New cell table of tile b (kCellTile cells): the offset before it from the
 // tile totals, then a block scan of the cells' net counts, which are cleared
 // for the next step.  A tile nothing entered or left only adds its offset.
-__global__ __launch_bounds__(kBlock) void k_inc_cells(uint32_t n_cells, const uint32_t* __restrict__ lb_old,
-                                                      const uint32_t* __restrict__ tin,
-                                                      const uint32_t* __restrict__ tout, uint4* __restrict__ cin,
-                                                      uint4* __restrict__ cout, uint32_t* __restrict__ lb) {
+template <bool CLEAR>
+__device__ inline void cell_tile(uint32_t b, uint32_t n_cells, const uint32_t* __restrict__ lb_old,
+                                 const uint32_t* __restrict__ tin, const uint32_t* __restrict__ tout,
+                                 uint4* __restrict__ cin, uint4* __restrict__ cout, uint32_t* __restrict__ lb) {
   static_assert(kCellTile == 4 * kBlock, "four cells per thread");
   __shared__ uint32_t s4[4];
-  const uint32_t b = blockIdx.x, t = threadIdx.x;
+  const uint32_t t = threadIdx.x;
   const bool busy = (tin[b] | tout[b]) != 0u;
   uint32_t part = 0;
   for (uint32_t k = t; k < b; k += kBlock) part += tin[k] - tout[k];
@@ -421,8 +422,8 @@ __global__ __launch_bounds__(kBlock) void k_inc_cells(uint32_t n_cells, const ui
     const uint32_t q = b * kBlock + t;
     const uint4 in = cin[q], out = cout[q];
     d[0] = in.x - out.x; d[1] = in.y - out.y; d[2] = in.z - out.z; d[3] = in.w - out.w;
-    if (in.x | in.y | in.z | in.w) cin[q] = make_uint4(0u, 0u, 0u, 0u);
-    if (out.x | out.y | out.z | out.w) cout[q] = make_uint4(0u, 0u, 0u, 0u);
+    if (CLEAR && (in.x | in.y | in.z | in.w)) cin[q] = make_uint4(0u, 0u, 0u, 0u);
+    if (CLEAR && (out.x | out.y | out.z | out.w)) cout[q] = make_uint4(0u, 0u, 0u, 0u);
     uint32_t total;
     run += block_excl_scan(d[0] + d[1] + d[2] + d[3], s4, &total);
   }
@@ -434,6 +435,13 @@ __global__ __launch_bounds__(kBlock) void k_inc_cells(uint32_t n_cells, const ui
   }
 }
 
+__global__ __launch_bounds__(kBlock) void k_inc_cells(uint32_t n_cells, const uint32_t* __restrict__ lb_old,
+                                                      const uint32_t* __restrict__ tin,
+                                                      const uint32_t* __restrict__ tout, uint4* __restrict__ cin,
+                                                      uint4* __restrict__ cout, uint32_t* __restrict__ lb) {
+  cell_tile<true>(blockIdx.x, n_cells, lb_old, tin, tout, cin, cout, lb);
+}
+
 // Set bits of the moved-slot mask in [a, b).
 __device__ inline uint32_t moved_in(const uint64_t* __restrict__ mask, uint32_t a, uint32_t b) {
   if (a >= b) return 0u;
@@ -443,6 +451,22 @@ __device__ inline uint32_t moved_in(const uint64_t* __restrict__ mask, uint32_t 
   for (uint32_t k = wa; k < wb; w = mask[++k]) cnt += (uint32_t)__popcll(w);
   const uint32_t top = b & 63u;   // 0: the last word counts whole
   return cnt + (uint32_t)__popcll(top ? w & ((1ull << top) - 1ull) : w);
+}
+
+// Place in the new order of slot i, now in cell c: o0, o1 and l0, l1 are the
+// cell's bounds in the old and the new table, hd its list's head.
+__device__ inline uint32_t place_of(uint32_t i, uint32_t o0, uint32_t o1, uint32_t l0, uint32_t l1, uint64_t hd,
+                                    uint32_t epoch, const uint64_t* __restrict__ mask,
+                                    const uint32_t* __restrict__ next) {
+  uint32_t below = 0, above = 0;   // incoming slots before i, and i or after it
+  if ((uint32_t)(hd >> 32) == epoch)
+    for (uint32_t e = (uint32_t)hd; e != kListEnd; e = next[e]) {
+      below += e < i ? 1u : 0u;
+      above += e < i ? 0u : 1u;
+    }
+  if (i < o0) return l0 + below;
+  if (i >= o1) return l1 - above;
+  return l0 + below + (i - o0) - moved_in(mask, o0, i);
 }
 
 // One thread per slot: its place in the new order; key, permutation and the
@@ -457,28 +481,109 @@ __global__ __launch_bounds__(kBlock) void k_inc_place(
   for (uint32_t k = i; k < cell_tiles; k += gridDim.x * (uint32_t)kBlock) tin[k] = tout[k] = 0u;
   if (i >= n) return;
   const uint32_t c = knew[i];
-  const uint32_t o0 = lb_old[c], l0 = lb[c];
-  const uint64_t hd = head[c];
-  uint32_t below = 0, above = 0;   // incoming slots before i, and i or after it
-  if ((uint32_t)(hd >> 32) == epoch)
-    for (uint32_t e = (uint32_t)hd; e != kListEnd; e = next[e]) {
-      below += e < i ? 1u : 0u;
-      above += e < i ? 0u : 1u;
-    }
-  uint32_t pos;
-  if (i < o0) pos = l0 + below;
-  else if (i >= lb_old[c + 1u]) pos = lb[c + 1u] - above;
-  else pos = l0 + below + (i - o0) - moved_in(mask, o0, i);
+  const uint32_t pos = place_of(i, lb_old[c], lb_old[c + 1u], lb[c], lb[c + 1u], head[c], epoch, mask, next);
   if (pos >= n) return;   // never, when the counts are consistent
   kout[pos] = c;
   perm[pos] = i;
   move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, c);
 }
 
+// Both in one launch, for small scenes, whose builds are bound by launches and
+// chains of dependent loads (two of 6-7 us; one of 7-9): the first place_blocks blocks place, each slot taking its cell's new
+// bounds from the counts themselves (the tiles before, scanned by the block;
+// the tile's groups before; the group's cells before: 24 independent loads that
+// neighbouring slots share), the others write the table.  Nothing here may be
+// cleared while another block reads it, so the table's blocks clear the set of
+// counts that the build before this one read.
+struct IncSet {
+  uint4 *cin, *cout, *gnet;
+  uint32_t *tin, *tout;
+};
+// Elements first, first + 1, ... of v whose number is below end, added up.
+__device__ inline uint32_t sum_below(uint4 v, uint32_t first, uint32_t end) {
+  return (first < end ? v.x : 0u) + (first + 1u < end ? v.y : 0u) + (first + 2u < end ? v.z : 0u) +
+         (first + 3u < end ? v.w : 0u);
+}
+template <class T4, bool OMEGA, bool PROBE, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_inc_one(
+    uint32_t n, uint32_t n_cells, uint32_t cell_tiles, uint32_t place_blocks, const uint32_t* __restrict__ knew,
+    const uint64_t* __restrict__ mask, const uint64_t* __restrict__ head, const uint32_t* __restrict__ next,
+    uint32_t epoch, const uint32_t* __restrict__ lb_old, uint32_t* __restrict__ lb, IncSet in, IncSet old,
+    uint32_t* __restrict__ kout, uint32_t* __restrict__ perm, ReorderIO<T4> io) {
+  constexpr uint32_t kGroups = kCellTile / kCellGroup;
+  const uint32_t t = threadIdx.x;
+  if (blockIdx.x >= place_blocks) {
+    const uint32_t b = blockIdx.x - place_blocks;
+    cell_tile<false>(b, n_cells, lb_old, in.tin, in.tout, in.cin, in.cout, lb);
+    const bool stale = (old.tin[b] | old.tout[b]) != 0u;
+    __syncthreads();
+    if (!stale) return;
+    old.cin[b * kBlock + t] = old.cout[b * kBlock + t] = make_uint4(0u, 0u, 0u, 0u);
+    if (t < kGroups / 4u) old.gnet[b * (kGroups / 4u) + t] = make_uint4(0u, 0u, 0u, 0u);
+    if (t == 0u) old.tin[b] = old.tout[b] = 0u;
+    return;
+  }
+  __shared__ uint32_t s4[4], s_off[kBlock];
+  __shared__ bool s_busy[kBlock];
+  const uint32_t i = blockIdx.x * (uint32_t)kBlock + t;
+  const uint32_t c = i < n ? knew[i] : 0u;
+  const uint32_t ti = t < cell_tiles ? in.tin[t] : 0u, to = t < cell_tiles ? in.tout[t] : 0u;
+  const uint32_t o0 = lb_old[c], o1 = lb_old[c + 1u];
+  const uint64_t hd = head[c];
+  uint32_t total;
+  s_off[t] = block_excl_scan(ti - to, s4, &total);
+  s_busy[t] = (ti | to) != 0u;
+  __syncthreads();
+  if (i >= n) return;
+  const uint32_t b = c / kCellTile;
+  uint32_t before = s_off[b], upto = before;   // what the cell's bounds move by
+  if (s_busy[b]) {
+    const uint4* __restrict__ g = in.gnet + b * (kGroups / 4u);
+    const uint32_t q = c / kCellGroup * (kCellGroup / 4u);
+    uint4 vg[kGroups / 4u], vi[kCellGroup / 4u], vo[kCellGroup / 4u];
+#pragma unroll
+    for (uint32_t k = 0; k < kGroups / 4u; ++k) vg[k] = g[k];
+#pragma unroll
+    for (uint32_t k = 0; k < kCellGroup / 4u; ++k) { vi[k] = in.cin[q + k]; vo[k] = in.cout[q + k]; }
+    const uint32_t ng = c / kCellGroup % kGroups, nc = c % kCellGroup;
+#pragma unroll
+    for (uint32_t k = 0; k < kGroups / 4u; ++k) before += sum_below(vg[k], 4u * k, ng);
+    upto = before;
+#pragma unroll
+    for (uint32_t k = 0; k < kCellGroup / 4u; ++k) {
+      const uint4 d = make_uint4(vi[k].x - vo[k].x, vi[k].y - vo[k].y, vi[k].z - vo[k].z, vi[k].w - vo[k].w);
+      before += sum_below(d, 4u * k, nc);
+      upto += sum_below(d, 4u * k, nc + 1u);
+    }
+  }
+  const uint32_t pos = place_of(i, o0, o1, o0 + before, o1 + upto, hd, epoch, mask, next);
+  if (pos >= n) return;   // never, when the counts are consistent
+  kout[pos] = c;
+  perm[pos] = i;
+  move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, c);
+}
+
+// One launch pays while a launch weighs more than the extra loads of every
+// slot.  Us a step, two launches / one: spheres 1,000 17.2 / 14.2, 10,000 19.8 /
+// 17.3, 100,000 42.0 / 39.5; slots of a dam break, 42,866 49.1 / 47.1, 196k mixed
+// 95.0 / 92.8, 329k 132.3 / 130.8, 664k F32 183.3 / 183.9.  A block scans the
+// tiles with a thread each, so there may be no more of them.
+constexpr uint64_t kIncOne = 400000;
+bool inc_in_one(uint64_t n, size_t cell_tiles) { return cell_tiles <= (size_t)kBlock && n <= kIncOne; }
+
 MovedOut moved_out(Ctx& c) {
   c.inc_counts = true;
-  return MovedOut{c.inc_mask.as<uint64_t>(), c.inc_cin(), c.inc_cout(), c.inc_tin(), c.inc_tout(), c.inc_head(),
-                  c.inc_next.as<uint32_t>(), ++c.inc_epoch, c.flags.as<uint32_t>()};
+  const int s = c.inc_set;
+  return MovedOut{c.inc_mask.as<uint64_t>(), c.inc_cin(s), c.inc_cout(s), c.inc_tin(s), c.inc_tout(s),
+                  c.inc_one ? c.inc_gnet(s) : nullptr, c.inc_head(), c.inc_next.as<uint32_t>(), ++c.inc_epoch,
+                  c.flags.as<uint32_t>()};
+}
+
+static void inc_taken(Ctx& c) {
+  std::swap(c.lb.p, c.lb_spare.p);
+  c.inc_counts = false;
+  c.cur_key ^= 1;
+  c.perm_buf = 0;
 }
 
 // Stable sort of keys[cur_key] from the previous build's order (keys[cur_key
@@ -488,11 +593,29 @@ static void incremental_sort(Ctx& c) {
   const uint32_t n = (uint32_t)c.n;
   const uint32_t cells = c.grid.n_cells;
   const uint32_t tiles = (uint32_t)c.inc_tiles;
+  if (c.inc_one) {
+    LaunchScope ls(&c, "sort_inc_one", 8.0 * cells + (12.0 + reorder_bytes(c)) * n);
+    auto set = [&](int s) {
+      return IncSet{reinterpret_cast<uint4*>(c.inc_cin(s)), reinterpret_cast<uint4*>(c.inc_cout(s)),
+                    reinterpret_cast<uint4*>(c.inc_gnet(s)), c.inc_tin(s), c.inc_tout(s)};
+    };
+    with_reorder_form(c, c.cur, c.cur ^ 1, [&](auto form, auto io) {
+      using F = decltype(form);
+      const uint32_t place_blocks = blocks_for(n);
+      k_inc_one<typename F::T, F::omega, F::probe, F::mixed><<<place_blocks + tiles, kBlock, 0, c.stream>>>(
+          n, cells, tiles, place_blocks, c.keys[c.cur_key].as<uint32_t>(), c.inc_mask.as<uint64_t>(), c.inc_head(),
+          c.inc_next.as<uint32_t>(), c.inc_epoch, c.lb.as<uint32_t>(), c.lb_spare.as<uint32_t>(), set(c.inc_set),
+          set(c.inc_set ^ 1), c.keys[c.cur_key ^ 1].as<uint32_t>(), c.vals[0].as<uint32_t>(), io);
+    });
+    PR_HIP(hipGetLastError());
+    c.inc_set ^= 1;
+    return inc_taken(c);
+  }
   {
     LaunchScope ls(&c, "sort_inc_cells", 8.0 * cells);
-    k_inc_cells<<<tiles, kBlock, 0, c.stream>>>(cells, c.lb.as<uint32_t>(), c.inc_tin(), c.inc_tout(),
-                                                reinterpret_cast<uint4*>(c.inc_cin()),
-                                                reinterpret_cast<uint4*>(c.inc_cout()), c.lb_spare.as<uint32_t>());
+    k_inc_cells<<<tiles, kBlock, 0, c.stream>>>(cells, c.lb.as<uint32_t>(), c.inc_tin(0), c.inc_tout(0),
+                                                reinterpret_cast<uint4*>(c.inc_cin(0)),
+                                                reinterpret_cast<uint4*>(c.inc_cout(0)), c.lb_spare.as<uint32_t>());
     PR_HIP(hipGetLastError());
   }
   {
@@ -501,15 +624,12 @@ static void incremental_sort(Ctx& c) {
       using F = decltype(form);
       k_inc_place<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(
           n, tiles, c.keys[c.cur_key].as<uint32_t>(), c.inc_mask.as<uint64_t>(), c.inc_head(),
-          c.inc_next.as<uint32_t>(), c.inc_epoch, c.lb.as<uint32_t>(), c.lb_spare.as<uint32_t>(), c.inc_tin(),
-          c.inc_tout(), c.keys[c.cur_key ^ 1].as<uint32_t>(), c.vals[0].as<uint32_t>(), io);
+          c.inc_next.as<uint32_t>(), c.inc_epoch, c.lb.as<uint32_t>(), c.lb_spare.as<uint32_t>(), c.inc_tin(0),
+          c.inc_tout(0), c.keys[c.cur_key ^ 1].as<uint32_t>(), c.vals[0].as<uint32_t>(), io);
     });
     PR_HIP(hipGetLastError());
   }
-  std::swap(c.lb.p, c.lb_spare.p);
-  c.inc_counts = false;
-  c.cur_key ^= 1;
-  c.perm_buf = 0;
+  inc_taken(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -755,7 +875,7 @@ void neighbors_build(Ctx& c) {
     incremental_sort(c);
   } else {
     if (c.inc_counts) {   // counts of a step this build does not continue
-      PR_HIP(hipMemsetAsync(c.inc_cin(), 0, c.inc_count_bytes(), c.stream));
+      PR_HIP(hipMemsetAsync(c.inc_cin(0), 0, c.inc_count_bytes(), c.stream));
       c.inc_counts = false;
     }
     if (!c.sort_radix && count_sort_fits(n, c.grid.n_cells)) {

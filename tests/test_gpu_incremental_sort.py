@@ -57,6 +57,33 @@ def test_same_build_as_the_radix_sort(cells, n, move, precision, monkeypatch):
     assert cells == 1 or any(np.any(g["perm"] != np.arange(n)) for g in inc)
 
 
+@pytest.mark.parametrize("cells", [61, 62])
+def test_largest_grid_of_one_launch_and_the_next(cells, monkeypatch):
+    """63^3 cells are 245 tiles, each block scans them with a thread each; 64^3 and the table's last entry are 257."""
+    test_same_build_as_the_radix_sort(cells, 30000, 0.3, pa.F64, monkeypatch)
+
+
+def test_counts_that_no_build_took(monkeypatch):
+    """An upload after a step drops what the step counted: the builds after it start from cleared counts."""
+    d, arrs = make_scene(pa.SCENE_DEM_POUR, n_target=3000, seed=5)
+    out = {}
+    for policy in ("incremental", "radix"):
+        monkeypatch.setenv("PRESTIGE_SORT", policy)
+        got = []
+        with pa.Context(d) as ctx:
+            upload_all(ctx, {**arrs, "vx": np.full(len(arrs["x"]), 0.2)})
+            for steps in (1, 2, 3):
+                ctx.step(steps)
+                ctx.upload("x", ctx.download("x"))
+                ctx.step(2)
+                ctx.neighbors_build()
+                got.append(ctx.neighbors_download())
+        out[policy] = got
+    for a, b in zip(out["incremental"], out["radix"]):
+        for k in ("keys", "perm", "ids", "lb"):
+            assert np.array_equal(a[k], b[k]), k
+
+
 def test_a_runaway_into_one_cell_stays_bounded():
     """70,000 spheres jump into one cell in one step: the error names the runaway, no sphere is lost, and at
     most 65,536 of them changed cell."""
