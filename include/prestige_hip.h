@@ -161,12 +161,6 @@ prestige_status prestige_field_upload(prestige_ctx* ctx, const char* name,
 prestige_status prestige_field_download(prestige_ctx* ctx, const char* name,
                                         double* out, uint64_t n);
 
-/* Pinned host memory for field arrays (free with prestige_host_free): transfers
- * to and from it run at the link's rate, where ordinary memory is staged.  Any
- * host memory may be passed to the calls above. */
-prestige_status prestige_host_alloc(size_t bytes, void** out);
-void prestige_host_free(void* p);
-
 /* Cell keys of the current positions, stable LSD radix sort, reorder of every
  * field into key order, cell lower-bound table.  The neighbour relation the
  * gathers use afterwards is |x_i - x_j| < cutoff over the 27 surrounding

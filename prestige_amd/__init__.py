@@ -14,11 +14,8 @@ importing the binding fails loudly when the library is missing.
 """
 from __future__ import annotations
 
-import collections
 import ctypes as C
 import os
-import threading
-import weakref
 from pathlib import Path
 
 import numpy as np
@@ -113,8 +110,6 @@ def _bind(lib):
         "prestige_desc_init": (None, [C.POINTER(Desc), C.c_int32]),
         "prestige_create": (S, [C.POINTER(Desc), C.POINTER(_P)]),
         "prestige_destroy": (None, [_P]),
-        "prestige_host_alloc": (S, [C.c_size_t, C.POINTER(_P)]),
-        "prestige_host_free": (None, [_P]),
         "prestige_field_upload": (S, [_P, C.c_char_p, _D, C.c_uint64]),
         "prestige_field_download": (S, [_P, C.c_char_p, _D, C.c_uint64]),
         "prestige_neighbors_build": (S, [_P]),
@@ -181,90 +176,6 @@ def _check(status: int, ctx_handle=None):
         raise PrestigeError(status, (msg or b"").decode(errors="replace"))
 
 
-class _PinnedPool:
-    """Arrays of pinned host memory for what the device returns.  A download into
-    fresh pageable memory is staged, and faults every page in (1.8M values: 876 us
-    where the array is dropped, 1833 where it is kept; pinned 293 and 350).  A block
-    comes back when its array and every view of it are gone, and is used again by
-    size.  At most LIMIT bytes are pinned at a time, of which at most IDLE wait
-    unused while a context is open and none when the last one is closed; an array
-    that does not fit is an ordinary one."""
-
-    LIMIT = 1 << 30
-    IDLE = 256 << 20
-    SMALL = 128 << 10   # up to here the library stages through pinned memory of its own
-
-    def __init__(self):
-        self._lock = threading.Lock()
-        # Blocks whose arrays are gone.  Finalizers run anywhere, also under the
-        # lock or while a stream is captured, so they only append here.
-        self._back = collections.deque()
-        self._free = {}     # bytes -> [address, ...], oldest first
-        self._total = 0     # pinned bytes, in use or idle
-        self._idle = 0
-        self._contexts = 0
-
-    def empty(self, n: int) -> np.ndarray:
-        nbytes = 8 * n
-        if nbytes <= self.SMALL:
-            return np.empty(n, np.float64)
-        with self._lock:
-            self._collect()
-            blocks = self._free.get(nbytes)
-            if blocks:
-                addr = blocks.pop()
-                self._idle -= nbytes
-            else:
-                self._trim(self.LIMIT - nbytes, self._idle)
-                addr = self._alloc(nbytes) if self._total + nbytes <= self.LIMIT else None
-            self._trim(self.LIMIT, self.IDLE)
-        if addr is None:
-            return np.empty(n, np.float64)
-        block = (C.c_char * nbytes).from_address(addr)
-        weakref.finalize(block, self._back.append, (addr, nbytes)).atexit = False
-        return np.frombuffer(block, np.float64)
-
-    def opened(self) -> None:
-        with self._lock:
-            self._contexts += 1
-
-    def closed(self) -> None:
-        with self._lock:
-            self._contexts -= 1
-            if self._contexts == 0:
-                self._collect()
-                self._trim(self.LIMIT, 0)
-
-    # (the rest under the lock)
-    def _alloc(self, nbytes: int):
-        p = _P()
-        if load_library().prestige_host_alloc(nbytes, C.byref(p)) != 0:
-            return None
-        self._total += nbytes
-        return p.value
-
-    def _collect(self) -> None:
-        while self._back:
-            addr, nbytes = self._back.popleft()
-            self._free.setdefault(nbytes, []).append(addr)
-            self._idle += nbytes
-
-    def _trim(self, total: int, idle: int) -> None:
-        """Gives idle blocks back, the largest first, while more than `total`
-        bytes are pinned or more than `idle` of them unused."""
-        for nbytes in sorted(self._free, reverse=True):
-            blocks = self._free[nbytes]
-            while blocks and (self._total > total or self._idle > idle):
-                load_library().prestige_host_free(blocks.pop(0))
-                self._total -= nbytes
-                self._idle -= nbytes
-            if not blocks:
-                del self._free[nbytes]
-
-
-_pinned = _PinnedPool()
-
-
 def desc_init(model: int) -> Desc:
     d = Desc()
     load_library().prestige_desc_init(C.byref(d), model)
@@ -284,14 +195,12 @@ class Context:
         _check(lib.prestige_create(C.byref(self.desc), C.byref(h)), None)
         self._h = h
         self.n = int(desc.n_particles)
-        _pinned.opened()
 
     # -- lifetime ------------------------------------------------------------
     def close(self):
         if getattr(self, "_h", None):
             self._lib.prestige_destroy(self._h)
             self._h = None
-            _pinned.closed()
 
     def __enter__(self):
         return self
@@ -316,7 +225,7 @@ class Context:
         self._c(self._lib.prestige_field_upload(self._h, name.encode(), _dptr(a), self.n))
 
     def download(self, name: str) -> np.ndarray:
-        out = _pinned.empty(self.n)
+        out = np.empty(self.n, dtype=np.float64)
         self._c(self._lib.prestige_field_download(self._h, name.encode(), _dptr(out), self.n))
         return out
 
@@ -374,7 +283,7 @@ class Context:
             if s is not None and s.shape != (3 * self.n,):
                 raise PrestigeError(1, "seeds must hold 3*n values")
         gp = np.zeros(n_params, np.float64)
-        gv = _pinned.empty(3 * self.n) if want_v0 else None   # the library writes every value
+        gv = np.empty(3 * self.n) if want_v0 else None   # the library writes every value
         self._c(self._lib.prestige_adjoint(self._h, None if sx is None else _dptr(sx),
                                            None if sv is None else _dptr(sv), _dptr(gp), n_params,
                                            None if gv is None else _dptr(gv)))

@@ -2,11 +2,16 @@
 // lifetime, SoA field transfer by the reference's slice names, step and
 // neighbour-build dispatch, timing and error reporting.  No C++ exception
 // crosses this boundary.
+#include <atomic>
 #include <cctype>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <system_error>
+#include <thread>
+
+#include <sys/mman.h>
 
 #include "common.hpp"
 
@@ -92,13 +97,102 @@ LaunchScope::~LaunchScope() noexcept(false) {
 // ---------------------------------------------------------------------------
 // Small transfers go through the context's pinned block: the runtime's own
 // staging of a pageable buffer costs more than a memcpy, and kernels queued
-// behind such an upload often start 55 us late.  Upload of 10,000 / 42,900 /
-// 100,000 values, pageable 55 / 91 / 50 us, through the block 25 / 33 / 49; above
-// 1 MiB the runtime is the faster one.  Downloads gain only while their memcpy is
-// short against the call (10,000 values 39 -> 26 us; at 42,900 into a pinned array
-// 31 us straight, 40 through the block), so the line lies lower there.  Both
-// wait before they touch the block again, so one serves all calls.
-constexpr size_t kPinBytes = 1u << 20, kPinDown = 128u << 10;
+// behind such an upload often start 55 us late.  Larger uploads are the
+// runtime's.  Larger downloads go through a ring of chunks: this thread drives the
+// link while a few others first have the kernel map the caller's pages, most of
+// the cost of a fresh array, and then copy from the ring.  The results are the
+// caller's ordinary memory: arrays of pinned memory would save all this, but a
+// process forked later does not have them.
+//
+// Us a field of 10,000 / 100,000 / 200,000 / 571,000 / 1.8M / 6.03M values, all
+// by the runtime and with the checks on the host, then now: upload 56 / 70 / 129 /
+// 289 / 807 / 3223 -> 26 / 50 / 87 / 176 / 445 / 1869, download into fresh arrays
+// 59 / 93 / 282 / 568 / 1369 / 4930 -> 27 / 92 / 199 / 277 / 566 / 2986 (into
+// pinned arrays 571,000 take 112).  At 1 MiB both ways of a download take 135; a
+// chunk of 1 MiB keeps the threads busy from a few MiB on, from 8 MiB on 2 MiB
+// ask for fewer events (1.8M values 597 -> 566).
+constexpr size_t kPinBytes = 1u << 20;
+constexpr size_t kRing = 8u << 20, kChunk = 1u << 20, kBigChunk = 2u << 20;   // the ring, what the link moves at a time
+constexpr size_t kUnit = 128u << 10, kPages = 2u << 20;   // what a thread copies, and has mapped, at a time
+constexpr uint32_t kCopyThreads = 6;
+
+namespace {
+// Threads that copy a transfer from the ring as open lets them.  They make no
+// HIP calls; whatever ends the transfer early ends them too.
+struct Copiers {
+  char* const host;
+  const char* const ring;
+  const size_t bytes, chunk;
+  const uint32_t chunks, units, per_chunk;
+  std::atomic<uint32_t> mapped{0}, next{0}, open{0};   // page runs and units taken, chunks that may be copied
+  std::atomic<bool> stop{false};
+  std::vector<std::atomic<uint32_t>> done;   // units copied of each chunk
+  std::vector<std::thread> threads;
+
+  Copiers(void* host_, const char* ring_, size_t bytes_)
+      : host(static_cast<char*>(host_)), ring(ring_), bytes(bytes_), chunk(bytes_ >= kRing ? kBigChunk : kChunk),
+        chunks((uint32_t)((bytes + chunk - 1) / chunk)), units((uint32_t)((bytes + kUnit - 1) / kUnit)),
+        per_chunk((uint32_t)(chunk / kUnit)), done(chunks) {
+    threads.reserve(kCopyThreads);
+  }
+  ~Copiers() {
+    stop = true;
+    for (auto& t : threads) t.join();
+  }
+  void start() {
+    try {
+      while (threads.size() < kCopyThreads) threads.emplace_back([this] { work(); });
+    } catch (const std::system_error&) {
+      // fewer threads, or none: then wait_for copies
+    }
+  }
+  void copy(uint32_t u) {
+    const size_t at = u * kUnit;
+    std::memcpy(host + at, ring + at % kRing, std::min(kUnit, bytes - at));
+  }
+  // Leaves what the pages hold as it is; where the kernel cannot, the copy faults.
+  void map_pages() {
+    const uintptr_t lo = (reinterpret_cast<uintptr_t>(host) + 4095u) & ~(uintptr_t)4095u;
+    const uintptr_t hi = (reinterpret_cast<uintptr_t>(host) + bytes) & ~(uintptr_t)4095u;
+    for (uintptr_t a; !stop && (a = (lo & ~(kPages - 1u)) + mapped.fetch_add(1) * kPages) < hi;) {
+      const uintptr_t from = std::max(a, lo), to = std::min<uintptr_t>(a + kPages, hi);
+      if (madvise(reinterpret_cast<void*>(from), to - from, MADV_POPULATE_WRITE) != 0) return;
+    }
+  }
+  void work() {
+    map_pages();
+    for (uint32_t u; (u = next.fetch_add(1)) < units;) {
+      while (open.load(std::memory_order_acquire) <= u / per_chunk) {
+        if (stop) return;
+        std::this_thread::yield();
+      }
+      copy(u);
+      done[u / per_chunk].fetch_add(1, std::memory_order_release);
+    }
+  }
+  // Chunk k, which is open, has been copied.
+  void wait_for(uint32_t k) {
+    const uint32_t n = std::min(per_chunk, units - k * per_chunk);
+    if (threads.empty())
+      for (; done[k] < n; ++done[k]) copy(k * per_chunk + done[k]);
+    while (done[k].load(std::memory_order_acquire) < n) std::this_thread::yield();
+  }
+};
+}  // namespace
+
+static char* ring(Ctx& c) {
+  if (!c.ring) {
+    void* p = nullptr;
+    PR_HIP(hipHostMalloc(&p, kRing, hipHostMallocDefault));
+    c.ring = p;
+  }
+  while (c.ring_ev.size() < kRing / kChunk) {
+    hipEvent_t e;
+    PR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    c.ring_ev.push_back(e);
+  }
+  return static_cast<char*>(c.ring);
+}
 
 void to_device(Ctx& c, void* dst, const void* host, size_t bytes) {
   if (!bytes) return;
@@ -112,13 +206,32 @@ void to_device(Ctx& c, void* dst, const void* host, size_t bytes) {
 
 // Waits for the stream.
 void to_host(Ctx& c, void* host, const void* src, size_t bytes) {
-  if (bytes) PR_HIP(hipMemcpyAsync(bytes <= kPinDown ? c.pin : host, src, bytes, hipMemcpyDeviceToHost, c.stream));
-  PR_HIP(hipStreamSynchronize(c.stream));
-  if (bytes && bytes <= kPinDown) std::memcpy(host, c.pin, bytes);
+  if (bytes <= kPinBytes) {
+    if (bytes) PR_HIP(hipMemcpyAsync(c.pin, src, bytes, hipMemcpyDeviceToHost, c.stream));
+    PR_HIP(hipStreamSynchronize(c.stream));
+    if (bytes) std::memcpy(host, c.pin, bytes);
+    return;
+  }
+  char* const r = ring(c);
+  Copiers w(host, r, bytes);
+  const uint32_t slots = (uint32_t)(kRing / w.chunk);
+  for (uint32_t k = 0, sent = 0; k < w.chunks; ++k) {
+    for (; sent < w.chunks && sent < k + slots; ++sent) {
+      if (sent >= slots) w.wait_for(sent - slots);
+      const size_t at = sent * w.chunk;
+      PR_HIP(hipMemcpyAsync(r + at % kRing, static_cast<const char*>(src) + at, std::min(w.chunk, bytes - at),
+                            hipMemcpyDeviceToHost, c.stream));
+      PR_HIP(hipEventRecord(c.ring_ev[sent % slots], c.stream));
+    }
+    if (k == 0) w.start();   // while the first chunks are on their way
+    PR_HIP(hipEventSynchronize(c.ring_ev[k % slots]));
+    w.open.store(k + 1u, std::memory_order_release);
+  }
+  for (uint32_t k = 0; k < w.chunks; ++k) w.wait_for(k);
 }
 
 // What a field's values must satisfy, found on the device beside the copy (an
-// upload of 571,000 / 6,030,000 values takes 193 / 1740 us; 289 / 3328 with the
+// upload of 571,000 / 6,030,000 values takes 176 / 1869 us; 289 / 3223 with the
 // test on the host).  A value that fails sets bit 0 (not finite), 1 (not
 // positive) or 2 (over the limit) of a device word, which holds the kernels that
 // follow back, and a word per bit for the host in the pinned block; all stay 0
@@ -666,24 +779,6 @@ void prestige_destroy(prestige_ctx* ctx) {
   hipStream_t s = ctx->stream;
   delete ctx;   // buffers and events released by their destructors
   if (s) (void)hipStreamDestroy(s);
-}
-
-prestige_status prestige_host_alloc(size_t bytes, void** out) {
-  if (!out) {
-    g_create_error = "null output pointer";
-    return PRESTIGE_E_INVALID;
-  }
-  *out = nullptr;
-  const hipError_t e = hipHostMalloc(out, bytes ? bytes : 1, hipHostMallocDefault);
-  if (e == hipSuccess) return PRESTIGE_OK;
-  (void)hipGetLastError();
-  *out = nullptr;
-  g_create_error = std::string("hipHostMalloc: ") + hipGetErrorString(e);
-  return PRESTIGE_E_OOM;
-}
-
-void prestige_host_free(void* p) {
-  if (p) (void)hipHostFree(p);
 }
 
 prestige_status prestige_field_upload(prestige_ctx* ctx, const char* name, const double* data, uint64_t n) {

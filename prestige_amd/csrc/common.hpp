@@ -263,6 +263,8 @@ struct Ctx {
   Ctx& operator=(const Ctx&) = delete;
   ~Ctx() {
     if (pin) (void)hipHostFree(pin);
+    if (ring) (void)hipHostFree(ring);
+    for (auto e : ring_ev) (void)hipEventDestroy(e);
   }
   prestige_desc desc{};
   int device = 0;
@@ -324,6 +326,8 @@ struct Ctx {
   void forget_dry() { dens_pass += 2; }   // state changed outside a step
   DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word
   void *pin = nullptr, *pin_dev = nullptr;   // pinned block for small transfers (host and device address)
+  void* ring = nullptr;                      // pinned chunks of large ones, from the first on
+  std::vector<hipEvent_t> ring_ev;
   // gather outputs
   DevBuf rp;                     // (rho, p/rho^2) per slot: double2 or float2
   DevBuf pres;                   // p per slot (double or float)

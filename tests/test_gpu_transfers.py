@@ -1,4 +1,4 @@
-"""Field transfers: what crosses the pinned block and what does not, the checks on
+"""Field transfers: what crosses the pinned block and what the ring of chunks, the checks on
 the device, and arrays that outlive later downloads."""
 
 import numpy as np
@@ -9,7 +9,8 @@ from helpers import make_scene
 
 pytestmark = pytest.mark.gpu
 
-BLOCK_UP, BLOCK_DOWN = (1 << 20) // 8, (128 << 10) // 8   # values that just fit the pinned block
+BLOCK = (1 << 20) // 8   # values that just fit the pinned block, and a chunk of the ring
+RING = 8 * BLOCK
 
 
 def pairs(n):
@@ -21,7 +22,7 @@ def pairs(n):
     return pa.Context(d)
 
 
-@pytest.mark.parametrize("n", [1, 255, BLOCK_DOWN, BLOCK_DOWN + 1, BLOCK_UP, BLOCK_UP + 1])
+@pytest.mark.parametrize("n", [1, 255, BLOCK, BLOCK + 1, 2 * BLOCK - 1, 2 * BLOCK, 2 * BLOCK + 1, RING - 1, RING, RING + 1, 2 * RING + BLOCK + 3])
 def test_values_come_back_and_bad_ones_change_nothing(n):
     rng = np.random.default_rng(n)
     x, y, m = rng.random(n), rng.random(n), rng.random(n) + 0.5
@@ -43,10 +44,11 @@ def test_values_come_back_and_bad_ones_change_nothing(n):
         c.upload("x", y)
         assert np.array_equal(c.download("x"), y)
     assert np.array_equal(first, x) and np.array_equal(view, y[n // 2:])
-    first[:] = 0.0   # an ordinary, writable array of the caller's
+    first[:] = 0.0
+    assert first.flags.owndata   # ordinary memory of the caller's, which a forked process has too
 
 
-@pytest.mark.parametrize("n", [300, BLOCK_UP + 1])
+@pytest.mark.parametrize("n", [300, BLOCK + 1])
 def test_sphere_checks(n):
     d, _ = make_scene(pa.SCENE_DEM_POUR, n_target=4, seed=0)
     d.n_particles = d.n_moving = n
@@ -73,22 +75,3 @@ def test_sphere_checks(n):
         assert np.array_equal(c.download("radius"), r)
         c.upload("radius", 0.5 * r)
         assert np.array_equal(c.download("radius"), 0.5 * r)
-
-
-def test_pool_is_bounded_and_given_back(monkeypatch):
-    pool = pa._PinnedPool()
-    monkeypatch.setattr(pa, "_pinned", pool)
-    monkeypatch.setattr(pool, "LIMIT", 40 << 20)
-    monkeypatch.setattr(pool, "IDLE", 16 << 20)
-    n = 1 << 20   # 8 MiB a field
-    x = np.random.default_rng(3).random(n)
-    with pairs(n) as c, pairs(1):
-        c.upload("x", x)
-        keep = [c.download("x") for _ in range(7)]
-        assert pool._total == 40 << 20                  # five blocks; the other two are ordinary arrays
-        assert all(np.array_equal(k, x) for k in keep)
-        del keep
-        again = c.download("x")
-        assert pool._idle <= pool.IDLE and pool._total == pool._idle + (8 << 20)
-    assert pool._idle == 0 and pool._total == 8 << 20   # the last context has gone
-    assert np.array_equal(again, x)
