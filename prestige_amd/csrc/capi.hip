@@ -380,11 +380,13 @@ static void allocate(Ctx& c) {
     c.inc_one = inc_in_one(n, c.inc_tiles);
     c.inc_mask.alloc(((nn + 63) / 64) * 8);
     c.inc_next.alloc(nn * 4);
+    PR_HIP(hipMemsetAsync(c.inc_next.p, 0xFF, nn * 4, c.stream));   // kListEnd
     c.lb_spare.alloc(cells * 4);
-    c.inc_cells.alloc(c.inc_tiles * kCellTile * 8 + c.inc_count_bytes());
+    c.inc_cells.alloc(c.inc_head_bytes() + c.inc_count_bytes());
     PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, c.inc_cells.bytes, c.stream));
   }
   if (const char* dr = std::getenv("PRESTIGE_DRY")) c.dry_reuse = std::string(dr) != "off";
+  if (const char* ep = std::getenv("PRESTIGE_EPOCH")) c.inc_epoch = (uint32_t)std::strtoul(ep, nullptr, 10);
   if (const char* sp = std::getenv("PRESTIGE_SORT")) c.sort_radix = std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc((FLAG_COUNT + 1) * 4);

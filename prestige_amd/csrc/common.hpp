@@ -151,9 +151,10 @@ bool inc_in_one(uint64_t n, size_t cell_tiles);
 // its new cell (cin) and out of its old one (cout), into the same totals per
 // tile of kCellTile cells (tin, tout), and is linked into its new cell's list:
 // head[c] holds (epoch << 32 | last slot linked), next[slot] the slot linked
-// before it (kListEnd for the first of this epoch, so heads need no clearing).
-// Word w of mask has bit l set when slot 64 w + l moved.  Contexts whose build is
-// one launch also take what came less what left per kCellGroup cells (gnet).
+// before it (kListEnd for the first of this epoch, so heads need no clearing but
+// when the 32-bit epochs start again, at 1).  Word w of mask has bit l set when
+// slot 64 w + l moved.  Contexts whose build is one launch also take what came
+// less what left per kCellGroup cells (gnet).
 constexpr uint32_t kCellTile = 1024;
 constexpr uint32_t kCellGroup = 32;
 constexpr uint32_t kListEnd = 0xFFFFFFFFu;
@@ -300,9 +301,10 @@ struct Ctx {
   DevBuf inc_mask, inc_next, lb_spare, inc_cells;
   size_t inc_tiles = 0;
   uint64_t* inc_head() const { return inc_cells.as<uint64_t>(); }
+  size_t inc_head_bytes() const { return inc_tiles * kCellTile * 8; }
   size_t inc_set_words() const { return (inc_tiles * (2 * kCellTile + kCellTile / kCellGroup + 2) + 3) / 4 * 4; }
   uint32_t* inc_cin(int set) const {
-    return reinterpret_cast<uint32_t*>(inc_head() + inc_tiles * kCellTile) + set * inc_set_words();
+    return reinterpret_cast<uint32_t*>(inc_cells.as<char>() + inc_head_bytes()) + set * inc_set_words();
   }
   uint32_t* inc_cout(int set) const { return inc_cin(set) + inc_tiles * kCellTile; }
   uint32_t* inc_gnet(int set) const { return inc_cout(set) + inc_tiles * kCellTile; }
@@ -311,7 +313,7 @@ struct Ctx {
   size_t inc_count_bytes() const { return (inc_one ? 2 : 1) * inc_set_words() * 4; }   // from inc_cin(0) on
   bool inc_one = false;          // the build after a step is one launch
   int inc_set = 0;
-  uint32_t inc_epoch = 1;
+  uint32_t inc_epoch = 0;        // of the last step (PRESTIGE_EPOCH starts it elsewhere, for tests)
   bool inc_ready = false;        // keys[cur_key] are the next keys of the last build's slots
   bool inc_counts = false;       // a step's counts are waiting (a build that does not use them clears them)
   bool sort_radix = false;       // PRESTIGE_SORT=radix: every build sorts anew (comparisons and tests)

@@ -574,8 +574,12 @@ bool inc_in_one(uint64_t n, size_t cell_tiles) { return cell_tiles <= (size_t)kB
 MovedOut moved_out(Ctx& c) {
   c.inc_counts = true;
   const int s = c.inc_set;
+  if (++c.inc_epoch == 0u) {   // wrapped: heads left 2^32 steps ago, or never written, would pass for this step's
+    PR_HIP(hipMemsetAsync(c.inc_head(), 0, c.inc_head_bytes(), c.stream));
+    c.inc_epoch = 1u;
+  }
   return MovedOut{c.inc_mask.as<uint64_t>(), c.inc_cin(s), c.inc_cout(s), c.inc_tin(s), c.inc_tout(s),
-                  c.inc_one ? c.inc_gnet(s) : nullptr, c.inc_head(), c.inc_next.as<uint32_t>(), ++c.inc_epoch,
+                  c.inc_one ? c.inc_gnet(s) : nullptr, c.inc_head(), c.inc_next.as<uint32_t>(), c.inc_epoch,
                   c.flags.as<uint32_t>()};
 }
 
