@@ -1048,7 +1048,8 @@ __global__ __launch_bounds__(64) void k_eq1_allpairs(uint32_t n, const double* _
 // added at once.  A wavefront in which some lane's candidate falls between (a
 // few pairs in 10^5) takes the exact FP64 test for it.  So the pairs and the
 // order are the plain loop's, and each force is its sum bit for bit.
-// A union wider than the stage takes the exact test throughout.
+// A union wider than the stage takes the exact test throughout, as do offsets too
+// large for FP32.
 // The masses come in slot order (smass[mstride j]): gathered by id in here they
 // were 18 of a wavefront's loads of 64 scattered lines each, and what bounded it
 // (236 us below).  Four candidates share the question whether any lane is in doubt.
@@ -1132,7 +1133,11 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
     }
     const float m2 = fmaxf(ss_max, wave_max_pos(mq));
     const float margin = 0x1.0p-18f * (m2 + __builtin_sqrtf(m2) + 1.0f);
-    const float lo = (1.0f - margin) - so.w, hi = (1.0f + margin) - so.w;
+    // offsets of more than 2^50 cutoffs could overflow in the form: then no pair is
+    // decided here (every comparison with a NaN is false)
+    const bool far = !(m2 < 0x1.0p100f);
+    const float lo = far ? __builtin_nanf("") : (1.0f - margin) - so.w;
+    const float hi = far ? __builtin_nanf("") : (1.0f + margin) - so.w;
     __builtin_amdgcn_wave_barrier();   // one wavefront: its LDS operations complete in order
     const uint32_t first = j0[r] - base;
     auto batch = [&](uint32_t b, uint32_t cnt) {
@@ -1147,7 +1152,7 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
       }
       uint64_t open = 0;   // lanes that cannot tell
 #pragma unroll
-      for (uint32_t u = 0; u < kEq1Batch; ++u) open |= __ballot(v[u] < lo) ^ __ballot(v[u] < hi);
+      for (uint32_t u = 0; u < kEq1Batch; ++u) open |= __ballot(v[u] < lo) ^ __ballot(!(v[u] >= hi));
       if (open == 0ull) {
 #pragma unroll
         for (uint32_t u = 0; u < kEq1Batch; ++u)
@@ -1160,7 +1165,7 @@ __global__ __launch_bounds__(64) void k_eq1_cells(uint32_t n, const T4* __restri
         for (uint32_t u = 0; u < kEq1Batch; ++u) {
           const float w = u == 0u ? v[0] : (u == 1u ? v[1] : (u == 2u ? v[2] : v[3]));
           const double mu = u == 0u ? m[0] : (u == 1u ? m[1] : (u == 2u ? m[2] : m[3]));
-          if (w < lo || (w < hi && exact(j0[r] + b + u))) acc += mu;
+          if (u < cnt && (w < lo || (!(w >= hi) && exact(j0[r] + b + u)))) acc += mu;
         }
       }
     };
