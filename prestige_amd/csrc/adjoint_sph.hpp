@@ -578,10 +578,10 @@ void ensure_adj_buffers(Ctx& c);
 // in rec[t].  Taken by swap: the pair geometry (sorted pre-step state or FP32
 // probes), the permutation, the row-run masks and (rho, p/rho^2), all of which
 // the next step regenerates, and the previous step's ids, whose order this
-// step's build left.  The segment's last step copies its ids, and the taped
-// run's last (rho, p/rho^2), which stay downloadable.
+// step's build left.  The segment's last step copies its ids and (rho, p/rho^2):
+// rho stays downloadable, of the same step as p and the accelerations.
 template <int F>
-void record_sph_step(Ctx& c, Tape& T, uint32_t t, bool last, bool keep_rp) {
+void record_sph_step(Ctx& c, Tape& T, uint32_t t, bool last) {
   StepRecord& r = *T.rec[t];
   const size_t n = c.n ? c.n : 1;
   const size_t r2 = (F == kF64) ? sizeof(double2) : sizeof(float2);
@@ -597,9 +597,8 @@ void record_sph_step(Ctx& c, Tape& T, uint32_t t, bool last, bool keep_rp) {
   take_buffer(c.nmeta, r.nmeta);
   take_buffer(c.nword, r.nword);
   if (t > 0) take_buffer(c.ids[c.cur_ids ^ 1], T.rec[t - 1]->ids);
-  if (keep_rp) copy_many(c, {{&r.rp, &c.rp, n * r2}});
+  if (last) copy_many(c, {{&r.ids, &c.ids[c.cur_ids], n * 4}, {&r.rp, &c.rp, n * r2}});
   else take_buffer(c.rp, r.rp);
-  if (last) copy_many(c, {{&r.ids, &c.ids[c.cur_ids], n * 4}});
 }
 
 // Steps taken while this is alive leave every particle usable row masks
@@ -628,7 +627,7 @@ void sph_tape_forward(Ctx& c, uint32_t nsteps, uint32_t every) {
     }
     c.record_all = s >= last0;   // only recorded steps need usable masks for every particle
     sph_step_impl<F>(c);
-    if (s >= last0) record_sph_step<F>(c, T, s - last0, s + 1 == nsteps, s + 1 == nsteps);
+    if (s >= last0) record_sph_step<F>(c, T, s - last0, s + 1 == nsteps);
   }
   T.last_recorded = true;
   if (!c.tape.final_state) c.tape.final_state.reset(new Snapshot());
@@ -659,7 +658,7 @@ void sph_adjoint(Ctx& c, const double* seed_x, const double* seed_v, double* gra
       RecordAll keep_masks(c);
       for (uint32_t t = 0; t < len; ++t) {
         sph_step_impl<F>(c);
-        record_sph_step<F>(c, T, t, t + 1 == len, false);
+        record_sph_step<F>(c, T, t, t + 1 == len);
       }
     }
     T.last_recorded = false;   // records are overwritten by the recompute of earlier segments
