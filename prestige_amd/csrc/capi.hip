@@ -255,18 +255,16 @@ __global__ __launch_bounds__(kBlock) void k_check_field(uint32_t n, const double
 static void check_field(Ctx& c, const double* d, uint32_t what, double limit) {
   if (!c.n) return;
   k_check_field<<<blocks_for(c.n), kBlock, 0, c.stream>>>((uint32_t)c.n, d, what, limit, c.flags.as<uint32_t>() + FLAG_COUNT,
-                                                          static_cast<uint32_t*>(c.pin_dev) + kPinBytes / 4);
+                                                          c.note_dev + kNoteField);
   PR_HIP(hipGetLastError());
 }
 
 // Waits for the stream; the bits the last check found, cleared.
 static uint32_t checked(Ctx& c) {
   PR_HIP(hipStreamSynchronize(c.stream));
-  uint32_t* w = static_cast<uint32_t*>(c.pin) + kPinBytes / 4;
   uint32_t bad = 0;
-  for (uint32_t q = 0; q < 3; ++q) bad |= (static_cast<volatile uint32_t*>(w)[q] & 1u) << q;
+  for (int q = 0; q < 3; ++q) bad |= (c.take_note(kNoteField + q) ? 1u : 0u) << q;
   if (bad) {
-    for (uint32_t q = 0; q < 3; ++q) w[q] = 0u;
     PR_HIP(hipMemsetAsync(c.flags.as<uint32_t>() + FLAG_COUNT, 0, 4, c.stream));
     PR_HIP(hipStreamSynchronize(c.stream));
   }
@@ -389,17 +387,21 @@ static void allocate(Ctx& c) {
   if (const char* ep = std::getenv("PRESTIGE_EPOCH")) c.inc_epoch = (uint32_t)std::strtoul(ep, nullptr, 10);
   if (const char* sp = std::getenv("PRESTIGE_SORT")) c.sort_radix = std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
-  c.flags.alloc((FLAG_COUNT + 1) * 4);
-  PR_HIP(hipHostMalloc(&c.pin, kPinBytes + 64, hipHostMallocMapped));
-  PR_HIP(hipHostGetDevicePointer(&c.pin_dev, c.pin, 0));
-  std::memset(static_cast<char*>(c.pin) + kPinBytes, 0, 64);
+  c.flags.alloc((FLAG_COUNT + 2) * 4);
+  PR_HIP(hipHostMalloc(&c.pin, kPinBytes + kNotes * 4, hipHostMallocMapped));
+  void* pin_dev = nullptr;
+  PR_HIP(hipHostGetDevicePointer(&pin_dev, c.pin, 0));
+  c.note = reinterpret_cast<uint32_t*>(static_cast<char*>(c.pin) + kPinBytes);
+  c.note_dev = reinterpret_cast<uint32_t*>(static_cast<char*>(pin_dev) + kPinBytes);
+  std::memset(c.note, 0, kNotes * 4);
+  PR_HIP(hipEventCreateWithFlags(&c.counted, hipEventDisableTiming));
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {
     c.movcell.alloc(((size_t)c.grid.n_cells + 1) * 4);
     PR_HIP(hipMemsetAsync(c.movcell.p, 0, ((size_t)c.grid.n_cells + 1) * 4, c.stream));
     c.dry_pass.alloc(nn * 4);
     PR_HIP(hipMemsetAsync(c.dry_pass.p, 0, nn * 4, c.stream));
   }
-  PR_HIP(hipMemsetAsync(c.flags.p, 0, (FLAG_COUNT + 1) * 4, c.stream));
+  PR_HIP(hipMemsetAsync(c.flags.p, 0, (FLAG_COUNT + 2) * 4, c.stream));
   const size_t es = f32 || (mixed && c.desc.model == PRESTIGE_MODEL_WCSPH) ? 4 : 8;
   c.rp.alloc(nn * 2 * es);
   c.pres.alloc(nn * es);

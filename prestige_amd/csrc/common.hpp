@@ -258,6 +258,9 @@ struct Tape {
   }
 };
 
+// Words of Ctx::note: what a field check found (kNoteField + bit), a crowded cell.
+enum Note : int { kNoteField = 0, kNoteCrowd = 3, kNotes = 4 };
+
 struct Ctx {
   Ctx() = default;
   Ctx(const Ctx&) = delete;
@@ -266,6 +269,7 @@ struct Ctx {
     if (pin) (void)hipHostFree(pin);
     if (ring) (void)hipHostFree(ring);
     for (auto e : ring_ev) (void)hipEventDestroy(e);
+    if (counted) (void)hipEventDestroy(counted);
   }
   prestige_desc desc{};
   int device = 0;
@@ -326,8 +330,17 @@ struct Ctx {
   bool record_all = false;
   bool dry_reuse = true;         // PRESTIGE_DRY=off turns the reuse off (comparisons and tests)
   void forget_dry() { dens_pass += 2; }   // state changed outside a step
-  DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word
-  void *pin = nullptr, *pin_dev = nullptr;   // pinned block for small transfers (host and device address)
+  DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word and a first build's (Crowd)
+  void* pin = nullptr;                       // pinned block for small transfers
+  // pinned words that kernels leave for the host (host and device address), 0 until then
+  uint32_t *note = nullptr, *note_dev = nullptr;
+  bool take_note(int k) {   // reads and clears; after the kernel has been waited for
+    volatile uint32_t* w = note + k;
+    const bool set = *w != 0u;
+    if (set) *w = 0u;
+    return set;
+  }
+  hipEvent_t counted = nullptr;              // the counting sort's table is written
   void* ring = nullptr;                      // pinned chunks of large ones, from the first on
   std::vector<hipEvent_t> ring_ev;
   // gather outputs

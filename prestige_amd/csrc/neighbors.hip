@@ -650,30 +650,48 @@ static void incremental_sort(Ctx& c) {
 //
 // The radix sort keeps what does not pay here.  The table costs 16 bytes a
 // cell: 4.1M cells with 300k particles 110 -> 59, but with 20k 107 either way, so
-// the line lies at kCountCells.  A slot reads its cell's whole list: 2,000
-// particles in one cell 81 -> 65, but 20,000 84 -> 340, so the mean may not pass
-// kCountMean (a crowd in one cell of many costs any pass over the cells far
-// more than the build).
+// the line lies at kCountCells.  A slot reads its cell's whole list: 3,000
+// particles in one cell take 92 us and 106 by radix, 20,000 344 and 113, a million
+// 110,000 and 160 (a particle outside the grid counts into cell 0, so that wrong
+// units put all of them there).  So a context's build turns back at a cell of more
+// than kCountMost, which the host hears of while the table and the lists are
+// written, and sorts by radix: 20,000 in 110, a million in 240.  Asking costs the
+// builds that go on 3-5 us.  eq1 without allocating does not ask, being quadratic
+// in a crowd itself.
 constexpr uint32_t kCountCells = 1u << 22;
-constexpr uint32_t kCountMean = 2048;
+constexpr uint32_t kCountMost = 2048;
 
 static bool count_sort_fits(uint32_t n, uint32_t n_cells) {
-  if ((uint64_t)n > (uint64_t)kCountMean * n_cells) return false;
+  if ((uint64_t)n > (uint64_t)kCountMost * n_cells) return false;   // some cell has more
   // the tile totals live in the radix sort's histogram
   const uint64_t tiles = ((uint64_t)n_cells + 1u + kCellTile - 1u) / kCellTile;
   return n_cells <= kCountCells && tiles <= (uint64_t)kBuckets * sort_tiles(n);
 }
 
-__global__ __launch_bounds__(kBlock) void k_count_clear(uint32_t n, uint32_t* __restrict__ cnt, uint32_t* flags) {
+// Also clears the first n_words of words.
+__global__ __launch_bounds__(kBlock) void k_count_clear(uint32_t n, uint32_t* __restrict__ cnt, uint32_t n_words,
+                                                        uint32_t* __restrict__ words) {
   const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
   if (i < n) cnt[i] = 0u;
-  if (flags && i < (uint32_t)FLAG_COUNT) flags[i] = 0u;
+  if (i < n_words) words[i] = 0u;
 }
+
+// What the count of a cell that passes kCountMost sets: a device word, after which
+// the counting sort's kernels may leave their outputs unwritten, and the host's.
+struct Crowd {
+  uint32_t *word, *note;
+  __device__ bool seen() const { return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u; }
+  __device__ void set() const {
+    __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(note, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
 
 // This lane's number in cell key; the lanes of a wavefront that follow each
 // other into one cell take theirs with one atomic (571k particles in tank order:
 // 40 -> 4.5 us; points in no order find nothing to share).  All lanes call.
-__device__ inline uint32_t cell_arrival(uint32_t* __restrict__ cnt, uint32_t key, bool live) {
+// crowd may be null.
+__device__ inline uint32_t cell_arrival(uint32_t* __restrict__ cnt, uint32_t key, bool live, const Crowd* crowd) {
   const uint32_t lane = __lane_id();
   const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
   const uint64_t starts = __ballot(lane == 0u || key != before || !live);
@@ -681,15 +699,21 @@ __device__ inline uint32_t cell_arrival(uint32_t* __restrict__ cnt, uint32_t key
   const uint64_t after = lane == 63u ? 0ull : starts & (~0ull << (lane + 1u));
   const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
   uint32_t base = 0;
-  if (live && first == lane) base = atomicAdd(&cnt[key], end - first);
+  if (live && first == lane) {
+    base = atomicAdd(&cnt[key], end - first);
+    if (crowd && base <= kCountMost && base + (end - first) > kCountMost) crowd->set();
+  }
   return (uint32_t)__shfl((int)base, (int)first, 64) + lane - first;
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_keys(uint32_t n, const uint32_t* __restrict__ keys,
-                                                       uint32_t* __restrict__ cnt, uint32_t* __restrict__ arr) {
+                                                       uint32_t* __restrict__ cnt, uint32_t* __restrict__ arr,
+                                                       Crowd crowd) {
   const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
   const bool live = i < n;
-  const uint32_t a = cell_arrival(cnt, live ? keys[i] : 0u, live);
+  const uint32_t key = live ? keys[i] : 0u;
+  if (crowd.seen()) return;   // a million atomics on one count would take longer than the radix sort
+  const uint32_t a = cell_arrival(cnt, key, live, &crowd);
   if (live) arr[i] = a;
 }
 
@@ -735,8 +759,10 @@ __global__ __launch_bounds__(kBlock) void k_count_table(uint32_t n_cells, const 
 
 __global__ __launch_bounds__(kBlock) void k_count_list(uint32_t n, const uint32_t* __restrict__ keys,
                                                        const uint32_t* __restrict__ arr,
-                                                       const uint32_t* __restrict__ lb, uint32_t* __restrict__ list) {
+                                                       const uint32_t* __restrict__ lb, uint32_t* __restrict__ list,
+                                                       Crowd crowd) {
   const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  if (crowd.seen()) return;   // arr is not complete
   if (i < n) list[lb[keys[i]] + arr[i]] = i;
 }
 
@@ -786,24 +812,36 @@ static void count_table(Ctx* c, uint32_t n_cells, uint32_t* cnt, uint32_t* tot, 
   k_count_table<<<tiles, kBlock, 0, st>>>(n_cells, tot, cnt);
   PR_HIP(hipGetLastError());
 }
+
 // The counting sort of keys[cur_key] with the state moved; same outputs as
-// radix_sort, k_reorder and k_cell_lb.
-static void context_count_sort(Ctx& c) {
+// radix_sort, k_reorder and k_cell_lb.  False, with keys[cur_key] and the state as
+// they were, when a cell has more than kCountMost slots.
+static bool context_count_sort(Ctx& c) {
   const uint32_t n = (uint32_t)c.n, cells = c.grid.n_cells;
   const uint32_t* keys = c.keys[c.cur_key].as<uint32_t>();
   uint32_t* arr = c.vals[0].as<uint32_t>();
+  const Crowd crowd{c.flags.as<uint32_t>() + FLAG_COUNT + 1, c.note_dev + kNoteCrowd};
+  const bool ask = n > kCountMost;
   {
     LaunchScope ls(&c, "sort_count", 4.0 * cells + 12.0 * n);
-    k_count_clear<<<blocks_for(cells + 1u), kBlock, 0, c.stream>>>(cells + 1u, c.lb.as<uint32_t>(), nullptr);
+    k_count_clear<<<blocks_for(cells + 1u), kBlock, 0, c.stream>>>(cells + 1u, c.lb.as<uint32_t>(), 1u, crowd.word);
     PR_HIP(hipGetLastError());
-    k_count_keys<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, c.lb.as<uint32_t>(), arr);
+    k_count_keys<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, c.lb.as<uint32_t>(), arr, crowd);
     PR_HIP(hipGetLastError());
   }
+  if (ask) PR_HIP(hipEventRecord(c.counted, c.stream));
   count_table(&c, cells, c.lb.as<uint32_t>(), c.sort_hist.as<uint32_t>(), c.stream);
-  LaunchScope ls(&c, "sort_count_place", (24.0 + reorder_bytes(c)) * n);
   uint32_t* list = c.vals[1].as<uint32_t>();
-  k_count_list<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, arr, c.lb.as<uint32_t>(), list);
-  PR_HIP(hipGetLastError());
+  {
+    LaunchScope ls(&c, "sort_count_list", 16.0 * n);
+    k_count_list<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, arr, c.lb.as<uint32_t>(), list, crowd);
+    PR_HIP(hipGetLastError());
+  }
+  if (ask) {
+    PR_HIP(hipEventSynchronize(c.counted));
+    if (c.take_note(kNoteCrowd)) return false;
+  }
+  LaunchScope ls(&c, "sort_count_place", (8.0 + reorder_bytes(c)) * n);
   with_reorder_form(c, c.cur, c.cur ^ 1, [&](auto form, auto io) {
     using F = decltype(form);
     k_count_place<typename F::T, F::omega, F::probe, F::mixed><<<blocks_for(n), kBlock, 0, c.stream>>>(
@@ -812,6 +850,7 @@ static void context_count_sort(Ctx& c) {
   PR_HIP(hipGetLastError());
   c.cur_key ^= 1;
   c.perm_buf = 0;
+  return true;
 }
 
 // lb[c] = first slot with key >= c, for c = 0 .. n_cells.  Thread k < n owns
@@ -882,9 +921,7 @@ void neighbors_build(Ctx& c) {
       PR_HIP(hipMemsetAsync(c.inc_cin(0), 0, c.inc_count_bytes(), c.stream));
       c.inc_counts = false;
     }
-    if (!c.sort_radix && count_sort_fits(n, c.grid.n_cells)) {
-      context_count_sort(c);
-    } else {
+    if (c.sort_radix || !count_sort_fits(n, c.grid.n_cells) || !context_count_sort(c)) {
       radix_sort(c);
       const uint32_t* skeys = c.keys[c.cur_key].as<uint32_t>();
       const uint32_t* perm = c.vals[c.perm_buf].as<uint32_t>();
@@ -1250,7 +1287,7 @@ __global__ __launch_bounds__(kBlock) void k_count_soa(uint32_t n, const double* 
   const uint32_t i = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
   const bool live = i < n;
   const uint32_t key = live ? cell_key_of(x[i], y[i], z[i], g, flags) : 0u;
-  const uint32_t a = cell_arrival(cnt, key, live);
+  const uint32_t a = cell_arrival(cnt, key, live, nullptr);
   if (live) {
     keys[i] = key;
     arr[i] = a;
@@ -1346,7 +1383,7 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
   double4* spos = reinterpret_cast<double4*>(base + kNaPos + na_round(32 * kNoAllocMaxN));
   uint32_t* lb = reinterpret_cast<uint32_t*>(base + kNaLb);
   uint32_t* tot = reinterpret_cast<uint32_t*>(base + kNaTot);
-  k_count_clear<<<blocks_for(g.n_cells + 1u), kBlock, 0, st>>>(g.n_cells + 1u, lb, flags);
+  k_count_clear<<<blocks_for(g.n_cells + 1u), kBlock, 0, st>>>(g.n_cells + 1u, lb, FLAG_COUNT, flags);
   PR_HIP(hipGetLastError());
   k_count_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, g, keys, lb, arr, flags);
   PR_HIP(hipGetLastError());
