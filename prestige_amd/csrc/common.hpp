@@ -153,10 +153,12 @@ bool inc_in_one(uint64_t n, size_t cell_tiles);
 // head[c] holds (epoch << 32 | last slot linked), next[slot] the slot linked
 // before it (kListEnd for the first of this epoch, so heads need no clearing but
 // when the 32-bit epochs start again, at 1).  Word w of mask has bit l set when
-// slot 64 w + l moved.  Contexts whose build is one launch also take what came
-// less what left per kCellGroup cells (gnet).
+// slot 64 w + l moved.  What came less what left is also taken per 2^net_shift
+// cells (net): per kCellGroup where the build is one launch, else per kTileGroup
+// tiles.
 constexpr uint32_t kCellTile = 1024;
-constexpr uint32_t kCellGroup = 32;
+constexpr uint32_t kCellGroup = 32;    // 2^5
+constexpr uint32_t kTileGroup = 256;   // 2^8 tiles of 2^10 cells
 constexpr uint32_t kListEnd = 0xFFFFFFFFu;
 // Slots one cell's list takes in one step.  Steps within the CFL bounds stay
 // far below; a runaway that throws more than this into one cell leaves the
@@ -165,10 +167,10 @@ constexpr uint32_t kListEnd = 0xFFFFFFFFu;
 constexpr uint32_t kMaxIn = 1u << 16;
 struct MovedOut {
   uint64_t* mask;
-  uint32_t *cin, *cout, *tin, *tout, *gnet;
+  uint32_t *cin, *cout, *tin, *tout, *net;
   uint64_t* head;
   uint32_t* next;
-  uint32_t epoch;
+  uint32_t epoch, net_shift;
   uint32_t* flags;
 };
 // Slot i goes from cell old_key to cell key: record it; false when it stays
@@ -184,9 +186,9 @@ __device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old
   atomicAdd(&mo.cout[old_key], 1u);
   atomicAdd(&mo.tin[key / kCellTile], 1u);
   atomicAdd(&mo.tout[old_key / kCellTile], 1u);
-  if (mo.gnet && key / kCellGroup != old_key / kCellGroup) {
-    atomicAdd(&mo.gnet[key / kCellGroup], 1u);
-    atomicSub(&mo.gnet[old_key / kCellGroup], 1u);
+  if (key >> mo.net_shift != old_key >> mo.net_shift) {
+    atomicAdd(&mo.net[key >> mo.net_shift], 1u);
+    atomicSub(&mo.net[old_key >> mo.net_shift], 1u);
   }
   const unsigned long long mine = ((unsigned long long)mo.epoch << 32) | i;
   const unsigned long long last = atomicExch(reinterpret_cast<unsigned long long*>(&mo.head[key]), mine);
@@ -299,20 +301,21 @@ struct Ctx {
   DevBuf sort_hist, sort_tot;    // per-tile digit counts, per-digit totals
   // incremental sort (MovedOut): moved-slot mask, links per slot, the spare
   // cell table, and in one buffer the list heads per cell and the counts cin,
-  // cout (inc_tiles * kCellTile each), gnet (a kCellGroup-th of that), tin, tout
-  // (inc_tiles each).  Where the build is one launch there are two sets of
+  // cout (inc_tiles * kCellTile each), net (inc_nets), tin, tout (inc_tiles each).  Where the build is one launch there are two sets of
   // counts: a step writes set inc_set, its build reads it and clears the other.
   DevBuf inc_mask, inc_next, lb_spare, inc_cells;
   size_t inc_tiles = 0;
   uint64_t* inc_head() const { return inc_cells.as<uint64_t>(); }
   size_t inc_head_bytes() const { return inc_tiles * kCellTile * 8; }
-  size_t inc_set_words() const { return (inc_tiles * (2 * kCellTile + kCellTile / kCellGroup + 2) + 3) / 4 * 4; }
+  uint32_t inc_net_shift() const { return inc_one ? 5u : 18u; }
+  size_t inc_nets() const { return ((inc_tiles * kCellTile - 1) >> inc_net_shift()) + 1; }
+  size_t inc_set_words() const { return (inc_tiles * (2 * kCellTile + 2) + inc_nets() + 3) / 4 * 4; }
   uint32_t* inc_cin(int set) const {
     return reinterpret_cast<uint32_t*>(inc_cells.as<char>() + inc_head_bytes()) + set * inc_set_words();
   }
   uint32_t* inc_cout(int set) const { return inc_cin(set) + inc_tiles * kCellTile; }
-  uint32_t* inc_gnet(int set) const { return inc_cout(set) + inc_tiles * kCellTile; }
-  uint32_t* inc_tin(int set) const { return inc_gnet(set) + inc_tiles * (kCellTile / kCellGroup); }
+  uint32_t* inc_net(int set) const { return inc_cout(set) + inc_tiles * kCellTile; }
+  uint32_t* inc_tin(int set) const { return inc_net(set) + inc_nets(); }
   uint32_t* inc_tout(int set) const { return inc_tin(set) + inc_tiles; }
   size_t inc_count_bytes() const { return (inc_one ? 2 : 1) * inc_set_words() * 4; }   // from inc_cin(0) on
   bool inc_one = false;          // the build after a step is one launch
