@@ -100,8 +100,9 @@ typedef struct prestige_desc {
   uint64_t n_particles;       /* total particles (< 2^32 - 1; < 2^31 in the MIXED WCSPH form); 0 is
                                  valid: steps and gathers then do nothing and fields are empty */
   uint64_t n_moving;          /* ids [0, n_moving) are integrated; [n_moving, n) stay fixed */
-  double grid_lo[3];          /* cell-grid origin; particles must stay in [lo, hi) */
-  double grid_hi[3];
+  double grid_lo[3];          /* cell-grid origin; particles must stay in [lo, hi); fewer than 4e9 cells */
+  double grid_hi[3];          /* (device memory: 4 bytes a cell, WCSPH 8, and 20 more (28 in small scenes) in a
+                                 context that steps, which does without these where they do not fit) */
   double cell_size;           /* >= interaction cutoff (2h for WCSPH, 2 r_max for DEM) */
   double gravity[3];
   double dt;

@@ -349,6 +349,26 @@ __global__ void k_iota_ids(uint32_t n, uint32_t* ids) {
   if (i < n) ids[i] = i;
 }
 
+// Allocates all of list, or none: false when the device is out of memory, or
+// (modest) when they would take a gigabyte and over a quarter of what is left.
+static bool alloc_if_fits(std::initializer_list<std::pair<DevBuf*, size_t>> list, bool modest) {
+  size_t want = 0, left = 0, all = 0;
+  for (auto& b : list) want += b.second;
+  if (modest && want >= (1ull << 30)) {
+    PR_HIP(hipMemGetInfo(&left, &all));
+    if (want > left / 4) return false;
+  }
+  try {
+    for (auto& b : list) b.first->alloc(b.second);
+  } catch (const Error& e) {
+    if (e.code != PRESTIGE_E_OOM) throw;
+    (void)hipGetLastError();
+    for (auto& b : list) b.first->release();
+    return false;
+  }
+  return true;
+}
+
 static void allocate(Ctx& c) {
   const uint64_t n = c.n;
   const bool f32 = c.desc.precision == PRESTIGE_F32;
@@ -377,15 +397,11 @@ static void allocate(Ctx& c) {
     c.inc_tiles = (cells + kCellTile - 1) / kCellTile;
     c.inc_one = inc_in_one(n, c.inc_tiles);
     c.inc_mask.alloc(((nn + 63) / 64) * 8);
-    c.inc_next.alloc(nn * 4);
-    PR_HIP(hipMemsetAsync(c.inc_next.p, 0xFF, nn * 4, c.stream));   // kListEnd
-    c.lb_spare.alloc(cells * 4);
-    c.inc_cells.alloc(c.inc_head_bytes() + c.inc_count_bytes());
-    PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, c.inc_cells.bytes, c.stream));
   }
   if (const char* dr = std::getenv("PRESTIGE_DRY")) c.dry_reuse = std::string(dr) != "off";
   if (const char* ep = std::getenv("PRESTIGE_EPOCH")) c.inc_epoch = (uint32_t)std::strtoul(ep, nullptr, 10);
-  if (const char* sp = std::getenv("PRESTIGE_SORT")) c.sort_radix = std::string(sp) == "radix";
+  const char* sp = std::getenv("PRESTIGE_SORT");
+  c.sort_radix = sp && std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc((FLAG_COUNT + 2) * 4);
   PR_HIP(hipHostMalloc(&c.pin, kPinBytes + kNotes * 4, hipHostMallocMapped));
@@ -445,10 +461,6 @@ static void allocate(Ctx& c) {
       if (std::string(e) == "on") c.quad = true;
       else if (std::string(e) == "off") c.quad = false;
     }
-    if (c.quad) {
-      c.nlist.alloc(((nn + 15) / 16) * 2048 * sizeof(uint32_t));
-      c.ncnt.alloc(nn * sizeof(uint32_t));
-    }
   }
   c.scratch.alloc(nn * 8);
   if (dem) {
@@ -462,6 +474,19 @@ static void allocate(Ctx& c) {
       PR_HIP(hipMemsetAsync(c.hcnt[b].p, 0, nn * 4, c.stream));
       PR_HIP(hipMemsetAsync(c.wxi[b].p, 0, nn * 18 * hr, c.stream));
     }
+  }
+  // Last, what a context can do without: the neighbour lists of the four-lane
+  // passes, and the lists and counts per cell of the incremental sort (20 bytes a
+  // cell, 28 in small scenes, where the keys' own sorts need 4), unless they would
+  // take a gigabyte and over a quarter of the memory left.
+  if (c.quad)
+    c.quad = alloc_if_fits({{&c.nlist, ((nn + 15) / 16) * 2048 * sizeof(uint32_t)}, {&c.ncnt, nn * sizeof(uint32_t)}}, false);
+  if (c.desc.model != PRESTIGE_MODEL_PAIRS && !(sp && std::string(sp) == "keys") &&
+      alloc_if_fits({{&c.inc_cells, c.inc_head_bytes() + c.inc_count_bytes()},
+                     {&c.lb_spare, ((size_t)c.grid.n_cells + 1) * 4},
+                     {&c.inc_next, nn * 4}}, true)) {
+    PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, c.inc_cells.bytes, c.stream));
+    PR_HIP(hipMemsetAsync(c.inc_next.p, 0xFF, nn * 4, c.stream));   // kListEnd
   }
   if (n) {
     k_iota_ids<<<blocks_for(n), kBlock, 0, c.stream>>>((uint32_t)n, c.ids[0].as<uint32_t>());

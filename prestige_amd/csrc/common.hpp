@@ -177,6 +177,7 @@ struct MovedOut {
 // (key is then old_key).
 __device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old_key, uint32_t& key) {
   if (key == old_key) return false;
+  if (!mo.cin) return true;   // a context without them sorts by the keys alone
   if (atomicAdd(&mo.cin[key], 1u) >= kMaxIn) {
     atomicSub(&mo.cin[key], 1u);
     atomicOr(&mo.flags[FLAG_CAPACITY], 1u);
@@ -303,8 +304,10 @@ struct Ctx {
   // cell table, and in one buffer the list heads per cell and the counts cin,
   // cout (inc_tiles * kCellTile each), net (inc_nets), tin, tout (inc_tiles each).  Where the build is one launch there are two sets of
   // counts: a step writes set inc_set, its build reads it and clears the other.
+  // A context they do not fit has the mask only, and every build sorts anew.
   DevBuf inc_mask, inc_next, lb_spare, inc_cells;
   size_t inc_tiles = 0;
+  bool inc_fits() const { return inc_cells.p != nullptr; }
   uint64_t* inc_head() const { return inc_cells.as<uint64_t>(); }
   size_t inc_head_bytes() const { return inc_tiles * kCellTile * 8; }
   uint32_t inc_net_shift() const { return inc_one ? 5u : 18u; }
@@ -323,7 +326,7 @@ struct Ctx {
   uint32_t inc_epoch = 0;        // of the last step (PRESTIGE_EPOCH starts it elsewhere, for tests)
   bool inc_ready = false;        // keys[cur_key] are the next keys of the last build's slots
   bool inc_counts = false;       // a step's counts are waiting (a build that does not use them clears them)
-  bool sort_radix = false;       // PRESTIGE_SORT=radix: every build sorts anew (comparisons and tests)
+  bool sort_radix = false;       // PRESTIGE_SORT=radix: every build is a radix sort (comparisons and tests)
   DevBuf lb;                     // n_cells + 1
   // WCSPH wall particles far from the fluid (DryWalls): cell stamps (n_cells),
   // last dry pass per particle id, pass counter, the pass the stamps describe,

@@ -583,6 +583,11 @@ constexpr uint64_t kIncOne = 400000;
 bool inc_in_one(uint64_t n, size_t cell_tiles) { return cell_tiles <= (size_t)kBlock && n <= kIncOne; }
 
 MovedOut moved_out(Ctx& c) {
+  if (!c.inc_fits()) {
+    MovedOut mo{};
+    mo.mask = c.inc_mask.as<uint64_t>();
+    return mo;
+  }
   c.inc_counts = true;
   const int s = c.inc_set;
   if (++c.inc_epoch == 0u) {   // wrapped: heads left 2^32 steps ago, or never written, would pass for this step's
@@ -924,7 +929,7 @@ void neighbors_build(Ctx& c) {
   // incremental when the state is still in the previous build's slot order
   // with fresh keys (right after a step)
   const int src = c.cur, dst = c.cur ^ 1;
-  if (c.inc_ready && !c.sort_radix) {
+  if (c.inc_ready && c.inc_fits() && !c.sort_radix) {
     incremental_sort(c);
   } else {
     if (c.inc_counts) {   // counts of a step this build does not continue
