@@ -160,10 +160,13 @@ constexpr uint32_t kCellTile = 1024;
 constexpr uint32_t kCellGroup = 32;    // 2^5
 constexpr uint32_t kTileGroup = 256;   // 2^8 tiles of 2^10 cells
 constexpr uint32_t kListEnd = 0xFFFFFFFFu;
-// Slots one cell's list takes in one step.  Steps within the CFL bounds stay
-// far below; a runaway that throws more than this into one cell leaves the
-// rest in their old cells and raises the capacity flag, so that every list
-// walk stays short.
+// Runaways (particles that outran the time step, which is an error) one cell's
+// list takes in one step; the others stay in their old cells.  A build walks a
+// cell's list once for every slot of the cell, a dependent load (some 0.4 us) an
+// entry: 65,536 take 30 ms.  Particles within the step's bound are all listed: they
+// enter in such numbers only where as many share the cell, and the contact pass
+// tests each of those against all others (more than 128 in a row of cells end a
+// WCSPH step).
 constexpr uint32_t kMaxIn = 1u << 16;
 struct MovedOut {
   uint64_t* mask;
@@ -171,16 +174,14 @@ struct MovedOut {
   uint64_t* head;
   uint32_t* next;
   uint32_t epoch, net_shift;
-  uint32_t* flags;
 };
 // Slot i goes from cell old_key to cell key: record it; false when it stays
 // (key is then old_key).
-__device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old_key, uint32_t& key) {
+__device__ inline bool move_to_cell(const MovedOut& mo, uint32_t i, uint32_t old_key, uint32_t& key, bool runaway) {
   if (key == old_key) return false;
   if (!mo.cin) return true;   // a context without them sorts by the keys alone
-  if (atomicAdd(&mo.cin[key], 1u) >= kMaxIn) {
+  if (atomicAdd(&mo.cin[key], 1u) >= kMaxIn && runaway) {
     atomicSub(&mo.cin[key], 1u);
-    atomicOr(&mo.flags[FLAG_CAPACITY], 1u);
     key = old_key;
     return false;
   }

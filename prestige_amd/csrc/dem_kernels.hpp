@@ -315,7 +315,8 @@ __global__ __launch_bounds__(64) void k_dem_force(
       if (sub == 0u) {
         uint32_t key = key_i;   // a sphere outside the grid keeps its cell
         if (ok) key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
-        mv = move_to_cell(moved, i, key_i, key);
+        const bool runaway = (v2.x * v2.x + v2.y * v2.y + v2.z * v2.z) * (kc.dt * kc.dt) > 0.0625 * (r64 * r64);
+        mv = move_to_cell(moved, i, key_i, key, runaway);
         opos[i] = x2;
         ovel[i] = v2;
         oom[i] = w2;
@@ -328,8 +329,7 @@ __global__ __launch_bounds__(64) void k_dem_force(
           events[(size_t)n + me] += ev_weight * nslip;
         }
         if (!isfinite(axx) || !isfinite(ayy) || !isfinite(azz)) atomicOr(&flags[FLAG_NONFINITE], 1u);
-        if ((v2.x * v2.x + v2.y * v2.y + v2.z * v2.z) * (kc.dt * kc.dt) > 0.0625 * (r64 * r64))
-          atomicOr(&flags[FLAG_CFL], 1u);
+        if (runaway) atomicOr(&flags[FLAG_CFL], 1u);
         if (!ok) atomicOr(&flags[FLAG_DOMAIN], 1u);
       }
     }

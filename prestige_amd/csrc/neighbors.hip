@@ -595,7 +595,7 @@ MovedOut moved_out(Ctx& c) {
     c.inc_epoch = 1u;
   }
   return MovedOut{c.inc_mask.as<uint64_t>(), c.inc_cin(s), c.inc_cout(s), c.inc_tin(s), c.inc_tout(s), c.inc_net(s),
-                  c.inc_head(), c.inc_next.as<uint32_t>(), c.inc_epoch, c.inc_net_shift(), c.flags.as<uint32_t>()};
+                  c.inc_head(), c.inc_next.as<uint32_t>(), c.inc_epoch, c.inc_net_shift()};
 }
 
 static void inc_taken(Ctx& c) {

@@ -1133,8 +1133,9 @@ __device__ inline bool force_store(uint32_t i, bool live, const Sum<typename Sph
   o.ovel[i] = v2;
   if (o.oacc) o.oacc[i] = S4{ax, ay, az, 0};
   if (!isfinite(ax) || !isfinite(ay) || !isfinite(az)) atomicOr(&o.flags[FLAG_NONFINITE], 1u);
-  if ((double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2)
-    atomicOr(&o.flags[FLAG_CFL], 1u);
+  const bool runaway =
+      (double)v2.x * (double)v2.x + (double)v2.y * (double)v2.y + (double)v2.z * (double)v2.z > kc.cfl_v2;
+  if (runaway) atomicOr(&o.flags[FLAG_CFL], 1u);
   // next step's cell key, same FP64 floor as the key kernel
   double fx = floor(((double)x2.x - g.lo[0]) * g.inv_cs);
   double fy = floor(((double)x2.y - g.lo[1]) * g.inv_cs);
@@ -1146,7 +1147,7 @@ __device__ inline bool force_store(uint32_t i, bool live, const Sum<typename Sph
     key = ((uint32_t)fz * (uint32_t)g.dims[1] + (uint32_t)fy) * (uint32_t)g.dims[0] + (uint32_t)fx;
   else
     atomicOr(&o.flags[FLAG_DOMAIN], 1u);
-  const bool mv = move_to_cell(o.moved, i, old_key, key);
+  const bool mv = move_to_cell(o.moved, i, old_key, key, runaway);
   o.okeys[i] = key;
   o.movcell[key] = o.next_pass;   // this cell holds a moving particle at the next density pass
   return mv;
