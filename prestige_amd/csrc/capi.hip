@@ -95,23 +95,29 @@ LaunchScope::~LaunchScope() noexcept(false) {
 // ---------------------------------------------------------------------------
 // host transfers
 // ---------------------------------------------------------------------------
-// Small transfers go through the context's pinned block: the runtime's own
-// staging of a pageable buffer costs more than a memcpy, and kernels queued
-// behind such an upload often start 55 us late.  Larger uploads are the
-// runtime's.  Larger downloads go through a ring of chunks: this thread drives the
-// link while a few others first have the kernel map the caller's pages, most of
-// the cost of a fresh array, and then copy from the ring.  The results are the
-// caller's ordinary memory: arrays of pinned memory would save all this, but a
-// process forked later does not have them.
+// The caller's own pinned memory takes the link directly.  Of ordinary memory,
+// small transfers go through the context's pinned block: the runtime's own staging
+// costs more than a memcpy, and kernels queued behind such an upload often start
+// 55 us late.  Larger uploads and downloads of up to kRingFrom are the runtime's.
+// Larger downloads go through a ring of chunks: this thread drives the link while a
+// few others first have the kernel map the caller's pages, most of the cost of a
+// fresh array, and then copy from the ring.  The results are the caller's ordinary
+// memory: arrays of pinned memory would save all this, but a process forked later
+// does not have them.
 //
-// Us a field of 10,000 / 100,000 / 200,000 / 571,000 / 1.8M / 6.03M values, all
-// by the runtime and with the checks on the host, then now: upload 56 / 70 / 129 /
-// 289 / 807 / 3223 -> 26 / 50 / 87 / 176 / 445 / 1869, download into fresh arrays
-// 59 / 93 / 282 / 568 / 1369 / 4930 -> 27 / 92 / 199 / 277 / 566 / 2986 (into
-// pinned arrays 571,000 take 112).  At 1 MiB both ways of a download take 135; a
-// chunk of 1 MiB keeps the threads busy from a few MiB on, from 8 MiB on 2 MiB
-// ask for fewer events (1.8M values 597 -> 566).
-constexpr size_t kPinBytes = 1u << 20;
+// Us a field of 10,000 / 100,000 / 571,000 / 1.8M / 6.03M values, all by the
+// runtime and with the checks on the host, then now: upload 24 / 65 / 281 / 784 /
+// 2954 -> 23 / 47 / 160 / 432 / 1551, download into fresh arrays 57 / 56 / 269 / 775
+// / 4483 -> 25 / 57 / 194 / 413 / 2636, into pinned ones 21 / 34 / 104 / 287 / 905
+// either way (by the ring 571,000 took 193).  The lines: values of an id-order field
+// downloaded again into one array, by the runtime / through the block, 10,000 41 /
+// 12, 100,000 40 / 41, 131,072 60 / 65; by the runtime / the ring, 200,000 87 / 101,
+// 230,000 94 / 103, 262,000 104 / 104, 300,000 135 / 107.  A chunk of 1 MiB keeps the
+// threads busy from a few MiB on, from 8 MiB on 2 MiB ask for fewer events (1.8M
+// values 597 -> 566).
+constexpr size_t kStage = 768u << 10;     // the largest pinned block, and what goes through it
+constexpr size_t kRingFrom = 2u << 20;    // downloads through the ring
+constexpr size_t kAsk = 64;               // from here on a pointer is asked about (flags and parameter sums are smaller)
 constexpr size_t kRing = 8u << 20, kChunk = 1u << 20, kBigChunk = 2u << 20;   // the ring, what the link moves at a time
 constexpr size_t kUnit = 128u << 10, kPages = 2u << 20;   // what a thread copies, and has mapped, at a time
 constexpr uint32_t kCopyThreads = 6;
@@ -194,9 +200,21 @@ static char* ring(Ctx& c) {
   return static_cast<char*>(c.ring);
 }
 
+// Whether host is an allocation the runtime knows, which the link reads and writes by
+// itself: the caller's own pinned memory.
+static bool is_pinned(const void* host, size_t bytes) {
+  hipPointerAttribute_t a;
+  if (bytes < kAsk) return false;
+  if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 void to_device(Ctx& c, void* dst, const void* host, size_t bytes) {
   if (!bytes) return;
-  if (bytes <= kPinBytes) {
+  if (bytes <= c.pin_bytes && !is_pinned(host, bytes)) {
     PR_HIP(hipStreamSynchronize(c.stream));   // the block may still be on its way
     std::memcpy(c.pin, host, bytes);
     host = c.pin;
@@ -206,7 +224,13 @@ void to_device(Ctx& c, void* dst, const void* host, size_t bytes) {
 
 // Waits for the stream.
 void to_host(Ctx& c, void* host, const void* src, size_t bytes) {
-  if (bytes <= kPinBytes) {
+  const bool direct = is_pinned(host, bytes) || (bytes > c.pin_bytes && bytes < kRingFrom);
+  if (direct) {
+    PR_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, c.stream));
+    PR_HIP(hipStreamSynchronize(c.stream));
+    return;
+  }
+  if (bytes <= c.pin_bytes) {
     if (bytes) PR_HIP(hipMemcpyAsync(c.pin, src, bytes, hipMemcpyDeviceToHost, c.stream));
     PR_HIP(hipStreamSynchronize(c.stream));
     if (bytes) std::memcpy(host, c.pin, bytes);
@@ -404,11 +428,13 @@ static void allocate(Ctx& c) {
   c.sort_radix = sp && std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc((FLAG_COUNT + 2) * 4);
-  PR_HIP(hipHostMalloc(&c.pin, kPinBytes + kNotes * 4, hipHostMallocMapped));
+  // three fields (seeds, gradients), up to kStage
+  c.pin_bytes = std::min(kStage, (nn * 24 + 4095) / 4096 * 4096);
+  PR_HIP(hipHostMalloc(&c.pin, c.pin_bytes + kNotes * 4, hipHostMallocMapped));
   void* pin_dev = nullptr;
   PR_HIP(hipHostGetDevicePointer(&pin_dev, c.pin, 0));
-  c.note = reinterpret_cast<uint32_t*>(static_cast<char*>(c.pin) + kPinBytes);
-  c.note_dev = reinterpret_cast<uint32_t*>(static_cast<char*>(pin_dev) + kPinBytes);
+  c.note = reinterpret_cast<uint32_t*>(static_cast<char*>(c.pin) + c.pin_bytes);
+  c.note_dev = reinterpret_cast<uint32_t*>(static_cast<char*>(pin_dev) + c.pin_bytes);
   std::memset(c.note, 0, kNotes * 4);
   PR_HIP(hipEventCreateWithFlags(&c.counted, hipEventDisableTiming));
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {

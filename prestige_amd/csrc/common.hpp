@@ -339,6 +339,7 @@ struct Ctx {
   void forget_dry() { dens_pass += 2; }   // state changed outside a step
   DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word and a first build's (Crowd)
   void* pin = nullptr;                       // pinned block for small transfers
+  size_t pin_bytes = 0;
   // pinned words that kernels leave for the host (host and device address), 0 until then
   uint32_t *note = nullptr, *note_dev = nullptr;
   bool take_note(int k) {   // reads and clears; after the kernel has been waited for
