@@ -96,3 +96,28 @@ def test_pinned_memory_takes_the_link():
     assert hip().hipFree(dev) == 0
     block.free()
     assert field < 1.5 * plain
+
+
+@pytest.mark.parametrize("n", [1, 3, 4095, 4096, 4097])   # checked on the host up to 4,096 values, then on the device
+@pytest.mark.parametrize("name,value,status", [("x", np.nan, 5), ("x", -np.inf, 5), ("radius", np.inf, 5), ("radius", 0.0, 1),
+                                               ("radius", -0.1, 1), ("radius", 0.6, 1), ("mass", np.nan, 1), ("mass", 0.0, 1)])
+def test_one_bad_value(n, name, value, status):
+    d = pa.desc_init(pa.MODEL_DEM)
+    d.n_particles = d.n_moving = n
+    d.cell_size, d.dt = 1.0, 1e-5
+    for a in range(3):
+        d.grid_lo[a], d.grid_hi[a] = 0.0, 10.0
+    good = np.random.default_rng(n).uniform(0.1, 0.5, n)
+    good[0] = 0.5   # a radius of half a cell is allowed
+    with pa.Context(d) as ctx:
+        ctx.upload(name, good)
+        for at in {0, n // 2, n - 1}:
+            bad = good.copy()
+            bad[at] = value
+            with pytest.raises(pa.PrestigeError) as e:
+                ctx.upload(name, bad)
+            assert e.value.status == status
+        if name != "mass":   # (the equations' mass is replaced before the check)
+            assert np.array_equal(ctx.download(name), good)
+        ctx.upload(name, good)
+        assert np.array_equal(ctx.download(name), good)
