@@ -354,8 +354,9 @@ void dem_step_impl(Ctx& c) {
   const double ge = (double)sizeof(real);
   const double lb_bytes = 4.0 * (double)c.grid.n_cells / (double)n;
   // gathered: pos 3 + r, vel 3 + m, omega 3; ids + key; state in/out (pos, vel, omega) 3 x 24 x 2;
-  // history in/out: count + (typical) 6 slots x (id + 3 reals) + walls 18 reals
-  double hist_bytes = 2.0 * (4.0 + 6.0 * (4.0 + 3.0 * ge) + 18.0 * ge);
+  // history in/out: count + (typical) 6 slots x (id + 3 reals); wall springs move for
+  // the few spheres that touch a wall only
+  double hist_bytes = 2.0 * (4.0 + 6.0 * (4.0 + 3.0 * ge));
   double bytes = (11.0 * ge + 8.0 + lb_bytes + 2.0 * 3.0 * 32.0 + 4.0 + hist_bytes) * n;
   LaunchScope ls(&c, F == kF64 ? "dem_force_f64" : "dem_force_mixed", bytes);
   const int dst = c.cur ^ 1, kdst = c.cur_key ^ 1;
