@@ -112,11 +112,11 @@ LaunchScope::~LaunchScope() noexcept(false) {
 // / 4483 -> 25 / 57 / 194 / 413 / 2636, into pinned ones 21 / 34 / 104 / 287 / 905
 // either way (by the ring 571,000 took 193).  The lines: values of an id-order field
 // downloaded again into one array, by the runtime / through the block, 10,000 41 /
-// 12, 100,000 40 / 41, 131,072 60 / 65; by the runtime / the ring, 200,000 87 / 101,
+// 12, 100,000 40 / 40, 125,000 48 / 48, 131,072 60 / 63; by the runtime / the ring, 200,000 87 / 101,
 // 230,000 94 / 103, 262,000 104 / 104, 300,000 135 / 107.  A chunk of 1 MiB keeps the
 // threads busy from a few MiB on, from 8 MiB on 2 MiB ask for fewer events (1.8M
 // values 597 -> 566).
-constexpr size_t kStage = 768u << 10;     // the largest pinned block, and what goes through it
+constexpr size_t kStage = 976u << 10;     // the largest pinned block, and what goes through it
 constexpr size_t kRingFrom = 2u << 20;    // downloads through the ring
 constexpr size_t kAsk = 64;               // from here on a pointer is asked about (flags and parameter sums are smaller)
 constexpr size_t kRing = 8u << 20, kChunk = 1u << 20, kBigChunk = 2u << 20;   // the ring, what the link moves at a time
