@@ -835,7 +835,7 @@ __global__ __launch_bounds__(kDensBlock, WALK ? kDensWaves<F> : 4) void k_sph_de
     if (__ballot(!keep) == 0ull) {
       if (live && dw.zero_masks)
         for (uint32_t r = 0; r < kRuns; ++r)
-        if (WALK || r == sph_run(blockIdx.y)) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
+          if (WALK || r == sph_run(blockIdx.y)) meta[meta_index(r, n, i)] = make_uint2(0u, 0u);
       if constexpr (WALK)
         if (live) density_keep<F>(i, id, pi, wvel, kc, dw, rp, pres);
       return;
@@ -1367,12 +1367,13 @@ void sph_density_launch(Ctx& c, const SphStepIO<F>& io, typename SphForm<F>::R2*
     if (F == kF64 && c.record_all) launch(k_sph_density_quad<F, F == kF64>);
     else launch(k_sph_density_quad<F, false>);
     PR_HIP(hipGetLastError());
-    if (F == kMixed && c.record_all) {
+    if constexpr (F == kMixed) {
+      if (!c.record_all) return;
       // the mixed reverse passes round by how a lane's hits pair up in its
       // walk, so their masks are the one-lane scan's to the last bit
       LaunchScope lm(&c, "sph_masks", 0.0);
       const uint32_t tiles = blocks_for(n, kDensBlock);
-      k_sph_density<F, F != kMixed><<<dim3(tile_grid(tiles), kRuns), kDensBlock, 0, c.stream>>>(
+      k_sph_density<F, false><<<dim3(tile_grid(tiles), kRuns), kDensBlock, 0, c.stream>>>(
           n, c.pos[c.cur].as<S4>(), io.gpos, io.skeys, c.lb.as<uint32_t>(), c.grid, c.sph, io.u, c.nmeta.as<uint2>(),
           c.nword.as<uint32_t>(), rp, wpos, wvel, pres, c.flags.as<uint32_t>(), tiles, io.dw);
       PR_HIP(hipGetLastError());
