@@ -496,7 +496,9 @@ static void allocate(Ctx& c) {
     // 228/211, 294/290, 329/335, 424/480; FP32 109/40, 126/82, 165/154, 206/202,
     // 229/233, 286/330; mixed 138/45, 172/99, 227/193, 257/258, 280/315, 344/440.
     // The line lies where the two meet (mixed earlier, 225/227 at 250k: its
-    // compensated sums run under a mask).  The lists take 516 B a particle, so a
+    // compensated sums run under a mask) in stirred fluid; in the first hundred steps
+    // from rest they meet at 200k to 250k (300k FP64 225/239, FP32 166/180, after a
+    // thousand 266/240 and 182/180).  The lists take 516 B a particle, so a
     // context of over a million particles does without.
     const uint64_t most = mixed ? 240000u : 320000u;
     c.quad = c.n_moving <= most && n <= 1000000u;

@@ -12,9 +12,9 @@
 // pair.  Here the nine runs' table entries are read at once, each run's
 // candidates are loaded while the previous run is scanned, the hits of all
 // runs become one list per particle, and the walk knows every neighbour's
-// address ahead.  Density / force, us, against one lane per particle: 42,866
-// particles FP64 67 / 55 -> 27 / 17, 196k mixed 109 / 63 -> 61 / 38, 571k FP32
-// 98 / 87 -> 120 / 55.  What bounds them now: at 42,866 particles a wavefront's
+// address ahead.  Density / force, us, against one lane per particle (steps
+// 30-150 of a dam break): 42,866 particles FP64 63 / 44 -> 27 / 16, 196k mixed 103 /
+// 51 -> 56 / 33, 571k FP32 85 / 61 -> 107 / 46.  What bounds them now: at 42,866 particles a wavefront's
 // own chain (alone on its SIMD a chunk of 64 candidates takes 1,700 cycles, five
 // trips through LDS and ten rounds of writing hits among them, and a round of
 // the walk 1,000; deeper prefetch changes nothing); at 571k instruction issue
