@@ -453,7 +453,6 @@ static void allocate(Ctx& c) {
   c.note = reinterpret_cast<uint32_t*>(static_cast<char*>(c.pin) + c.pin_bytes);
   c.note_dev = reinterpret_cast<uint32_t*>(static_cast<char*>(pin_dev) + c.pin_bytes);
   std::memset(c.note, 0, kNotes * 4);
-  PR_HIP(hipEventCreateWithFlags(&c.counted, hipEventDisableTiming));
   if (c.desc.model == PRESTIGE_MODEL_WCSPH) {
     c.movcell.alloc(((size_t)c.grid.n_cells + 1) * 4);
     PR_HIP(hipMemsetAsync(c.movcell.p, 0, ((size_t)c.grid.n_cells + 1) * 4, c.stream));

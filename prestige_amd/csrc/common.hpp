@@ -262,7 +262,7 @@ struct Tape {
   }
 };
 
-// Words of Ctx::note: what a field check found (kNoteField + bit), a crowded cell.
+// Words of Ctx::note: what a field check found (kNoteField + bit), a first build's (Crowd).
 enum Note : int { kNoteField = 0, kNoteCrowd = 3, kNotes = 4 };
 
 struct Ctx {
@@ -273,7 +273,6 @@ struct Ctx {
     if (pin) (void)hipHostFree(pin);
     if (ring) (void)hipHostFree(ring);
     for (auto e : ring_ev) (void)hipEventDestroy(e);
-    if (counted) (void)hipEventDestroy(counted);
   }
   prestige_desc desc{};
   int device = 0;
@@ -340,7 +339,7 @@ struct Ctx {
   DevBuf flags;                  // FLAG_COUNT uint32, then the field check's word and a first build's (Crowd)
   void* pin = nullptr;                       // pinned block for small transfers
   size_t pin_bytes = 0;
-  // pinned words that kernels leave for the host (host and device address), 0 until then
+  // pinned words that kernels leave for the host (host and device address)
   uint32_t *note = nullptr, *note_dev = nullptr;
   bool take_note(int k) {   // reads and clears; after the kernel has been waited for
     volatile uint32_t* w = note + k;
@@ -348,7 +347,7 @@ struct Ctx {
     if (set) *w = 0u;
     return set;
   }
-  hipEvent_t counted = nullptr;              // the counting sort's table is written
+  uint32_t count_builds = 0;                 // first builds that asked for a crowded cell (Crowd)
   void* ring = nullptr;                      // pinned chunks of large ones, from the first on
   std::vector<hipEvent_t> ring_ev;
   // gather outputs

@@ -5,7 +5,9 @@
 // The sorted layout is what every gather kernel iterates: for a particle in
 // cell (cx, cy, cz) the three cells cx-1..cx+1 of each of the nine (dy, dz)
 // rows are one contiguous run [lb[row + cx-1], lb[row + cx+2]) of slots.
+#include <chrono>
 #include <mutex>
+#include <thread>
 
 #include "common.hpp"
 
@@ -671,7 +673,7 @@ static void incremental_sort(Ctx& c) {
 // units put all of them there).  So a context's build turns back at a cell of more
 // than kCountMost, which the host hears of while the table and the lists are
 // written, and sorts by radix: 20,000 in 110, a million in 240.  Asking costs the
-// builds that go on 3-5 us.  eq1 without allocating does not ask, being quadratic
+// builds that go on up to 4 us.  eq1 without allocating does not ask, being quadratic
 // in a crowd itself.
 constexpr uint32_t kCountCells = 1u << 22;
 constexpr uint32_t kCountMost = 2048;
@@ -691,14 +693,16 @@ __global__ __launch_bounds__(kBlock) void k_count_clear(uint32_t n, uint32_t* __
   if (i < n_words) words[i] = 0u;
 }
 
-// What the count of a cell that passes kCountMost sets: a device word, after which
-// the counting sort's kernels may leave their outputs unwritten, and the host's.
+// A device word that the count of a cell sets when it passes kCountMost; the counting
+// sort's kernels may then leave their outputs unwritten.  The kernel after the counts
+// tells the host: note is 2 build + (the word).
 struct Crowd {
   uint32_t *word, *note;
+  uint32_t build;
   __device__ bool seen() const { return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u; }
-  __device__ void set() const {
-    __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(note, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __device__ void set() const { __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  __device__ void tell() const {
+    __hip_atomic_store(note, 2u * build + (seen() ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 };
 
@@ -733,8 +737,9 @@ __global__ __launch_bounds__(kBlock) void k_count_keys(uint32_t n, const uint32_
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_tiles(uint32_t n_cells, const uint32_t* __restrict__ cnt,
-                                                        uint32_t* __restrict__ tot) {
+                                                        uint32_t* __restrict__ tot, Crowd crowd) {
   __shared__ uint32_t s4[4];
+  if (crowd.note && blockIdx.x == 0u && threadIdx.x == 0u) crowd.tell();
   uint32_t sum = 0;
 #pragma unroll
   for (uint32_t k = 0; k < kCellTile / kBlock; ++k) {
@@ -818,11 +823,12 @@ __global__ __launch_bounds__(kBlock) void k_count_place(uint32_t n, const uint32
   move_slot<T4, OMEGA, PROBE, MIXED>(io, i, pos, c);
 }
 
-// n_cells + 1 counts (the last unused) to the cell table; tot: a total per tile.
-static void count_table(Ctx* c, uint32_t n_cells, uint32_t* cnt, uint32_t* tot, hipStream_t st) {
+// n_cells + 1 counts (the last unused) to the cell table; tot: a total per tile;
+// crowd.note may be null.
+static void count_table(Ctx* c, uint32_t n_cells, uint32_t* cnt, uint32_t* tot, const Crowd& crowd, hipStream_t st) {
   LaunchScope ls(c, "sort_count_cells", 12.0 * n_cells);
   const uint32_t tiles = blocks_for((uint64_t)n_cells + 1u, (int)kCellTile);
-  k_count_tiles<<<tiles, kBlock, 0, st>>>(n_cells, cnt, tot);
+  k_count_tiles<<<tiles, kBlock, 0, st>>>(n_cells, cnt, tot, crowd);
   PR_HIP(hipGetLastError());
   k_count_table<<<tiles, kBlock, 0, st>>>(n_cells, tot, cnt);
   PR_HIP(hipGetLastError());
@@ -835,8 +841,9 @@ static bool context_count_sort(Ctx& c) {
   const uint32_t n = (uint32_t)c.n, cells = c.grid.n_cells;
   const uint32_t* keys = c.keys[c.cur_key].as<uint32_t>();
   uint32_t* arr = c.vals[0].as<uint32_t>();
-  const Crowd crowd{c.flags.as<uint32_t>() + FLAG_COUNT + 1, c.note_dev + kNoteCrowd};
   const bool ask = n > kCountMost;
+  const uint32_t build = ask ? ++c.count_builds & 0x7FFFFFFFu : 0u;
+  const Crowd crowd{c.flags.as<uint32_t>() + FLAG_COUNT + 1, ask ? c.note_dev + kNoteCrowd : nullptr, build};
   {
     LaunchScope ls(&c, "sort_count", 4.0 * cells + 12.0 * n);
     k_count_clear<<<blocks_for(cells + 1u), kBlock, 0, c.stream>>>(cells + 1u, c.lb.as<uint32_t>(), 1u, crowd.word);
@@ -844,8 +851,7 @@ static bool context_count_sort(Ctx& c) {
     k_count_keys<<<blocks_for(n), kBlock, 0, c.stream>>>(n, keys, c.lb.as<uint32_t>(), arr, crowd);
     PR_HIP(hipGetLastError());
   }
-  if (ask) PR_HIP(hipEventRecord(c.counted, c.stream));
-  count_table(&c, cells, c.lb.as<uint32_t>(), c.sort_hist.as<uint32_t>(), c.stream);
+  count_table(&c, cells, c.lb.as<uint32_t>(), c.sort_hist.as<uint32_t>(), crowd, c.stream);
   uint32_t* list = c.vals[1].as<uint32_t>();
   {
     LaunchScope ls(&c, "sort_count_list", 16.0 * n);
@@ -853,8 +859,15 @@ static bool context_count_sort(Ctx& c) {
     PR_HIP(hipGetLastError());
   }
   if (ask) {
-    PR_HIP(hipEventSynchronize(c.counted));
-    if (c.take_note(kNoteCrowd)) return false;
+    // A wait for an event leaves the device idle twice as long (in the segments of an
+    // adjoint sweep, where the host is a millisecond ahead, 15 us against 5); a wait
+    // of more than 2 ms is left to the runtime.
+    volatile const uint32_t* told = c.note + kNoteCrowd;
+    const auto from = std::chrono::steady_clock::now();
+    while (*told >> 1 != build && std::chrono::steady_clock::now() - from < std::chrono::milliseconds(2))
+      std::this_thread::yield();
+    if (*told >> 1 != build) PR_HIP(hipStreamSynchronize(c.stream));
+    if (*told & 1u) return false;
   }
   LaunchScope ls(&c, "sort_count_place", (8.0 + reorder_bytes(c)) * n);
   with_reorder_form(c, c.cur, c.cur ^ 1, [&](auto form, auto io) {
@@ -1402,7 +1415,7 @@ static void eq1_cells_noalloc(const double* x, const double* y, const double* z,
   PR_HIP(hipGetLastError());
   k_count_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, g, keys, lb, arr, flags);
   PR_HIP(hipGetLastError());
-  count_table(nullptr, g.n_cells, lb, tot, st);
+  count_table(nullptr, g.n_cells, lb, tot, Crowd{}, st);
   k_count_scatter_soa<<<blocks_for(n), kBlock, 0, st>>>(n, x, y, z, keys, arr, lb, upos);
   PR_HIP(hipGetLastError());
   k_count_rank_soa<<<blocks_for(n), kBlock, 0, st>>>(n, upos, lb, mass, spos, skeys, perm);
