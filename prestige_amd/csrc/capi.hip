@@ -390,33 +390,26 @@ __global__ void k_iota_ids(uint32_t n, uint32_t* ids) {
   if (i < n) ids[i] = i;
 }
 
-// Allocates all of list, or none: false when the device is out of memory, or
-// (modest) when they would take a gigabyte and over a quarter of what is left.
-static bool alloc_if_fits(std::initializer_list<std::pair<DevBuf*, size_t>> list, bool modest) {
-  size_t want = 0, left = 0, all = 0;
-  for (auto& b : list) want += b.second;
-  if (modest && want >= (1ull << 30)) {
-    PR_HIP(hipMemGetInfo(&left, &all));
-    if (want > left / 4) return false;
-  }
-  try {
-    for (auto& b : list) b.first->alloc(b.second);
-  } catch (const Error& e) {
-    if (e.code != PRESTIGE_E_OOM) throw;
-    (void)hipGetLastError();
-    for (auto& b : list) b.first->release();
-    return false;
-  }
-  return true;
+// Whether bytes are less than a gigabyte or than a quarter of the device memory left.
+static bool is_modest(size_t bytes) {
+  size_t left = 0, all = 0;
+  if (bytes < (1ull << 30)) return true;
+  PR_HIP(hipMemGetInfo(&left, &all));
+  return bytes < left / 4;
 }
 
-static void allocate(Ctx& c) {
+// extras: with what a context can do without: the neighbour lists of the four-lane
+// passes, and the lists and counts per cell of the incremental sort (20 bytes a cell,
+// 28 in small scenes, where the keys' own sorts need 4).  May be called again without.
+static void allocate(Ctx& c, bool extras) {
   const uint64_t n = c.n;
   const bool f32 = c.desc.precision == PRESTIGE_F32;
   const bool mixed = c.desc.precision == PRESTIGE_MIXED;
   const bool dem = c.desc.model == PRESTIGE_MODEL_DEM;
   const size_t e4 = f32 ? sizeof(float4) : sizeof(double4);
   const size_t nn = n ? n : 1;
+  const char* sp = std::getenv("PRESTIGE_SORT");
+  c.sort_radix = sp && std::string(sp) == "radix";
   for (int b = 0; b < 2; ++b) {
     c.pos[b].alloc(nn * e4);
     c.vel[b].alloc(nn * e4);
@@ -438,16 +431,29 @@ static void allocate(Ctx& c) {
     c.inc_tiles = (cells + kCellTile - 1) / kCellTile;
     c.inc_one = inc_in_one(n, c.inc_tiles);
     c.inc_mask.alloc(((nn + 63) / 64) * 8);
+    const size_t inc_bytes = c.inc_head_bytes() + c.inc_count_bytes();
+    if (extras && is_modest(inc_bytes + cells * 4) && !(sp && std::string(sp) == "keys")) {
+      c.inc_next.alloc(nn * 4);
+      PR_HIP(hipMemsetAsync(c.inc_next.p, 0xFF, nn * 4, c.stream));   // kListEnd
+      c.lb_spare.alloc(cells * 4);
+      c.inc_cells.alloc(inc_bytes);
+      PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, inc_bytes, c.stream));
+    } else {
+      for (DevBuf* b : {&c.inc_next, &c.lb_spare, &c.inc_cells}) b->release();
+    }
   }
   if (const char* dr = std::getenv("PRESTIGE_DRY")) c.dry_reuse = std::string(dr) != "off";
   if (const char* ep = std::getenv("PRESTIGE_EPOCH")) c.inc_epoch = (uint32_t)std::strtoul(ep, nullptr, 10);
-  const char* sp = std::getenv("PRESTIGE_SORT");
-  c.sort_radix = sp && std::string(sp) == "radix";
   c.lb.alloc(((size_t)c.grid.n_cells + 1) * 4);
   c.flags.alloc((FLAG_COUNT + 2) * 4);
-  // three fields (seeds, gradients), up to kStage
-  c.pin_bytes = std::min(kStage, (nn * 24 + 4095) / 4096 * 4096);
-  PR_HIP(hipHostMalloc(&c.pin, c.pin_bytes + kNotes * 4, hipHostMallocMapped));
+  // three fields (seeds, gradients), up to kStage; the blocks in powers of two, which
+  // the runtime keeps for the next context sooner (976 KiB: the first eight creations
+  // of a program 0.8 ms longer)
+  size_t block = 4096;
+  while (block < nn * 24 && block < (1u << 20)) block *= 2;
+  c.pin_bytes = std::min(kStage, block);
+  if (!c.pin) PR_HIP(hipHostMalloc(&c.pin, block + 64, hipHostMallocMapped));
+  static_assert(kStage <= (1u << 20) && kNotes * 4 <= 64, "a block holds what goes through it and the notes");
   void* pin_dev = nullptr;
   PR_HIP(hipHostGetDevicePointer(&pin_dev, c.pin, 0));
   c.note = reinterpret_cast<uint32_t*>(static_cast<char*>(c.pin) + c.pin_bytes);
@@ -505,6 +511,13 @@ static void allocate(Ctx& c) {
       if (std::string(e) == "on") c.quad = true;
       else if (std::string(e) == "off") c.quad = false;
     }
+    c.quad = c.quad && extras;
+    if (c.quad) {
+      c.nlist.alloc(((nn + 15) / 16) * 2048 * sizeof(uint32_t));
+      c.ncnt.alloc(nn * sizeof(uint32_t));
+    } else {
+      for (DevBuf* b : {&c.nlist, &c.ncnt}) b->release();
+    }
   }
   c.scratch.alloc(nn * 8);
   if (dem) {
@@ -518,19 +531,6 @@ static void allocate(Ctx& c) {
       PR_HIP(hipMemsetAsync(c.hcnt[b].p, 0, nn * 4, c.stream));
       PR_HIP(hipMemsetAsync(c.wxi[b].p, 0, nn * 18 * hr, c.stream));
     }
-  }
-  // Last, what a context can do without: the neighbour lists of the four-lane
-  // passes, and the lists and counts per cell of the incremental sort (20 bytes a
-  // cell, 28 in small scenes, where the keys' own sorts need 4), unless they would
-  // take a gigabyte and over a quarter of the memory left.
-  if (c.quad)
-    c.quad = alloc_if_fits({{&c.nlist, ((nn + 15) / 16) * 2048 * sizeof(uint32_t)}, {&c.ncnt, nn * sizeof(uint32_t)}}, false);
-  if (c.desc.model != PRESTIGE_MODEL_PAIRS && !(sp && std::string(sp) == "keys") &&
-      alloc_if_fits({{&c.inc_cells, c.inc_head_bytes() + c.inc_count_bytes()},
-                     {&c.lb_spare, ((size_t)c.grid.n_cells + 1) * 4},
-                     {&c.inc_next, nn * 4}}, true)) {
-    PR_HIP(hipMemsetAsync(c.inc_cells.p, 0, c.inc_cells.bytes, c.stream));
-    PR_HIP(hipMemsetAsync(c.inc_next.p, 0xFF, nn * 4, c.stream));   // kListEnd
   }
   if (n) {
     k_iota_ids<<<blocks_for(n), kBlock, 0, c.stream>>>((uint32_t)n, c.ids[0].as<uint32_t>());
@@ -824,7 +824,13 @@ prestige_status prestige_create(const prestige_desc* desc, prestige_ctx** out) {
     derive_constants(*c);
     PR_HIP(hipGetDevice(&c->device));
     PR_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    allocate(*c);
+    try {
+      allocate(*c, true);
+    } catch (const Error& e) {
+      if (e.code != PRESTIGE_E_OOM) throw;
+      (void)hipGetLastError();
+      allocate(*c, false);
+    }
   } catch (const Error& e) {
     g_create_error = e.what();
     if (c) {

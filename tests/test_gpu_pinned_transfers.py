@@ -43,7 +43,7 @@ def _ptr(a):
 
 
 # 64 bytes, 976 KiB (also a small context's whole block), 2 MiB, and past the ring's size
-@pytest.mark.parametrize("n", [1, 7, 8, 170, 171, 124927, 124928, 124929, 262143, 262144, 262145, 1100003])
+@pytest.mark.parametrize("n", [1, 7, 8, 511, 512, 513, 124927, 124928, 124929, 262143, 262144, 262145, 1100003])
 def test_values_and_edges(n):
     lib = pa.load_library()
     rng = np.random.default_rng(n)
